@@ -241,6 +241,14 @@ int mxl_grouped_gemm_wgrad(const void* a_codes, const void* a_scales, int a_fmt,
  * (primus_turbo_mxfp4_local.py:319-331; the first operand's codes are plain there).  E2M1 x E2M1, block scales in
  * the plain row-major layout, n % 16 == 0.  Same results bit for bit as on the plain codes. */
 #define MXL_GF_B_SHUFFLED 16u
+/* With MXL_GF_KSTEP (and without MXL_GF_ACCUM_F32): the output tile of the launch, 64 x 64, 64 x 128, 128 x 128 or
+ * 256 x 256 (64 x 64 stands for 64 x 128 where b is read transposed).  Without one of these the library picks by the
+ * size of the problem.  The result is the same bit for bit. */
+#define MXL_GF_TILE_64 0x100u
+#define MXL_GF_TILE_64X128 0x200u
+#define MXL_GF_TILE_128 0x300u
+#define MXL_GF_TILE_256 0x400u
+#define MXL_GF_TILE_MASK 0x700u
 int mxl_grouped_gemm_nt_ex(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes,
                            const void* b_scales, int b_fmt, void* c_bf16, const int64_t* group_lens,
                            int num_groups, int64_t total_m, int64_t n, int64_t k, uint32_t flags, void* stream);

@@ -32,6 +32,7 @@ GF_KCHUNK = 1                               # flag of the GEMM _ex entry points:
 GF_KSTEP = 4                                # ... K-step-major codes and scales (ring kernel)
 GF_ACCUM_F32 = 2                            # wgrad: the output is float32 and the result is added to it
 GF_B_SHUFFLED = 16                          # forward / dgrad, row-major E2M1: b's codes are in the pre-shuffled byte order
+GF_TILES = {None: 0, "64": 0x100, "64x128": 0x200, "128": 0x300, "256": 0x400}   # output tile of a launch on K-step-major operands
 GF_B_TRANSPOSED = 8                         # forward / dgrad: b's codes are those of the transposed matrices (row-wise weight copy)
 BF_B_KN, BF_ACCUM_F32, BF_TILE_128, BF_TILE_256 = 1, 2, 4, 8    # flags of the bf16 grouped GEMMs
 

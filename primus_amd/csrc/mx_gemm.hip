@@ -27,35 +27,13 @@
 // 8-byte bf16 store).
 #include <type_traits>
 
-#include "mx_device.h"
-#include "mx_gemm_addr.h"
+#include "mx_gemm_common.h"
+#include "mx_gemm_tile.h"
 
 namespace mxl {
 
-constexpr int BM = 256, BN = 256;
-constexpr int BK = 64;     // one MFMA K step (two MX blocks)
 constexpr int BKP = 128;   // K per LDS slot: two K steps, one full 128-byte line per FP8 row
 constexpr int NSLOT = 2;
-constexpr int GTHREADS = 256;
-constexpr int MODE_FWD = 0;    // rows of A ragged by group; B = [G, N, K]
-constexpr int MODE_WGRAD = 1;  // contraction ragged by group; C = [G, M, N]
-constexpr int GROUP_M = 4;     // tile-order super-row height (L2 locality)
-
-struct GemmArgs {
-    const uint8_t* a;   // M-side codes
-    const uint8_t* sa;  // M-side scales
-    const uint8_t* b;   // N-side codes
-    const uint8_t* sb;  // N-side scales
-    uint16_t* c;        // bf16 out
-    const int64_t* group_lens;  // device, may be null (one group)
-    int num_groups;     // >= 1
-    int64_t total_m;    // FWD: rows of a; WGRAD: tokens (sum of lens)
-    int64_t m;          // WGRAD: rows of a (fixed)   | FWD: unused
-    int64_t n;          // columns of c / rows of b (per group in FWD)
-    int64_t k;          // FWD: contraction length; WGRAD: padded width W
-    const float* alpha_a;   // ALPHA kernels: the output is multiplied by *alpha_a * *alpha_b (per-tensor
-    const float* alpha_b;   // scales of tensor-wise quantised operands) before it is rounded
-};
 
 template <int FMT> struct Op {
     static constexpr bool fp4 = (FMT == kFmtE2M1);
@@ -67,54 +45,6 @@ template <int FMT> struct Op {
     // 32 consecutive rows): 8 chunks per 128-byte row, 4 chunks per 64-byte row.
     static __device__ __forceinline__ int swz(int row) { return fp4 ? ((row >> 2) & 3) : ((row >> 1) & 7); }
 };
-
-// ---- asynchronous global -> LDS loads ------------------------------------
-// Written as inline assembly on purpose: the compiler then keeps no record of
-// LDS writes in flight and does not put a full vmcnt wait in front of every
-// LDS read; completion is waited for explicitly (wait_vm) before the barrier
-// that publishes a stage.  The hardware writes lane i's data to LDS address
-// M0 + size*i, so the XOR swizzle is applied on the global side: the lane that
-// owns physical chunk (row, pch) fetches logical chunk pch ^ swz(row).
-__device__ __forceinline__ v4i make_rsrc(const void* base, int64_t bytes) {
-    const uint64_t p = (uint64_t)base;
-    const uint32_t n = bytes > 0xFFFFFFFFll ? 0xFFFFFFFFu : (uint32_t)(bytes < 0 ? 0 : bytes);
-    v4i r;
-    r[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)p);
-    r[1] = __builtin_amdgcn_readfirstlane((int)(uint32_t)(p >> 32) & 0xFFFF);  // stride 0: raw buffer
-    r[2] = __builtin_amdgcn_readfirstlane((int)n);                             // bytes; reads past it give 0
-    r[3] = 0x00020000;
-    return r;
-}
-// The statement writes M0 (the LDS address of an LDS-direct load).  M0 cannot be named in the clobber list: the
-// compiler diagnoses clobbers of reserved registers.  Nothing else in these kernels lives in M0: LDS instructions do
-// not take it on gfx950 and the kernels use no relative moves, messages or interpolation, and every use here
-// reloads it first.
-__device__ __forceinline__ void dma16(v4i rsrc, uint32_t lds_off, uint32_t voff, uint32_t soff) {
-    asm volatile("" : "+s"(soff));   // the scalar offset has to sit in a register, also when it is a known constant
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :
-                 : "s"(lds_off), "v"(voff), "s"(rsrc), "s"(soff)
-                 : "memory");
-}
-template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-// The same load with the LDS address formed in M0 by one scalar add (base register + constant) and the scalar
-// offset taken as it is: the ring kernel keeps a round's row offset in the per-lane offset instead of adding it to
-// the scalar one, which leaves two scalar instructions per request.
-template <int LDS_IMM>
-__device__ __forceinline__ void dma16_at(v4i rsrc, uint32_t lds_base, uint32_t voff, uint32_t soff) {
-    asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds"
-                 :
-                 : "s"(lds_base), "n"(LDS_IMM), "v"(voff), "s"(rsrc), "s"(soff)
-                 : "memory", "scc");
-}
-
-// Output stores are marked non-temporal: the kernel never reads its output back, and keeping it
-// out of the way leaves L2 to the operand tiles that neighbouring workgroups share.
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void store16_streaming(uint8_t* dst, const uint4& v) {
-    const u32x4 t = {v.x, v.y, v.z, v.w};
-    __builtin_nontemporal_store(t, (u32x4*)dst);
-}
 
 // LDS -> MFMA fragment of one 32-row tile for K step ks (0 or 1) of a slot.
 template <int FMT>
@@ -147,15 +77,6 @@ struct Frags {
     v8i a[4], b[4];
     int sa[4], sb[4];
 };
-
-// compile-time loop: f(integral_constant<int, I>) for I .. N - 1
-template <int I, int N, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<I + 1, N>(f);
-    }
-}
 
 // LAYOUT 0: operand codes row-major [rows, K].  LAYOUT 1: K-chunk-major [K / 128][rows][128 elements] (what the
 // quantisers write with MXL_QF_KCHUNK): the rows of a tile's K slot are one contiguous block, so a load round
@@ -1373,6 +1294,69 @@ static int launch_gemm_ring(const GemmArgs& a, int64_t max_tiles, hipStream_t st
     return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;
 }
 
+// Tile of a launch on K-step-major operands: what the caller's flag says, or by size.
+static bool tile_flag_ok(uint32_t flags) {
+    const uint32_t t = flags & MXL_GF_TILE_MASK;
+    return t <= MXL_GF_TILE_256 && (t == 0 || ((flags & MXL_GF_KSTEP) && !(flags & MXL_GF_ACCUM_F32)));
+}
+// Which tile is fastest is a matter of how many tiles there are.  Measured cost of a tile in us per CU and 4096 elements of
+// FP8 contraction (E2M1 x E2M1: all of them about 0.7 of it): 64 x 64 6.5, 64 x 128 9.7, 128 x 128 14.2, the ring kernel's
+// 256 x 256 53 -- per flop the ring kernel is the cheapest (1 : 0.93 : 0.69 : 0.51), but it needs 256 tiles to occupy the
+// chip, and its launches cost whole rounds of 256.  A dense launch takes the tile with the least ceil(tiles / 256) * cost.
+// Only the first two rounds are priced as whole ones, in backward GEMMs only the first: there the input and the weight
+// gradient run side by side and fill each other's last round ([4096, 14336] x [4096, 14336] tensor-wise, 3.5 rounds each
+// in the backward: 0.80 ms on ring tiles, 0.94 on 128 x 128 ones).
+//   [256, 4096] x [4096, 4096]: ring 41.2 us, 128 13.2, 64 x 128 10.4, 64 x 64 8.9.   [1024, ...]: 42.4, 18.4, 22.2, 27.6
+//   [1999, 2880] x [5760, 2880]: 39.2, 34.0, 45.7, 54.4.   [4096, 4096] x [4096, 4096]: 56.3, 60.1, 80.6, 106
+// A grouped launch does not know its tile counts (they are on the device): a group's last row tile is taken as half full.
+// Up to about one round of the ring kernel the same rule holds.  Beyond that a launch is bound by reading the weights,
+// which the ring kernel does best from about 32 rows per group on; with fewer its two and a half rounds of mostly empty
+// tiles cost more than the smaller tiles' shorter reads.  E2M1 weights against FP8 rows are half the bytes, which shifts
+// the line up.
+//   128 groups, [5760, 2880]: 4 rows per group ring 378 us, 64 x 128 317 (E2M1 weights 272, 183); 64 rows 474, 530 (413, 333)
+//   32 groups, [4096, 7168]: 32 rows per group ring 185, 128 180 (transposed codes 238, 196); 64 rows 187, 208 (243, 217)
+// The weight gradient's tiles are all output and little contraction: dense ones take 128 x 128 while the contraction is
+// short (256 tokens, 14336 x 4096: 43 -> 29 us); grouped ones run the ring kernel at the rate the board writes, except
+// where the gradient is a few tiles.
+template <int MODE> static int tile_choice(const GemmArgs& a, bool e2m1_weights, bool bt, uint32_t flags) {
+    switch (flags & MXL_GF_TILE_MASK) {
+        case MXL_GF_TILE_64: return TILE_64;
+        case MXL_GF_TILE_64X128: return TILE_64x128;
+        case MXL_GF_TILE_128: return TILE_128;
+        case MXL_GF_TILE_256: return TILE_RING;
+    }
+    const bool grouped = a.group_lens != nullptr;
+    auto cdiv = [](int64_t x, int64_t y) { return (x + y - 1) / y; };
+    auto tiles = [&](int64_t tm, int64_t tn) {
+        const int64_t cols = cdiv(a.n, tn);
+        if (MODE == MODE_WGRAD) return a.num_groups * cdiv(a.m, tm) * cols;
+        if (!grouped) return cdiv(a.total_m, tm) * cols;
+        const int64_t live = a.total_m < a.num_groups ? a.total_m : a.num_groups;
+        return (a.total_m / tm + (live + 1) / 2) * cols;
+    };
+    const int64_t ring_tiles = tiles(256, 256);
+    if (MODE == MODE_WGRAD && grouped) return ring_tiles < 256 ? TILE_128 : TILE_RING;
+    if (grouped && ring_tiles > 300) {
+        const int64_t rows = a.total_m / a.num_groups;
+        if (e2m1_weights) return rows <= 96 ? TILE_64x128 : rows <= 192 ? TILE_128 : TILE_RING;
+        return rows <= 16 ? TILE_64x128 : rows <= (bt ? 64 : 32) ? TILE_128 : TILE_RING;
+    }
+    auto cost = [&](int64_t tm, int64_t tn, double c) { return (double)cdiv(tiles(tm, tn), 256) * c; };
+    int best = TILE_RING;
+    const bool whole_rounds = ring_tiles <= 256 || (MODE == MODE_FWD && !bt && ring_tiles <= 512);
+    double least = whole_rounds ? cost(256, 256, 53.0) : ring_tiles / 256.0 * 53.0;
+    auto consider = [&](int tile, double c) {
+        if (c < least) least = c, best = tile;
+    };
+    // (a short weight gradient is mostly output: the small tiles overlap theirs, see tile_wgrad_shallow)
+    consider(TILE_128, cost(128, 128, MODE == MODE_WGRAD && tile_wgrad_shallow(a) ? 9.0 : 14.2));
+    if (MODE == MODE_FWD) {
+        consider(TILE_64x128, cost(64, 128, 9.7));
+        if (!e2m1_weights && !bt) consider(TILE_64, cost(64, 64, 6.5));
+    }
+    return best;
+}
+
 // The 4-slot ring kernel serves operands in the K-step-major layout with at most RING_MAX_GROUPS groups: FP8 x FP8,
 // and FP8 rows against an FP4 weight operand in the forward / dgrad GEMM.
 template <int MODE>
@@ -1451,19 +1435,20 @@ static int dispatch_wgrad_accum_ring(int afmt, int bfmt, const GemmArgs& a, int6
 
 // forward / dgrad on the row-wise codes of the transposed weight (MXL_GF_B_TRANSPOSED): E4M3 weights with E4M3 or E5M2
 // rows, or E2M1 weights with E2M1 rows (128-element steps)
-static int dispatch_gemm_ring_bt(int afmt, int bfmt, const GemmArgs& a, int64_t max_tiles, hipStream_t st) {
+static int dispatch_gemm_ring_bt(int afmt, int bfmt, const GemmArgs& a, int64_t max_tiles, hipStream_t st, uint32_t flags) {
     if (a.num_groups > RING_MAX_GROUPS) return MXL_EINVAL;
+    const int tile = tile_choice<MODE_FWD>(a, false, true, flags);
     if (bfmt == MXL_FMT_E2M1) {
         if (afmt != MXL_FMT_E2M1 || a.alpha_a != nullptr) return MXL_EINVAL;
+        if (tile != TILE_RING) return gemm_tile_bt(afmt, bfmt, a, tile, st);
         return launch_gemm_ring<MXL_FMT_E2M1, MXL_FMT_E2M1, MODE_FWD, false, false, true>(a, max_tiles, st);
     }
-    if (bfmt != MXL_FMT_E4M3) return MXL_EINVAL;
+    if (bfmt != MXL_FMT_E4M3 || (afmt != MXL_FMT_E4M3 && (afmt != MXL_FMT_E5M2 || a.alpha_a == nullptr))) return MXL_EINVAL;
+    if (tile != TILE_RING) return gemm_tile_bt(afmt, bfmt, a, tile, st);
     if (a.alpha_a != nullptr) {
         if (afmt == MXL_FMT_E5M2) return launch_gemm_ring<MXL_FMT_E5M2, MXL_FMT_E4M3, MODE_FWD, true, false, true>(a, max_tiles, st);
-        if (afmt == MXL_FMT_E4M3) return launch_gemm_ring<MXL_FMT_E4M3, MXL_FMT_E4M3, MODE_FWD, true, false, true>(a, max_tiles, st);
-        return MXL_EINVAL;
+        return launch_gemm_ring<MXL_FMT_E4M3, MXL_FMT_E4M3, MODE_FWD, true, false, true>(a, max_tiles, st);
     }
-    if (afmt != MXL_FMT_E4M3) return MXL_EINVAL;
     return launch_gemm_ring<MXL_FMT_E4M3, MXL_FMT_E4M3, MODE_FWD, false, false, true>(a, max_tiles, st);
 }
 
@@ -1471,7 +1456,7 @@ static int dispatch_gemm_ring_bt(int afmt, int bfmt, const GemmArgs& a, int64_t 
 // layout: 0 row-major codes, 1 K-chunk-major codes, 2 K-step-major codes and scales
 template <int MODE>
 static int dispatch_gemm(int afmt, int bfmt, const GemmArgs& a, int64_t max_tiles, int layout, int64_t a_rows, int64_t b_rows,
-                         hipStream_t st, bool accum = false) {
+                         hipStream_t st, bool accum = false, uint32_t flags = 0) {
     const bool kchunk = layout == 1;
     if (layout == 2) {
         if ((accum && MODE != MODE_WGRAD) || !ring_serves<MODE>(afmt, bfmt, a)) return MXL_EINVAL;
@@ -1480,6 +1465,8 @@ static int dispatch_gemm(int afmt, int bfmt, const GemmArgs& a, int64_t max_tile
         // the kernel keeps a tile's first output row in 32 bits
         if ((MODE == MODE_WGRAD ? (int64_t)a.num_groups * a.m : a.total_m) >= ((int64_t)1 << 31)) return MXL_EINVAL;
         if (accum) return dispatch_wgrad_accum_ring(afmt, bfmt, a, max_tiles, st);
+        const int tile = tile_choice<MODE>(a, bfmt == MXL_FMT_E2M1 && afmt != MXL_FMT_E2M1, false, flags);
+        if (tile != TILE_RING) return MODE == MODE_FWD ? gemm_tile_fwd(afmt, bfmt, a, tile, st) : gemm_tile_wgrad(afmt, bfmt, a, tile, st);
         return dispatch_gemm_ring<MODE>(afmt, bfmt, a, max_tiles, st);
     }
     if (accum) {
@@ -1511,7 +1498,8 @@ __global__ __launch_bounds__(256) void zero_fill_kernel(uint32_t* dst, int64_t w
 static int grouped_gemm_nt(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes, const void* b_scales,
                            int b_fmt, void* c_bf16, const int64_t* group_lens, int num_groups, int64_t total_m, int64_t n,
                            int64_t k, const float* alpha_a, const float* alpha_b, uint32_t flags, void* stream) {
-    if (flags & ~(uint32_t)(MXL_GF_KCHUNK | MXL_GF_KSTEP | MXL_GF_B_TRANSPOSED | MXL_GF_B_SHUFFLED)) return MXL_EINVAL;
+    if (flags & ~(uint32_t)(MXL_GF_KCHUNK | MXL_GF_KSTEP | MXL_GF_B_TRANSPOSED | MXL_GF_B_SHUFFLED | MXL_GF_TILE_MASK)) return MXL_EINVAL;
+    if (!tile_flag_ok(flags)) return MXL_EINVAL;
     if ((flags & MXL_GF_KCHUNK) && (flags & MXL_GF_KSTEP)) return MXL_EINVAL;
     // pre-shuffled weight codes: row-major E2M1 x E2M1, block scales, whole 16-row blocks per group
     if ((flags & MXL_GF_B_SHUFFLED) && (flags != MXL_GF_B_SHUFFLED || a_fmt != MXL_FMT_E2M1 || b_fmt != MXL_FMT_E2M1 || alpha_a || n % 16 != 0))
@@ -1546,10 +1534,10 @@ static int grouped_gemm_nt(const void* a_codes, const void* a_scales, int a_fmt,
         const int64_t n_ld = (n + 127) / 128 * 128;
         if (total_m * k >= ((int64_t)1 << 32) || (int64_t)num_groups * k * n_ld >= ((int64_t)1 << 32) || total_m >= ((int64_t)1 << 31))
             return MXL_EINVAL;
-        return dispatch_gemm_ring_bt(a_fmt, b_fmt, a, max_tiles, (hipStream_t)stream);
+        return dispatch_gemm_ring_bt(a_fmt, b_fmt, a, max_tiles, (hipStream_t)stream, flags);
     }
     return dispatch_gemm<MODE_FWD>(a_fmt, b_fmt, a, max_tiles, (flags & MXL_GF_KSTEP) ? 2 : (flags & MXL_GF_KCHUNK) ? 1 : 0, total_m,
-                                   (int64_t)num_groups * n, (hipStream_t)stream);
+                                   (int64_t)num_groups * n, (hipStream_t)stream, false, flags);
 }
 
 extern "C" int mxl_grouped_gemm_nt_ex(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes,
@@ -1585,7 +1573,8 @@ static int grouped_gemm_wgrad(const void* a_codes, const void* a_scales, int a_f
                               const void* b_scales, int b_fmt, void* c_bf16, const int64_t* group_lens, int num_groups,
                               int64_t total_m, int64_t n, int64_t k, const float* alpha_a, const float* alpha_b,
                               uint32_t flags, void* stream) {
-    if (flags & ~(uint32_t)(MXL_GF_KCHUNK | MXL_GF_KSTEP | MXL_GF_ACCUM_F32)) return MXL_EINVAL;
+    if (flags & ~(uint32_t)(MXL_GF_KCHUNK | MXL_GF_KSTEP | MXL_GF_ACCUM_F32 | MXL_GF_TILE_MASK)) return MXL_EINVAL;
+    if (!tile_flag_ok(flags)) return MXL_EINVAL;
     if ((flags & MXL_GF_KCHUNK) && (flags & MXL_GF_KSTEP)) return MXL_EINVAL;
     const bool accum = (flags & MXL_GF_ACCUM_F32) != 0;
     if (accum && !(flags & (MXL_GF_KCHUNK | MXL_GF_KSTEP))) return MXL_EINVAL;
@@ -1630,7 +1619,7 @@ static int grouped_gemm_wgrad(const void* a_codes, const void* a_scales, int a_f
     a.alpha_b = alpha_b;
     const int64_t max_tiles = (int64_t)G * ((n + BM - 1) / BM) * ((k + BN - 1) / BN);
     return dispatch_gemm<MODE_WGRAD>(a_fmt, b_fmt, a, max_tiles, (flags & MXL_GF_KSTEP) ? 2 : (flags & MXL_GF_KCHUNK) ? 1 : 0, n, k,
-                                     (hipStream_t)stream, accum);
+                                     (hipStream_t)stream, accum, flags);
 }
 
 extern "C" int mxl_grouped_gemm_wgrad_ex(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes,

@@ -106,6 +106,10 @@ MXL_HD Desc ring_panel_desc(int64_t rows_total, int64_t panels, int64_t row0) {
 }
 MXL_HD uint32_t ring_panel_lane(int t) { return (uint32_t)(t * 16); }
 
+// A scalar offset no request survives: operands end below 4 GiB and are a multiple of 32 bytes, so num_records is at most
+// 2^32 - 32 and the sum of the offsets (no wrap-around) is past it.
+constexpr uint32_t kDropped = 0xFFFFFFF0u;
+
 // The hardware's decision for dword c (0 .. 3) of a 16-byte request
 MXL_HD bool accepted(const Desc& d, uint32_t voff, uint32_t soff, int c) {
     const uint64_t rec = d.records <= 0 ? 0u : (d.records > 0xFFFFFFFFll ? 0xFFFFFFFFull : (uint64_t)d.records);

@@ -127,8 +127,8 @@ def _qflag(kchunk) -> int:
     return (0, _lib.QF_KCHUNK, _lib.QF_KSTEP, _lib.QF_KSTEP | _lib.QF_KSTEP128)[_layout(kchunk)]
 
 
-def _gflag(kchunk) -> int:
-    return (0, _lib.GF_KCHUNK, _lib.GF_KSTEP, _lib.GF_KSTEP)[_layout(kchunk)]
+def _gflag(kchunk, tile: Optional[str] = None) -> int:
+    return (0, _lib.GF_KCHUNK, _lib.GF_KSTEP, _lib.GF_KSTEP)[_layout(kchunk)] | _lib.GF_TILES[tile]
 
 
 def pick_layout(groups: int, n: int, k: int, rows: int = 0, fp8: bool = True, fp4: bool = False) -> int:
@@ -497,14 +497,15 @@ def gemm_mx_nt_impl(a, a_scale, b, b_scale, out_dtype=torch.bfloat16, kchunk=Fal
 
 
 def grouped_gemm_mx_nt_impl(a, a_scale, b, b_scale, group_lens, out_dtype=torch.bfloat16, kchunk=False,
-                            b_transposed: bool = False) -> torch.Tensor:
+                            b_transposed: bool = False, tile: Optional[str] = None) -> torch.Tensor:
     """Forward / dgrad grouped GEMM: rows of ``a[total_m, k]`` split by
     ``group_lens``; ``b`` is ``[G, n, k]``.  ``kchunk``: both code tensors are K-chunk-major,
     ``a [k / 128, total_m, 128]`` and ``b [k / 128, G * n, 128]``; ``b_scale`` is ``[G, n, k / 32]`` as always.
     ``b_transposed`` (K-step-major FP8 operands, or E2M1 operands in 128-element steps): ``b`` holds the codes of the
     transposed matrices, ``[n_ld / 64, G * k, 64]`` (E2M1: ``[n_ld / 128, G * k, 64 bytes]``) -- the row-wise copy of a
     weight ``[G, k, n]`` serving its dgrad GEMM -- and ``b_scale`` the scale panels of ``[G * n, k]`` (the transposed
-    copy's scales)."""
+    copy's scales).  ``tile`` (K-step-major layouts): the output tile, a key of ``_lib.GF_TILES`` (None: by the size of
+    the problem); the result is the same bit for bit."""
     _check_out_dtype(out_dtype)
     _require_cuda(a, a_scale, b, b_scale, group_lens)
     G = _check_group_lens(group_lens, a.device)
@@ -529,7 +530,7 @@ def grouped_gemm_mx_nt_impl(a, a_scale, b, b_scale, group_lens, out_dtype=torch.
         with _hooked("grouped_gemm_nt" if G else "gemm_nt", m=total_m, n=n, k=k):
             rc = _lib.load().mxl_grouped_gemm_nt_ex(
                 _ptr(a), _ptr(a_scale), a_fmt, _ptr(b), _ptr(b_scale), b_fmt, _ptr(c), _ptr(group_lens), groups, total_m, n, k,
-                _lib.GF_KSTEP | _lib.GF_B_TRANSPOSED, _stream()
+                _gflag(kchunk, tile) | _lib.GF_B_TRANSPOSED, _stream()
             )
         _lib.check(rc, "mxl_grouped_gemm_nt_ex")
         return c
@@ -553,7 +554,7 @@ def grouped_gemm_mx_nt_impl(a, a_scale, b, b_scale, group_lens, out_dtype=torch.
         with _hooked("grouped_gemm_nt" if G else "gemm_nt", m=total_m, n=n, k=k):
             rc = _lib.load().mxl_grouped_gemm_nt_ex(
                 _ptr(a), _ptr(a_scale), a_fmt, _ptr(b), _ptr(b_scale), b_fmt, _ptr(c), _ptr(group_lens), groups, total_m, n, k,
-                _gflag(kchunk), _stream()
+                _gflag(kchunk, tile), _stream()
             )
         _lib.check(rc, "mxl_grouped_gemm_nt_ex")
         return c
@@ -585,7 +586,7 @@ def _accum_target(accum_into, shape, kchunk, device):
 
 
 def grouped_gemm_mx_wgrad_impl(a_t, a_t_scale, b_t, b_t_scale, group_lens, total_m, out_dtype=torch.bfloat16,
-                               kchunk=False, accum_into: Optional[torch.Tensor] = None) -> torch.Tensor:
+                               kchunk=False, accum_into: Optional[torch.Tensor] = None, tile: Optional[str] = None) -> torch.Tensor:
     """Variable-K (wgrad) grouped GEMM on segment-padded transposed operands:
     ``a_t`` = dY^T codes ``[n, W]``, ``b_t`` = X^T codes ``[k, W]``; returns
     ``[G, n, k]`` (``[n, k]`` when ``group_lens`` is None).  An expert with no
@@ -610,7 +611,7 @@ def grouped_gemm_mx_wgrad_impl(a_t, a_t_scale, b_t, b_t_scale, group_lens, total
     elif tuple(a_t_scale.shape) != (n, W // BLOCK) or tuple(b_t_scale.shape) != (k, W // BLOCK):
         raise ValueError("scale shapes must be [rows, W/32]")
     shape = (n, k) if group_lens is None else (G, n, k)
-    flags = _gflag(kchunk)
+    flags = _gflag(kchunk, tile)
     if accum_into is not None:
         # the result is added, in float32, to accum_into (which is returned)
         c = _accum_target(accum_into, shape, kchunk, a_t.device)
@@ -888,7 +889,7 @@ def _alpha_ok(*alphas):
 
 
 def gemm_tw_nt_impl(a, a_unit, a_scale_inv, b, b_unit, b_scale_inv, group_lens=None, kchunk: bool = False,
-                    b_transposed_n: Optional[int] = None) -> torch.Tensor:
+                    b_transposed_n: Optional[int] = None, tile: Optional[str] = None) -> torch.Tensor:
     """``c = (a . b^T) * a_scale_inv * b_scale_inv`` on tensor-wise scaled codes, dense (``group_lens`` None,
     ``b [n, k]``) or grouped (``b [G, n, k]``); layouts and the unit block scales as the quantisers above
     return them (``b_unit`` is ``[n, k/32]`` or ``[G, n, k/32]``).  The contraction dim must be padded to 128.
@@ -912,7 +913,7 @@ def gemm_tw_nt_impl(a, a_unit, a_scale_inv, b, b_unit, b_scale_inv, group_lens=N
         with _hooked("grouped_gemm_nt" if G else "gemm_nt", m=total_m, n=n, k=k):
             rc = _lib.load().mxl_grouped_gemm_nt_scaled(
                 _ptr(a), _ptr(a_unit), a_fmt, _ptr(b), None, b_fmt, _ptr(c), _ptr(group_lens), groups, total_m, n, k,
-                _ptr(a_scale_inv), _ptr(b_scale_inv), _lib.GF_KSTEP | _lib.GF_B_TRANSPOSED, _stream(),
+                _ptr(a_scale_inv), _ptr(b_scale_inv), _gflag(kchunk, tile) | _lib.GF_B_TRANSPOSED, _stream(),
             )
         _lib.check(rc, "mxl_grouped_gemm_nt_scaled")
         return c
@@ -941,14 +942,14 @@ def gemm_tw_nt_impl(a, a_unit, a_scale_inv, b, b_unit, b_scale_inv, group_lens=N
     with _hooked("grouped_gemm_nt" if G else "gemm_nt", m=total_m, n=n, k=k):
         rc = _lib.load().mxl_grouped_gemm_nt_scaled(
             _ptr(a), _ptr(a_unit), a_fmt, _ptr(b), _ptr(b_unit), b_fmt, _ptr(c), _ptr(group_lens), groups, total_m, n, k,
-            _ptr(a_scale_inv), _ptr(b_scale_inv), _gflag(kchunk), _stream(),
+            _ptr(a_scale_inv), _ptr(b_scale_inv), _gflag(kchunk, tile), _stream(),
         )
     _lib.check(rc, "mxl_grouped_gemm_nt_scaled")
     return c
 
 
 def gemm_tw_wgrad_impl(a_t, a_t_unit, a_scale_inv, b_t, b_t_unit, b_scale_inv, group_lens, total_m,
-                       kchunk: bool = False, accum_into: Optional[torch.Tensor] = None) -> torch.Tensor:
+                       kchunk: bool = False, accum_into: Optional[torch.Tensor] = None, tile: Optional[str] = None) -> torch.Tensor:
     """Variable-K (wgrad) GEMM on tensor-wise scaled transposed operands, times the two factors; shapes as
     ``grouped_gemm_mx_wgrad_impl`` (also ``accum_into``)."""
     _require_cuda(a_t, a_t_unit, b_t, b_t_unit, group_lens)
@@ -970,7 +971,7 @@ def gemm_tw_wgrad_impl(a_t, a_t_unit, a_scale_inv, b_t, b_t_unit, b_scale_inv, g
     elif tuple(a_t_unit.shape) != (n, W // BLOCK) or tuple(b_t_unit.shape) != (k, W // BLOCK):
         raise ValueError("scale shapes must be [rows, W/32]")
     shape = (n, k) if group_lens is None else (G, n, k)
-    flags = _gflag(kchunk)
+    flags = _gflag(kchunk, tile)
     if accum_into is not None:
         c = _accum_target(accum_into, shape, kchunk, a_t.device)
         flags |= _lib.GF_ACCUM_F32
