@@ -490,6 +490,53 @@ int mxl_blockwise_gemm_plan(int64_t m, int64_t n, int mode, int num_groups, int6
 int mxl_shuffle_codes(const void* src, int64_t rows, int64_t row_bytes, void* dst, int inverse, void* stream);
 int mxl_shuffle_scales(const void* src, int64_t rows, int64_t cols, void* dst, int inverse, void* stream);
 
+/* ---- a linear in two calls -------------------------------------------------------------------------------------
+ * What ops.gemm_fp8 / gemm_fp4 / grouped_gemm_fp8 / grouped_gemm_fp4 launch for one linear
+ * (primus/backends/megatron/core/extensions/primus_turbo.py:1095-1150, :2122-2178) issued by one call per direction, on
+ * operands in the K-step-major layouts (at most 256 groups, every operand below 4 GiB).  The caller fills in the first
+ * block of fields, mxl_linear_sizes the sizes of the three buffers; pointers are device memory, 256-byte aligned buffers,
+ * and nothing is kept between calls.
+ *   forward   x -> y; `saved` receives what the backward reads, `scratch` (fwd_bytes) is free afterwards.
+ *   backward  in parts (a caller may put MXL_LINEAR_DW on another stream once MXL_LINEAR_QUANTIZE is done): dy is
+ *             quantised, dx and dw are written (dw_flags: 0 or MXL_GF_ACCUM_F32); `scratch` (bwd_bytes) is shared by the parts.
+ *   input     what x is: the GEMM's input itself; the [rows, 2k] tensor a gated activation turns into it (aux0 =
+ *             probabilities, aux1 = row mask or NULL; daux = their fp32 gradient); or the tensor an RMSNorm turns
+ *             into it (aux0 = norm weight; daux = its bf16 gradient).
+ *   w         bf16 [groups, n, k], or with w_quantized the row-wise codes (w_scales: their scales); the backward is then
+ *             given the transposed copy (wt, wt_scales).
+ *   dx_from_rows  the backward reads the row-wise codes transposed (MXL_GF_B_TRANSPOSED); n and k multiples of 128.
+ * recipe MXL_LINEAR_TENSORWISE takes plain inputs and bf16 weights.  rows > 0. */
+#define MXL_LINEAR_MX 0
+#define MXL_LINEAR_TENSORWISE 1
+#define MXL_LINEAR_PLAIN 0
+#define MXL_LINEAR_SILU 1
+#define MXL_LINEAR_GELU 2
+#define MXL_LINEAR_RMSNORM 3
+#define MXL_LINEAR_QUANTIZE 1
+#define MXL_LINEAR_DX 2
+#define MXL_LINEAR_DW 4
+typedef struct mxl_linear {
+    int64_t rows, n, k;
+    int64_t groups;                      /* 0: dense */
+    int64_t recipe;
+    int64_t act_fmt, w_fmt, grad_fmt;
+    int64_t scale_mode;
+    int64_t input, probs_dtype;
+    int64_t need_dx, need_dw, w_quantized, dx_from_rows;
+    int64_t grad_sr;                     /* E2M1 gradients rounded stochastically (sr_seed of the backward) */
+    int64_t rht_signs;                   /* Hadamard signs of both wgrad operands, or -1 */
+    double eps;                          /* of the RMSNorm */
+    int64_t saved_bytes, fwd_bytes, bwd_bytes;   /* written by mxl_linear_sizes */
+} mxl_linear;
+int mxl_linear_sizes(mxl_linear* p);
+int mxl_linear_forward(const mxl_linear* p, const void* x, const void* aux0, const void* aux1, const void* w,
+                       const void* w_scales, const int64_t* group_lens, void* saved, void* scratch, void* y_bf16,
+                       void* stream);
+int mxl_linear_backward(const mxl_linear* p, int parts, const void* dy_bf16, const void* x, const void* aux0,
+                        const void* aux1, const void* wt, const void* wt_scales, const int64_t* group_lens, void* saved,
+                        void* scratch, void* dx_bf16, void* daux, void* dw, uint32_t dw_flags, uint64_t sr_seed,
+                        void* stream);
+
 /* ---- calibration (no counterpart in the reference: a measuring aid of this library's benchmark) ----
  *
  * mxl_calibrate_mfma launches a register-only loop of the GEMM kernels' scaled MFMA (32 x 32 x 64; a_fmt / b_fmt:

@@ -77,6 +77,9 @@ EXPORTS = (
     "mxl_grouped_gemm_wgrad_blockwise",
     "mxl_blockwise_gemm_tile",
     "mxl_blockwise_gemm_plan",
+    "mxl_linear_sizes",
+    "mxl_linear_forward",
+    "mxl_linear_backward",
     "mxl_shuffle_codes",
     "mxl_shuffle_scales",
     "mxl_calibrate_mfma",
@@ -86,6 +89,20 @@ EXPORTS = (
     "mxl_calibrate_tile_copy",
     "mxl_calibrate_range_check",
 )
+
+
+class Linear(ctypes.Structure):
+    """``mxl_linear``: one linear's sizes and options, and the sizes of the buffers its two calls work in."""
+
+    _fields_ = [(name, ctypes.c_int64) for name in (
+        "rows", "n", "k", "groups", "recipe", "act_fmt", "w_fmt", "grad_fmt", "scale_mode", "input", "probs_dtype", "need_dx",
+        "need_dw", "w_quantized", "dx_from_rows", "grad_sr", "rht_signs")] + [("eps", ctypes.c_double)] + [
+        (name, ctypes.c_int64) for name in ("saved_bytes", "fwd_bytes", "bwd_bytes")]
+
+
+LINEAR_MX, LINEAR_TENSORWISE = 0, 1
+LINEAR_PLAIN, LINEAR_SILU, LINEAR_GELU, LINEAR_RMSNORM = 0, 1, 2, 3
+LINEAR_QUANTIZE, LINEAR_DX, LINEAR_DW = 1, 2, 4
 
 
 class MXLinearError(RuntimeError):
@@ -206,6 +223,12 @@ def load() -> ctypes.CDLL:
         lib.mxl_calibrate_mfma_bf16_flops.argtypes = [i64]
         lib.mxl_gemm_nt_blockwise.restype = i32
         lib.mxl_gemm_nt_blockwise.argtypes = [vp, vp, i32, vp, vp, i32, i32, vp, i64, i64, i64, vp]
+        lib.mxl_linear_sizes.restype = i32
+        lib.mxl_linear_sizes.argtypes = [vp]
+        lib.mxl_linear_forward.restype = i32
+        lib.mxl_linear_forward.argtypes = [vp] * 11
+        lib.mxl_linear_backward.restype = i32
+        lib.mxl_linear_backward.argtypes = [vp, i32] + [vp] * 12 + [u32, ctypes.c_uint64, vp]
         lib.mxl_blockwise_gemm_tile.restype = i32
         lib.mxl_blockwise_gemm_tile.argtypes = [i32]
         lib.mxl_blockwise_gemm_plan.restype = i32

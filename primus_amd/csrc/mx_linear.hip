@@ -1,0 +1,235 @@
+// One linear as two calls: everything its forward launches, and everything its backward launches (host code only).
+//
+// A linear is 3 to 5 launches forward and 4 to 7 backward, and a dozen buffers.  Issued one by one from Python, with an
+// allocation per buffer and a stream look-up per launch, they take 230 us for a pass whose kernels need 60.  Here the
+// caller allocates three buffers -- what the backward needs, and a scratch buffer per direction -- and makes one call per
+// direction; the layout of the buffers is arithmetic on the sizes and is worked out again in every call.
+#include "mx_device.h"
+
+namespace {
+
+int64_t rup(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
+
+// hands out pieces of a buffer; with base null it only counts
+struct Arena {
+    uint8_t* base;
+    int64_t used = 0;
+    explicit Arena(void* b) : base((uint8_t*)b) {}
+    uint8_t* take(int64_t bytes) {
+        uint8_t* p = base ? base + used : nullptr;
+        used += rup(bytes, 256);
+        return p;
+    }
+};
+
+struct Copy {          // one quantised copy: codes, scales
+    uint8_t *q = nullptr, *s = nullptr;
+};
+
+struct Linear {
+    const mxl_linear& p;
+    int64_t batch, k_ld, n_ld, width;
+    int f44;
+    explicit Linear(const mxl_linear* d) : p(*d) {
+        batch = p.groups > 0 ? p.groups : 1;
+        k_ld = rup(p.k, 128);
+        n_ld = rup(p.n, 128);
+        width = mxl_padded_width(p.rows, (int)p.groups);
+        f44 = p.act_fmt == MXL_FMT_E2M1 && p.w_fmt == MXL_FMT_E2M1;
+    }
+    bool mx() const { return p.recipe == MXL_LINEAR_MX; }
+    bool tensorwise() const { return p.recipe == MXL_LINEAR_TENSORWISE; }
+    uint32_t qf() const { return MXL_QF_KSTEP | (f44 ? MXL_QF_KSTEP128 : 0u); }
+
+    // K-step-major copies of [rows, ld] (ld padded): codes, scale panels
+    static Copy rows_copy(Arena& a, int64_t rows, int64_t ld, int64_t fmt, int64_t restarts = 0) {
+        Copy c;
+        c.q = a.take(rows * ld / (fmt == MXL_FMT_E2M1 ? 2 : 1));
+        c.s = a.take(((ld + 511) / 512 + restarts) * rows * 16);
+        return c;
+    }
+    Copy x_row(Arena& a) const { return rows_copy(a, p.rows, k_ld, p.act_fmt); }
+    Copy cols_copy(Arena& a, int64_t cols, int64_t fmt) const { return rows_copy(a, cols, width, fmt, p.groups > 0 ? p.groups + 1 : 0); }
+    Copy w_row(Arena& a) const { return rows_copy(a, batch * p.n, k_ld, p.w_fmt); }
+    Copy w_col(Arena& a) const {
+        Copy c;
+        if (!p.dx_from_rows) c.q = a.take(batch * p.k * n_ld / (p.w_fmt == MXL_FMT_E2M1 ? 2 : 1));
+        c.s = a.take((n_ld + 511) / 512 * batch * p.k * 16);
+        return c;
+    }
+};
+
+// what the forward leaves for the backward
+struct Saved {
+    Copy x_col, w_row, w_col;
+    float *rstd = nullptr, *x_si = nullptr, *w_si = nullptr;
+    Saved(const Linear& l, Arena& a) {
+        const mxl_linear& p = l.p;
+        if (p.need_dw) x_col = l.cols_copy(a, p.k, p.act_fmt);
+        if (p.need_dx && !p.w_quantized) {
+            if (p.dx_from_rows) w_row = l.w_row(a);
+            if (!(l.tensorwise() && p.dx_from_rows)) w_col = l.w_col(a);
+        }
+        if (p.input == MXL_LINEAR_RMSNORM) rstd = (float*)a.take(p.rows * 4);
+        if (l.tensorwise()) {
+            x_si = (float*)a.take(4);
+            w_si = (float*)a.take(4);
+        }
+    }
+};
+struct ForwardScratch {
+    Copy x_row, w_row;
+    float *x_amax = nullptr, *w_amax = nullptr;
+    ForwardScratch(const Linear& l, Arena& a) {
+        x_row = l.x_row(a);
+        if (!l.p.w_quantized && !(l.p.need_dx && l.p.dx_from_rows)) w_row = l.w_row(a);
+        if (l.tensorwise()) {
+            x_amax = (float*)a.take(4);
+            w_amax = (float*)a.take(4);
+        }
+    }
+};
+struct BackwardScratch {
+    Copy d_row, d_col;
+    float *amax = nullptr, *d_si = nullptr, *norm_ws = nullptr;
+    int64_t norm_bytes = 0;
+    void* dxi = nullptr;          // gradient of the GEMM's input where the operator's input is something else
+    BackwardScratch(const Linear& l, Arena& a) {
+        const mxl_linear& p = l.p;
+        if (p.need_dx) d_row = Linear::rows_copy(a, p.rows, l.n_ld, p.grad_fmt);
+        if (p.need_dw) d_col = l.cols_copy(a, p.n, p.grad_fmt);
+        if (l.tensorwise()) {
+            amax = (float*)a.take(4);
+            d_si = (float*)a.take(4);
+        }
+        if (p.input != MXL_LINEAR_PLAIN && p.need_dx) dxi = a.take(p.rows * p.k * 2);
+        if (p.input == MXL_LINEAR_RMSNORM && p.need_dx) {
+            norm_bytes = mxl_rmsnorm_bwd_workspace_bytes(p.rows, p.k);
+            norm_bytes = norm_bytes < 16 ? 16 : norm_bytes;
+            norm_ws = (float*)a.take(norm_bytes);
+        }
+    }
+};
+
+bool valid(const mxl_linear* p) {
+    if (!p || p->rows <= 0 || p->n <= 0 || p->k <= 0 || p->n % MXL_BLOCK || p->k % MXL_BLOCK || p->groups < 0 || p->groups > MXL_MAX_GROUPS) return false;
+    if (p->recipe != MXL_LINEAR_MX && p->recipe != MXL_LINEAR_TENSORWISE) return false;
+    if (p->recipe == MXL_LINEAR_TENSORWISE && (p->input != MXL_LINEAR_PLAIN || p->w_quantized)) return false;
+    if (p->input < MXL_LINEAR_PLAIN || p->input > MXL_LINEAR_RMSNORM) return false;
+    return !(p->dx_from_rows && (p->n % 128 || p->k % 128 || p->w_quantized));
+}
+
+}  // namespace
+
+#define MXL_TRY(call)                    \
+    do {                                 \
+        const int rc_ = (call);          \
+        if (rc_ != MXL_OK) return rc_;   \
+    } while (0)
+
+extern "C" int mxl_linear_sizes(mxl_linear* p) {
+    if (!valid(p)) return MXL_EINVAL;
+    const Linear l(p);
+    Arena s(nullptr), f(nullptr), b(nullptr);
+    Saved saved(l, s);
+    ForwardScratch fwd(l, f);
+    BackwardScratch bwd(l, b);
+    p->saved_bytes = s.used;
+    p->fwd_bytes = f.used;
+    p->bwd_bytes = b.used;
+    return MXL_OK;
+}
+
+extern "C" int mxl_linear_forward(const mxl_linear* p, const void* x, const void* aux0, const void* aux1, const void* w,
+                                  const void* w_scales, const int64_t* lens, void* saved_buf, void* scratch, void* y,
+                                  void* stream) {
+    if (!valid(p) || !x || !w || !scratch || !y || (p->saved_bytes > 0 && !saved_buf)) return MXL_EINVAL;
+    const Linear l(p);
+    const int G = (int)p->groups, batch = (int)l.batch;
+    Arena sa(saved_buf), fa(scratch);
+    const Saved sv(l, sa);
+    const ForwardScratch f(l, fa);
+    const int af = (int)p->act_fmt, wf = (int)p->w_fmt;
+    const bool from_rows = p->need_dx && p->dx_from_rows;
+    const Copy wr = from_rows ? sv.w_row : f.w_row;
+    if (l.tensorwise()) {
+        MXL_TRY(mxl_amax(x, p->rows * p->k, f.x_amax, stream));
+        MXL_TRY(mxl_quantize_tensorwise(x, p->rows, p->k, l.k_ld, af, f.x_amax, p->need_dw ? lens : nullptr, p->need_dw ? G : 0, f.x_row.q, f.x_row.s,
+                                        sv.x_col.q, sv.x_col.s, sv.x_si, l.qf(), stream));
+        MXL_TRY(mxl_amax(w, l.batch * p->n * p->k, f.w_amax, stream));
+        MXL_TRY(mxl_quantize_weight_tensorwise(w, l.batch, p->n, p->k, l.k_ld, l.n_ld, wf, f.w_amax, wr.q, wr.s, sv.w_col.q, sv.w_col.s, sv.w_si,
+                                               l.qf(), stream));
+        return mxl_grouped_gemm_nt_scaled(f.x_row.q, f.x_row.s, af, wr.q, wr.s, wf, y, lens, batch, p->rows, p->n, l.k_ld, sv.x_si, sv.w_si,
+                                          MXL_GF_KSTEP, stream);
+    }
+    if (p->input == MXL_LINEAR_RMSNORM) {
+        MXL_TRY(mxl_rmsnorm_fwd(x, aux0, (float)p->eps, p->rows, p->k, nullptr, sv.rstd, stream));
+        MXL_TRY(mxl_rmsnorm_quantize(x, aux0, sv.rstd, p->rows, p->k, l.k_ld, af, (int)p->scale_mode, nullptr, 0, f.x_row.q, f.x_row.s,
+                                     sv.x_col.q, sv.x_col.s, l.qf(), stream));
+    } else if (p->input != MXL_LINEAR_PLAIN) {
+        MXL_TRY(mxl_glu_probs_quantize(x, aux0, (int)p->probs_dtype, (const uint8_t*)aux1, p->rows, p->k, l.k_ld,
+                                       p->input == MXL_LINEAR_SILU ? MXL_ACT_SILU : MXL_ACT_GELU, af, (int)p->scale_mode, lens, G, f.x_row.q,
+                                       f.x_row.s, sv.x_col.q, sv.x_col.s, l.qf(), stream));
+    } else {
+        const bool rht = p->rht_signs >= 0 && p->need_dw;
+        MXL_TRY(mxl_quantize_ex(x, p->rows, p->k, l.k_ld, af, (int)p->scale_mode, lens, G, f.x_row.q, f.x_row.s, sv.x_col.q, sv.x_col.s,
+                                l.qf() | (rht ? MXL_QF_RHT_COL : 0u), 0, rht ? (uint32_t)p->rht_signs : 0u, stream));
+    }
+    if (p->w_quantized) {
+        if (!w_scales) return MXL_EINVAL;
+        return mxl_grouped_gemm_nt_ex(f.x_row.q, f.x_row.s, af, w, w_scales, wf, y, lens, batch, p->rows, p->n, l.k_ld, MXL_GF_KSTEP, stream);
+    }
+    MXL_TRY(mxl_quantize_weight_2d_ex(w, l.batch, p->n, p->k, l.k_ld, l.n_ld, wf, (int)p->scale_mode, wr.q, wr.s, sv.w_col.q, sv.w_col.s, l.qf(),
+                                      stream));
+    return mxl_grouped_gemm_nt_ex(f.x_row.q, f.x_row.s, af, wr.q, wr.s, wf, y, lens, batch, p->rows, p->n, l.k_ld, MXL_GF_KSTEP, stream);
+}
+
+extern "C" int mxl_linear_backward(const mxl_linear* p, int parts, const void* dy, const void* x, const void* aux0, const void* aux1,
+                                   const void* wt, const void* wt_scales, const int64_t* lens, void* saved_buf, void* scratch, void* dx,
+                                   void* daux, void* dw, uint32_t dw_flags, uint64_t sr_seed, void* stream) {
+    if (!valid(p) || !scratch || (dw_flags & ~(uint32_t)MXL_GF_ACCUM_F32)) return MXL_EINVAL;
+    const Linear l(p);
+    const int G = (int)p->groups, batch = (int)l.batch;
+    Arena sa(saved_buf), ba(scratch);
+    const Saved sv(l, sa);
+    const BackwardScratch b(l, ba);
+    const int gf = (int)p->grad_fmt, wf = (int)p->w_fmt;
+    const bool sr = p->grad_sr && gf == MXL_FMT_E2M1;
+    if (parts & MXL_LINEAR_QUANTIZE) {
+        if (!dy) return MXL_EINVAL;
+        if (l.tensorwise()) {
+            MXL_TRY(mxl_amax(dy, p->rows * p->n, b.amax, stream));
+            MXL_TRY(mxl_quantize_tensorwise(dy, p->rows, p->n, p->need_dx ? l.n_ld : 0, gf, b.amax, p->need_dw ? lens : nullptr, p->need_dw ? G : 0,
+                                            b.d_row.q, b.d_row.s, b.d_col.q, b.d_col.s, b.d_si, l.qf(), stream));
+        } else {
+            const bool rht = p->rht_signs >= 0 && p->need_dw;
+            MXL_TRY(mxl_quantize_ex(dy, p->rows, p->n, l.n_ld, gf, (int)p->scale_mode, lens, G, b.d_row.q, b.d_row.s, b.d_col.q, b.d_col.s,
+                                    l.qf() | (rht ? MXL_QF_RHT_COL : 0u) | (sr ? MXL_QF_SR : 0u), sr ? sr_seed : 0,
+                                    rht ? (uint32_t)p->rht_signs : 0u, stream));
+        }
+    }
+    if ((parts & MXL_LINEAR_DX) && p->need_dx) {
+        void* out = b.dxi ? b.dxi : dx;
+        if (!out) return MXL_EINVAL;
+        const uint32_t flags = MXL_GF_KSTEP | (p->dx_from_rows ? MXL_GF_B_TRANSPOSED : 0u);
+        const void* bq = p->w_quantized ? wt : p->dx_from_rows ? sv.w_row.q : sv.w_col.q;
+        const void* bs = p->w_quantized ? wt_scales : sv.w_col.s;
+        if (l.tensorwise())
+            MXL_TRY(mxl_grouped_gemm_nt_scaled(b.d_row.q, b.d_row.s, gf, bq, bs, wf, out, lens, batch, p->rows, p->k, l.n_ld, b.d_si, sv.w_si, flags, stream));
+        else
+            MXL_TRY(mxl_grouped_gemm_nt_ex(b.d_row.q, b.d_row.s, gf, bq, bs, wf, out, lens, batch, p->rows, p->k, l.n_ld, flags, stream));
+        if (p->input == MXL_LINEAR_RMSNORM)
+            MXL_TRY(mxl_rmsnorm_bwd(b.dxi, x, aux0, sv.rstd, p->rows, p->k, dx, daux, b.norm_ws, b.norm_bytes, stream));
+        else if (p->input != MXL_LINEAR_PLAIN)
+            MXL_TRY(mxl_glu_probs_bwd(b.dxi, x, aux0, (int)p->probs_dtype, (const uint8_t*)aux1, p->rows, p->k,
+                                      p->input == MXL_LINEAR_SILU ? MXL_ACT_SILU : MXL_ACT_GELU, dx, daux, stream));
+    }
+    if ((parts & MXL_LINEAR_DW) && p->need_dw) {
+        const uint32_t flags = MXL_GF_KSTEP | dw_flags;
+        if (l.tensorwise())
+            return mxl_grouped_gemm_wgrad_scaled(b.d_col.q, b.d_col.s, gf, sv.x_col.q, sv.x_col.s, (int)p->act_fmt, dw, lens, G, p->rows, p->n, p->k,
+                                                 b.d_si, sv.x_si, flags, stream);
+        return mxl_grouped_gemm_wgrad_ex(b.d_col.q, b.d_col.s, gf, sv.x_col.q, sv.x_col.s, (int)p->act_fmt, dw, lens, G, p->rows, p->n, p->k, flags, stream);
+    }
+    return MXL_OK;
+}

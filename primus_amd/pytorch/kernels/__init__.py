@@ -10,6 +10,8 @@ stream, allocates only its outputs and never reads device data from the host.
 
 from __future__ import annotations
 
+import ctypes
+import functools
 from typing import Optional, Tuple
 
 import torch
@@ -202,7 +204,8 @@ def _ptr(t: Optional[torch.Tensor]):
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    # the handle alone: torch.cuda.current_stream() builds a Stream object around it (3 us a launch)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _require_cuda(*tensors: torch.Tensor) -> None:
@@ -625,6 +628,62 @@ def grouped_gemm_mx_wgrad_impl(a_t, a_t_scale, b_t, b_t_scale, group_lens, total
         )
     _lib.check(rc, "mxl_grouped_gemm_wgrad")
     return c
+
+
+# --------------------------------------------------------------------------
+# a whole linear in two calls (mxl_linear_forward / mxl_linear_backward)
+# --------------------------------------------------------------------------
+class LinearPlan:
+    """Sizes and options of one linear and of the buffers its two calls work in; depends on nothing else, so linears of
+    the same sizes share it."""
+
+    __slots__ = ("struct", "ptr", "saved_bytes", "fwd_bytes", "bwd_bytes", "rows", "n", "k")
+
+    def __init__(self, **fields):
+        self.struct = _lib.Linear(**fields)
+        self.ptr = ctypes.addressof(self.struct)
+        _lib.check(_lib.load().mxl_linear_sizes(self.ptr), "mxl_linear_sizes")
+        self.saved_bytes, self.fwd_bytes, self.bwd_bytes = self.struct.saved_bytes, self.struct.fwd_bytes, self.struct.bwd_bytes
+        self.rows, self.n, self.k = self.struct.rows, self.struct.n, self.struct.k
+
+
+@functools.lru_cache(maxsize=512)
+def linear_plan(rows, n, k, groups, recipe, act_fmt, w_fmt, grad_fmt, scale_mode, need_dx, need_dw, dx_from_rows=False,
+                w_quantized=False, input=_lib.LINEAR_PLAIN, probs_dtype=0, grad_sr=False, rht_signs=None, eps=0.0) -> LinearPlan:
+    """``rows`` > 0, operands in the K-step-major layouts (``pick_layout``); the fields are those of ``mxl_linear``."""
+    return LinearPlan(rows=rows, n=n, k=k, groups=groups, recipe=recipe, act_fmt=act_fmt, w_fmt=w_fmt, grad_fmt=grad_fmt,
+                      scale_mode=scale_mode, need_dx=need_dx, need_dw=need_dw, dx_from_rows=dx_from_rows, w_quantized=w_quantized,
+                      input=input, probs_dtype=probs_dtype, grad_sr=grad_sr, rht_signs=-1 if rht_signs is None else rht_signs & 0xFFFF, eps=eps)
+
+
+def linear_forward_impl(plan: LinearPlan, x, w, w_scales=None, group_lens=None, aux0=None, aux1=None):
+    """``(y, saved)``: every launch of the linear's forward; ``saved`` is what ``linear_backward_impl`` reads (None if
+    the plan needs no gradient)."""
+    dev = x.device
+    saved = torch.empty(plan.saved_bytes, dtype=torch.uint8, device=dev) if plan.saved_bytes else None
+    scratch = torch.empty(plan.fwd_bytes, dtype=torch.uint8, device=dev)
+    y = torch.empty((plan.rows, plan.n), dtype=torch.bfloat16, device=dev)
+    rc = _lib.load().mxl_linear_forward(
+        plan.ptr, x.data_ptr(), None if aux0 is None else aux0.data_ptr(), None if aux1 is None else aux1.data_ptr(), w.data_ptr(),
+        None if w_scales is None else w_scales.data_ptr(), None if group_lens is None else group_lens.data_ptr(),
+        None if saved is None else saved.data_ptr(), scratch.data_ptr(), y.data_ptr(), _stream())
+    if rc:
+        _lib.check(rc, "mxl_linear_forward")
+    return y, saved
+
+
+def linear_backward_impl(plan: LinearPlan, parts: int, dy, saved, scratch, dx=None, dw=None, daux=None, x=None, wt=None, wt_scales=None,
+                         group_lens=None, aux0=None, aux1=None, accumulate: bool = False, sr_seed: int = 0) -> None:
+    """``parts`` of the linear's backward (``_lib.LINEAR_*``, or'ed) on the current stream; ``scratch``
+    (``plan.bwd_bytes``) carries the quantised gradient from one part to the others."""
+    def ptr(t):
+        return None if t is None else t.data_ptr()
+
+    rc = _lib.load().mxl_linear_backward(
+        plan.ptr, parts, ptr(dy), ptr(x), ptr(aux0), ptr(aux1), ptr(wt), ptr(wt_scales), ptr(group_lens), ptr(saved), ptr(scratch),
+        ptr(dx), ptr(daux), ptr(dw), _lib.GF_ACCUM_F32 if accumulate else 0, sr_seed, _stream())
+    if rc:
+        _lib.check(rc, "mxl_linear_backward")
 
 
 # --------------------------------------------------------------------------

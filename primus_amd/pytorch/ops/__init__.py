@@ -151,6 +151,122 @@ def _cache_layout(b: QuantizedTensor, b_t, kc: int, fp8: bool, groups: int, fp4:
     return lay if kc else 0
 
 
+# The two GEMMs of a backward run side by side from this many operations each on.  Below it they are a few tens of
+# microseconds, and the events between the two streams cost more than the overlap gives.
+_OVERLAP_MIN_FLOPS = 1.0e11
+
+
+def _two_calls(a, b, group_lens, cached: bool, norm_weight=None) -> bool:
+    """Whether a linear on K-step-major operands can go through ``mxl_linear_forward`` / ``_backward``: on the GPU, in
+    sizes the kernels take (anything else raises on the launch-by-launch route), and nobody is watching the launches."""
+    if K._launch_hook is not None or not a.is_cuda or b.shape[-1] % _lib.BLOCK or b.shape[-2] % _lib.BLOCK:
+        return False
+    if not cached and not b.is_cuda:
+        return False
+    if norm_weight is not None:
+        K._norm_args(a, norm_weight)
+    K._check_group_lens(group_lens, a.device)
+    return True
+
+
+def _mx_forward(ctx, a, b, b_t, group_lens, act_fmt, w_fmt, scale_mode, probs, row_mask, activation, grad_sr, rht_signs, norm_weight,
+                norm_eps, accum, kc, need_dgrad, need_wgrad):
+    """Forward of ``_MXLinearFunction`` on K-step-major operands: one call."""
+    cached = isinstance(b, QuantizedTensor)
+    w, w_scales, wt, wt_scales = b, None, None, None
+    if cached:
+        if b.axis != -1:
+            raise ValueError("the forward weight copy must be quantised along axis=-1")
+        if b.tensor_scale_inv is not None:
+            raise ValueError("the cached weight copy is tensor-wise scaled, the operator's config is an MX recipe")
+        w, w_scales = _cached_codes(b, kc), _cached_scales(b, kc)
+        if need_dgrad:
+            if b_t is None:
+                raise ValueError("dgrad needs the transposed weight copy (QuantizedTensorPair.data_t)")
+            if b_t.axis != -2:
+                raise ValueError("QuantizedTensorPair.data_t must be quantised along axis=-2")
+            wt, wt_scales = _cached_codes(b_t, kc), _cached_scales(b_t, kc)
+    n, k = b.shape[-2], b.shape[-1]
+    # dgrad on the row-wise weight codes: see the launch-by-launch route below
+    bt = (need_dgrad and not cached and _dgrad_reads_rowwise and act_fmt == w_fmt and n % K.GEMM_K_ALIGN == 0 and k % K.GEMM_K_ALIGN == 0)
+    inp, pd, aux0, aux1 = _lib.LINEAR_PLAIN, 0, None, None
+    if activation is not None:
+        act, pd, row_mask = K._glu_args(a, probs, row_mask, activation)
+        inp = _lib.LINEAR_SILU if act == _lib.ACT_SILU else _lib.LINEAR_GELU
+        aux0, aux1 = probs, row_mask
+    elif norm_weight is not None:
+        inp, aux0 = _lib.LINEAR_RMSNORM, norm_weight
+    sr = bool(grad_sr) and act_fmt == _lib.FMT_E2M1
+    plan = K.linear_plan(a.shape[0], n, k, 0 if group_lens is None else b.shape[0], _lib.LINEAR_MX, act_fmt, w_fmt, act_fmt, scale_mode,
+                         need_dgrad, need_wgrad, bt, cached, inp, pd, sr, rht_signs, norm_eps)
+    y, saved = K.linear_forward_impl(plan, a, w, w_scales, group_lens, aux0, aux1)
+    if need_dgrad or need_wgrad:
+        ctx.plan, ctx.sr, ctx.accum = plan, sr, accum
+        ctx.needs = (need_dgrad, need_wgrad, tuple(b.shape))
+        keep = need_dgrad and inp != _lib.LINEAR_PLAIN
+        ctx.save_for_backward(saved, group_lens, wt, wt_scales, a if keep else None, aux0 if keep else None, aux1 if keep else None)
+    return y
+
+
+def _mx_backward(ctx, dy):
+    plan = ctx.plan
+    saved, group_lens, wt, wt_scales, x, aux0, aux1 = ctx.saved_tensors
+    need_dgrad, need_wgrad, w_shape = ctx.needs
+    dx = daux = None
+    if need_dgrad:
+        inp = plan.struct.input
+        if inp == _lib.LINEAR_PLAIN:
+            dx = torch.empty((plan.rows, plan.k), dtype=torch.bfloat16, device=dy.device)
+        else:
+            dx = torch.empty_like(x)
+            daux = torch.empty_like(aux0) if inp == _lib.LINEAR_RMSNORM else torch.empty((plan.rows,), dtype=torch.float32, device=dy.device)
+    dw = _backward_in_parts(plan, dy, saved, group_lens, ctx.accum, need_dgrad, need_wgrad, w_shape, dx, daux, x, wt, wt_scales, aux0, aux1,
+                            K.next_sr_seed() if ctx.sr else 0)
+    grad_p = grad_nw = None
+    if daux is not None:
+        if plan.struct.input == _lib.LINEAR_RMSNORM:
+            grad_nw = daux
+        else:
+            grad_p = daux.to(aux0.dtype)
+    return dx, dw, None, None, None, None, None, grad_p, None, None, None, None, grad_nw, None, None, None
+
+
+def _backward_in_parts(plan, dy, saved, group_lens, accum, need_dgrad, need_wgrad, w_shape, dx, daux=None, x=None, wt=None,
+                       wt_scales=None, aux0=None, aux1=None, sr_seed=0):
+    """The backward of one linear: one call, or its weight gradient on the side stream.  Returns the weight gradient."""
+    dy = dy.contiguous()
+    if dy.dtype != torch.bfloat16:
+        dy = dy.to(torch.bfloat16)
+    dev = dy.device
+    scratch = torch.empty(plan.bwd_bytes, dtype=torch.uint8, device=dev)
+    dw, fused, target = None, False, None
+    if need_wgrad:
+        target = accum[0] if accum is not None else None
+        fused = _fusable(target)      # the GEMM's epilogue adds into the float32 buffer
+    overlap = (_wgrad_overlap and need_dgrad and need_wgrad and 2.0 * plan.rows * plan.n * plan.k >= _OVERLAP_MIN_FLOPS)
+    if not overlap:
+        if need_wgrad:
+            dw = target if fused else torch.empty(w_shape, dtype=torch.bfloat16, device=dev)
+        K.linear_backward_impl(plan, _lib.LINEAR_QUANTIZE | _lib.LINEAR_DX | _lib.LINEAR_DW, dy, saved, scratch, dx, dw, daux, x, wt, wt_scales,
+                               group_lens, aux0, aux1, fused, sr_seed)
+    else:
+        K.linear_backward_impl(plan, _lib.LINEAR_QUANTIZE, dy, saved, scratch, group_lens=group_lens, sr_seed=sr_seed)
+        main = torch.cuda.current_stream(dev)
+        side = _side_stream(dev)
+        side.wait_stream(main)   # the quantised operands are ready
+        K.linear_backward_impl(plan, _lib.LINEAR_DX, None, saved, scratch, dx, None, daux, x, wt, wt_scales, group_lens, aux0, aux1)
+        with torch.cuda.stream(side):
+            dw = target if fused else torch.empty(w_shape, dtype=torch.bfloat16, device=dev)
+            K.linear_backward_impl(plan, _lib.LINEAR_DW, None, saved, scratch, None, dw, group_lens=group_lens, accumulate=fused)
+        for t in (saved, scratch) + (() if group_lens is None else (group_lens,)):
+            t.record_stream(side)
+        dw.record_stream(main)
+        main.wait_stream(side)
+    if need_wgrad and accum is not None:
+        return _finish_wgrad(dw, accum, fused, w_shape)
+    return dw
+
+
 class _MXLinearFunction(torch.autograd.Function):
     """Y = X . W^T on MX operands, dense (``group_lens is None``) or grouped.
 
@@ -160,11 +276,11 @@ class _MXLinearFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, a, b, b_t, group_lens, act_fmt, w_fmt, scale_mode, probs=None, row_mask=None, activation=None,
-                grad_sr=False, rht_signs=None, norm_weight=None, norm_eps=0.0, accum=None):
+                grad_sr=False, rht_signs=None, norm_weight=None, norm_eps=0.0, accum=None, need_grad=True):
         glu = activation is not None
         norm = norm_weight is not None
-        need_dgrad = a.requires_grad or (glu and probs.requires_grad) or (norm and norm_weight.requires_grad)
-        need_wgrad = b.requires_grad
+        need_dgrad = need_grad and (a.requires_grad or (glu and probs.requires_grad) or (norm and norm_weight.requires_grad))
+        need_wgrad = need_grad and b.requires_grad
         grouped = group_lens is not None
         # Every operand of the three GEMMs is stored in one layout, K-chunk-major unless an operand is
         # too large for it (or the layout is switched off): same codes, same results, faster loads.
@@ -175,8 +291,13 @@ class _MXLinearFunction(torch.autograd.Function):
         # E2M1 x E2M1 runs on the ring kernel too, in steps of 128 elements (two MFMAs per step)
         fp4 = act_fmt == _lib.FMT_E2M1 and w_fmt == _lib.FMT_E2M1
         kc = K.pick_layout(groups, b.shape[-2], b.shape[-1], a.shape[0], fp8=fp8, fp4=fp4)
-        if isinstance(b, QuantizedTensor):   # cached copies decide: the call uses the layout they are stored in
+        cached = isinstance(b, QuantizedTensor)
+        if cached:   # cached copies decide: the call uses the layout they are stored in
             kc = _cache_layout(b, b_t, kc, fp8, groups, fp4)
+        if kc in (K.LAYOUT_KSTEP, K.LAYOUT_KSTEP128) and a.shape[0] > 0 and _two_calls(a, b, group_lens, cached, norm_weight):
+            return _mx_forward(ctx, a, b, b_t, group_lens, act_fmt, w_fmt, scale_mode, probs, row_mask, activation, grad_sr, rht_signs,
+                               norm_weight, norm_eps, accum, kc, need_dgrad, need_wgrad)
+        ctx.plan = None
         # (a weight gradient that is added to a float32 buffer inside the GEMM runs on either chunked layout)
         # activations: row-wise for the forward GEMM, transposed col-wise kept for wgrad
         # (row-wise copies are padded to the GEMM's K granularity, like the reference pads its
@@ -246,6 +367,8 @@ class _MXLinearFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy):
+        if ctx.plan is not None:
+            return _mx_backward(ctx, dy)
         a_col, a_cs, w_col, w_cs, group_lens = ctx.saved_tensors[:5]
         act_fmt, scale_mode, total_m, need_dgrad, need_wgrad, w_shape = ctx.cfg
         grouped = group_lens is not None
@@ -300,7 +423,7 @@ class _MXLinearFunction(torch.autograd.Function):
             # grad_a so far is dL/dX for X = rmsnorm(a); take it through the normalisation
             pre, nw, rstd = ctx.saved_tensors[5:8]
             grad_a, grad_nw = K.rmsnorm_bwd_impl(grad_a, pre, nw, rstd)
-        return grad_a, grad_b, None, None, None, None, None, grad_p, None, None, None, None, grad_nw, None, None
+        return grad_a, grad_b, None, None, None, None, None, grad_p, None, None, None, None, grad_nw, None, None, None
 
 
 def _transposed_cache(q: QuantizedTensor, kchunk: bool):
@@ -336,9 +459,9 @@ class _TWLinearFunction(torch.autograd.Function):
     transposed copies that dgrad and wgrad read."""
 
     @staticmethod
-    def forward(ctx, a, b, b_t, group_lens, fwd_fmt, bwd_fmt, accum=None):
-        need_dgrad = a.requires_grad
-        need_wgrad = b.requires_grad
+    def forward(ctx, a, b, b_t, group_lens, fwd_fmt, bwd_fmt, accum=None, need_grad=True):
+        need_dgrad = need_grad and a.requires_grad
+        need_wgrad = need_grad and b.requires_grad
         grouped = group_lens is not None
         groups = b.shape[0] if grouped else 1
         if isinstance(b, QuantizedTensor):
@@ -352,6 +475,17 @@ class _TWLinearFunction(torch.autograd.Function):
                 kc = 0
         else:
             kc = K.pick_layout(groups, b.shape[-2], b.shape[-1], a.shape[0], fp8=True)
+        if kc == K.LAYOUT_KSTEP and a.shape[0] > 0 and not isinstance(b, QuantizedTensor) and _two_calls(a, b, group_lens, False):
+            n, k = b.shape[-2], b.shape[-1]
+            bt = need_dgrad and _dgrad_reads_rowwise and fwd_fmt == _lib.FMT_E4M3 and n % K.GEMM_K_ALIGN == 0 and k % K.GEMM_K_ALIGN == 0
+            plan = K.linear_plan(a.shape[0], n, k, groups if grouped else 0, _lib.LINEAR_TENSORWISE, fwd_fmt, fwd_fmt, bwd_fmt, 0,
+                                 need_dgrad, need_wgrad, bt)
+            y, saved = K.linear_forward_impl(plan, a, b, None, group_lens)
+            ctx.plan, ctx.accum = plan, accum
+            ctx.needs = (need_dgrad, need_wgrad, tuple(b.shape))
+            ctx.save_for_backward(saved, group_lens)
+            return y
+        ctx.plan = None
         a_row, a_ru, a_col, a_cu, a_si = K.quantize_tensorwise_impl(
             a, fwd_fmt, rowwise=True, colwise=need_wgrad, group_lens=group_lens, pad_to=K.GEMM_K_ALIGN, kchunk=kc)
         if isinstance(b, QuantizedTensor):
@@ -383,6 +517,12 @@ class _TWLinearFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dy):
+        if ctx.plan is not None:
+            saved, group_lens = ctx.saved_tensors
+            need_dgrad, need_wgrad, w_shape = ctx.needs
+            dx = torch.empty((ctx.plan.rows, ctx.plan.k), dtype=torch.bfloat16, device=dy.device) if need_dgrad else None
+            dw = _backward_in_parts(ctx.plan, dy, saved, group_lens, ctx.accum, need_dgrad, need_wgrad, w_shape, dx)
+            return dx, dw, None, None, None, None, None, None
         a_col, a_cu, a_si, w_col, w_cu, w_si, group_lens = ctx.saved_tensors
         bwd_fmt, total_m, need_dgrad, need_wgrad, w_shape, kc = ctx.cfg
         dy = dy.contiguous()
@@ -417,7 +557,7 @@ class _TWLinearFunction(torch.autograd.Function):
             else:
                 grad_b = wgrad()
             grad_b = _finish_wgrad(grad_b, ctx.accum, fused, w_shape)
-        return grad_a, grad_b, None, None, None, None, None
+        return grad_a, grad_b, None, None, None, None, None, None
 
 
 class _BWLinearFunction(torch.autograd.Function):
@@ -487,6 +627,21 @@ def _formats(config, fp4: bool):
     return f, f
 
 
+class _NoGradContext:
+    """Stands in for the autograd context where no gradient will be asked for."""
+
+    def save_for_backward(self, *tensors):
+        pass
+
+
+def _apply(fn, *args):
+    """``fn.apply(*args)``, or its forward alone when nothing needs a gradient: no graph node, and no copies for a
+    backward that cannot come (``requires_grad`` of a leaf says nothing under ``torch.no_grad``)."""
+    if torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in args):
+        return fn.apply(*args)
+    return fn.forward(_NoGradContext(), *args, need_grad=False)
+
+
 def _run(a, b, group_lens, trans_a, trans_b, out_dtype, config, fuse_bgrad_accum_pattern, fp4, glu=None, norm=None):
     if trans_a or not trans_b:
         raise ValueError("the MX linear path is NT only: trans_a=False, trans_b=True (primus_turbo.py:1095-1103)")
@@ -540,7 +695,7 @@ def _run(a, b, group_lens, trans_a, trans_b, out_dtype, config, fuse_bgrad_accum
     if tensorwise:
         if glu is not None or norm is not None:
             raise NotImplementedError("the activation / normalisation prologues exist for the MX recipes only")
-        return _TWLinearFunction.apply(a, b, b_t, group_lens, fwd_fmt, bwd_fmt, accum)
+        return _apply(_TWLinearFunction, a, b, b_t, group_lens, fwd_fmt, bwd_fmt, accum)
     # stochastic rounding applies to E2M1 gradients; with E4M3 activations the gradients are MXFP8
     grad_sr = bool(fp4 and config.use_gradient_sr and act_fmt == _lib.FMT_E2M1)
     rht = getattr(config, "colwise_rht_signs", None) if fp4 and act_fmt == _lib.FMT_E2M1 else None
@@ -550,10 +705,10 @@ def _run(a, b, group_lens, trans_a, trans_b, out_dtype, config, fuse_bgrad_accum
         norm_weight, eps = norm
         if norm_weight.dtype != torch.bfloat16 or tuple(norm_weight.shape) != (a.shape[-1],):
             raise ValueError("the norm weight must be a bfloat16 vector of the contraction length")
-        return _MXLinearFunction.apply(a, b, b_t, None, act_fmt, w_fmt, config.scale_mode.value,
+        return _apply(_MXLinearFunction, a, b, b_t, None, act_fmt, w_fmt, config.scale_mode.value,
                                        None, None, None, grad_sr, None, norm_weight.contiguous(), float(eps), accum)
     if glu is None:
-        return _MXLinearFunction.apply(a, b, b_t, group_lens, act_fmt, w_fmt, config.scale_mode.value,
+        return _apply(_MXLinearFunction, a, b, b_t, group_lens, act_fmt, w_fmt, config.scale_mode.value,
                                        None, None, None, grad_sr, rht, None, 0.0, accum)
     if rht is not None:
         raise NotImplementedError("the activation prologue and the Hadamard transform cannot be combined")
@@ -562,7 +717,7 @@ def _run(a, b, group_lens, trans_a, trans_b, out_dtype, config, fuse_bgrad_accum
         raise ValueError(f"activation must be 'silu' or 'gelu', got {activation!r}")
     if probs.dim() != 1 or probs.shape[0] != a.shape[0]:
         raise ValueError("probs must be 1-D with one entry per row of the activations")
-    return _MXLinearFunction.apply(a, b, b_t, group_lens, act_fmt, w_fmt, config.scale_mode.value,
+    return _apply(_MXLinearFunction, a, b, b_t, group_lens, act_fmt, w_fmt, config.scale_mode.value,
                                    probs.contiguous(), row_mask, activation, grad_sr, None, None, 0.0, accum)
 
 
@@ -577,6 +732,14 @@ def gemm_fp4(a, b, trans_a: bool = False, trans_b: bool = True, out_dtype: Optio
              config: Optional[Float4QuantConfig] = None, fuse_bgrad_accum_pattern: Optional[str] = None):
     """Same with MXFP4 weights (activations per ``config.activation_format``)."""
     return _run(a, b, None, trans_a, trans_b, out_dtype, config, fuse_bgrad_accum_pattern, fp4=True)
+
+
+def mxfp4_linear_2d(a, b, use_gradient_sr: bool, colwise_rht_signs: Optional[int]):
+    """``gemm_fp4`` with every operand E2M1 and the options given one by one: the MXFP4 linear of the local transformer
+    spec (primus/backends/megatron/core/extensions/primus_turbo_mxfp4_local.py:291-461), whose weight-gradient operands
+    go through the Hadamard transform."""
+    return _run(a, b, None, False, True, None, Float4QuantConfig(use_gradient_sr=use_gradient_sr, colwise_rht_signs=colwise_rht_signs),
+                None, fp4=True)
 
 
 class _RMSNormFunction(torch.autograd.Function):
