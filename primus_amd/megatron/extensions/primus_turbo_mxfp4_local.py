@@ -39,6 +39,7 @@ import torch
 
 from ... import _lib
 from ...pytorch import kernels as K
+from ...pytorch import ops
 from ...pytorch.core.low_precision import ScalingGranularity, dtype_to_fmt_code, float4_e2m1fn_x2, float8_e5m2, float8_e8m0
 
 MXFP4_BLOCK_SIZE = 32
@@ -286,6 +287,8 @@ class MXFP4LinearFunction(torch.autograd.Function):
     @staticmethod
     def setup_context(ctx, inputs, output):
         input, weight, preshuffle, backward_is_fp8, fp8_bwd_dtype, _, _, use_gradient_sr = inputs
+        # no zero gradients for the kept copies: they are not differentiable (four fill kernels of their size a pass)
+        ctx.set_materialize_grads(False)
         ctx.preshuffle = preshuffle
         ctx.backward_is_fp8 = backward_is_fp8
         ctx.use_gradient_sr = use_gradient_sr
@@ -301,6 +304,8 @@ class MXFP4LinearFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output, *_):
+        if grad_output is None:
+            return (None,) * 8
         grad_2d = grad_output.contiguous().reshape(-1, grad_output.shape[-1])
         if grad_2d.dtype != torch.bfloat16:
             grad_2d = grad_2d.to(torch.bfloat16)
@@ -327,5 +332,13 @@ def mxfp4_linear(input, weight, preshuffle: bool = False, backward_precision: st
     if backward_precision not in ("mxfp4", "fp8"):
         raise ValueError("backward_precision must be 'mxfp4' or 'fp8'")
     fp8 = backward_precision == "fp8"
+    if not fp8 and not torch.compiler.is_compiling():
+        # The operators' MXFP4 linear is the same arithmetic on the same codes (the pre-shuffled byte order changes no
+        # result) in the layout the ring GEMM reads, without a transposed weight copy and without the custom ops, which
+        # exist for torch.compile.
+        if input.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
+            raise ValueError("MXFP4LinearFunction expects bfloat16 operands")
+        out = ops.mxfp4_linear_2d(input.reshape(-1, input.shape[-1]).contiguous(), weight.contiguous(), use_gradient_sr, RHT_SIGNS)
+        return out.reshape(*input.shape[:-1], weight.shape[0])
     return MXFP4LinearFunction.apply(input, weight, preshuffle, fp8, float8_e5m2 if fp8 else None,
                                      ScalingGranularity.TENSORWISE.value if fp8 else 0, 0, use_gradient_sr)[0]
