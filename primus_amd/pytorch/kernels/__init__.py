@@ -637,14 +637,14 @@ class LinearPlan:
     """Sizes and options of one linear and of the buffers its two calls work in; depends on nothing else, so linears of
     the same sizes share it."""
 
-    __slots__ = ("struct", "ptr", "saved_bytes", "fwd_bytes", "bwd_bytes", "rows", "n", "k")
+    __slots__ = ("struct", "ptr", "saved_bytes", "fwd_bytes", "bwd_bytes", "rows", "n", "k", "groups")
 
     def __init__(self, **fields):
         self.struct = _lib.Linear(**fields)
         self.ptr = ctypes.addressof(self.struct)
         _lib.check(_lib.load().mxl_linear_sizes(self.ptr), "mxl_linear_sizes")
         self.saved_bytes, self.fwd_bytes, self.bwd_bytes = self.struct.saved_bytes, self.struct.fwd_bytes, self.struct.bwd_bytes
-        self.rows, self.n, self.k = self.struct.rows, self.struct.n, self.struct.k
+        self.rows, self.n, self.k, self.groups = self.struct.rows, self.struct.n, self.struct.k, self.struct.groups
 
 
 @functools.lru_cache(maxsize=512)

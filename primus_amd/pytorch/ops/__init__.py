@@ -70,7 +70,7 @@ def set_dgrad_reads_rowwise_weight(enabled: bool) -> None:
 
 
 def set_wgrad_overlap(enabled: bool) -> None:
-    """Run wgrad on a side stream next to dgrad (default on)."""
+    """Let wgrad run on a side stream next to dgrad where that is faster (default on)."""
     global _wgrad_overlap
     _wgrad_overlap = bool(enabled)
 
@@ -151,9 +151,20 @@ def _cache_layout(b: QuantizedTensor, b_t, kc: int, fp8: bool, groups: int, fp4:
     return lay if kc else 0
 
 
-# The two GEMMs of a backward run side by side from this many operations each on.  Below it they are a few tens of
-# microseconds, and the events between the two streams cost more than the overlap gives.
-_OVERLAP_MIN_FLOPS = 1.0e11
+def _overlaps(plan) -> bool:
+    """Whether the weight gradient runs on the side stream next to dgrad.  Both are persistent kernels on every CU, so what
+    the overlap gives is their last, partial rounds of tiles and their epilogues under the other's MFMAs; what it costs is
+    the events between the streams, operand panels of two GEMMs in the same L2s, and buffers the allocator must keep for
+    two streams.  Measured, together / one after the other: dense [8192, 4096] x 14336 1.29 / 1.28 ms, [2048, 4096] x 4096
+    217 / 144 us; Mixtral experts MXFP8, 16384 tokens, 16.5 / 16.3 ms.  Grouped E2M1 operands gain (Mixtral MXFP4, 4096
+    tokens 3.81 / 3.88 ms, 16384 10.6 / 10.7; at 2048 tokens and 4096 x 4096 experts 936 / 936 us), FP8 ones with groups of up
+    to about 1000 rows a little (DeepSeek shard, 4096 tokens, 5.59 / 5.63; 8192 tokens 9.39 / 9.37)."""
+    flops = 2.0 * plan.rows * plan.n * plan.k
+    if plan.groups == 0:
+        return False
+    if plan.struct.act_fmt == _lib.FMT_E2M1:
+        return flops >= 5e11
+    return flops >= 1.5e12 and plan.rows <= 1024 * plan.groups
 
 
 def _two_calls(a, b, group_lens, cached: bool, norm_weight=None) -> bool:
@@ -243,7 +254,7 @@ def _backward_in_parts(plan, dy, saved, group_lens, accum, need_dgrad, need_wgra
     if need_wgrad:
         target = accum[0] if accum is not None else None
         fused = _fusable(target)      # the GEMM's epilogue adds into the float32 buffer
-    overlap = (_wgrad_overlap and need_dgrad and need_wgrad and 2.0 * plan.rows * plan.n * plan.k >= _OVERLAP_MIN_FLOPS)
+    overlap = _wgrad_overlap and need_dgrad and need_wgrad and _overlaps(plan)
     if not overlap:
         if need_wgrad:
             dw = target if fused else torch.empty(w_shape, dtype=torch.bfloat16, device=dev)

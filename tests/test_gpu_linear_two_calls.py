@@ -31,7 +31,7 @@ def _config(recipe):
     return Float4QuantConfig(use_gradient_sr=True, colwise_rht_signs=0xA6C9)
 
 
-def _check(run, leaves, overlap_flops=None):
+def _check(run, leaves):
     from primus_amd.pytorch import ops
 
     def step():
@@ -42,17 +42,17 @@ def _check(run, leaves, overlap_flops=None):
             y0 = run()
         return (y, y0) + torch.autograd.grad(y, leaves, dy)
 
-    saved = ops._OVERLAP_MIN_FLOPS
+    rule = ops._overlaps
     try:
         want = _launch_by_launch(step)
-        for floor in (0.0, 1e30):          # the weight gradient on the side stream, and everything in one call
-            ops._OVERLAP_MIN_FLOPS = floor
+        for together in (True, False):     # the weight gradient on the side stream, and everything in one call
+            ops._overlaps = lambda plan: together
             got = step()
             torch.cuda.synchronize()
             assert all(torch.equal(a, b) for a, b in zip(got, want))
         assert torch.equal(want[0], want[1])
     finally:
-        ops._OVERLAP_MIN_FLOPS = saved
+        ops._overlaps = rule
         ops.manual_sr_seed(None)
 
 
