@@ -602,6 +602,12 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
     static_assert(AFMT != kFmtE2M1 || (F44 && !ALPHA), "an FP4 row operand needs an FP4 weight operand (MX recipe)");
     static_assert(BFMT != kFmtE2M1 || F44 || (MODE == MODE_FWD && !ALPHA), "an E2M1 weight operand against FP8 rows: forward / dgrad of the MX recipe");
     constexpr bool B4 = BFMT == kFmtE2M1 && !F44;     // FP4 weights against FP8 rows: 32 bytes per row and K step
+    // PEEL: a tile's first MFMAs start from the constant 0 instead of cleared accumulators.  The compiler clears the 256
+    // accumulators of an E2M1 tile twice over, 2048 clocks that nothing covers (one wave per SIMD): the weight gradient of
+    // 1024 rows per group, [8, 28672, 4096], 903 -> 734 us; dgrad on the row-wise codes 1-3 % (fc1 of the same, 556 -> 537).
+    // The peeled step is another copy of the loop body, which the forward GEMM gains nothing from and the FP8
+    // instantiations do not survive (16 -> 160 spilled registers, 1081 -> 1236 us).
+    constexpr bool PEEL = F44 && (MODE == MODE_WGRAD || BT);
     constexpr int KS = F44 ? 2 * BK : BK;             // elements of the contraction per step
     constexpr int PSTEPS = 512 / KS;                  // steps per scale panel
     constexpr int B_ROW = B4 ? BK / 2 : BK;           // bytes of a row of b in a K step
@@ -837,7 +843,7 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
 
 #define MXL_MFMA(F, I, J) \
     do { if (MF && (I) < LIVE) { \
-             acc[I][J] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(F.b[J], F.a[I], acc[I][J], CB, BL, 0, F.sb[J], 0, F.sa[I]); \
+             acc[I][J] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(F.b[J], F.a[I], FIRST ? v16f{} : acc[I][J], CB, BL, 0, F.sb[J], 0, F.sa[I]); \
              if (F44) acc[I][J] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4( \
                  __builtin_shufflevector(F.b[J], F.b[J], 4, 5, 6, 7, 4, 5, 6, 7), __builtin_shufflevector(F.a[I], F.a[I], 4, 5, 6, 7, 4, 5, 6, 7), \
                  acc[I][J], CB, BL, 1, F.sb[J], 1, F.sa[I]); } } while (0)
@@ -987,13 +993,14 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
                 MXL_RD_B(f0, 0); MXL_RD_B(f0, 1); MXL_RD_B(f0, 2); MXL_RD_B(f0, 3);
                 MXL_RD_A(f0, 0); MXL_RD_A(f0, 1); MXL_RD_A(f0, 2); MXL_RD_A(f0, 3);
                 MXL_PIN;
-                // the accumulators are cleared while those reads are on their way
+                if (!PEEL) {    // the accumulators are cleared while those reads are on their way
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+                    for (int i = 0; i < 4; ++i)
 #pragma unroll
-                    for (int j = 0; j < 4; ++j)
+                        for (int j = 0; j < 4; ++j)
 #pragma unroll
-                        for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+                            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+                }
                 MXL_PIN;
                 MXL_SC_B(f0, 0); MXL_SC_B(f0, 1); MXL_SC_B(f0, 2); MXL_SC_B(f0, 3);
                 MXL_SC_A(f0, 0); MXL_SC_A(f0, 1); MXL_SC_A(f0, 2); MXL_SC_A(f0, 3);
@@ -1005,10 +1012,11 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
             using E2 = std::integral_constant<int, 2>; using E3 = std::integral_constant<int, 3>;
             using E4 = std::integral_constant<int, 4>; using E5 = std::integral_constant<int, 5>;
             using E6 = std::integral_constant<int, 6>; using E7 = std::integral_constant<int, 7>;
-            auto kstep = [&](auto par_tag, auto mf_tag, auto last_tag, int s, Frags& cur, Frags& nxt) __attribute__((always_inline)) {
+            auto kstep = [&](auto par_tag, auto mf_tag, auto last_tag, auto first_tag, int s, Frags& cur, Frags& nxt) __attribute__((always_inline)) {
                 constexpr int PAR = decltype(par_tag)::value;
                 constexpr bool MF = decltype(mf_tag)::value;
                 constexpr bool LAST = decltype(last_tag)::value;
+                constexpr bool FIRST = decltype(first_tag)::value;
                 const uint32_t slot_prev = wave_base + (uint32_t)(((gs + 3) & 3) * STAGE);   // group of step gs + 3
                 const uint32_t slot_new = wave_base + (uint32_t)((gs & 3) * STAGE);          // group of step gs + 4
                 MXL_MFMA(cur, 0, 0); if (ROUNDS == 8) issue_e(E6{}, slot_prev); MXL_PIN;
@@ -1046,34 +1054,37 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
             using P1 = std::integral_constant<int, 1>;
             using Yes = std::integral_constant<bool, true>;
             using No = std::integral_constant<bool, false>;
-            if (nst_real >= 3) {
-                for (int s = 0; s < nst - 2; s += 2) {
-                    if (s == nst - 4) {
-                        // the request stream moves on to the workgroup's next tile: its scale panel 0 first
-                        pb_is = next3(pb_is);
-                        issue_s(dn, 0, pb_is);
-                        stream_enter(dn);
-                    } else if ((s & (PSTEPS - 1)) == PSTEPS - 4 && s + 4 < nst) {
-                        // this tile's next scale panel (K steps s + 4 ...): first read three barriers from here
-                        pb_is = next3(pb_is);
-                        issue_s(d, (s + 4) / PSTEPS, pb_is);
-                    }
-                    kstep(P0{}, Yes{}, No{}, s, f0, f1);
-                    kstep(P1{}, Yes{}, No{}, s + 1, f1, f0);
+            auto pair = [&](auto first_tag, int s) __attribute__((always_inline)) {
+                if (s == nst - 4) {
+                    // the request stream moves on to the workgroup's next tile: its scale panel 0 first
+                    pb_is = next3(pb_is);
+                    issue_s(dn, 0, pb_is);
+                    stream_enter(dn);
+                } else if ((s & (PSTEPS - 1)) == PSTEPS - 4 && s + 4 < nst) {
+                    // this tile's next scale panel (K steps s + 4 ...): first read three barriers from here
+                    pb_is = next3(pb_is);
+                    issue_s(d, (s + 4) / PSTEPS, pb_is);
                 }
-                kstep(P0{}, Yes{}, No{}, nst - 2, f0, f1);
-                if (!F44 || nst_real == nst) kstep(P1{}, Yes{}, Yes{}, nst - 1, f1, f0);
-                else kstep(P1{}, No{}, Yes{}, nst - 1, f1, f0);          // an odd range: the padding step does not multiply
+                kstep(P0{}, Yes{}, No{}, first_tag, s, f0, f1);
+                kstep(P1{}, Yes{}, No{}, No{}, s + 1, f1, f0);
+            };
+            using First = std::integral_constant<bool, PEEL>;
+            if (nst_real >= 3) {
+                if constexpr (PEEL) pair(Yes{}, 0);
+                for (int s = PEEL ? 2 : 0; s < nst - 2; s += 2) pair(No{}, s);
+                kstep(P0{}, Yes{}, No{}, No{}, nst - 2, f0, f1);
+                if (!F44 || nst_real == nst) kstep(P1{}, Yes{}, Yes{}, No{}, nst - 1, f1, f0);
+                else kstep(P1{}, No{}, Yes{}, No{}, nst - 1, f1, f0);          // an odd range: the padding step does not multiply
             } else {
                 // a contraction range of one or two steps: four steps run, the others without multiplying
                 pb_is = next3(pb_is);
                 issue_s(dn, 0, pb_is);
                 stream_enter(dn);
-                kstep(P0{}, Yes{}, No{}, 0, f0, f1);
-                if (!F44 || nst_real == 2) kstep(P1{}, Yes{}, No{}, 1, f1, f0);
-                else kstep(P1{}, No{}, No{}, 1, f1, f0);
-                kstep(P0{}, No{}, No{}, 2, f0, f1);
-                kstep(P1{}, No{}, Yes{}, 3, f1, f0);
+                kstep(P0{}, Yes{}, No{}, First{}, 0, f0, f1);
+                if (!F44 || nst_real == 2) kstep(P1{}, Yes{}, No{}, No{}, 1, f1, f0);
+                else kstep(P1{}, No{}, No{}, No{}, 1, f1, f0);
+                kstep(P0{}, No{}, No{}, No{}, 2, f0, f1);
+                kstep(P1{}, No{}, Yes{}, No{}, 3, f1, f0);
             }
         };
         {
