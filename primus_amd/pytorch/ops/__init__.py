@@ -647,8 +647,12 @@ class _NoGradContext:
 
 def _apply(fn, *args):
     """``fn.apply(*args)``, or its forward alone when nothing needs a gradient: no graph node, and no copies for a
-    backward that cannot come (``requires_grad`` of a leaf says nothing under ``torch.no_grad``)."""
+    backward that cannot come (``requires_grad`` of a leaf says nothing under ``torch.no_grad``).  Inside a function
+    transform or a forward-mode level ``apply`` is called all the same: it refuses what the operator has no rule for,
+    where the forward alone would drop the tangent."""
     if torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in args):
+        return fn.apply(*args)
+    if torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0:
         return fn.apply(*args)
     return fn.forward(_NoGradContext(), *args, need_grad=False)
 
