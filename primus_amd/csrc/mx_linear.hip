@@ -153,10 +153,9 @@ extern "C" int mxl_linear_forward(const mxl_linear* p, const void* x, const void
     const bool from_rows = p->need_dx && p->dx_from_rows;
     const Copy wr = from_rows ? sv.w_row : f.w_row;
     if (l.tensorwise()) {
-        MXL_TRY(mxl_amax(x, p->rows * p->k, f.x_amax, stream));
+        MXL_TRY(mxl::amax_pair(x, p->rows * p->k, f.x_amax, w, l.batch * p->n * p->k, f.w_amax, stream));
         MXL_TRY(mxl_quantize_tensorwise(x, p->rows, p->k, l.k_ld, af, f.x_amax, p->need_dw ? lens : nullptr, p->need_dw ? G : 0, f.x_row.q, f.x_row.s,
                                         sv.x_col.q, sv.x_col.s, sv.x_si, l.qf(), stream));
-        MXL_TRY(mxl_amax(w, l.batch * p->n * p->k, f.w_amax, stream));
         MXL_TRY(mxl_quantize_weight_tensorwise(w, l.batch, p->n, p->k, l.k_ld, l.n_ld, wf, f.w_amax, wr.q, wr.s, sv.w_col.q, sv.w_col.s, sv.w_si,
                                                l.qf(), stream));
         return mxl_grouped_gemm_nt_scaled(f.x_row.q, f.x_row.s, af, wr.q, wr.s, wf, y, lens, batch, p->rows, p->n, l.k_ld, sv.x_si, sv.w_si,

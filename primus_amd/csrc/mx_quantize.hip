@@ -619,18 +619,43 @@ static int dispatch_quant_tensor(int fmt, QuantArgs& a, int64_t tiles_r, int64_t
     return MXL_EINVAL;
 }
 
-// abs-max of a bf16 tensor: non-negative floats order like their bit patterns, so an integer atomic max on the
-// fp32 pattern does it (a NaN pattern is larger than every number and wins).  One atomic per workgroup.
-__global__ __launch_bounds__(256) void amax_kernel(const uint16_t* x, int64_t n8, int64_t n, uint32_t* out) {
+// abs-max of one or two bf16 tensors: non-negative floats order like their bit patterns, so an integer atomic max on
+// the fp32 pattern does it (a NaN pattern is larger than every number and wins).  One atomic per workgroup.
+//
+// Bound by reading the tensor once, if enough loads are in flight and few enough atomics meet at the one result: a
+// workgroup takes pieces of 32 KiB, eight 16-byte loads per lane issued together, and at most AMAX_MAX_WG of them share
+// a tensor.  [4096, 14336] twice: 103 us with one load in flight per lane and up to 4096 workgroups, 41 (5.8 TB/s) so;
+// [4096, 4096]: 17.4 -> 11.8 us (16.6 with 1024 workgroups).
+// The loads are ordinary ones: the quantiser reads the same tensor next, and up to 256 MiB of it then come from the
+// memory-side cache.
+constexpr int AMAX_LOADS = 8, AMAX_PIECE = 256 * AMAX_LOADS, AMAX_MAX_WG = 512;
+struct AmaxArgs {
+    const uint16_t* x[2];
+    int64_t n[2];
+    uint32_t* out[2];
+    uint32_t wg[2];          // workgroups of each tensor
+};
+__global__ __launch_bounds__(256) void amax_kernel(AmaxArgs p) {
     __shared__ uint32_t part[4];
+    const int second = blockIdx.x >= p.wg[0];
+    const uint16_t* x = p.x[second];
+    const int64_t n = p.n[second], n8 = n / 8, wg = p.wg[second];
+    const int64_t blk = (int64_t)blockIdx.x - (second ? p.wg[0] : 0u);
     uint32_t m = 0;
-    const int64_t stride = (int64_t)gridDim.x * 256;
-    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n8; i += stride) {
-        const uint4 v = load16_streaming(x + i * 8);
-        m = pk_max16(m, pk_max16(pk_max16(v.x & 0x7FFF7FFFu, v.y & 0x7FFF7FFFu), pk_max16(v.z & 0x7FFF7FFFu, v.w & 0x7FFF7FFFu)));
+    for (int64_t i0 = blk * AMAX_PIECE; i0 < n8; i0 += wg * AMAX_PIECE) {
+        uint4 v[AMAX_LOADS];
+#pragma unroll
+        for (int u = 0; u < AMAX_LOADS; ++u) {
+            // past the end: the last piece once more
+            const int64_t i = i0 + u * 256 + threadIdx.x;
+            v[u] = *(const uint4*)(x + (i < n8 ? i : n8 - 1) * 8);
+        }
+#pragma unroll
+        for (int u = 0; u < AMAX_LOADS; ++u)
+            m = pk_max16(m, pk_max16(pk_max16(v[u].x & 0x7FFF7FFFu, v[u].y & 0x7FFF7FFFu), pk_max16(v[u].z & 0x7FFF7FFFu, v[u].w & 0x7FFF7FFFu)));
     }
     m = hmax16(m);
-    if (blockIdx.x == 0 && threadIdx.x == 0)
+    if (blk == 0 && threadIdx.x == 0)
         for (int64_t i = n8 * 8; i < n; ++i) m = max(m, (uint32_t)(x[i] & 0x7FFFu));   // tail of fewer than 8 elements
 #pragma unroll
     for (int s = 32; s > 0; s >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, s));
@@ -638,29 +663,44 @@ __global__ __launch_bounds__(256) void amax_kernel(const uint16_t* x, int64_t n8
     __syncthreads();
     if (threadIdx.x == 0) {
         m = max(max(part[0], part[1]), max(part[2], part[3]));
-        atomicMax(out, m << 16);   // bf16 pattern -> fp32 pattern
+        atomicMax(p.out[second], m << 16);   // bf16 pattern -> fp32 pattern
     }
 }
 
-__global__ void amax_init_kernel(uint32_t* out) { *out = 0u; }
+__global__ void amax_init_kernel(uint32_t* a, uint32_t* b) {
+    *a = 0u;
+    *b = 0u;
+}
+
+static uint32_t amax_workgroups(int64_t n) {
+    const int64_t pieces = (n / 8 + AMAX_PIECE - 1) / AMAX_PIECE;
+    if (pieces <= 0) return n > 0 ? 1 : 0;
+    const int64_t rounds = (pieces + AMAX_MAX_WG - 1) / AMAX_MAX_WG;
+    return (uint32_t)((pieces + rounds - 1) / rounds);      // every workgroup the same number of pieces
+}
+
+// out_a = max |a| over na values, out_b = max |b| (b may be null: one tensor), in two launches
+int amax_pair(const void* a, int64_t na, void* out_a, const void* b, int64_t nb, void* out_b, void* stream) {
+    if (na < 0 || nb < 0 || !out_a || (na > 0 && !a) || ((uintptr_t)a & 15) != 0) return MXL_EINVAL;
+    if (nb > 0 && (!b || !out_b || ((uintptr_t)b & 15) != 0)) return MXL_EINVAL;
+    if (!device_is_gfx950()) return MXL_ENODEV;
+    hipStream_t st = (hipStream_t)stream;
+    AmaxArgs p{{(const uint16_t*)a, (const uint16_t*)b}, {na, nb}, {(uint32_t*)out_a, (uint32_t*)(out_b ? out_b : out_a)},
+               {amax_workgroups(na), amax_workgroups(nb)}};
+    // a fill kernel, not a memset: callers may be capturing the stream into a graph
+    hipLaunchKernelGGL(amax_init_kernel, dim3(1), dim3(1), 0, st, p.out[0], p.out[1]);
+    if (hipGetLastError() != hipSuccess) return MXL_ELAUNCH;
+    if (p.wg[0] + p.wg[1] == 0) return MXL_OK;
+    hipLaunchKernelGGL(amax_kernel, dim3(p.wg[0] + p.wg[1]), dim3(256), 0, st, p);
+    return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;
+}
 
 }  // namespace mxl
 
 using namespace mxl;
 
 extern "C" int mxl_amax(const void* x_bf16, int64_t n, void* amax_f32, void* stream) {
-    if (n < 0 || !amax_f32 || (n > 0 && !x_bf16) || ((uintptr_t)x_bf16 & 15) != 0) return MXL_EINVAL;
-    if (!device_is_gfx950()) return MXL_ENODEV;
-    hipStream_t st = (hipStream_t)stream;
-    // a fill kernel, not a memset: callers may be capturing the stream into a graph
-    hipLaunchKernelGGL(amax_init_kernel, dim3(1), dim3(1), 0, st, (uint32_t*)amax_f32);
-    if (hipGetLastError() != hipSuccess) return MXL_ELAUNCH;
-    if (n == 0) return MXL_OK;
-    const int64_t n8 = n / 8;
-    int64_t grid = (n8 + 256 * 8 - 1) / (256 * 8);   // about 8 loads per lane
-    grid = grid < 1 ? 1 : grid > 4096 ? 4096 : grid;
-    hipLaunchKernelGGL(amax_kernel, dim3((unsigned)grid), dim3(256), 0, st, (const uint16_t*)x_bf16, n8, n, (uint32_t*)amax_f32);
-    return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;
+    return amax_pair(x_bf16, n, amax_f32, nullptr, 0, nullptr, stream);
 }
 
 extern "C" int64_t mxl_padded_width(int64_t total_rows, int num_groups) {
