@@ -7,19 +7,17 @@
 //                                                                   or . b_g          b_g = [k, n]   (MXL_BF_B_KN)
 //   wgrad           :  c[g][m_out, n_out] = sum over the tokens t of group g of p[t, m_out] * q[t, n_out]
 //
-// One workgroup (4 waves, 2 x 2) per BM x 256 output tile, in two sizes chosen per launch: BM = 256 (a wave owns
-// 128 x 128 = 4 x 4 MFMA tiles of 32 x 32, 256 fp32 accumulators, one workgroup per CU, a ring of four 32 KiB LDS
-// stages filled three K slots ahead) for groups of many rows, and BM = 128 (64 x 128 per wave, two workgroups per CU,
-// two stages) for groups of a few hundred rows, where a 256-row tile would mostly hold padding.  K advances in slots
-// of 32 elements (64 bytes per row), filled by LDS-direct loads (buffer_load ... lds); loads complete in order, so a
-// partial s_waitcnt leaves the younger slots in flight, and there is one barrier per slot.  An operand whose contraction dim is contiguous in memory is
-// staged [rows][32] and read with ds_read_b128; one whose contraction dim is the slow one (the [k, n] weight, both
-// operands of wgrad) is staged as it lies, [32][columns], and read with the transposing LDS read ds_read_b64_tr_b16,
+// Two kernels, chosen per launch, 256 output columns per tile each: 256 rows (bf16_gemm_tall_kernel: 8 waves, one
+// workgroup per CU) and, for forward / dgrad over groups of fewer rows, where a 256-row tile would mostly hold padding,
+// 128 rows (bf16_gemm_kernel: 4 waves of 64 x 128, two workgroups per CU, two stages of 32 contraction elements).  Both
+// fill LDS by LDS-direct loads (buffer_load ... lds).  An operand whose contraction dim is contiguous in memory is
+// staged by rows and read with ds_read_b128; one whose contraction dim is the slow one (the [k, n] weight, both
+// operands of wgrad) is staged as it lies, [contraction][columns], and read with the transposing LDS read ds_read_b64_tr_b16,
 // which hands every lane four consecutive contraction elements of its own column.  Measured lane mapping of that
 // read: inside each block of 16 lanes, lane 4 a + e receives element e of the 8-byte pieces addressed by lanes a,
 // a + 4, a + 8, a + 12 (in this order).  16-byte pieces are XOR-swizzled on the global side so that both kinds of
 // read are spread over the LDS banks.  The tile list is derived from group_lens by every workgroup; the workgroups
-// are persistent and walk it in rounds.
+// are persistent and walk it in rounds.  Both kernels add every output element's products in the same order: the same bits.
 #include "mx_device.h"
 
 #include <type_traits>
@@ -77,29 +75,66 @@ __device__ __forceinline__ void bf_dma16_at(v4i rsrc, uint32_t lds_base, uint32_
                  : "memory", "scc");
 }
 
-constexpr int bf16_lds_bytes(int bm, int nst) {
-    return nst * (bm * 64 + BF_B_BYTES) + (MXL_MAX_GROUPS + 2) * 4 + (MXL_MAX_GROUPS + 2) * 8;
+// one dword per lane into LDS: the line it lies in is in the L2 afterwards
+__device__ __forceinline__ void bf_dma4(v4i rsrc, uint32_t lds_off, uint32_t voff, uint32_t soff) {
+    asm volatile("" : "+s"(soff));
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+                 :
+                 : "s"(lds_off), "v"(voff), "s"(rsrc), "s"(soff)
+                 : "memory");
 }
-// number of gaps g in [first, m) that are not wave ph's request gaps (g % 4 == ph): the index of the fragment read
-// that the gap behind MFMA m holds
-constexpr int bf_read_index(int m, int first, int ph) {
-    int n = 0;
-    for (int g = first; g < m; ++g) n += (g & 3) != ph;
-    return n;
+
+constexpr int bf16_lds_bytes() {
+    return 2 * (128 * 64 + BF_B_BYTES) + (MXL_MAX_GROUPS + 2) * 4 + (MXL_MAX_GROUPS + 2) * 8;
 }
 template <int N>
 __device__ __forceinline__ void bf_wait_vm() {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// prefix sums over the groups of their rows and of their row tiles; lens clamped to what the buffers hold
+template <int BM>
+__device__ __forceinline__ void bf16_group_table(const Bf16Args& p, int64_t* pre_rows, int* pre_tiles, int t, int threads) {
+    const int G = p.num_groups;
+    for (int i = t; i < G; i += threads) pre_rows[i + 1] = p.group_lens ? p.group_lens[i] : p.total_m;
+    __syncthreads();
+    if (t == 0) {
+        int tiles = 0;
+        int64_t rows = 0;
+        pre_tiles[0] = 0;
+        pre_rows[0] = 0;
+        for (int i = 0; i < G; ++i) {
+            int64_t len = pre_rows[i + 1];
+            len = len < 0 ? 0 : len;
+            len = len > p.total_m - rows ? p.total_m - rows : len;
+            tiles += (int)((len + BM - 1) / BM);
+            rows += len;
+            pre_tiles[i + 1] = tiles;
+            pre_rows[i + 1] = rows;
+        }
+    }
+    __syncthreads();
+}
+// a fragment's 8 contraction elements of step ks from an operand staged [contraction row][256 columns]
+__device__ __forceinline__ v8bf bf16_read_trans(uint8_t* lane, int ks) {
+    v8bf out;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const v4s v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(lane + ks * 8192 + h * 2048));
+        const v4bf q = __builtin_bit_cast(v4bf, v);
+        out[4 * h] = q[0]; out[4 * h + 1] = q[1]; out[4 * h + 2] = q[2]; out[4 * h + 3] = q[3];
+    }
+    return out;
+}
+
 // A_T / B_T: the operand's contraction dim is the slow one in memory (staged [32][cols], transposing reads).
 // WGRAD: contraction over the tokens of a group (both operands A_T / B_T), one output matrix per group.
 // ACCUM (wgrad): c is float32 and the result is added to it.
-template <int BF_BM, int NST, bool A_T, bool B_T, bool WGRAD, bool ACCUM>
-__global__ __launch_bounds__(BF_THREADS, BF_BM == 256 ? 1 : 2) void bf16_gemm_kernel(Bf16Args p) {
+template <bool A_T, bool B_T, bool WGRAD, bool ACCUM>
+__global__ __launch_bounds__(BF_THREADS, 2) void bf16_gemm_kernel(Bf16Args p) {
     static_assert(!WGRAD || (A_T && B_T), "wgrad contracts over tokens: both operands are token-major");
     static_assert(!ACCUM || WGRAD, "only the weight gradient accumulates");
-    static_assert((BF_BM == 128 && NST == 2) || (BF_BM == 256 && NST == 4), "tile sizes built");
+    constexpr int BF_BM = 128, NST = 2;
     constexpr int BF_A_BYTES = BF_BM * 64, BF_STAGE = BF_A_BYTES + BF_B_BYTES;
     constexpr int MI = BF_BM / 64;             // 32-row fragments per wave
     constexpr int AR = BF_BM / 64;             // load rounds of 4 KiB for a (b: 4)
@@ -115,25 +150,7 @@ __global__ __launch_bounds__(BF_THREADS, BF_BM == 256 ? 1 : 2) void bf16_gemm_ke
     const int G = p.num_groups;
     const uint32_t smem_base = (uint32_t)(uintptr_t)smem;
 
-    // ---- group tables: prefix of rows and of 128-row tiles; lens clamped to what the buffers hold ----
-    for (int i = t; i < G; i += BF_THREADS) pre_rows[i + 1] = p.group_lens ? p.group_lens[i] : p.total_m;
-    __syncthreads();
-    if (t == 0) {
-        int tiles = 0;
-        int64_t rows = 0;
-        pre_tiles[0] = 0;
-        pre_rows[0] = 0;
-        for (int i = 0; i < G; ++i) {
-            int64_t len = pre_rows[i + 1];
-            len = len < 0 ? 0 : len;
-            len = len > p.total_m - rows ? p.total_m - rows : len;
-            tiles += (int)((len + BF_BM - 1) / BF_BM);
-            rows += len;
-            pre_tiles[i + 1] = tiles;
-            pre_rows[i + 1] = rows;
-        }
-    }
-    __syncthreads();
+    bf16_group_table<BF_BM>(p, pre_rows, pre_tiles, t, BF_THREADS);
 
     const int tiles_n = (int)((p.n + BF_BN - 1) / BF_BN);
     const int tiles_m = WGRAD ? (int)((p.m + BF_BM - 1) / BF_BM) : pre_tiles[G];
@@ -281,144 +298,34 @@ __global__ __launch_bounds__(BF_THREADS, BF_BM == 256 ? 1 : 2) void bf16_gemm_ke
         return out;
     };
 
-    // row fragments of this wave that hold rows of the tile (the others are neither read nor multiplied)
-    int live = (m_valid - wm * (BF_BM / 2) + 31) >> 5;
-    live = __builtin_amdgcn_readfirstlane(live < 0 ? 0 : (live > MI ? MI : live));
+    // does this wave hold rows of the tile?  (if not it only keeps the requests going)
+    const bool live = __builtin_amdgcn_readfirstlane(m_valid > wm * (BF_BM / 2));
 
-    // slot s has landed when at most the requests of the younger slots in flight are outstanding
-    auto wait_slot = [&](int s) __attribute__((always_inline)) {
-        const int younger = nslots - 1 - s;
-        if (NST >= 4 && younger >= 2) bf_wait_vm<2 * LOADS>();
-        else if (NST >= 3 && younger >= 1) bf_wait_vm<LOADS>();
-        else bf_wait_vm<0>();
-    };
     auto read_a = [&](uint8_t* sa, int i, int ks) __attribute__((always_inline)) {
         return A_T ? read_trans(sa, BF_BM * 2, wm * (BF_BM / 2) + 32 * i, ks) : read_contig(sa, ca_row + 32 * i, ks);
     };
     auto read_b = [&](uint8_t* sb, int j, int ks) __attribute__((always_inline)) {
         return B_T ? read_trans(sb, 512, wn * 128 + 32 * j, ks) : read_contig(sb, cb_row + 32 * j, ks);
     };
-    if constexpr (NST >= 4) {
-      if (live == MI && nslots > 0) {
-        // One wave per SIMD: nothing but this wave's own instruction order keeps the MFMA pipe fed, so the order is
-        // written out and pinned (sched_barrier): every fragment read and every load request sits between two MFMAs.
-        // A slot is two halves of 16 MFMAs (4 x 4 fragments, 16 contraction elements).  While the MFMAs of half 0 run,
-        // the fragments of half 1 are read; the first four MFMAs of half 1 are issued in front of the slot barrier (so
-        // the pipe has work while the waves meet), the fragments of the next slot's half 0 are read behind it.
-        // The 8 requests of slot s + 3 go out four per half, and the four waves -- which run in lockstep between the
-        // barriers, one per SIMD -- take turns: wave PH issues behind MFMA 4 e + PH, so the address unit sees one
-        // request per MFMA time instead of four at once and no wave waits at the unit's queue with its MFMA pipe
-        // running empty (a bf16 MFMA is over in 32 clocks, a request occupies the unit for about 16).
-        // Requests past the last slot fetch the last slot again (into a stage nobody reads any more): the request
-        // count per slot is then the same in every iteration and the partial waits are constants.
-        // The N-side fragment is MFMA source 0, so that a lane holds 4 consecutive output columns per register quad.
-        static_assert(MI == 4 && AR == 4, "written out for the 256-row tile");
-        const int last = nslots - 1;
+    if (nslots > 0) issue(0, 0);
+    for (int s = 0; s < nslots; ++s) {
+        bf_wait_vm<0>();
+        __syncthreads();     // slot s is in LDS for every wave, and every wave has left the stage of slot s - 1
+        if (s + 1 < nslots) issue(s + 1, (s + 1) & 1);
+        uint8_t* sa = smem + (s & 1) * BF_STAGE;
+        uint8_t* sb = sa + BF_A_BYTES;
+        if (!live) continue;
 #pragma unroll
-        for (int s = 0; s < NST - 1; ++s) issue(s < last ? s : last, s);
-        bf_wait_vm<2 * LOADS>();
-        __syncthreads();
-        auto run = [&](auto ph_tag) __attribute__((always_inline)) {
-            constexpr int PH = decltype(ph_tag)::value;
-            v8bf fa0[4], fb0[4], fa1[4], fb1[4];
+        for (int ks = 0; ks < 2; ++ks) {
+            v8bf fb[4], fa[MI];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) fb0[j] = read_b(smem + BF_A_BYTES, j, 0);
+            for (int j = 0; j < 4; ++j) fb[j] = read_b(sb, j, ks);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) fa0[i] = read_a(smem, i, 0);
-#define BF_PIN __builtin_amdgcn_sched_barrier(0)
-            // The gap behind MFMA number M = 4 j + i of a half holds at most one other instruction of weight: wave PH's
-            // load request (M - PH) / 4 of the half when M % 4 == PH, else the next fragment read (eight per half,
-            // in the order the next half's MFMAs need them: b0, a0 .. a3, b1 .. b3), from gap FIRST on.
-            auto rd = [&](auto r_tag, v8bf (&fa)[4], v8bf (&fb)[4], uint8_t* pa, uint8_t* pb, int ks) __attribute__((always_inline)) {
-                constexpr int R = decltype(r_tag)::value;
-                if constexpr (R == 0) fb[0] = read_b(pb, 0, ks);
-                else if constexpr (R <= 4) fa[R - 1] = read_a(pa, R - 1, ks);
-                else fb[R - 4] = read_b(pb, R - 4, ks);
-            };
-#define BF_STEP(FA, FB, M, R, VO, SO, OFF, RFA, RFB, PA, PB, KS, FIRST)                                                    \
-    acc[(M) & 3][(M) >> 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(FB[(M) >> 2], FA[(M) & 3], acc[(M) & 3][(M) >> 2], 0, 0, 0); \
-    if constexpr (((M) & 3) == PH) bf_dma16_at<(OFF) + ((M) >> 2) * 4096>(R, in_base, VO[(M) >> 2], SO);                     \
-    else if constexpr ((M) >= (FIRST) && bf_read_index(M, FIRST, PH) < 8)                                                  \
-        rd(std::integral_constant<int, bf_read_index(M, FIRST, PH)>{}, RFA, RFB, PA, PB, KS);                              \
-    BF_PIN
-#define BF_HALF0(M) BF_STEP(fa0, fb0, M, ra, va, in_sa, 0, fa1, fb1, sa, sb, 1, 0)
-#define BF_HALF1(M) BF_STEP(fa1, fb1, M, rb, vb, in_sb, BF_A_BYTES, fa0, fb0, na, nb, 0, 4)
-            int stage = 0;                            // stage of slot s; slot s + 3 goes into the stage in front of it
-            for (int s = 0; s < nslots; ++s) {
-                uint8_t* sa = smem + stage * BF_STAGE;
-                uint8_t* sb = sa + BF_A_BYTES;
-                const int in_slot = s + NST - 1 < last ? s + NST - 1 : last;
-                const uint32_t in_base = smem_base + (uint32_t)((stage == 0 ? NST - 1 : stage - 1) * BF_STAGE) + (uint32_t)(w * 1024);
-                const uint32_t in_sa = (uint32_t)in_slot * a_step, in_sb = (uint32_t)in_slot * b_step;
-                stage = stage == NST - 1 ? 0 : stage + 1;
-                uint8_t* na = smem + stage * BF_STAGE;
-                uint8_t* nb = na + BF_A_BYTES;
-                // ---- half 0 multiplies, half 1 is read; requests: the a rows of slot s + 3 ----
-                BF_HALF0(0); BF_HALF0(1); BF_HALF0(2); BF_HALF0(3); BF_HALF0(4); BF_HALF0(5); BF_HALF0(6); BF_HALF0(7);
-                BF_HALF0(8); BF_HALF0(9); BF_HALF0(10); BF_HALF0(11); BF_HALF0(12); BF_HALF0(13); BF_HALF0(14); BF_HALF0(15);
-                // ---- half 1 multiplies; behind the barrier the next slot's half 0 is read; requests: the b rows ----
-                BF_HALF1(0); BF_HALF1(1); BF_HALF1(2); BF_HALF1(3);
-                // slot s + 1 has landed when only slot s + 2, the a rows of slot s + 3 and its first b request are outstanding
-                // (waves of a ragged tile that run the generic loop below meet the same barriers: one per slot)
-                if (s + 1 < nslots) {
-                    bf_wait_vm<LOADS + AR + 1>();
-                    __syncthreads();   // slot s + 1 is in LDS for every wave; every wave holds its fragments of slot s
-                }
-                BF_PIN;
-                BF_HALF1(4); BF_HALF1(5); BF_HALF1(6); BF_HALF1(7); BF_HALF1(8); BF_HALF1(9);
-                BF_HALF1(10); BF_HALF1(11); BF_HALF1(12); BF_HALF1(13); BF_HALF1(14); BF_HALF1(15);
-            }
-#undef BF_HALF0
-#undef BF_HALF1
-#undef BF_STEP
-#undef BF_PIN
-        };
-        if (w == 0) run(std::integral_constant<int, 0>{});
-        else if (w == 1) run(std::integral_constant<int, 1>{});
-        else if (w == 2) run(std::integral_constant<int, 2>{});
-        else run(std::integral_constant<int, 3>{});
-        bf_wait_vm<0>();     // the repeated requests of the last slots must not land in the output staging area
-      }
-    }
-    if (NST < 4 || live != MI) {
+            for (int i = 0; i < MI; ++i) fa[i] = read_a(sa, i, ks);
 #pragma unroll
-        for (int s = 0; s < NST - 1; ++s)
-            if (s < nslots) issue(s, s);
-        int stage = 0, stage_in = NST - 1;        // stage of slot s; stage that slot s + NST - 1 goes into
-        for (int s = 0; s < nslots; ++s) {
-            wait_slot(s);
-            __syncthreads();     // slot s is in LDS for every wave, and every wave has left the stage of slot s - 1
-            if (s + NST - 1 < nslots) issue(s + NST - 1, stage_in);
-            uint8_t* sa = smem + stage * BF_STAGE;
-            uint8_t* sb = sa + BF_A_BYTES;
-            if (live > 0) {
+            for (int i = 0; i < MI; ++i)
 #pragma unroll
-                for (int ks = 0; ks < 2; ++ks) {
-                    v8bf fb[4];
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) fb[j] = read_b(sb, j, ks);
-                    if (NST == 2 || live == MI) {
-                        v8bf fa[MI];
-#pragma unroll
-                        for (int i = 0; i < MI; ++i) fa[i] = read_a(sa, i, ks);
-#pragma unroll
-                        for (int i = 0; i < MI; ++i)
-#pragma unroll
-                            for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < MI; ++i) {
-                            if (i < live) {
-                                const v8bf fa = read_a(sa, i, ks);
-#pragma unroll
-                                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j], fa, acc[i][j], 0, 0, 0);
-                            }
-                        }
-                    }
-                }
-            }
-            stage = stage == NST - 1 ? 0 : stage + 1;
-            stage_in = stage_in == NST - 1 ? 0 : stage_in + 1;
+                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[j], fa[i], acc[i][j], 0, 0, 0);
         }
     }
     __syncthreads();         // every wave is done with the stages: they become the output staging area
@@ -477,6 +384,382 @@ __global__ __launch_bounds__(BF_THREADS, BF_BM == 256 ? 1 : 2) void bf16_gemm_ke
   }
 }
 
+// ---- the 256-row tile: 8 waves (2 x 4) of 128 x 64, two per SIMD, K slots of 64 elements ----
+// Bound by the board's power limit where the groups are long (MFMA busy 0.80 at 1.55 GHz; the vendor library's dense
+// kernel on the same problem 0.88 at 1.51, 7 % faster), by the padding of the groups' last tiles where they are short.
+// What the split is for:
+//   * two waves per SIMD: one's requests, reads and barriers run under the other's MFMAs.  Four waves of 128 x 128, one
+//     per SIMD, had MFMA busy 0.58 whatever the order of their instructions;
+//   * slots of 64 elements: a request moves whole 128-byte lines of a contiguous operand (32 elements: half lines);
+//   * requests close behind the barrier that frees their stage (spread over 15 MFMAs; over 22: -3 %, over 30: -6 %): they
+//     have one slot, about a microsecond, to land;
+//   * the L2 is asked four slots ahead for the lines this tile's neighbours on the XCD will want, each line by one of
+//     them: a fifth of the requests missed the L2 and every slot waited for some of those (-15 % cycles);
+//   * the next tile's first slot is requested in front of the output's way out (wgrad of 1000 tokens: +1.5 %).
+// Mixtral experts [32768, 4096] x [8, 28672, 4096], forward / dgrad / wgrad: 1.07 / 1.19 / 1.17 -> 1.27 / 1.30 / 1.36 PFLOP/s;
+// 32 ragged groups of about 1024 rows, [4096, 7168]: 0.88 / 0.97 / 0.98 -> 1.10 / 1.15 / 1.13; 128 groups of about 512,
+// [5760, 2880]: 0.75 / 0.81 / 0.70 -> 0.89 / 0.88 / 0.72.
+constexpr int TL_THREADS = 512;
+constexpr int TL_KS = 64;                               // contraction elements per slot: 128 bytes of a row, four MFMA steps
+constexpr int TL_HALF = 256 * TL_KS * 2;                // 32 KiB: one operand of a slot
+constexpr int TL_STAGE = 2 * TL_HALF, TL_OPS = 2;       // two stages
+constexpr int TL_REQ = 8;                               // requests per wave and slot: four rounds of 8 KiB per operand
+constexpr int TL_AHEAD = 4;                             // slots the L2 is asked ahead
+constexpr int TL_TABLES = (MXL_MAX_GROUPS + 2) * 4 + (MXL_MAX_GROUPS + 2) * 8;
+constexpr int tall_lds_bytes() { return TL_OPS * TL_STAGE + TL_TABLES + 256; }      // (256: where the L2 requests' dwords land)
+
+template <int I, int N, class F>
+__device__ __forceinline__ void bf_static_for(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        bf_static_for<I + 1, N>(f);
+    }
+}
+
+template <bool A_T, bool B_T, bool WGRAD, bool ACCUM>
+__global__ __launch_bounds__(TL_THREADS, 2) void bf16_gemm_tall_kernel(Bf16Args p) {
+    static_assert(!WGRAD || (A_T && B_T), "wgrad contracts over tokens: both operands are token-major");
+    static_assert(!ACCUM || WGRAD, "only the weight gradient accumulates");
+    extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+    int* pre_tiles = (int*)(smem + TL_OPS * TL_STAGE);
+    int64_t* pre_rows = (int64_t*)(pre_tiles + MXL_MAX_GROUPS + 2);
+    const int t = threadIdx.x;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int l = t & 63, lr = l & 31, g = l >> 5;
+    const int wm = w >> 2, wn = w & 3;      // the two waves of a SIMD hold different rows: a tile of <= 128 rows keeps one busy on each
+    const int G = p.num_groups;
+    const uint32_t smem_base = (uint32_t)(uintptr_t)smem;
+    bf16_group_table<256>(p, pre_rows, pre_tiles, t, TL_THREADS);
+
+    const int tiles_n = (int)((p.n + BF_BN - 1) / BF_BN);
+    const int tiles_m = WGRAD ? (int)((p.m + 255) / 256) : pre_tiles[G];
+    const int total_tiles = WGRAD ? G * tiles_m * tiles_n : tiles_m * tiles_n;
+    const int nwg = gridDim.x;
+    const int vwg = (nwg & 7) ? (int)blockIdx.x : ((int)(blockIdx.x & 7) * (nwg >> 3) + (int)(blockIdx.x >> 3));
+
+    // ---- per-lane constants ----
+    // requests: lane's place in a round of 8 KiB (contiguous operand: 64 rows of 128 bytes; transposed: 16 rows of 512)
+    const int c_row = t >> 3, c_piece = (t & 7) ^ ((c_row >> 1) & 7);
+    const int t_row = t >> 5, t_piece = (t & 31) ^ ((t_row & 3) << 2);
+    // fragment reads: contiguous, row lr of a fragment, piece 2 ks + g XOR (row / 2) % 8 (16 lanes are served at a time,
+    // 256 bytes: 16 rows have to put the piece into 16 different places of two rows; with row % 8 half of them met)
+    const int lane_c = lr * 128 + 16 * (g ^ ((lr >> 1) & 7));
+    const int a_c = wm * 128 * 128 + lane_c, b_c = TL_HALF + wn * 64 * 128 + lane_c;
+    // transposed: this lane addresses row tj of a 4-row group, 8-byte piece ta4 of its 16-lane block's 16 columns
+    const int tj = (l & 15) >> 2, ta4 = l & 3, tblk = (l >> 4) & 1;
+    const int lane_t = (8 * g + tj) * 512 + 8 * (ta4 & 1), t_col16 = 2 * tblk + (ta4 >> 1);
+
+    struct Tile {
+        int64_t n0, c_row0;             // first output column and row (forward: token row; wgrad: row inside the group's matrix)
+        int grp, m_valid, n_valid;
+        int halves;                     // contraction in halves of a slot (32 elements)
+        uint32_t a_step, b_step;        // bytes from one K slot to the next
+        v4i ra, rb;
+        uint32_t va[4], vb[4];          // per-lane offsets of the load rounds
+        v4i rp;                         // the L2 request: descriptor, bytes from slot to slot, per-lane offset
+        uint32_t p_step, vp;
+    };
+    auto setup = [&](int tile) __attribute__((always_inline)) {
+        Tile q;
+        int grp = 0;
+        if (WGRAD) {
+            grp = tile / (tiles_m * tiles_n);
+            tile -= grp * tiles_m * tiles_n;
+        }
+        int pid_m, pid_n;
+        {
+            const int width = BF_GROUP_M * tiles_n;
+            const int first = (tile / width) * BF_GROUP_M;
+            const int gsz = (tiles_m - first) < BF_GROUP_M ? (tiles_m - first) : BF_GROUP_M;
+            pid_m = first + (tile % width) % gsz;
+            pid_n = (tile % width) / gsz;
+        }
+        const int64_t n0 = (int64_t)pid_n * BF_BN;
+        const int n_valid = (p.n - n0) < BF_BN ? (int)(p.n - n0) : BF_BN;
+        int64_t klen, c_row0;
+        int m_valid;
+        uint32_t a_step, b_step;
+        if (!WGRAD) {
+            int lo = 0, hi = G;
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (pre_tiles[mid] <= pid_m) lo = mid; else hi = mid;
+            }
+            grp = lo;
+            const int64_t g_row0 = pre_rows[grp], g_rows = pre_rows[grp + 1] - g_row0;
+            const int64_t r = (int64_t)(pid_m - pre_tiles[grp]) * 256;
+            c_row0 = g_row0 + r;
+            m_valid = (g_rows - r) < 256 ? (int)(g_rows - r) : 256;
+            klen = p.k;
+            const int64_t lda = p.k * 2;
+            q.ra = bf_rsrc(p.a + c_row0 * lda, (p.total_m - c_row0) * lda);
+            a_step = TL_KS * 2;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) q.va[e] = (uint32_t)((c_row + 64 * e) * lda + 16 * c_piece);
+            if (!B_T) {
+                const int64_t ldb = p.k * 2, b_row0 = (int64_t)grp * p.n + n0;
+                q.rb = bf_rsrc(p.b + b_row0 * ldb, ((int64_t)G * p.n - b_row0) * ldb);
+                b_step = TL_KS * 2;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) q.vb[e] = (uint32_t)((c_row + 64 * e) * ldb + 16 * c_piece);
+            } else {
+                const int64_t ldb = p.n * 2;
+                q.rb = bf_rsrc(p.b + ((int64_t)grp * p.k * p.n + n0) * 2, (p.k * p.n - n0) * 2);
+                b_step = (uint32_t)(TL_KS * ldb);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) q.vb[e] = (uint32_t)((t_row + 16 * e) * ldb + 16 * t_piece);
+            }
+        } else {
+            const int64_t m0 = (int64_t)pid_m * 256;
+            c_row0 = m0;
+            m_valid = (p.m - m0) < 256 ? (int)(p.m - m0) : 256;
+            const int64_t t0 = pre_rows[grp];
+            klen = pre_rows[grp + 1] - t0;
+            // the descriptors end with the group's last token: the rows of a partly filled last slot read as zero
+            const int64_t lda = p.m * 2, ldb = p.n * 2;
+            q.ra = bf_rsrc(p.a + t0 * lda + m0 * 2, klen * lda - m0 * 2);
+            q.rb = bf_rsrc(p.b + t0 * ldb + n0 * 2, klen * ldb - n0 * 2);
+            a_step = (uint32_t)(TL_KS * lda);
+            b_step = (uint32_t)(TL_KS * ldb);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                q.va[e] = (uint32_t)((t_row + 16 * e) * lda + 16 * t_piece);
+                q.vb[e] = (uint32_t)((t_row + 16 * e) * ldb + 16 * t_piece);
+            }
+        }
+        q.a_step = (uint32_t)__builtin_amdgcn_readfirstlane((int)a_step);
+        q.b_step = (uint32_t)__builtin_amdgcn_readfirstlane((int)b_step);
+        {
+            // lines of 128 bytes this tile asks the L2 for: a quarter of a's 256 of a slot (waves 0 .. 3, 16 lanes each),
+            // an eighth of b's (waves 4 .. 7, 8 lanes).  Rows of a at a power of two apart are left out (an empty
+            // descriptor drops the request): asking for them costs more than it gives (k = 4096: 1.17 with, 1.22 without).
+            const bool of_a = w < 4, trans = of_a ? A_T : B_T;
+            const int line = of_a ? (pid_n & 3) * 64 + w * 16 + (l & 15) : (pid_m & 7) * 32 + (w - 4) * 8 + (l & 7);
+            const int64_t ld = (of_a ? (WGRAD ? p.m : p.k) : (WGRAD || B_T ? p.n : p.k)) * 2;
+            const bool ask = trans || !of_a || (ld & (ld - 1)) != 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) q.rp[i] = __builtin_amdgcn_readfirstlane(of_a ? q.ra[i] : q.rb[i]);
+            if (!ask) q.rp[2] = 0;
+            q.p_step = (uint32_t)__builtin_amdgcn_readfirstlane(ask ? (int)(of_a ? a_step : b_step) : 0);
+            q.vp = (uint32_t)(trans ? (line >> 2) * ld + (line & 3) * 128 : line * ld);
+        }
+        q.halves = __builtin_amdgcn_readfirstlane((int)((klen + 31) / 32));
+        q.m_valid = __builtin_amdgcn_readfirstlane(m_valid);
+        q.n_valid = n_valid;
+        q.grp = grp;
+        q.n0 = n0;
+        q.c_row0 = c_row0;
+        return q;
+    };
+    // requests of a slot; past the last slot the descriptors are empty, so the range check drops them
+    struct In {
+        v4i ra, rb;
+        uint32_t base, sa, sb;
+    };
+    auto in_begin = [&](const Tile& q, int slot) __attribute__((always_inline)) {
+        In r{q.ra, q.rb, smem_base + (uint32_t)((slot & 1) * TL_STAGE) + (uint32_t)(w * 1024), (uint32_t)slot * q.a_step, (uint32_t)slot * q.b_step};
+        if (2 * slot >= q.halves) r.ra[2] = 0, r.rb[2] = 0, r.sa = 0, r.sb = 0;
+        return r;
+    };
+    auto request = [&](auto e_tag, const In& r, const Tile& q) __attribute__((always_inline)) {
+        constexpr int e = decltype(e_tag)::value;       // the operands in turn
+        if constexpr ((e & 1) == 0) bf_dma16_at<(e >> 1) * 8192>(r.ra, r.base, q.va[e >> 1], r.sa);
+        else bf_dma16_at<TL_HALF + (e >> 1) * 8192>(r.rb, r.base, q.vb[e >> 1], r.sb);
+    };
+    const uint32_t ahead_lds = smem_base + TL_OPS * TL_STAGE + TL_TABLES;
+    auto ask_l2 = [&](const Tile& q, int slot) __attribute__((always_inline)) {
+        v4i r = q.rp;
+        uint32_t so = (uint32_t)slot * q.p_step;
+        if (2 * slot >= q.halves) r[2] = 0, so = 0;
+        if (l < (w < 4 ? 16 : 8)) bf_dma4(r, ahead_lds, q.vp, so);
+    };
+    auto first_slot = [&](const Tile& q) __attribute__((always_inline)) {
+        const In r = in_begin(q, 0);
+        bf_static_for<0, TL_REQ>([&](auto e) { request(e, r, q); });
+    };
+
+    if (vwg >= total_tiles) return;
+    Tile tl = setup(vwg);
+    first_slot(tl);
+    for (int tile_id = vwg;;) {
+        // an odd half is the first half of a last slot (what lies past it in the slot belongs to the next row and is not
+        // multiplied)
+        const int halves = tl.halves, nfull = halves >> 1;
+        v16f acc[4][2];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+        // row fragments of this wave that hold rows of the tile
+        int live = (tl.m_valid - wm * 128 + 31) >> 5;
+        live = live < 0 || wn * 64 >= tl.n_valid ? 0 : live;
+
+        auto read_a = [&](uint8_t* st, auto i_tag, auto ks_tag) __attribute__((always_inline)) {
+            constexpr int i = decltype(i_tag)::value, ks = decltype(ks_tag)::value;
+            if constexpr (!A_T) return *(const v8bf*)(st + (a_c ^ (32 * ks)) + i * 4096);
+            else return bf16_read_trans(st + lane_t + 16 * ((16 * wm + 4 * i + t_col16) ^ (tj << 2)), ks);
+        };
+        auto read_b = [&](uint8_t* st, auto j_tag, auto ks_tag) __attribute__((always_inline)) {
+            constexpr int j = decltype(j_tag)::value, ks = decltype(ks_tag)::value;
+            if constexpr (!B_T) return *(const v8bf*)(st + (b_c ^ (32 * ks)) + j * 4096);
+            else return bf16_read_trans(st + TL_HALF + lane_t + 16 * ((8 * wn + 4 * j + t_col16) ^ (tj << 2)), ks);
+        };
+
+        // One MFMA step (16 elements) multiplies while the next one's fragments are read; every read and request sits
+        // between two MFMAs (pinned).  The slot's barrier stands one MFMA into its last step: by then every wave holds
+        // all its fragments of the slot, so the stage is free for the slot after next, whose requests are spread over
+        // the rest of this step and the next one.  With two waves per SIMD one's barrier and waits run under the other's MFMAs.
+        auto run = [&](auto live_tag) __attribute__((always_inline)) {
+            constexpr int L = decltype(live_tag)::value;
+            constexpr int NM = 2 * L, NR = L + 2, NB = 1;             // MFMAs, reads per step; MFMAs in front of the barrier
+            constexpr int Q = (NM - NB) + NM;                         // gaps the requests are spread over
+            constexpr int E3 = (NM - NB) * TL_REQ / Q;                // of them behind the barrier of the slot
+            In in = in_begin(tl, 1);
+            bf_static_for<0, E3>([&](auto e) { request(e, in, tl); });
+            bf_wait_vm<E3>();
+            __syncthreads();
+            v8bf fa[2][L], fb[2][2];
+            auto read = [&](auto x_tag, auto ks_tag, uint8_t* st) __attribute__((always_inline)) {
+                constexpr int x = decltype(x_tag)::value, ks = decltype(ks_tag)::value;
+                if constexpr (x == 0) fb[ks & 1][0] = read_b(st, std::integral_constant<int, 0>{}, ks_tag);
+                else if constexpr (x <= L) fa[ks & 1][x - 1] = read_a(st, std::integral_constant<int, x - 1>{}, ks_tag);
+                else fb[ks & 1][1] = read_b(st, std::integral_constant<int, 1>{}, ks_tag);
+            };
+            auto multiply = [&](auto m_tag, auto ks_tag) __attribute__((always_inline)) {
+                constexpr int m = decltype(m_tag)::value, ks = decltype(ks_tag)::value, j = m / L, i = m % L;
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[ks & 1][j], fa[ks & 1][i], acc[i][j], 0, 0, 0);
+            };
+            bf_static_for<0, NR>([&](auto x) { read(x, std::integral_constant<int, 0>{}, smem); });
+            for (int s = 0; s < nfull; ++s) {
+                uint8_t* cur = smem + (s & 1) * TL_STAGE;
+                uint8_t* nxt = smem + ((s & 1) ^ 1) * TL_STAGE;
+                bf_static_for<0, 3>([&](auto ks_tag) {
+                    constexpr int ks = decltype(ks_tag)::value;
+                    bf_static_for<0, NM>([&](auto m_tag) {
+                        constexpr int m = decltype(m_tag)::value;
+                        multiply(m_tag, ks_tag);
+                        bf_static_for<(m * NR + NM - 1) / NM, ((m + 1) * NR + NM - 1) / NM>([&](auto x) { read(x, std::integral_constant<int, ks + 1>{}, cur); });
+                        if constexpr (ks < 1) {
+                            constexpr int q = (NM - NB) + ks * NM + m;
+                            bf_static_for<q * TL_REQ / Q, (q + 1) * TL_REQ / Q>([&](auto e) { request(e, in, tl); });
+                        }
+                        if constexpr (ks == 1 && m == 1) ask_l2(tl, s + TL_AHEAD);
+                        __builtin_amdgcn_sched_barrier(0);
+                    });
+                });
+                bf_static_for<0, NB>([&](auto m_tag) { multiply(m_tag, std::integral_constant<int, 3>{}); });
+                in = in_begin(tl, s + 2);
+                bf_wait_vm<1>();        // slot s + 1 has landed (the L2 request may still be on its way)
+                __syncthreads();        // ... for every wave, and every wave holds its fragments of slot s
+                __builtin_amdgcn_sched_barrier(0);
+                bf_static_for<NB, NM>([&](auto m_tag) {
+                    constexpr int m = decltype(m_tag)::value, q = m - NB;
+                    multiply(m_tag, std::integral_constant<int, 3>{});
+                    bf_static_for<(q * NR + NM - NB - 1) / (NM - NB), ((q + 1) * NR + NM - NB - 1) / (NM - NB)>([&](auto x) { read(x, std::integral_constant<int, 0>{}, nxt); });
+                    bf_static_for<q * TL_REQ / Q, (q + 1) * TL_REQ / Q>([&](auto e) { request(e, in, tl); });
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+            }
+            if (halves & 1) {           // the last slot's first half
+                uint8_t* cur = smem + (nfull & 1) * TL_STAGE;
+                bf_static_for<0, NR>([&](auto x) { read(x, std::integral_constant<int, 1>{}, cur); });
+                bf_static_for<0, 2>([&](auto ks_tag) { bf_static_for<0, NM>([&](auto m_tag) { multiply(m_tag, ks_tag); }); });
+            }
+        };
+        if (halves > 0) {
+            if (live > 2) run(std::integral_constant<int, 4>{});
+            else if (live > 0) run(std::integral_constant<int, 2>{});
+            else {
+                // no row or column of the tile is this wave's: it only keeps its share of the requests going
+                In in = in_begin(tl, 1);
+                bf_static_for<0, TL_REQ>([&](auto e) { request(e, in, tl); });
+                bf_wait_vm<TL_REQ>();
+                __syncthreads();
+                for (int s = 0; s < nfull; ++s) {
+                    ask_l2(tl, s + TL_AHEAD);
+                    bf_wait_vm<1>();
+                    __syncthreads();
+                    in = in_begin(tl, s + 2);
+                    bf_static_for<0, TL_REQ>([&](auto e) { request(e, in, tl); });
+                }
+            }
+        }
+        bf_wait_vm<0>();
+        __syncthreads();         // every wave is done with the stages
+
+        // the next tile's first slot goes into stage 0 while this tile's output leaves through stage 1
+        const int grp = tl.grp, m_valid = tl.m_valid, n_valid = tl.n_valid;
+        const int64_t n0 = tl.n0, c_row0 = tl.c_row0;
+        tile_id += nwg;
+        const bool more = tile_id < total_tiles;
+        if (more) {
+            tl = setup(tile_id);
+            first_slot(tl);
+        }
+
+        // lane (lr, g) of fragment (i, j) holds row 32 i + lr, columns 32 j + 8 q + 4 g .. + 3 in registers 4 q .. 4 q + 3
+        if (ACCUM) {
+            float* c = (float*)p.c + ((int64_t)grp * p.m + c_row0) * p.n + n0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int row = wm * 128 + 32 * i + lr;
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const int col = wn * 64 + 32 * j + 8 * q + 4 * g;
+                        if (row < m_valid && col < n_valid) {      // n_out is a multiple of 8: a quad is in or out as a whole
+                            v4f* dst = (v4f*)(c + (int64_t)row * p.n + col);
+                            v4f o = *dst;
+                            o[0] += acc[i][j][4 * q]; o[1] += acc[i][j][4 * q + 1]; o[2] += acc[i][j][4 * q + 2]; o[3] += acc[i][j][4 * q + 3];
+                            *dst = o;
+                        }
+                    }
+            }
+        } else {
+            uint16_t* c = (uint16_t*)p.c + ((WGRAD ? (int64_t)grp * p.m : 0) + c_row0) * p.n + n0;
+            // in two passes of 128 rows of 512 bytes, 16-byte pieces XOR row % 32; every wave stores whole rows
+            uint8_t* out = smem + TL_STAGE;
+            int to = t;
+            asm("" : "+v"(to));          // the store addresses are formed here, not kept in registers across the main loop
+            const int col = (to & 31) * 8, row0 = to >> 5;
+            uint16_t* cl = c + (int64_t)row0 * p.n + col;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                if (h) __syncthreads();
+                if (wm == h) {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int j = 0; j < 2; ++j)
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) {
+                                const v4bf o = {(__bf16)acc[i][j][4 * q], (__bf16)acc[i][j][4 * q + 1], (__bf16)acc[i][j][4 * q + 2], (__bf16)acc[i][j][4 * q + 3]};
+                                *(v4bf*)(out + (32 * i + lr) * 512 + 16 * ((8 * wn + 4 * j + q) ^ lr) + 8 * g) = o;
+                            }
+                }
+                __syncthreads();
+                uint4 v[8];
+#pragma unroll
+                for (int x = 0; x < 8; ++x) {
+                    const int row = x * 16 + row0;
+                    v[x] = *(const uint4*)(out + row * 512 + 16 * ((to & 31) ^ (row & 31)));
+                }
+#pragma unroll
+                for (int x = 0; x < 8; ++x) {
+                    const int row = h * 128 + x * 16;
+                    if (row + row0 < m_valid && col < n_valid) *(uint4*)(cl + (int64_t)row * p.n) = v[x];
+                }
+            }
+        }
+        if (!more) break;
+        __syncthreads();         // every wave has left the staging area: the next tile's requests may overwrite it
+    }
+}
+
 static int bf16_num_cus(int dev) {
     static std::atomic<int> cached[64];
     int v = cached[dev & 63].load(std::memory_order_relaxed);
@@ -487,14 +770,17 @@ static int bf16_num_cus(int dev) {
     return pr.multiProcessorCount;
 }
 
-template <int BM, int NST, bool A_T, bool B_T, bool WGRAD, bool ACCUM>
+template <int BM, bool A_T, bool B_T, bool WGRAD, bool ACCUM>
 static int launch_bf16(const Bf16Args& a, int64_t max_tiles, hipStream_t st) {
-    constexpr int lds = bf16_lds_bytes(BM, NST);
+    constexpr bool TALL = BM == 256;
+    constexpr int lds = TALL ? tall_lds_bytes() : bf16_lds_bytes();
     if (!device_is_gfx950()) return MXL_ENODEV;
     static std::atomic<bool> attr_set[64];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return MXL_ELAUNCH;
-    auto kern = bf16_gemm_kernel<BM, NST, A_T, B_T, WGRAD, ACCUM>;
+    void (*kern)(Bf16Args) = nullptr;
+    if constexpr (TALL) kern = bf16_gemm_tall_kernel<A_T, B_T, WGRAD, ACCUM>;
+    else kern = bf16_gemm_kernel<A_T, B_T, WGRAD, ACCUM>;
     if (!attr_set[dev & 63].load(std::memory_order_acquire)) {
         if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess) return MXL_ELAUNCH;
         attr_set[dev & 63].store(true, std::memory_order_release);
@@ -506,16 +792,16 @@ static int launch_bf16(const Bf16Args& a, int64_t max_tiles, hipStream_t st) {
     grid = grid / 8 * 8;
     if (grid < 8) grid = 8;
     if ((max_tiles + 7) / 8 * 8 < grid) grid = (max_tiles + 7) / 8 * 8;
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(BF_THREADS), lds, st, a);
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(TALL ? TL_THREADS : BF_THREADS), lds, st, a);
     return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;
 }
 
 // Tile height of a launch: the caller's choice (MXL_BF_TILE_128 / MXL_BF_TILE_256), else from the average number of
-// rows per group -- the counts live on the device, the average is all the host knows.  Measured: forward / dgrad
-// tiles are cut from a group's rows, and 256-row tiles win from a few hundred rows per group on (512 rows: +7 %, 4096:
-// +18-24 %; below, most of a group's last tile is padding).  The weight gradient reads both operands through the
-// transposing LDS reads (twice the LDS instructions per MFMA): two workgroups per CU hide that better than one, and the
-// 128-row tile wins at every shape tried (+2 % at 4096 rows per group, +50 % at 512), so it is the default there.
+// rows per group -- the counts live on the device, the average is all the host knows.  Forward / dgrad tiles are cut from
+// a group's rows, and 256-row tiles win from about 256 rows per group on (32 groups, [4096, 7168], forward + dgrad with
+// 256-row against 128-row tiles: 1024 rows 3.42 against 4.16 ms, 256 rows 1.49 against 1.55, 128 rows 1.23 against 1.16).
+// The weight gradient's are cut from the output: 256 rows are as fast or faster at every length (1024 rows 1.71 against
+// 1.94 ms, 256 rows 0.72 against 0.78, 64 rows 0.43 against 0.44).
 static bool bf16_tall_tiles(uint32_t flags, int64_t rows_per_group, int64_t threshold) {
     if (flags & MXL_BF_TILE_256) return true;
     if (flags & MXL_BF_TILE_128) return false;
@@ -542,8 +828,8 @@ extern "C" int mxl_grouped_gemm_bf16(const void* a_bf16, const void* b_bf16, voi
     const int64_t max_tiles = (total_m / (tall ? 256 : 128) + num_groups) * ((n + BF_BN - 1) / BF_BN);
     hipStream_t st = (hipStream_t)stream;
     if (flags & MXL_BF_B_KN)
-        return tall ? launch_bf16<256, 4, false, true, false, false>(a, max_tiles, st) : launch_bf16<128, 2, false, true, false, false>(a, max_tiles, st);
-    return tall ? launch_bf16<256, 4, false, false, false, false>(a, max_tiles, st) : launch_bf16<128, 2, false, false, false, false>(a, max_tiles, st);
+        return tall ? launch_bf16<256, false, true, false, false>(a, max_tiles, st) : launch_bf16<128, false, true, false, false>(a, max_tiles, st);
+    return tall ? launch_bf16<256, false, false, false, false>(a, max_tiles, st) : launch_bf16<128, false, false, false, false>(a, max_tiles, st);
 }
 
 extern "C" int mxl_grouped_gemm_bf16_wgrad(const void* p_bf16, const void* q_bf16, void* c, const int64_t* group_lens,
@@ -559,11 +845,12 @@ extern "C" int mxl_grouped_gemm_bf16_wgrad(const void* p_bf16, const void* q_bf1
     if (total_m * m_out * 2 >= ((int64_t)1 << 32) || total_m * n_out * 2 >= ((int64_t)1 << 32)) return MXL_EINVAL;
     Bf16Args a{(const uint8_t*)p_bf16, (const uint8_t*)q_bf16, c, group_lens, num_groups, total_m, m_out, n_out, 0};
     // the tiles are cut from the [m_out, n_out] matrix of every group; the contraction runs over the group's tokens
-    const bool tall = bf16_tall_tiles(flags, total_m / num_groups, INT64_MAX);
+    // (the last K slot may reach 63 tokens past the operand's end, where 32-bit offsets must not wrap around)
+    const bool tall = bf16_tall_tiles(flags, total_m / num_groups, 0) && (total_m + 64) * (m_out > n_out ? m_out : n_out) * 2 < ((int64_t)1 << 32);
     const int bm = tall ? 256 : 128;
     const int64_t max_tiles = (int64_t)num_groups * ((m_out + bm - 1) / bm) * ((n_out + BF_BN - 1) / BF_BN);
     hipStream_t st = (hipStream_t)stream;
     if (flags & MXL_BF_ACCUM_F32)
-        return tall ? launch_bf16<256, 4, true, true, true, true>(a, max_tiles, st) : launch_bf16<128, 2, true, true, true, true>(a, max_tiles, st);
-    return tall ? launch_bf16<256, 4, true, true, true, false>(a, max_tiles, st) : launch_bf16<128, 2, true, true, true, false>(a, max_tiles, st);
+        return tall ? launch_bf16<256, true, true, true, true>(a, max_tiles, st) : launch_bf16<128, true, true, true, true>(a, max_tiles, st);
+    return tall ? launch_bf16<256, true, true, true, false>(a, max_tiles, st) : launch_bf16<128, true, true, true, false>(a, max_tiles, st);
 }
