@@ -1314,9 +1314,10 @@ static bool tile_flag_ok(uint32_t flags) {
 // FP8 contraction (E2M1 x E2M1: all of them about 0.7 of it): 64 x 64 6.5, 64 x 128 9.7, 128 x 128 14.2, the ring kernel's
 // 256 x 256 53 -- per flop the ring kernel is the cheapest (1 : 0.93 : 0.69 : 0.51), but it needs 256 tiles to occupy the
 // chip, and its launches cost whole rounds of 256.  A dense launch takes the tile with the least ceil(tiles / 256) * cost.
-// Only the first two rounds are priced as whole ones, in backward GEMMs only the first: there the input and the weight
-// gradient run side by side and fill each other's last round ([4096, 14336] x [4096, 14336] tensor-wise, 3.5 rounds each
-// in the backward: 0.80 ms on ring tiles, 0.94 on 128 x 128 ones).
+// Only the first two rounds are priced as whole ones: from the third on a partly filled round runs at a higher clock, and at
+// the board's power limit the small tiles' LDS reads cost what the empty CUs would ([4096, 14336] x [4096, 14336]
+// tensor-wise, 3.5 rounds each in the backward, whole linear 699 us on ring tiles, 746 on 128 x 128 ones; 1.08 rounds, the
+// weight gradient of 1999 tokens, 5760 x 2880: 57 and 41 us; 1.5 rounds, 3333 tokens, 3072 x 8192: 96 and 76).
 //   [256, 4096] x [4096, 4096]: ring 41.2 us, 128 13.2, 64 x 128 10.4, 64 x 64 8.9.   [1024, ...]: 42.4, 18.4, 22.2, 27.6
 //   [1999, 2880] x [5760, 2880]: 39.2, 34.0, 45.7, 54.4.   [4096, 4096] x [4096, 4096]: 56.3, 60.1, 80.6, 106
 // A grouped launch does not know its tile counts (they are on the device): a group's last row tile is taken as half full.
@@ -1354,8 +1355,7 @@ template <int MODE> static int tile_choice(const GemmArgs& a, bool e2m1_weights,
     }
     auto cost = [&](int64_t tm, int64_t tn, double c) { return (double)cdiv(tiles(tm, tn), 256) * c; };
     int best = TILE_RING;
-    const bool whole_rounds = ring_tiles <= 256 || (MODE == MODE_FWD && !bt && ring_tiles <= 512);
-    double least = whole_rounds ? cost(256, 256, 53.0) : ring_tiles / 256.0 * 53.0;
+    double least = ring_tiles <= 512 ? cost(256, 256, 53.0) : ring_tiles / 256.0 * 53.0;
     auto consider = [&](int tile, double c) {
         if (c < least) least = c, best = tile;
     };
