@@ -1444,18 +1444,32 @@ static int dispatch_wgrad_accum_ring(int afmt, int bfmt, const GemmArgs& a, int6
     return MXL_EINVAL;
 }
 
+// an input gradient on small tiles: put off into `hold` where a launch with the weight gradient exists
+static int hold_or_launch(bool bt, int afmt, int bfmt, const GemmArgs& a, int tile, HeldGemm* hold, hipStream_t st) {
+    HeldGemm h;
+    h.held = true;
+    h.bt = bt;
+    h.afmt = afmt;
+    h.bfmt = bfmt;
+    h.tile = tile;
+    h.args = a;
+    if (!hold || !gemm_pair_takes(h)) return h.flush(st);
+    *hold = h;
+    return MXL_OK;
+}
+
 // forward / dgrad on the row-wise codes of the transposed weight (MXL_GF_B_TRANSPOSED): E4M3 weights with E4M3 or E5M2
 // rows, or E2M1 weights with E2M1 rows (128-element steps)
-static int dispatch_gemm_ring_bt(int afmt, int bfmt, const GemmArgs& a, int64_t max_tiles, hipStream_t st, uint32_t flags) {
+static int dispatch_gemm_ring_bt(int afmt, int bfmt, const GemmArgs& a, int64_t max_tiles, hipStream_t st, uint32_t flags, HeldGemm* hold) {
     if (a.num_groups > RING_MAX_GROUPS) return MXL_EINVAL;
     const int tile = tile_choice<MODE_FWD>(a, false, true, flags);
     if (bfmt == MXL_FMT_E2M1) {
         if (afmt != MXL_FMT_E2M1 || a.alpha_a != nullptr) return MXL_EINVAL;
-        if (tile != TILE_RING) return gemm_tile_bt(afmt, bfmt, a, tile, st);
+        if (tile != TILE_RING) return hold_or_launch(true, afmt, bfmt, a, tile, hold, st);
         return launch_gemm_ring<MXL_FMT_E2M1, MXL_FMT_E2M1, MODE_FWD, false, false, true>(a, max_tiles, st);
     }
     if (bfmt != MXL_FMT_E4M3 || (afmt != MXL_FMT_E4M3 && (afmt != MXL_FMT_E5M2 || a.alpha_a == nullptr))) return MXL_EINVAL;
-    if (tile != TILE_RING) return gemm_tile_bt(afmt, bfmt, a, tile, st);
+    if (tile != TILE_RING) return hold_or_launch(true, afmt, bfmt, a, tile, hold, st);
     if (a.alpha_a != nullptr) {
         if (afmt == MXL_FMT_E5M2) return launch_gemm_ring<MXL_FMT_E5M2, MXL_FMT_E4M3, MODE_FWD, true, false, true>(a, max_tiles, st);
         return launch_gemm_ring<MXL_FMT_E4M3, MXL_FMT_E4M3, MODE_FWD, true, false, true>(a, max_tiles, st);
@@ -1467,7 +1481,7 @@ static int dispatch_gemm_ring_bt(int afmt, int bfmt, const GemmArgs& a, int64_t 
 // layout: 0 row-major codes, 1 K-chunk-major codes, 2 K-step-major codes and scales
 template <int MODE>
 static int dispatch_gemm(int afmt, int bfmt, const GemmArgs& a, int64_t max_tiles, int layout, int64_t a_rows, int64_t b_rows,
-                         hipStream_t st, bool accum = false, uint32_t flags = 0) {
+                         hipStream_t st, bool accum = false, uint32_t flags = 0, HeldGemm* hold = nullptr) {
     const bool kchunk = layout == 1;
     if (layout == 2) {
         if ((accum && MODE != MODE_WGRAD) || !ring_serves<MODE>(afmt, bfmt, a)) return MXL_EINVAL;
@@ -1477,7 +1491,13 @@ static int dispatch_gemm(int afmt, int bfmt, const GemmArgs& a, int64_t max_tile
         if ((MODE == MODE_WGRAD ? (int64_t)a.num_groups * a.m : a.total_m) >= ((int64_t)1 << 31)) return MXL_EINVAL;
         if (accum) return dispatch_wgrad_accum_ring(afmt, bfmt, a, max_tiles, st);
         const int tile = tile_choice<MODE>(a, bfmt == MXL_FMT_E2M1 && afmt != MXL_FMT_E2M1, false, flags);
-        if (tile != TILE_RING) return MODE == MODE_FWD ? gemm_tile_fwd(afmt, bfmt, a, tile, st) : gemm_tile_wgrad(afmt, bfmt, a, tile, st);
+        if (tile != TILE_RING && MODE == MODE_FWD) return hold_or_launch(false, afmt, bfmt, a, tile, hold, st);
+        // the weight gradient of what is held: the same rows' format, and the columns' is the weight's
+        if (tile != TILE_RING && hold && hold->held && hold->afmt == afmt && hold->bfmt == bfmt) {
+            hold->held = false;
+            return gemm_pair(*hold, a, st);
+        }
+        if (tile != TILE_RING) return gemm_tile_wgrad(afmt, bfmt, a, tile, st);
         return dispatch_gemm_ring<MODE>(afmt, bfmt, a, max_tiles, st);
     }
     if (accum) {
@@ -1508,7 +1528,7 @@ __global__ __launch_bounds__(256) void zero_fill_kernel(uint32_t* dst, int64_t w
 
 static int grouped_gemm_nt(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes, const void* b_scales,
                            int b_fmt, void* c_bf16, const int64_t* group_lens, int num_groups, int64_t total_m, int64_t n,
-                           int64_t k, const float* alpha_a, const float* alpha_b, uint32_t flags, void* stream) {
+                           int64_t k, const float* alpha_a, const float* alpha_b, uint32_t flags, void* stream, HeldGemm* hold = nullptr) {
     if (flags & ~(uint32_t)(MXL_GF_KCHUNK | MXL_GF_KSTEP | MXL_GF_B_TRANSPOSED | MXL_GF_B_SHUFFLED | MXL_GF_TILE_MASK)) return MXL_EINVAL;
     if (!tile_flag_ok(flags)) return MXL_EINVAL;
     if ((flags & MXL_GF_KCHUNK) && (flags & MXL_GF_KSTEP)) return MXL_EINVAL;
@@ -1545,10 +1565,10 @@ static int grouped_gemm_nt(const void* a_codes, const void* a_scales, int a_fmt,
         const int64_t n_ld = (n + 127) / 128 * 128;
         if (total_m * k >= ((int64_t)1 << 32) || (int64_t)num_groups * k * n_ld >= ((int64_t)1 << 32) || total_m >= ((int64_t)1 << 31))
             return MXL_EINVAL;
-        return dispatch_gemm_ring_bt(a_fmt, b_fmt, a, max_tiles, (hipStream_t)stream, flags);
+        return dispatch_gemm_ring_bt(a_fmt, b_fmt, a, max_tiles, (hipStream_t)stream, flags, hold);
     }
     return dispatch_gemm<MODE_FWD>(a_fmt, b_fmt, a, max_tiles, (flags & MXL_GF_KSTEP) ? 2 : (flags & MXL_GF_KCHUNK) ? 1 : 0, total_m,
-                                   (int64_t)num_groups * n, (hipStream_t)stream, false, flags);
+                                   (int64_t)num_groups * n, (hipStream_t)stream, false, flags, hold);
 }
 
 extern "C" int mxl_grouped_gemm_nt_ex(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes,
@@ -1583,7 +1603,7 @@ extern "C" int mxl_gemm_nt(const void* a_codes, const void* a_scales, int a_fmt,
 static int grouped_gemm_wgrad(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes,
                               const void* b_scales, int b_fmt, void* c_bf16, const int64_t* group_lens, int num_groups,
                               int64_t total_m, int64_t n, int64_t k, const float* alpha_a, const float* alpha_b,
-                              uint32_t flags, void* stream) {
+                              uint32_t flags, void* stream, HeldGemm* hold = nullptr) {
     if (flags & ~(uint32_t)(MXL_GF_KCHUNK | MXL_GF_KSTEP | MXL_GF_ACCUM_F32 | MXL_GF_TILE_MASK)) return MXL_EINVAL;
     if (!tile_flag_ok(flags)) return MXL_EINVAL;
     if ((flags & MXL_GF_KCHUNK) && (flags & MXL_GF_KSTEP)) return MXL_EINVAL;
@@ -1630,8 +1650,23 @@ static int grouped_gemm_wgrad(const void* a_codes, const void* a_scales, int a_f
     a.alpha_b = alpha_b;
     const int64_t max_tiles = (int64_t)G * ((n + BM - 1) / BM) * ((k + BN - 1) / BN);
     return dispatch_gemm<MODE_WGRAD>(a_fmt, b_fmt, a, max_tiles, (flags & MXL_GF_KSTEP) ? 2 : (flags & MXL_GF_KCHUNK) ? 1 : 0, n, k,
-                                     (hipStream_t)stream, accum, flags);
+                                     (hipStream_t)stream, accum, flags, hold);
 }
+
+namespace mxl {
+int gemm_nt_held(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes, const void* b_scales, int b_fmt, void* c,
+                 const int64_t* group_lens, int num_groups, int64_t total_m, int64_t n, int64_t k, const float* alpha_a,
+                 const float* alpha_b, uint32_t flags, HeldGemm* hold, void* stream) {
+    return grouped_gemm_nt(a_codes, a_scales, a_fmt, b_codes, b_scales, b_fmt, c, group_lens, num_groups, total_m, n, k, alpha_a, alpha_b, flags,
+                           stream, hold);
+}
+int gemm_wgrad_held(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes, const void* b_scales, int b_fmt, void* c,
+                    const int64_t* group_lens, int num_groups, int64_t total_m, int64_t n, int64_t k, const float* alpha_a,
+                    const float* alpha_b, uint32_t flags, HeldGemm* hold, void* stream) {
+    return grouped_gemm_wgrad(a_codes, a_scales, a_fmt, b_codes, b_scales, b_fmt, c, group_lens, num_groups, total_m, n, k, alpha_a, alpha_b,
+                              flags, stream, hold);
+}
+}  // namespace mxl
 
 extern "C" int mxl_grouped_gemm_wgrad_ex(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes,
                                          const void* b_scales, int b_fmt, void* c_bf16, const int64_t* group_lens,

@@ -4,7 +4,7 @@
 // allocation per buffer and a stream look-up per launch, they take 230 us for a pass whose kernels need 60.  Here the
 // caller allocates three buffers -- what the backward needs, and a scratch buffer per direction -- and makes one call per
 // direction; the layout of the buffers is arithmetic on the sizes and is worked out again in every call.
-#include "mx_device.h"
+#include "mx_gemm_tile.h"
 
 namespace {
 
@@ -207,28 +207,36 @@ extern "C" int mxl_linear_backward(const mxl_linear* p, int parts, const void* d
                                     rht ? (uint32_t)p->rht_signs : 0u, stream));
         }
     }
-    if ((parts & MXL_LINEAR_DX) && p->need_dx) {
+    // the two GEMMs: where both run on small tiles, in one launch
+    const bool dx_part = (parts & MXL_LINEAR_DX) && p->need_dx, dw_part = (parts & MXL_LINEAR_DW) && p->need_dw;
+    mxl::HeldGemm hold;
+    if (dx_part) {
         void* out = b.dxi ? b.dxi : dx;
         if (!out) return MXL_EINVAL;
         const uint32_t flags = MXL_GF_KSTEP | (p->dx_from_rows ? MXL_GF_B_TRANSPOSED : 0u);
         const void* bq = p->w_quantized ? wt : p->dx_from_rows ? sv.w_row.q : sv.w_col.q;
         const void* bs = p->w_quantized ? wt_scales : sv.w_col.s;
-        if (l.tensorwise())
-            MXL_TRY(mxl_grouped_gemm_nt_scaled(b.d_row.q, b.d_row.s, gf, bq, bs, wf, out, lens, batch, p->rows, p->k, l.n_ld, b.d_si, sv.w_si, flags, stream));
+        const bool tw = l.tensorwise();
+        if (tw && (!b.d_si || !sv.w_si)) return MXL_EINVAL;
+        MXL_TRY(mxl::gemm_nt_held(b.d_row.q, b.d_row.s, gf, bq, bs, wf, out, lens, batch, p->rows, p->k, l.n_ld, tw ? b.d_si : nullptr,
+                                  tw ? sv.w_si : nullptr, flags, dw_part ? &hold : nullptr, stream));
+    }
+    int rc = MXL_OK;
+    if (dw_part) {
+        const bool tw = l.tensorwise();
+        if (tw && (!b.d_si || !sv.x_si)) rc = MXL_EINVAL;
         else
-            MXL_TRY(mxl_grouped_gemm_nt_ex(b.d_row.q, b.d_row.s, gf, bq, bs, wf, out, lens, batch, p->rows, p->k, l.n_ld, flags, stream));
+            rc = mxl::gemm_wgrad_held(b.d_col.q, b.d_col.s, gf, sv.x_col.q, sv.x_col.s, (int)p->act_fmt, dw, lens, G, p->rows, p->n, p->k,
+                                      tw ? b.d_si : nullptr, tw ? sv.x_si : nullptr, MXL_GF_KSTEP | dw_flags, &hold, stream);
+    }
+    MXL_TRY(hold.flush((hipStream_t)stream));
+    MXL_TRY(rc);
+    if (dx_part) {
         if (p->input == MXL_LINEAR_RMSNORM)
             MXL_TRY(mxl_rmsnorm_bwd(b.dxi, x, aux0, sv.rstd, p->rows, p->k, dx, daux, b.norm_ws, b.norm_bytes, stream));
         else if (p->input != MXL_LINEAR_PLAIN)
             MXL_TRY(mxl_glu_probs_bwd(b.dxi, x, aux0, (int)p->probs_dtype, (const uint8_t*)aux1, p->rows, p->k,
                                       p->input == MXL_LINEAR_SILU ? MXL_ACT_SILU : MXL_ACT_GELU, dx, daux, stream));
-    }
-    if ((parts & MXL_LINEAR_DW) && p->need_dw) {
-        const uint32_t flags = MXL_GF_KSTEP | dw_flags;
-        if (l.tensorwise())
-            return mxl_grouped_gemm_wgrad_scaled(b.d_col.q, b.d_col.s, gf, sv.x_col.q, sv.x_col.s, (int)p->act_fmt, dw, lens, G, p->rows, p->n, p->k,
-                                                 b.d_si, sv.x_si, flags, stream);
-        return mxl_grouped_gemm_wgrad_ex(b.d_col.q, b.d_col.s, gf, sv.x_col.q, sv.x_col.s, (int)p->act_fmt, dw, lens, G, p->rows, p->n, p->k, flags, stream);
     }
     return MXL_OK;
 }
