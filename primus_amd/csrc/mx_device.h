@@ -173,26 +173,39 @@ __device__ __forceinline__ uint32_t sr_mix(uint32_t x) {
     x ^= x >> 16;
     return x;
 }
-__device__ __forceinline__ uint32_t sr_word(uint64_t counter, uint64_t seed, uint32_t stream) {
-    const uint32_t h = sr_mix((uint32_t)counter ^ (uint32_t)seed);
-    return sr_mix(h + (uint32_t)(counter >> 32) * 0x9E3779B9u + (uint32_t)(seed >> 32) + stream * 0x85EBCA6Bu);
+// The word of counter `key + i`, i < 4, key a multiple of 4: `low` = key's low word ^ the seed's, `high` = sr_high(), the
+// part that the four words of a key share.
+__device__ __forceinline__ uint32_t sr_high(uint64_t key, uint64_t seed, uint32_t stream) {
+    return (uint32_t)(key >> 32) * 0x9E3779B9u + (uint32_t)(seed >> 32) + stream * 0x85EBCA6Bu;
 }
-__device__ __forceinline__ uint32_t sr1_e2m1(float x, float inv, uint32_t rnd16) {
+__device__ __forceinline__ uint32_t sr_word(uint32_t low, uint32_t i, uint32_t high) { return sr_mix(sr_mix(low ^ i) + high); }
+// (The products of the counter and the shared part are worked out once: the random words are four 32-bit multiplications a pair, each the
+// time of four other instructions, and bound the kernel.  Quantising [4096, 14336] both ways with stochastic rounding and
+// the Hadamard transform: 90 -> 79 us, 46 without stochastic rounding.)
+// The magnitude without a branch: in units of 2^-23, w itself below 1 and its fp32 pattern (less that of 0.5) from 1 on.
+// The pattern is the smaller of the two from 1 on and the larger never below, so the one wanted is the median with 1.
+__device__ __forceinline__ uint32_t sr_mag_e2m1(float x, float inv, uint32_t rnd16) {
     const float w = fabsf(x) * inv;
-    const uint32_t sign = (__float_as_uint(x) >> 28) & 0x8u;
-    const uint32_t add = rnd16 << 6;
-    uint32_t mag;
-    if (w < 1.f) {
-        mag = ((uint32_t)(w * 8388608.f) + add) >> 22;
-    } else {
-        mag = ((__float_as_uint(w) + add) >> 22) - 252u;
-        mag = mag > 7u ? 7u : mag;
-    }
-    return sign | mag;
+    const int fixed = (int)(w * 8388608.f), line = (int)__float_as_uint(w) - 0x3F000000;
+    const int base = max(min(line, fixed), min(max(line, fixed), 1 << 23));
+    return (uint32_t)min(base + (int)(rnd16 << 6), 0x1FFFFFF) >> 22;
 }
-// two bf16 (packed) -> two nibbles in bits 7:0, element 0 (random bits 15:0) in bits 3:0
-__device__ __forceinline__ uint32_t sr2_e2m1(uint32_t pair, float inv, uint32_t rnd) {
-    return sr1_e2m1(bf16_lo(pair), inv, rnd & 0xFFFFu) | (sr1_e2m1(bf16_hi(pair), inv, rnd >> 16) << 4);
+// four packed bf16 pairs -> eight nibbles, element 0 (random bits 15:0 of the first word) in bits 3:0; the signs are
+// gathered for all eight at once.  key: the first pair's counter, a multiple of 4
+__device__ __forceinline__ uint32_t sr8_e2m1(uint32_t p0, uint32_t p1, uint32_t p2, uint32_t p3, float inv, uint64_t key,
+                                             uint64_t seed, uint32_t stream) {
+    const uint32_t p[4] = {p0, p1, p2, p3};
+    const uint32_t low = (uint32_t)key ^ (uint32_t)seed, high = sr_high(key, seed, stream);
+    uint32_t o = 0;
+#pragma unroll
+    for (int i = 3; i >= 0; --i) {
+        const uint32_t rnd = sr_word(low, (uint32_t)i, high);
+        o = (o << 4) | sr_mag_e2m1(bf16_hi(p[i]), inv, rnd >> 16);
+        o = (o << 4) | sr_mag_e2m1(bf16_lo(p[i]), inv, rnd & 0xFFFFu);
+    }
+    const uint32_t x = __builtin_amdgcn_perm(p1, p0, 0x07030501u), y = __builtin_amdgcn_perm(p3, p2, 0x07030501u);
+    const uint32_t even = __builtin_amdgcn_perm(y, x, 0x05040100u), odd = __builtin_amdgcn_perm(y, x, 0x07060302u);
+    return o | ((even >> 4) & 0x08080808u) | (odd & 0x80808080u);
 }
 
 // ---- gated activation of the expert MLP (shared by the activation kernels and the fused

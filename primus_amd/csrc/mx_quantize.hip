@@ -278,6 +278,8 @@ __global__ __launch_bounds__(QTHREADS) void mx_quant_kernel(QuantArgs a) {
 
     // ---- row-wise copy ----
     if (ROW) {
+        // (products of 64 bits once per lane: a multiplication costs four other instructions)
+        const uint64_t sr_row = SR ? (uint64_t)(src_row0 + 32 * w + 8 * rg) * (uint64_t)(a.cols >> 1) + (uint64_t)(col >> 1) : 0;
         uint2 o_even = make_uint2(0u, 0u);   // FP8: codes of the even row of a row pair, kept until its partner is done
 #pragma unroll
         for (int it = 0; it < 8; ++it) {
@@ -321,11 +323,8 @@ __global__ __launch_bounds__(QTHREADS) void mx_quant_kernel(QuantArgs a) {
                 uint32_t o;
                 if (SR && byte != 255u) {
                     const float inv = inv_scale(byte);
-                    const uint64_t key = (uint64_t)(src_row0 + r) * (uint64_t)(a.cols >> 1) + (uint64_t)(col >> 1);
-                    o = sr2_e2m1(d[it].x, inv, sr_word(key, a.sr_seed, 0)) |
-                        (sr2_e2m1(d[it].y, inv, sr_word(key + 1, a.sr_seed, 0)) << 8) |
-                        (sr2_e2m1(d[it].z, inv, sr_word(key + 2, a.sr_seed, 0)) << 16) |
-                        (sr2_e2m1(d[it].w, inv, sr_word(key + 3, a.sr_seed, 0)) << 24);
+                    const uint64_t key = sr_row + (uint64_t)it * (uint64_t)(a.cols >> 1);
+                    o = sr8_e2m1(d[it].x, d[it].y, d[it].z, d[it].w, inv, key, a.sr_seed, 0);
                 } else if (byte != 255u) {
                     const float sc = fwd_scale(byte);
                     o = cvt2_e2m1(d[it].x, sc) | (cvt2_e2m1(d[it].y, sc) << 8) | (cvt2_e2m1(d[it].z, sc) << 16) |
@@ -396,6 +395,8 @@ __global__ __launch_bounds__(QTHREADS) void mx_quant_kernel(QuantArgs a) {
 
     // ---- column-wise (transposed) copy into the LDS tile ----
     if (COL) {
+        // position of the lane's 8 rows along the padded token axis, in its first column
+        const uint64_t sr_col = SR ? (uint64_t)col * (uint64_t)(a.W >> 1) + (((uint64_t)pt * QT + (uint64_t)(32 * w + 8 * rg)) >> 1) : 0;
         const uint32_t* dw = (const uint32_t*)d;  // dw[it*4 + j]: columns 2j, 2j+1 of row `it`
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -428,12 +429,8 @@ __global__ __launch_bounds__(QTHREADS) void mx_quant_kernel(QuantArgs a) {
                 uint32_t o;
                 if (SR && byte != 255u) {
                     const float inv = inv_scale(byte);
-                    const uint64_t pos = (uint64_t)pt * QT + (uint64_t)(32 * w + 8 * rg);   // along the padded token axis
-                    const uint64_t key = (uint64_t)(col0 + c) * (uint64_t)(a.W >> 1) + (pos >> 1);
-                    o = sr2_e2m1(pr[0], inv, sr_word(key, a.sr_seed, 1)) |
-                        (sr2_e2m1(pr[1], inv, sr_word(key + 1, a.sr_seed, 1)) << 8) |
-                        (sr2_e2m1(pr[2], inv, sr_word(key + 2, a.sr_seed, 1)) << 16) |
-                        (sr2_e2m1(pr[3], inv, sr_word(key + 3, a.sr_seed, 1)) << 24);
+                    const uint64_t key = sr_col + (uint64_t)j * (uint64_t)(a.W >> 1);
+                    o = sr8_e2m1(pr[0], pr[1], pr[2], pr[3], inv, key, a.sr_seed, 1);
                 } else if (byte != 255u) {
                     const float sc = fwd_scale(byte);
                     o = cvt2_e2m1(pr[0], sc) | (cvt2_e2m1(pr[1], sc) << 8) | (cvt2_e2m1(pr[2], sc) << 16) |
