@@ -167,12 +167,32 @@ def _overlaps(plan) -> bool:
     return flops >= 1.5e12 and plan.rows <= 1024 * plan.groups
 
 
-def _two_calls(a, b, group_lens, cached: bool, norm_weight=None) -> bool:
+def _holds(q: QuantizedTensor, rows: int, ld: int, fmt: int, kc: int, device) -> bool:
+    """Whether a cached copy is ``[rows, ld]`` codes of ``fmt`` and their scales on ``device``, in layout ``kc`` without
+    gaps: all that the two calls, which are handed its pointers, take for granted about it."""
+    codes, scales = q.codes, q.scales
+    ld = K._round_up(ld, K.GEMM_K_ALIGN)
+    return (q.fmt == fmt and int(q.kchunk) == int(kc) and codes.device == device and scales.device == device
+            and codes.is_contiguous() and scales.is_contiguous()
+            and tuple(codes.shape) == K._code_shape(rows, ld, K._per_byte(fmt), kc)
+            and tuple(scales.shape) == K._scale_shape(rows, ld, kc))
+
+
+def _two_calls(a, b, group_lens, norm_weight=None, cache=None) -> bool:
     """Whether a linear on K-step-major operands can go through ``mxl_linear_forward`` / ``_backward``: on the GPU, in
-    sizes the kernels take (anything else raises on the launch-by-launch route), and nobody is watching the launches."""
+    sizes the kernels take (anything else raises on the launch-by-launch route), and nobody is watching the launches.
+    ``cache``: the transposed copy that goes with the cached copy ``b`` (None: not needed), the weight's format and the
+    layout; a copy that holds anything but what its logical shape and that format say is left to the launch-by-launch
+    route, whose wrappers look at the payload itself."""
     if K._launch_hook is not None or not a.is_cuda or b.shape[-1] % _lib.BLOCK or b.shape[-2] % _lib.BLOCK:
         return False
-    if not cached and not b.is_cuda:
+    if cache is not None:
+        b_t, fmt, kc = cache
+        n, k = b.shape[-2], b.shape[-1]
+        groups = 1 if group_lens is None else b.shape[0]
+        if not _holds(b, groups * n, k, fmt, kc, a.device) or (b_t is not None and not _holds(b_t, groups * k, n, fmt, kc, a.device)):
+            return False
+    elif not b.is_cuda:
         return False
     if norm_weight is not None:
         K._norm_args(a, norm_weight)
@@ -305,7 +325,8 @@ class _MXLinearFunction(torch.autograd.Function):
         cached = isinstance(b, QuantizedTensor)
         if cached:   # cached copies decide: the call uses the layout they are stored in
             kc = _cache_layout(b, b_t, kc, fp8, groups, fp4)
-        if kc in (K.LAYOUT_KSTEP, K.LAYOUT_KSTEP128) and a.shape[0] > 0 and _two_calls(a, b, group_lens, cached, norm_weight):
+        if kc in (K.LAYOUT_KSTEP, K.LAYOUT_KSTEP128) and a.shape[0] > 0 and _two_calls(
+                a, b, group_lens, norm_weight, (b_t if need_dgrad else None, w_fmt, kc) if cached else None):
             return _mx_forward(ctx, a, b, b_t, group_lens, act_fmt, w_fmt, scale_mode, probs, row_mask, activation, grad_sr, rht_signs,
                                norm_weight, norm_eps, accum, kc, need_dgrad, need_wgrad)
         ctx.plan = None
@@ -486,7 +507,7 @@ class _TWLinearFunction(torch.autograd.Function):
                 kc = 0
         else:
             kc = K.pick_layout(groups, b.shape[-2], b.shape[-1], a.shape[0], fp8=True)
-        if kc == K.LAYOUT_KSTEP and a.shape[0] > 0 and not isinstance(b, QuantizedTensor) and _two_calls(a, b, group_lens, False):
+        if kc == K.LAYOUT_KSTEP and a.shape[0] > 0 and not isinstance(b, QuantizedTensor) and _two_calls(a, b, group_lens):
             n, k = b.shape[-2], b.shape[-1]
             bt = need_dgrad and _dgrad_reads_rowwise and fwd_fmt == _lib.FMT_E4M3 and n % K.GEMM_K_ALIGN == 0 and k % K.GEMM_K_ALIGN == 0
             plan = K.linear_plan(a.shape[0], n, k, groups if grouped else 0, _lib.LINEAR_TENSORWISE, fwd_fmt, fwd_fmt, bwd_fmt, 0,
