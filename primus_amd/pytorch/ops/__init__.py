@@ -274,6 +274,8 @@ def _backward_in_parts(plan, dy, saved, group_lens, accum, need_dgrad, need_wgra
     if need_wgrad:
         target = accum[0] if accum is not None else None
         fused = _fusable(target)      # the GEMM's epilogue adds into the float32 buffer
+        if fused:
+            K._accum_target(target, w_shape, K.LAYOUT_KSTEP, dev)
     overlap = _wgrad_overlap and need_dgrad and need_wgrad and _overlaps(plan)
     if not overlap:
         if need_wgrad:
