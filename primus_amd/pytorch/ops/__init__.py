@@ -672,10 +672,12 @@ def _apply(fn, *args):
     """``fn.apply(*args)``, or its forward alone when nothing needs a gradient: no graph node, and no copies for a
     backward that cannot come (``requires_grad`` of a leaf says nothing under ``torch.no_grad``).  Inside a function
     transform or a forward-mode level ``apply`` is called all the same: it refuses what the operator has no rule for,
-    where the forward alone would drop the tangent."""
+    where the forward alone would drop the tangent.  So it is under ``torch.jit.trace``, which records the function as one
+    call; of the forward alone it would record the allocations and none of the launches."""
     if torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in args):
         return fn.apply(*args)
-    if torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0:
+    if (torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._get_tracing_state() is not None):
         return fn.apply(*args)
     return fn.forward(_NoGradContext(), *args, need_grad=False)
 
