@@ -324,18 +324,30 @@ class MXFP4LinearFunction(torch.autograd.Function):
         return (grad_input, grad_weight) + (None,) * 6
 
 
+def _plain_eager(*tensors) -> bool:
+    """Whether a call on these tensors may hand their addresses to native code behind torch's back: nothing is traced or
+    transformed, no dispatch mode looks on and no tensor is a stand-in (fake tensors) or a wrapper of others.
+    ``MXFP4LinearFunction`` with its custom ops serves those calls."""
+    if torch.compiler.is_compiling() or torch._C._are_functorch_transforms_active() or torch._C._len_torch_dispatch_stack() > 0:
+        return False
+    return all(type(t).__torch_dispatch__ is torch.Tensor.__torch_dispatch__ for t in tensors)
+
+
 def mxfp4_linear(input, weight, preshuffle: bool = False, backward_precision: str = "mxfp4",
                  use_gradient_sr: bool = False):
     """``MXFP4LinearFunction`` with the arguments the reference's parallel linears derive from their config
     (:476-511): ``backward_precision`` "mxfp4" or "fp8" (``mxfp4_backward_precision``; FP8 means E5M2 codes, one
-    scale per tensor), ``use_gradient_sr`` (``mxfp4_gradient_stochastic_rounding``).  Returns the output only."""
+    scale per tensor), ``use_gradient_sr`` (``mxfp4_gradient_stochastic_rounding``).  Returns the output only.
+
+    ``preshuffle`` chooses the byte order between the quantiser and the GEMM inside ``MXFP4LinearFunction``, which changes
+    no result; plain eager calls with the MXFP4 backward do not run on it and have one order."""
     if backward_precision not in ("mxfp4", "fp8"):
         raise ValueError("backward_precision must be 'mxfp4' or 'fp8'")
     fp8 = backward_precision == "fp8"
-    if not fp8 and not torch.compiler.is_compiling():
+    if not fp8 and _plain_eager(input, weight):
         # The operators' MXFP4 linear is the same arithmetic on the same codes (the pre-shuffled byte order changes no
         # result) in the layout the ring GEMM reads, without a transposed weight copy and without the custom ops, which
-        # exist for torch.compile.
+        # exist for torch.compile, function transforms and fake tensors.
         if input.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16:
             raise ValueError("MXFP4LinearFunction expects bfloat16 operands")
         out = ops.mxfp4_linear_2d(input.reshape(-1, input.shape[-1]).contiguous(), weight.contiguous(), use_gradient_sr, RHT_SIGNS)
