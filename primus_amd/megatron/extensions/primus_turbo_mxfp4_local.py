@@ -304,8 +304,8 @@ class MXFP4LinearFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, grad_output, *_):
-        if grad_output is None:
-            return (None,) * 8
+        if grad_output is None:     # a gradient of the other outputs only: the linear's own is zero
+            grad_output = torch.zeros((*ctx.orig_shape[:-1], ctx.n_out), dtype=ctx.out_dtype, device=ctx.saved_tensors[0].device)
         grad_2d = grad_output.contiguous().reshape(-1, grad_output.shape[-1])
         if grad_2d.dtype != torch.bfloat16:
             grad_2d = grad_2d.to(torch.bfloat16)

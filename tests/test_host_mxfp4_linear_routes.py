@@ -61,3 +61,14 @@ def test_a_dispatch_mode_sees_the_custom_ops(on_the_host, monkeypatch):
     monkeypatch.setattr(ops, "mxfp4_linear_2d", lambda *a: pytest.fail("not the custom ops"))
     with Mode():
         assert local.mxfp4_linear(*_operands()).unique().tolist() == [1.0]
+
+
+def test_a_gradient_of_another_output_only(on_the_host, monkeypatch):
+    """The FP8 mode hands out its kept operands; where only they have a gradient, the linear's own is zero."""
+    from primus_amd.pytorch.core.low_precision import ScalingGranularity, float8_e5m2
+
+    monkeypatch.setattr(local, "_fp8_tw_backward_op", lambda g, x, w, fmt: (g.sum() * x, g.sum() * w))
+    x, w = (t.requires_grad_() for t in _operands())
+    out = local.MXFP4LinearFunction.apply(x, w, False, True, float8_e5m2, ScalingGranularity.TENSORWISE.value, 0, False)
+    dx, dw = torch.autograd.grad(out[1].sum() + out[2].sum(), [x, w])
+    assert torch.equal(dx, torch.zeros_like(x)) and torch.equal(dw, torch.zeros_like(w))
