@@ -133,3 +133,30 @@ def test_accumulating_weight_gradient(gpu):
 
     want = _launch_by_launch(step)
     assert all(torch.equal(a, b) for a, b in zip(step(), want))
+
+
+@pytest.mark.parametrize("sr", [False, True])
+@pytest.mark.parametrize("shape,n", [((3, 100, 256), 192), ((71, 160), 96)])
+def test_local_mxfp4_linear_and_its_function(gpu, sr, shape, n):
+    """``mxfp4_linear`` in eager mode runs on the operators; output and both gradients have the bits of
+    ``MXFP4LinearFunction``, which serves everything else, in either byte order."""
+    from primus_amd.megatron.extensions.primus_turbo_mxfp4_local import MXFP4LinearFunction, mxfp4_linear
+    from primus_amd.pytorch import ops
+
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn(*shape, generator=g).bfloat16().to(gpu).requires_grad_()
+    w = (torch.randn(n, shape[-1], generator=g) * 0.05).bfloat16().to(gpu).requires_grad_()
+    dy = torch.randn(*shape[:-1], n, generator=g).bfloat16().to(gpu)
+
+    def step(linear):
+        ops.manual_sr_seed(23)
+        y = linear()
+        return (y,) + torch.autograd.grad(y, [x, w], dy)
+
+    try:
+        got = step(lambda: mxfp4_linear(x, w, use_gradient_sr=sr))
+        for pre in (False, True):
+            want = step(lambda: MXFP4LinearFunction.apply(x, w, pre, False, None, 0, 0, sr)[0])
+            assert all(torch.equal(a, b) for a, b in zip(got, want)), pre
+    finally:
+        ops.manual_sr_seed(None)
