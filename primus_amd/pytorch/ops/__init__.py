@@ -167,30 +167,30 @@ def _overlaps(plan) -> bool:
     return flops >= 1.5e12 and plan.rows <= 1024 * plan.groups
 
 
-def _holds(q: QuantizedTensor, rows: int, ld: int, fmt: int, kc: int, device) -> bool:
-    """Whether a cached copy is ``[rows, ld]`` codes of ``fmt`` and their scales on ``device``, in layout ``kc`` without
-    gaps: all that the two calls, which are handed its pointers, take for granted about it."""
+def _holds(q: QuantizedTensor, rows: int, ld: int, fmt: int, kc: int, device: int) -> bool:
+    """Whether a cached copy is ``[rows, ld]`` codes of ``fmt`` and their scales on GPU ``device``, in the K-step-major layout
+    ``kc`` without gaps: all that the two calls, which are handed its pointers, take for granted about it."""
     codes, scales = q.codes, q.scales
-    ld = K._round_up(ld, K.GEMM_K_ALIGN)
-    return (q.fmt == fmt and int(q.kchunk) == int(kc) and codes.device == device and scales.device == device
-            and codes.is_contiguous() and scales.is_contiguous()
-            and tuple(codes.shape) == K._code_shape(rows, ld, K._per_byte(fmt), kc)
-            and tuple(scales.shape) == K._scale_shape(rows, ld, kc))
+    step = K.KSTEP if kc == K.LAYOUT_KSTEP else K.KCHUNK
+    ld = (ld + K.GEMM_K_ALIGN - 1) // K.GEMM_K_ALIGN * K.GEMM_K_ALIGN
+    return (q.fmt == fmt and q.kchunk == kc
+            and codes.shape == (ld // step, rows, step // (2 if fmt == _lib.FMT_E2M1 else 1)) and codes.is_contiguous()
+            and scales.shape == ((ld + K.PANEL - 1) // K.PANEL, rows, 16) and scales.is_contiguous()
+            and codes.get_device() == device and scales.get_device() == device)
 
 
-def _two_calls(a, b, group_lens, norm_weight=None, cache=None) -> bool:
+def _two_calls(a, b, n, k, group_lens, norm_weight=None, cache=None) -> bool:
     """Whether a linear on K-step-major operands can go through ``mxl_linear_forward`` / ``_backward``: on the GPU, in
     sizes the kernels take (anything else raises on the launch-by-launch route), and nobody is watching the launches.
-    ``cache``: the transposed copy that goes with the cached copy ``b`` (None: not needed), the weight's format and the
-    layout; a copy that holds anything but what its logical shape and that format say is left to the launch-by-launch
-    route, whose wrappers look at the payload itself."""
-    if K._launch_hook is not None or not a.is_cuda or b.shape[-1] % _lib.BLOCK or b.shape[-2] % _lib.BLOCK:
+    ``cache``: the transposed copy that goes with the cached copy ``b`` (None: not needed), the weight's format, the
+    layout and the groups; a copy that holds anything but what its logical shape and that format say is left to the
+    launch-by-launch route, whose wrappers look at the payload itself."""
+    if K._launch_hook is not None or not a.is_cuda or k % _lib.BLOCK or n % _lib.BLOCK:
         return False
     if cache is not None:
-        b_t, fmt, kc = cache
-        n, k = b.shape[-2], b.shape[-1]
-        groups = 1 if group_lens is None else b.shape[0]
-        if not _holds(b, groups * n, k, fmt, kc, a.device) or (b_t is not None and not _holds(b_t, groups * k, n, fmt, kc, a.device)):
+        b_t, fmt, kc, groups = cache
+        device = a.get_device()
+        if not _holds(b, groups * n, k, fmt, kc, device) or (b_t is not None and not _holds(b_t, groups * k, n, fmt, kc, device)):
             return False
     elif not b.is_cuda:
         return False
@@ -200,7 +200,7 @@ def _two_calls(a, b, group_lens, norm_weight=None, cache=None) -> bool:
     return True
 
 
-def _mx_forward(ctx, a, b, b_t, group_lens, act_fmt, w_fmt, scale_mode, probs, row_mask, activation, grad_sr, rht_signs, norm_weight,
+def _mx_forward(ctx, a, b, w_shape, b_t, group_lens, act_fmt, w_fmt, scale_mode, probs, row_mask, activation, grad_sr, rht_signs, norm_weight,
                 norm_eps, accum, kc, need_dgrad, need_wgrad):
     """Forward of ``_MXLinearFunction`` on K-step-major operands: one call."""
     cached = isinstance(b, QuantizedTensor)
@@ -217,7 +217,7 @@ def _mx_forward(ctx, a, b, b_t, group_lens, act_fmt, w_fmt, scale_mode, probs, r
             if b_t.axis != -2:
                 raise ValueError("QuantizedTensorPair.data_t must be quantised along axis=-2")
             wt, wt_scales = _cached_codes(b_t, kc), _cached_scales(b_t, kc)
-    n, k = b.shape[-2], b.shape[-1]
+    n, k = w_shape[-2], w_shape[-1]
     # dgrad on the row-wise weight codes: see the launch-by-launch route below
     bt = (need_dgrad and not cached and _dgrad_reads_rowwise and act_fmt == w_fmt and n % K.GEMM_K_ALIGN == 0 and k % K.GEMM_K_ALIGN == 0)
     inp, pd, aux0, aux1 = _lib.LINEAR_PLAIN, 0, None, None
@@ -228,12 +228,12 @@ def _mx_forward(ctx, a, b, b_t, group_lens, act_fmt, w_fmt, scale_mode, probs, r
     elif norm_weight is not None:
         inp, aux0 = _lib.LINEAR_RMSNORM, norm_weight
     sr = bool(grad_sr) and act_fmt == _lib.FMT_E2M1
-    plan = K.linear_plan(a.shape[0], n, k, 0 if group_lens is None else b.shape[0], _lib.LINEAR_MX, act_fmt, w_fmt, act_fmt, scale_mode,
+    plan = K.linear_plan(a.shape[0], n, k, 0 if group_lens is None else w_shape[0], _lib.LINEAR_MX, act_fmt, w_fmt, act_fmt, scale_mode,
                          need_dgrad, need_wgrad, bt, cached, inp, pd, sr, rht_signs, norm_eps)
     y, saved = K.linear_forward_impl(plan, a, w, w_scales, group_lens, aux0, aux1)
     if need_dgrad or need_wgrad:
         ctx.plan, ctx.sr, ctx.accum = plan, sr, accum
-        ctx.needs = (need_dgrad, need_wgrad, tuple(b.shape))
+        ctx.needs = (need_dgrad, need_wgrad, tuple(w_shape))
         keep = need_dgrad and inp != _lib.LINEAR_PLAIN
         ctx.save_for_backward(saved, group_lens, wt, wt_scales, a if keep else None, aux0 if keep else None, aux1 if keep else None)
     return y
@@ -317,19 +317,20 @@ class _MXLinearFunction(torch.autograd.Function):
         grouped = group_lens is not None
         # Every operand of the three GEMMs is stored in one layout, K-chunk-major unless an operand is
         # too large for it (or the layout is switched off): same codes, same results, faster loads.
-        groups = b.shape[0] if grouped else 1
+        w_shape = b.shape
+        groups = w_shape[0] if grouped else 1
         # K-step-major operands (the ring kernel) whenever the activations are FP8: against FP8 weights in all three
         # GEMMs, against E2M1 weights in forward and dgrad (wgrad is FP8 x FP8 then)
         fp8 = act_fmt != _lib.FMT_E2M1
         # E2M1 x E2M1 runs on the ring kernel too, in steps of 128 elements (two MFMAs per step)
         fp4 = act_fmt == _lib.FMT_E2M1 and w_fmt == _lib.FMT_E2M1
-        kc = K.pick_layout(groups, b.shape[-2], b.shape[-1], a.shape[0], fp8=fp8, fp4=fp4)
+        kc = K.pick_layout(groups, w_shape[-2], w_shape[-1], a.shape[0], fp8=fp8, fp4=fp4)
         cached = isinstance(b, QuantizedTensor)
         if cached:   # cached copies decide: the call uses the layout they are stored in
             kc = _cache_layout(b, b_t, kc, fp8, groups, fp4)
         if kc in (K.LAYOUT_KSTEP, K.LAYOUT_KSTEP128) and a.shape[0] > 0 and _two_calls(
-                a, b, group_lens, norm_weight, (b_t if need_dgrad else None, w_fmt, kc) if cached else None):
-            return _mx_forward(ctx, a, b, b_t, group_lens, act_fmt, w_fmt, scale_mode, probs, row_mask, activation, grad_sr, rht_signs,
+                a, b, w_shape[-2], w_shape[-1], group_lens, norm_weight, (b_t if need_dgrad else None, w_fmt, kc, groups) if cached else None):
+            return _mx_forward(ctx, a, b, w_shape, b_t, group_lens, act_fmt, w_fmt, scale_mode, probs, row_mask, activation, grad_sr, rht_signs,
                                norm_weight, norm_eps, accum, kc, need_dgrad, need_wgrad)
         ctx.plan = None
         # (a weight gradient that is added to a float32 buffer inside the GEMM runs on either chunked layout)
@@ -509,7 +510,7 @@ class _TWLinearFunction(torch.autograd.Function):
                 kc = 0
         else:
             kc = K.pick_layout(groups, b.shape[-2], b.shape[-1], a.shape[0], fp8=True)
-        if kc == K.LAYOUT_KSTEP and a.shape[0] > 0 and not isinstance(b, QuantizedTensor) and _two_calls(a, b, group_lens):
+        if kc == K.LAYOUT_KSTEP and a.shape[0] > 0 and not isinstance(b, QuantizedTensor) and _two_calls(a, b, b.shape[-2], b.shape[-1], group_lens):
             n, k = b.shape[-2], b.shape[-1]
             bt = need_dgrad and _dgrad_reads_rowwise and fwd_fmt == _lib.FMT_E4M3 and n % K.GEMM_K_ALIGN == 0 and k % K.GEMM_K_ALIGN == 0
             plan = K.linear_plan(a.shape[0], n, k, groups if grouped else 0, _lib.LINEAR_TENSORWISE, fwd_fmt, fwd_fmt, bwd_fmt, 0,

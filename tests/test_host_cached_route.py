@@ -24,6 +24,9 @@ class _OnDevice(torch.Tensor):
     def device(self):
         return torch.device("cuda", 0)
 
+    def get_device(self):
+        return 0
+
     @classmethod
     def __torch_function__(cls, func, types, args=(), kwargs=None):
         with torch._C.DisableTorchFunctionSubclass():
