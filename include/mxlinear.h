@@ -559,7 +559,8 @@ int64_t mxl_calibrate_mfma_bf16_flops(int64_t iters);
  * descriptor over `buf` with that num_records, per-lane offset and scalar offset, and out[4 i .. 4 i + 3] (uint32,
  * device) receives the four dwords that arrived -- zeros where the range check dropped them.  max_offset_host = the
  * largest voffset + soffset of the cases as the caller states it; the call is refused unless that plus 16 fits
- * buf_bytes, so no case can leave `buf` whatever the hardware decides. */
+ * buf_bytes, so no case can leave `buf` whatever the hardware decides (a sum past 2^32 counts modulo 2^32: it is
+ * dropped, or it wraps around). */
 int mxl_calibrate_range_check(const void* buf, int64_t buf_bytes, const void* cases, int num_cases, void* out,
                               int64_t max_offset_host, void* stream);
 

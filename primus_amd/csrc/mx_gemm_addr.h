@@ -5,7 +5,8 @@
 //     address = descriptor base + per-lane offset (voffset) + scalar offset (soffset).
 // On gfx950 a raw buffer descriptor's range check covers BOTH offsets, dword by dword: dword c of a request is
 // fetched iff  voffset + soffset + 4 c + 4 <= num_records,  otherwise nothing is read and zeros arrive (in the
-// register or, for an LDS-direct load, in LDS); there is no wrap-around when soffset alone exceeds num_records.
+// register or, for an LDS-direct load, in LDS); there is no wrap-around, neither when soffset alone exceeds num_records nor
+// when the sum passes 2^32.
 // (Measured on the device; tests/test_gpu_range_check.py pins it through mxl_calibrate_range_check.)
 // The rule of these kernels: the descriptor of a tile starts at the tile's first row and its num_records ends with
 // the OPERAND.  Whatever a request adds -- the row of a ragged last tile, a load round, a K slot beyond the
@@ -105,6 +106,24 @@ MXL_HD Desc ring_panel_desc(int64_t rows_total, int64_t panels, int64_t row0) {
     return Desc{row0 * 16, rows_total * panels * 16 - row0 * 16};
 }
 MXL_HD uint32_t ring_panel_lane(int t) { return (uint32_t)(t * 16); }
+
+// ---------------- bf16 grouped GEMM, 256-row tile (bf16_gemm_tall_kernel) ----------------
+// An operand whose contraction dim is contiguous, [rows_total, ld bytes]: descriptor from the tile's first row to the
+// operand's end; thread t of 512 fetches a 16-byte piece of row t / 8 + 64 e (128 bytes of a row per K slot).
+MXL_HD Desc tall_rows_desc(int64_t rows_total, int64_t row0, int64_t ld) { return Desc{row0 * ld, (rows_total - row0) * ld}; }
+MXL_HD uint32_t tall_rows_lane(int t, int e, int64_t ld) {
+    const int row = t >> 3;
+    return (uint32_t)((row + 64 * e) * ld + 16 * ((t & 7) ^ ((row >> 1) & 7)));
+}
+// One whose contraction dim is the slow one: descriptor from column byte col0 of the first contraction row (of the
+// group's matrix, or the group's first token) to the end of the last one; a K slot is 64 contraction rows.
+MXL_HD Desc tall_cols_desc(int64_t row0, int64_t rows, int64_t ld, int64_t col0) { return Desc{row0 * ld + col0, rows * ld - col0}; }
+MXL_HD uint32_t tall_cols_lane(int t, int e, int64_t ld) {
+    const int row = t >> 5;
+    return (uint32_t)((row + 16 * e) * ld + 16 * ((t & 31) ^ ((row & 3) << 2)));
+}
+// The L2 request, one dword per 128-byte line: line 0 .. 255 of a slot of the operand.
+MXL_HD uint32_t tall_l2_lane(int line, bool cols, int64_t ld) { return (uint32_t)(cols ? (line >> 2) * ld + (line & 3) * 128 : line * ld); }
 
 // A scalar offset no request survives: operands end below 4 GiB and are a multiple of 32 bytes, so num_records is at most
 // 2^32 - 32 and the sum of the offsets (no wrap-around) is past it.

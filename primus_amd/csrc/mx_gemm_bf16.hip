@@ -19,6 +19,7 @@
 // read are spread over the LDS banks.  The tile list is derived from group_lens by every workgroup; the workgroups
 // are persistent and walk it in rounds.  Both kernels add every output element's products in the same order: the same bits.
 #include "mx_device.h"
+#include "mx_gemm_addr.h"
 
 #include <type_traits>
 
@@ -56,6 +57,7 @@ __device__ __forceinline__ v4i bf_rsrc(const void* base, int64_t bytes) {
     r[3] = 0x00020000;
     return r;
 }
+__device__ __forceinline__ v4i bf_desc(const uint8_t* operand, const addr::Desc& d) { return bf_rsrc(operand + d.base, d.records); }
 // LDS-direct 16-byte load: lane i's data lands at lds_off + 16 i.  (M0 holds nothing else in this kernel.)
 __device__ __forceinline__ void bf_dma16(v4i rsrc, uint32_t lds_off, uint32_t voff, uint32_t soff) {
     asm volatile("" : "+s"(soff));
@@ -438,9 +440,6 @@ __global__ __launch_bounds__(TL_THREADS, 2) void bf16_gemm_tall_kernel(Bf16Args 
     const int vwg = (nwg & 7) ? (int)blockIdx.x : ((int)(blockIdx.x & 7) * (nwg >> 3) + (int)(blockIdx.x >> 3));
 
     // ---- per-lane constants ----
-    // requests: lane's place in a round of 8 KiB (contiguous operand: 64 rows of 128 bytes; transposed: 16 rows of 512)
-    const int c_row = t >> 3, c_piece = (t & 7) ^ ((c_row >> 1) & 7);
-    const int t_row = t >> 5, t_piece = (t & 31) ^ ((t_row & 3) << 2);
     // fragment reads: contiguous, row lr of a fragment, piece 2 ks + g XOR (row / 2) % 8 (16 lanes are served at a time,
     // 256 bytes: 16 rows have to put the piece into 16 different places of two rows; with row % 8 half of them met)
     const int lane_c = lr * 128 + 16 * (g ^ ((lr >> 1) & 7));
@@ -492,22 +491,22 @@ __global__ __launch_bounds__(TL_THREADS, 2) void bf16_gemm_tall_kernel(Bf16Args 
             m_valid = (g_rows - r) < 256 ? (int)(g_rows - r) : 256;
             klen = p.k;
             const int64_t lda = p.k * 2;
-            q.ra = bf_rsrc(p.a + c_row0 * lda, (p.total_m - c_row0) * lda);
+            q.ra = bf_desc(p.a, addr::tall_rows_desc(p.total_m, c_row0, lda));
             a_step = TL_KS * 2;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) q.va[e] = (uint32_t)((c_row + 64 * e) * lda + 16 * c_piece);
+            for (int e = 0; e < 4; ++e) q.va[e] = addr::tall_rows_lane(t, e, lda);
             if (!B_T) {
                 const int64_t ldb = p.k * 2, b_row0 = (int64_t)grp * p.n + n0;
-                q.rb = bf_rsrc(p.b + b_row0 * ldb, ((int64_t)G * p.n - b_row0) * ldb);
+                q.rb = bf_desc(p.b, addr::tall_rows_desc((int64_t)G * p.n, b_row0, ldb));
                 b_step = TL_KS * 2;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) q.vb[e] = (uint32_t)((c_row + 64 * e) * ldb + 16 * c_piece);
+                for (int e = 0; e < 4; ++e) q.vb[e] = addr::tall_rows_lane(t, e, ldb);
             } else {
                 const int64_t ldb = p.n * 2;
-                q.rb = bf_rsrc(p.b + ((int64_t)grp * p.k * p.n + n0) * 2, (p.k * p.n - n0) * 2);
+                q.rb = bf_desc(p.b, addr::tall_cols_desc(grp * p.k, p.k, ldb, n0 * 2));
                 b_step = (uint32_t)(TL_KS * ldb);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) q.vb[e] = (uint32_t)((t_row + 16 * e) * ldb + 16 * t_piece);
+                for (int e = 0; e < 4; ++e) q.vb[e] = addr::tall_cols_lane(t, e, ldb);
             }
         } else {
             const int64_t m0 = (int64_t)pid_m * 256;
@@ -517,14 +516,14 @@ __global__ __launch_bounds__(TL_THREADS, 2) void bf16_gemm_tall_kernel(Bf16Args 
             klen = pre_rows[grp + 1] - t0;
             // the descriptors end with the group's last token: the rows of a partly filled last slot read as zero
             const int64_t lda = p.m * 2, ldb = p.n * 2;
-            q.ra = bf_rsrc(p.a + t0 * lda + m0 * 2, klen * lda - m0 * 2);
-            q.rb = bf_rsrc(p.b + t0 * ldb + n0 * 2, klen * ldb - n0 * 2);
+            q.ra = bf_desc(p.a, addr::tall_cols_desc(t0, klen, lda, m0 * 2));
+            q.rb = bf_desc(p.b, addr::tall_cols_desc(t0, klen, ldb, n0 * 2));
             a_step = (uint32_t)(TL_KS * lda);
             b_step = (uint32_t)(TL_KS * ldb);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                q.va[e] = (uint32_t)((t_row + 16 * e) * lda + 16 * t_piece);
-                q.vb[e] = (uint32_t)((t_row + 16 * e) * ldb + 16 * t_piece);
+                q.va[e] = addr::tall_cols_lane(t, e, lda);
+                q.vb[e] = addr::tall_cols_lane(t, e, ldb);
             }
         }
         q.a_step = (uint32_t)__builtin_amdgcn_readfirstlane((int)a_step);
@@ -541,7 +540,7 @@ __global__ __launch_bounds__(TL_THREADS, 2) void bf16_gemm_tall_kernel(Bf16Args 
             for (int i = 0; i < 4; ++i) q.rp[i] = __builtin_amdgcn_readfirstlane(of_a ? q.ra[i] : q.rb[i]);
             if (!ask) q.rp[2] = 0;
             q.p_step = (uint32_t)__builtin_amdgcn_readfirstlane(ask ? (int)(of_a ? a_step : b_step) : 0);
-            q.vp = (uint32_t)(trans ? (line >> 2) * ld + (line & 3) * 128 : line * ld);
+            q.vp = addr::tall_l2_lane(line, trans, ld);
         }
         q.halves = __builtin_amdgcn_readfirstlane((int)((klen + 31) / 32));
         q.m_valid = __builtin_amdgcn_readfirstlane(m_valid);

@@ -131,7 +131,139 @@ static void check_ring_bt4(int64_t groups, int64_t kc, int64_t planes, int64_t g
                 request(d, ring_bt4_lane(t, e, rows_total), (uint32_t)(st * 128 * 64), bytes, plane0 + (e >> 1) < planes, "ring E2M1 codes transposed");
 }
 
+// ---- small-tile kernel (mx_gemm_tile_body.h): TM or TN rows per tile, ST K steps requested ahead.  A request past the
+// contraction range carries the scalar offset kDropped and has to be dropped whole. ----
+static void dropped(const Desc& d, uint32_t voff, const char* what) {
+    for (int c = 0; c < 4; ++c) {
+        ++n_checked;
+        if (accepted(d, voff, kDropped, c)) fail(what, d.base, d.records, voff, c);
+        else ++n_dropped;
+    }
+}
+
+// codes of one operand: `rows` tile rows from row0 on, K steps st0 .. st0 + nst - 1 of `steps`
+static void check_tile_codes(int rows, int row_bytes, int64_t rows_total, int64_t steps, int64_t row0, int64_t st0, int64_t nst) {
+    const bool half = row_bytes == 32;
+    const int rounds = half ? (rows + 127) / 128 : rows / 64;
+    const int64_t bytes = steps * rows_total * row_bytes;
+    const Desc d = ring_code_desc(rows_total, steps, row0, row_bytes);
+    for (int64_t s = 0; s < nst + 4; ++s)
+        for (int e = 0; e < rounds; ++e)
+            for (int t = 0; t < 256; ++t) {
+                const uint32_t voff = ring_code_lane(t, e, half);
+                const int row = half ? (t >> 1) + 128 * e : (t >> 2) + 64 * e;
+                if (s >= nst) dropped(d, voff, "tile codes past the range");
+                else request(d, voff, (uint32_t)(st0 + s) * (uint32_t)(rows_total * row_bytes), bytes, row0 + row < rows_total, "tile codes");
+            }
+}
+
+// its scale panels pan0 .. pan0 + count - 1 of `panels`
+static void check_tile_panels(int rows, int64_t rows_total, int64_t panels, int64_t row0, int64_t pan0, int64_t count) {
+    const Desc d = ring_panel_desc(rows_total, panels, row0);
+    for (int64_t pn = 0; pn < count + 1; ++pn)
+        for (int r = 0; r < rows; ++r) {
+            const uint32_t voff = ring_panel_lane(r);
+            if (pn >= count) dropped(d, voff, "tile panels past the range");
+            else request(d, voff, (uint32_t)(pan0 + pn) * (uint32_t)(rows_total * 16), panels * rows_total * 16, row0 + r < rows_total, "tile panels");
+        }
+}
+
+// 128 columns of b read transposed: two planes of 64 (FP8) or one of 128 (E2M1, `step_rows` 128)
+static void check_tile_bt(int64_t groups, int64_t kc, int64_t planes, int64_t grp, int64_t plane0, int step_rows) {
+    const int64_t rows_total = groups * kc, bytes = planes * rows_total * 64, steps = kc / step_rows;
+    const Desc d = ring_bt_desc(rows_total, planes, grp * kc, plane0);
+    for (int64_t s = 0; s < steps + 4; ++s)
+        for (int e = 0; e < 2; ++e)
+            for (int t = 0; t < 256; ++t) {
+                const uint32_t voff = step_rows == 128 ? ring_bt4_lane(t, e, rows_total) : ring_bt_lane(t, e, rows_total);
+                if (s >= steps) dropped(d, voff, "tile transposed codes past the range");
+                else request(d, voff, (uint32_t)(s * step_rows * 64), bytes, plane0 + (step_rows == 128 ? 0 : e) < planes, "tile transposed codes");
+            }
+}
+
+static void check_tiles() {
+    for (int64_t rows_total : {1, 31, 33, 64, 127, 129, 300, 513})
+        for (int64_t row0 = 0; row0 < rows_total; row0 += rows_total > 130 ? 37 : 11)
+            for (int rows : {64, 128})
+                for (int64_t steps : {2, 4, 18}) {
+                    for (int row_bytes : {64, 32})
+                        for (int64_t st0 = 0; st0 < steps; st0 += 2) check_tile_codes(rows, row_bytes, rows_total, steps, row0, st0, steps - st0 < 4 ? steps - st0 : 3);
+                    const int64_t panels = (steps * 64 + 511) / 512 + 4;       // (a weight gradient over three groups)
+                    for (int64_t pan0 = 0; pan0 < panels; ++pan0) check_tile_panels(rows, rows_total, panels, row0, pan0, panels - pan0);
+                }
+    for (int64_t groups : {1, 3})
+        for (int64_t kc : {128, 384})
+            for (int64_t planes : {1, 2, 3, 6})
+                for (int64_t grp = 0; grp < groups; ++grp)
+                    for (int64_t plane0 = 0; plane0 < planes; ++plane0) {
+                        check_tile_bt(groups, kc, planes, grp, plane0, 128);
+                        if (plane0 % 2 == 0) check_tile_bt(groups, kc, planes, grp, plane0, 64);
+                    }
+    // the largest operand the entry points admit: num_records 32 bytes short of 2^32
+    for (int t = 0; t < 256; ++t)
+        for (int e = 0; e < 2; ++e) dropped(Desc{0, (1ll << 32) - 32}, ring_code_lane(t, e, false), "largest operand");
+}
+
+// ---- the 256-row bf16 tile (bf16_gemm_tall_kernel): slots of 64 contraction elements, eight requests a slot and wave and
+// one dword per line for the L2.  An odd number of halves leaves the last slot's second half past the range. ----
+static void line_request(const Desc& d, uint32_t voff, uint32_t soff, int64_t bytes, const char* what) {
+    ++n_checked;
+    if (!accepted(d, voff, soff, 0)) {
+        ++n_dropped;
+        return;
+    }
+    const int64_t a = d.base + (int64_t)voff + (int64_t)soff;
+    if (a < 0 || a + 4 > bytes) fail(what, a, bytes, voff, soff);
+}
+
+static void check_tall_rows(int64_t rows_total, int64_t k, int64_t row0) {
+    const int64_t ld = k * 2, bytes = rows_total * ld, halves = k / 32;
+    const Desc d = tall_rows_desc(rows_total, row0, ld);
+    for (int64_t slot = 0; 2 * slot < halves; ++slot) {      // (later slots have an empty descriptor)
+        const uint32_t soff = (uint32_t)(slot * 128);
+        for (int e = 0; e < 4; ++e)
+            for (int t = 0; t < 512; ++t) {
+                const int piece = (t & 7) ^ ((t >> 4) & 7);
+                const bool exists = row0 + (t >> 3) + 64 * e < rows_total && slot * 128 + 16 * piece < ld;
+                request(d, tall_rows_lane(t, e, ld), soff, bytes, exists, "tall rows");
+            }
+        for (int line = 0; line < 256; ++line) line_request(d, tall_l2_lane(line, false, ld), soff, bytes, "tall rows, L2");
+    }
+}
+
+// rows [row0, row0 + klen) of an operand of `rows_total` contraction rows and n columns, tile columns from n0 on
+static void check_tall_cols(int64_t rows_total, int64_t row0, int64_t klen, int64_t n, int64_t n0) {
+    const int64_t ld = n * 2, bytes = rows_total * ld, halves = (klen + 31) / 32;
+    const Desc d = tall_cols_desc(row0, klen, ld, n0 * 2);
+    for (int64_t slot = 0; 2 * slot < halves; ++slot) {
+        const uint32_t soff = (uint32_t)(slot * 64 * ld);
+        for (int e = 0; e < 4; ++e)
+            for (int t = 0; t < 512; ++t) {
+                const int row = (t >> 5) + 16 * e, piece = (t & 31) ^ (((t >> 5) & 3) << 2);
+                const uint32_t voff = tall_cols_lane(t, e, ld);
+                request(d, voff, soff, bytes, slot * 64 + row < klen && n0 + 8 * piece < n, "tall columns");
+                // a token past the group's last one has to read as zero: it is multiplied
+                if (slot * 64 + row >= klen)
+                    for (int c = 0; c < 4; ++c)
+                        if (accepted(d, voff, soff, c)) fail("tall columns past the group", slot, row, klen, c);
+            }
+        for (int line = 0; line < 256; ++line) line_request(d, tall_l2_lane(line, true, ld), soff, bytes, "tall columns, L2");
+    }
+}
+
+static void check_tall() {
+    for (int64_t rows_total : {1, 33, 255, 256, 257, 700})
+        for (int64_t row0 = 0; row0 < rows_total; row0 += rows_total > 100 ? 61 : 7)
+            for (int64_t k : {32, 64, 96, 288}) check_tall_rows(rows_total, k, row0);
+    for (int64_t klen : {1, 31, 32, 63, 64, 65, 200})
+        for (int64_t row0 : {0, 5, 77})
+            for (int64_t n : {8, 120, 256, 264, 520})
+                for (int64_t n0 = 0; n0 < n; n0 += 256) check_tall_cols(row0 + klen + (row0 == 5 ? 90 : 0), row0, klen, n, n0);
+}
+
 int main() {
+    check_tiles();
+    check_tall();
     for (int64_t groups : {1, 3})
         for (int64_t kc : {128, 384})
             for (int64_t planes : {1, 2, 3, 5})

@@ -49,3 +49,19 @@ def test_range_check_covers_per_lane_and_scalar_offset(gpu):
     # the entry point refuses cases that could leave the buffer
     assert lib.mxl_calibrate_range_check(ctypes.c_void_p(buf.data_ptr()), 4096, ctypes.c_void_p(dc.data_ptr()), len(cases),
                                          ctypes.c_void_p(out.data_ptr()), top, st) == -1
+
+
+def test_a_sum_past_32_bits_is_dropped(gpu):
+    """The small-tile kernel drops a request by a scalar offset of 2^32 - 16: the range check has to add the per-lane offset
+    without wrapping around.  (Were it to wrap, every case would fetch from the start of the buffer.)"""
+    lib = _lib.load()
+    words, soff = 16384, 0xFFFFFFF0
+    buf = (torch.arange(words, dtype=torch.int32, device=gpu) + 1)
+    cases = [(voff, soff, records) for voff in (0, 16, 32, 1040, 4096, 32768) for records in (64, 8192, 65536)]
+    dc = torch.from_numpy(np.array(cases, dtype=np.uint32).view(np.int32).copy()).to(gpu)
+    out = torch.full((len(cases) * 4,), -1, dtype=torch.int32, device=gpu)
+    rc = lib.mxl_calibrate_range_check(ctypes.c_void_p(buf.data_ptr()), words * 4, ctypes.c_void_p(dc.data_ptr()), len(cases),
+                                       ctypes.c_void_p(out.data_ptr()), max((v + soff) % (1 << 32) for v, _, _ in cases if v >= 16),
+                                       ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    assert not out.cpu().any()
