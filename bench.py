@@ -561,6 +561,7 @@ def main():
         step()
     torch.cuda.synchronize()
     t1 = time.perf_counter()
+    overlapped = bool(pt.ops._side_streams)      # made when a linear first puts its weight gradient on one
 
     # Per-kernel accounting in a pass of its own, every launch bracketed with events on its stream and
     # wgrad kept behind dgrad: two kernels sharing the chip would inflate each other's duration.
@@ -603,7 +604,7 @@ def main():
     peak = BF16_PEAK_TFLOPS if spec.get("bf16") else FP4_PEAK_TFLOPS if act_fp4 else FP8_PEAK_TFLOPS
     roofline = {
         # the MX and tensor-wise workloads run on the 4-slot ring kernel
-        "kernel": "bf16_gemm_kernel<fwd/dgrad> (grouped_gemm_bf16)" if spec.get("bf16") else
+        "kernel": "%s<fwd/dgrad> (grouped_gemm_bf16)" % ("bf16_gemm_tall_kernel" if M // G >= 256 else "bf16_gemm_kernel") if spec.get("bf16") else
                   "bw_gemm256_kernel<e4m3|e5m2,weight factors> (%s)" % fwd_name if spec.get("blockwise") else
                   "%s<%s,%s,fwd/dgrad%s> (%s)" % ("mx_gemm_ring_kernel",
                                                    "e4m3|e5m2" if spec.get("tensorwise") else "e2m1" if act_fp4 else "e4m3",
@@ -664,7 +665,7 @@ def main():
         ("frac_bf16_mfma_peak_whole_step" if spec.get("bf16") else "frac_fp4_mfma_peak_whole_step" if act_fp4 else "frac_fp8_mfma_peak_whole_step"): round(value / peak, 4),
         "gemm_only_TFLOP/s": round(gemm_flops / gemm_sec / 1e12, 2),
         ("gemm_only_frac_bf16_mfma_peak" if spec.get("bf16") else "gemm_only_frac_fp4_mfma_peak" if act_fp4 else "gemm_only_frac_fp8_mfma_peak"): round(gemm_flops / gemm_sec / 1e12 / peak, 4),
-        "wgrad_overlaps_dgrad": not args.no_wgrad_overlap,
+        "wgrad_overlaps_dgrad": overlapped,
         "kernels_note": "per-kernel figures: separate pass of %d steps after the timed region, wgrad serialised behind dgrad" % kernel_steps,
         "kernels": kernels,
         "roofline": roofline,

@@ -603,8 +603,9 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
     static_assert(BFMT != kFmtE2M1 || F44 || (MODE == MODE_FWD && !ALPHA), "an E2M1 weight operand against FP8 rows: forward / dgrad of the MX recipe");
     constexpr bool B4 = BFMT == kFmtE2M1 && !F44;     // FP4 weights against FP8 rows: 32 bytes per row and K step
     // PEEL: a tile's first MFMAs start from the constant 0 instead of cleared accumulators.  The compiler clears the 256
-    // accumulators of an E2M1 tile twice over, 2048 clocks that nothing covers (one wave per SIMD): the weight gradient of
-    // 1024 rows per group, [8, 28672, 4096], 903 -> 734 us; dgrad on the row-wise codes 1-3 % (fc1 of the same, 556 -> 537).
+    // accumulators of an E2M1 tile twice over, 2048 clocks that nothing covers (one wave per SIMD).  Launches alone, 1024
+    // rows in each of 8 groups: weight gradient [8, 28672, 4096] 814 -> 776 us, [8, 4096, 14336] 370 -> 348; dgrad on the
+    // row-wise codes of the same weights 523 -> 516 and 260 -> 262.
     // The peeled step is another copy of the loop body, which the forward GEMM gains nothing from and the FP8
     // instantiations do not survive (16 -> 160 spilled registers, 1081 -> 1236 us).
     constexpr bool PEEL = F44 && (MODE == MODE_WGRAD || BT);
@@ -1328,8 +1329,9 @@ static bool tile_flag_ok(uint32_t flags) {
 //   128 groups, [5760, 2880]: 4 rows per group ring 378 us, 64 x 128 317 (E2M1 weights 272, 183); 64 rows 474, 530 (413, 333)
 //   32 groups, [4096, 7168]: 32 rows per group ring 185, 128 180 (transposed codes 238, 196); 64 rows 187, 208 (243, 217)
 // The weight gradient's tiles are all output and little contraction: dense ones take 128 x 128 while the contraction is
-// short (256 tokens, 14336 x 4096: 43 -> 29 us); grouped ones run the ring kernel at the rate the board writes, except
-// where the gradient is a few tiles.
+// short (256 tokens, 14336 x 4096: 43 -> 29 us).  Grouped ones run the ring kernel, which writes more per second on
+// expert-sized gradients, if far from what a fill does (256 rows in each of 32 groups, [4096, 7168]: 458 us, a fill of its
+// 1.9 GB 273; skewed rows, ring 474, 128 x 128 tiles 541), except where the gradient is a few tiles.
 template <int MODE> static int tile_choice(const GemmArgs& a, bool e2m1_weights, bool bt, uint32_t flags) {
     switch (flags & MXL_GF_TILE_MASK) {
         case MXL_GF_TILE_64: return TILE_64;

@@ -398,9 +398,10 @@ __global__ __launch_bounds__(BF_THREADS, 2) void bf16_gemm_kernel(Bf16Args p) {
 //   * the L2 is asked four slots ahead for the lines this tile's neighbours on the XCD will want, each line by one of
 //     them: a fifth of the requests missed the L2 and every slot waited for some of those (-15 % cycles);
 //   * the next tile's first slot is requested in front of the output's way out (wgrad of 1000 tokens: +1.5 %).
-// Mixtral experts [32768, 4096] x [8, 28672, 4096], forward / dgrad / wgrad: 1.07 / 1.19 / 1.17 -> 1.27 / 1.30 / 1.36 PFLOP/s;
-// 32 ragged groups of about 1024 rows, [4096, 7168]: 0.88 / 0.97 / 0.98 -> 1.10 / 1.15 / 1.13; 128 groups of about 512,
-// [5760, 2880]: 0.75 / 0.81 / 0.70 -> 0.89 / 0.88 / 0.72.
+// Against its 4-wave predecessor (wgrad: the 128-row tile it ran on), ragged groups, forward / dgrad / wgrad in PFLOP/s:
+// Mixtral experts [32768, 4096] x [8, 28672, 4096] 1.04 / 1.03 / 1.12 -> 1.23 / 1.12 / 1.28; 32 groups of about 1024 rows,
+// [4096, 7168], 0.89 / 0.94 / 0.96 -> 1.07 / 1.09 / 1.09; 128 groups of about 512, [5760, 2880], 0.68 / 0.78 / 0.75 ->
+// 0.87 / 0.86 / 0.81.  (At the power limit the rate follows the box and the data: up to 1.27 / 1.30 / 1.36 on the first.)
 constexpr int TL_THREADS = 512;
 constexpr int TL_KS = 64;                               // contraction elements per slot: 128 bytes of a row, four MFMA steps
 constexpr int TL_HALF = 256 * TL_KS * 2;                // 32 KiB: one operand of a slot

@@ -40,9 +40,9 @@ __all__ = ["gemm", "grouped_gemm", "gemm_fp8", "gemm_fp4", "grouped_gemm_fp8", "
            "swiglu_with_probs", "geglu_with_probs", "tokens_per_expert_to_mask", "glu_grouped_gemm_fp8",
            "glu_grouped_gemm_fp4", "manual_sr_seed", "set_kchunk_layout", "rmsnorm", "rmsnorm_gemm_fp8", "rmsnorm_gemm_fp4", "pad_groups", "unpad_groups"]
 
-# dgrad and wgrad of one linear are independent once dY is quantised.  Both GEMMs are persistent
-# kernels with one workgroup per CU, so launching wgrad on a second stream lets its workgroups move in
-# as dgrad's last, partial wave of tiles drains instead of leaving those CUs idle.
+# dgrad and wgrad of one linear are independent once dY is quantised, so wgrad may run on a second stream, where its
+# workgroups move in as dgrad's last, partial round of tiles drains.  The default is one stream: _overlaps() names the
+# linears that gain, and what the overlap costs the others.  (The launch-by-launch route overlaps whenever this is on.)
 _wgrad_overlap = True
 _side_streams = {}
 
