@@ -167,13 +167,16 @@ def _overlaps(plan) -> bool:
     return flops >= 1.5e12 and plan.rows <= 1024 * plan.groups
 
 
+_CODE_DTYPES = {fmt: K._code_dtype(fmt) for fmt in (_lib.FMT_E4M3, _lib.FMT_E2M1, _lib.FMT_E5M2)}
+
+
 def _holds(q: QuantizedTensor, rows: int, ld: int, fmt: int, kc: int, device: int) -> bool:
     """Whether a cached copy is ``[rows, ld]`` codes of ``fmt`` and their scales on GPU ``device``, in the K-step-major layout
     ``kc`` without gaps: all that the two calls, which are handed its pointers, take for granted about it."""
-    codes, scales = q.codes, q.scales
+    codes, scales = q._codes, q._scales
     step = K.KSTEP if kc == K.LAYOUT_KSTEP else K.KCHUNK
     ld = (ld + K.GEMM_K_ALIGN - 1) // K.GEMM_K_ALIGN * K.GEMM_K_ALIGN
-    return (q.fmt == fmt and q.kchunk == kc
+    return (codes.dtype == _CODE_DTYPES[fmt] and q._kchunk == kc
             and codes.shape == (ld // step, rows, step // (2 if fmt == _lib.FMT_E2M1 else 1)) and codes.is_contiguous()
             and scales.shape == ((ld + K.PANEL - 1) // K.PANEL, rows, 16) and scales.is_contiguous()
             and codes.get_device() == device and scales.get_device() == device)
@@ -196,7 +199,8 @@ def _two_calls(a, b, n, k, group_lens, norm_weight=None, cache=None) -> bool:
         return False
     if norm_weight is not None:
         K._norm_args(a, norm_weight)
-    K._check_group_lens(group_lens, a.device)
+    if group_lens is not None:
+        K._check_group_lens(group_lens, a.device)
     return True
 
 
