@@ -570,6 +570,7 @@ constexpr int RING_MAX_GROUPS = 256;          // what the group tables may take 
 constexpr int RING_PANEL = 256 * 16;              // scale panel of one operand: 16 bytes per row = 8 K steps
 constexpr int RING_PANEL_BUFS = 3;
 constexpr int RING_TBL = RING_MAX_GROUPS + 2;
+constexpr int HALF_ROWS = 128;                    // rows of a tile that the first two of every wave's fragments hold
 
 constexpr int ring_lds_bytes() {
     return RING_SLOTS * RING_STAGE + RING_PANEL_BUFS * 2 * RING_PANEL + RING_TBL * 4 + RING_TBL * 8 + RING_TBL * 4 + RING_TBL * 4;
@@ -808,9 +809,11 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
     // lra / lrb: descriptors of the tile the stream is in; lca / lcb: byte offset of the K chunk the next group
     // starts in; ga / gb: byte offset (chunk + half) of the group in flight.
     v4i lra, lrb, crb;
-    uint32_t lca, lcb, lla, llb, ga = 0, gb = 0, cgb = 0;
+    // lup: rounds 2 and 3 of a half tile (rows HALF_ROWS ..) are sent to an offset the range check drops
+    uint32_t lca, lcb, lla, llb, ga = 0, gb = 0, cgb = 0, gup = 0, lup = 0;
     auto stream_enter = [&](const Tile& d) __attribute__((always_inline)) {
         lra = d.ra; lrb = d.rb; lca = d.ca0; lcb = d.cb0; lla = d.cal; llb = d.cbl;
+        if (MODE == MODE_FWD) lup = d.m_valid > HALF_ROWS ? 0u : addr::kDropped;
     };
     // start the group of the stream's next K step: fixes ga / gb and moves the stream on.  A step past the tile's
     // contraction range (a range of two steps is padded to four) requests the range's last step again: every
@@ -818,6 +821,7 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
     auto group_begin = [&]() __attribute__((always_inline)) {
         ga = lca < lla ? lca : lla;
         gb = lcb < llb ? lcb : llb;
+        gup = ga | lup;
         lca += a_cstride;
         lcb += b_cstride;
         // rounds 6 and 7 of this group go out at the start of the next step, possibly after the stream has
@@ -829,7 +833,8 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
     // (slot_base already holds the wave's 1 KiB share, w * 1024; the round's 4 KiB come in as a constant)
     auto issue_e = [&](auto e_tag, uint32_t slot_base) __attribute__((always_inline)) {
         constexpr int e = decltype(e_tag)::value;
-        if constexpr (e < 4) dma16_at<e * 4096>(lra, slot_base, va[e], ga);
+        if constexpr (e < 2) dma16_at<e * 4096>(lra, slot_base, va[e], ga);
+        else if constexpr (e < 4) dma16_at<e * 4096>(lra, slot_base, va[e], MODE == MODE_FWD ? gup : ga);
         else if constexpr (e >= 6) dma16_at<A_BYTES + (e - 4) * 4096>(crb, slot_base, vb[e - 4], cgb);
         else dma16_at<A_BYTES + (e - 4) * 4096>(lrb, slot_base, vb[e - 4], gb);
     };
@@ -851,7 +856,7 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
 #define MXL_PIN __builtin_amdgcn_sched_barrier(0)
     // fragment (+ scale byte) reads of the K step in ring slot at `sn`, panel bytes at `pan`
 #define MXL_RD_A(F, I) \
-    do { if ((I) < LIVE) { const uint8_t* r_ = sn + a_frag + (I) * (32 * BK); \
+    do { if ((I) < LIVE) { const uint8_t* r_ = sn + a_frag + (I) * (64 * BK); \
          const uint4 lo_ = *(const uint4*)(r_ + a_lo), hi_ = *(const uint4*)(r_ + a_hi); \
          F.a[I][0] = lo_.x; F.a[I][1] = lo_.y; F.a[I][2] = lo_.z; F.a[I][3] = lo_.w; \
          F.a[I][4] = hi_.x; F.a[I][5] = hi_.y; F.a[I][6] = hi_.z; F.a[I][7] = hi_.w; } } while (0)
@@ -883,7 +888,7 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
 #define MXL_SC_B(F, J) do { F.sb[J] = ALPHA ? 127 : (int)(uint32_t)(psb[J] >> psh); } while (0)
     // per-lane constants of the fragment reads: 64-byte rows, piece index XOR (row / 4) % 4
     const int sw = (lr >> 2) & 3;
-    const int a_frag = (wm * 128 + lr) * BK, b_frag = (wn * 128 + lr) * B_ROW;
+    const int a_frag = (wm * 32 + lr) * BK, b_frag = (wn * 128 + lr) * B_ROW;
     const int b4_lo = 16 * (g ^ ((lr >> 3) & 1));      // FP4: lane (row, g) holds elements 32 g .. 32 g + 31 of the K step
     // BT: this lane ADDRESSES contraction row 16 g + 8 h + tj (+ 32 for the second half of the step) and the 8-byte
     // piece of its 16-lane block's 16 columns: bt_off[h][J & 1] inside a plane's 64 rows x 64 bytes (same swizzle
@@ -915,11 +920,11 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
     // Scale bytes: a panel row holds [g][K step] = 2 x 8 bytes, so the 8 bytes at (row, g) are the lane's scale
     // bytes of the panel's 8 K steps.  They are read once per panel (8 reads of 8 bytes per wave, 512 consecutive
     // bytes each) and the byte of a step is shifted down in registers: the MFMA takes byte 0 of its scale operand.
-    const int a_sc = (wm * 128 + lr) * 16 + 8 * g, b_sc = (wn * 128 + lr) * 16 + 8 * g;
+    const int a_sc = (wm * 32 + lr) * 16 + 8 * g, b_sc = (wn * 128 + lr) * 16 + 8 * g;
     uint64_t psa[4], psb[4];
 #define MXL_RD_PANEL(PAN) \
     do { if (!ALPHA) _Pragma("unroll") for (int i_ = 0; i_ < 4; ++i_) { \
-             psa[i_] = *(const uint64_t*)((PAN) + a_sc + i_ * (32 * 16)); \
+             psa[i_] = *(const uint64_t*)((PAN) + a_sc + i_ * (64 * 16)); \
              psb[i_] = *(const uint64_t*)((PAN) + PANEL + b_sc + i_ * (32 * 16)); } } while (0)
 
     // The workgroup's tiles: one per round of nwg tiles, at position vwg of the round -- in wgrad at position
@@ -982,9 +987,13 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
         v16f acc[4][4];
         Frags f0, f1;
         const int nst = d.nst, nst_real = d.nst_real;
-        // LIVE: how many of the wave's four 32-row fragments hold rows of the tile (4, 2 or 0).  A tile at the ragged end of
-        // a group has fewer than 256 rows; fragments beyond them are neither read nor multiplied (loads, barriers and the
-        // request stream are the same for every wave).
+        // LIVE: how many of the wave's four 32-row fragments are run (4, 3 or 2).  Fragment i of the two wave rows holds tile
+        // rows 64 i .. 64 i + 63, so that the tile at a group's ragged end is less work for all four waves alike, and one of
+        // at most 128 rows fetches only those.  (Two halves of 128 consecutive rows, the waves of a short tile's second one
+        // idle while the first one's take as long as ever: 32 groups of 2 .. 777 rows, [4096, 7168], forward 333 -> 314 us,
+        // transposed codes 338 -> 317; 128 groups of about 512 rows, E2M1 [5760, 2880], 1066 -> 1031.  A fourth variant,
+        // LIVE 1, costs 116 spilled registers.  Two tiles of at most 128 rows as one position of the tile order, for equal
+        // shares, lose: such tiles wait for the weights' bytes, 172 -> 217 us on 32 groups of [7168, 2048].)
         auto run_tile = [&](auto live_tag) __attribute__((always_inline)) {
             constexpr int LIVE = decltype(live_tag)::value;
             {   // fragments of K step 0
@@ -994,7 +1003,8 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
                 MXL_RD_B(f0, 0); MXL_RD_B(f0, 1); MXL_RD_B(f0, 2); MXL_RD_B(f0, 3);
                 MXL_RD_A(f0, 0); MXL_RD_A(f0, 1); MXL_RD_A(f0, 2); MXL_RD_A(f0, 3);
                 MXL_PIN;
-                if (!PEEL) {    // the accumulators are cleared while those reads are on their way
+                if (!PEEL) {    // the accumulators are cleared while those reads are on their way (all of them, whatever LIVE is:
+                                // registers left unset cost 110 spilled ones)
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -1089,10 +1099,9 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
             }
         };
         {
-            const int live = (MODE == MODE_FWD) ? d.m_valid - wm * 128 : 128;
-            if (MODE != MODE_FWD || live > 64) run_tile(std::integral_constant<int, 4>{});
-            else if (live > 0) run_tile(std::integral_constant<int, 2>{});
-            else run_tile(std::integral_constant<int, 0>{});
+            if (MODE != MODE_FWD || d.m_valid > HALF_ROWS + 64) run_tile(std::integral_constant<int, 4>{});
+            else if (d.m_valid > HALF_ROWS) run_tile(std::integral_constant<int, 3>{});
+            else run_tile(std::integral_constant<int, 2>{});
         }
         // K step 0 of the next tile (and its scale panel) has landed; every wave is done reading the ring
         wait_vm<2 * ROUNDS>();
@@ -1131,12 +1140,13 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
             // the stores of patch n, which wait for those reads, come behind the conversions and writes of patch n + 1
             // and find their data there.  The loop exists twice, for whole tiles (nothing predicated) and for tiles at
             // an edge.
-            auto write_out = [&](auto full_tag) __attribute__((always_inline)) {
+            auto write_out = [&](auto full_tag, auto count_tag) __attribute__((always_inline)) {
                 constexpr bool FULL = decltype(full_tag)::value;
+                constexpr int COUNT = decltype(count_tag)::value;
                 uint4 v[4];
-                static_for<0, 9>([&](auto it_tag) {
+                static_for<0, COUNT + 1>([&](auto it_tag) {
                     constexpr int it = decltype(it_tag)::value;
-                    if constexpr (it < 8) {
+                    if constexpr (it < COUNT) {
                         constexpr int i = it >> 1, jh = it & 1;
 #pragma unroll
                         for (int jl = 0; jl < 2; ++jl)
@@ -1155,15 +1165,15 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
                     if constexpr (it > 0) {
                         constexpr int i = (it - 1) >> 1, jh = (it - 1) & 1;
                         // uniform base of the patch's rows; the lane adds a 32-bit offset
-                        uint8_t* rowbase = (uint8_t*)(ctile + (int64_t)(wm * 128 + i * 32) * p.n + wn * 128 + jh * 64);
+                        uint8_t* rowbase = (uint8_t*)(ctile + (int64_t)(i * 64 + wm * 32) * p.n + wn * 128 + jh * 64);
                         const int cc = wn * 128 + jh * 64 + rch * 8;
 #pragma unroll
                         for (int u = 0; u < 4; ++u)
-                            if (FULL || (wm * 128 + i * 32 + 8 * u + rrow < m_valid && cc < n_valid))
+                            if (FULL || (i * 64 + wm * 32 + 8 * u + rrow < m_valid && cc < n_valid))
                                 store16_streaming(rowbase + (int64_t)(8 * u) * p.n * 2 + lane_off,
                                                   u >= 2 ? make_uint4(v[u].z, v[u].w, v[u].x, v[u].y) : v[u]);
                     }
-                    if constexpr (it < 8) {
+                    if constexpr (it < COUNT) {
 #pragma unroll
                         for (int u = 0; u < 4; ++u) v[u] = *(const uint4*)(((u & 1) ? rd1 : rd0) + u * (8 * 128));
                     }
@@ -1197,11 +1207,11 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
                     }
                     if constexpr (it > 0) {
                         constexpr int i = (it - 1) >> 2, j = (it - 1) & 3;
-                        float* base = ctile32 + (int64_t)(wm * 128 + i * 32) * p.n + wn * 128 + j * 32;   // uniform
+                        float* base = ctile32 + (int64_t)(i * 64 + wm * 32) * p.n + wn * 128 + j * 32;   // uniform
                         const bool col_ok = FULL || wn * 128 + j * 32 + rw < n_valid;
 #pragma unroll
                         for (int v = 0; v < 16; ++v)
-                            if (FULL || (col_ok && wm * 128 + i * 32 + 2 * v + rr2 < m_valid))
+                            if (FULL || (col_ok && i * 64 + wm * 32 + 2 * v + rr2 < m_valid))
                                 unsafeAtomicAdd(base + (int64_t)(2 * v) * p.n + lane_off32, val[v]);
                     }
                     if constexpr (it < 16) {
@@ -1216,8 +1226,9 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
                 if (full) add_out(std::true_type{});
                 else add_out(std::false_type{});
             } else {
-                if (full) write_out(std::true_type{});
-                else write_out(std::false_type{});
+                if (full) write_out(std::true_type{}, std::integral_constant<int, 8>{});
+                else if (MODE != MODE_FWD || m_valid > HALF_ROWS) write_out(std::false_type{}, std::integral_constant<int, 8>{});
+                else write_out(std::false_type{}, std::integral_constant<int, 4>{});      // (acc[2 ..] of a half tile hold nothing)
             }
         }
         if (tile_n >= total_tiles) break;

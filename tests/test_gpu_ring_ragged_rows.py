@@ -1,0 +1,60 @@
+"""The ring kernel's tiles at a group's ragged end: row counts on both sides of every number of live fragments (64, 128, 192,
+256 rows), alone and behind a whole tile, and column counts on both sides of the output patches (64 and 128 columns).  Compared
+bit for bit with the 128 x 128 tile, which runs the same MFMAs per output element; rows and columns next to the tile must stay
+untouched, so the output is one part of a larger buffer filled beforehand."""
+
+import ctypes
+
+import pytest
+import torch
+
+from primus_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+LENS = [1, 63, 64, 65, 0, 127, 128, 129, 191, 192, 193, 255, 256, 257, 320, 384, 448, 449]
+GUARD = 512
+
+
+@pytest.mark.parametrize("recipe", ["mxfp8", "mxfp4w8", "mxfp4"])
+@pytest.mark.parametrize("n,k", [(32, 128), (64, 256), (96, 384), (160, 128), (320, 640), (512, 128)])
+def test_ragged_tiles(gpu, recipe, n, k):
+    from primus_amd.pytorch import kernels as K
+
+    afmt, wfmt, lay = {"mxfp8": (0, 0, 2), "mxfp4w8": (0, 1, 2), "mxfp4": (1, 1, 3)}[recipe]
+    g = torch.Generator().manual_seed(n + k)
+    m, G = sum(LENS), len(LENS)
+    x = torch.randn(m, k, generator=g).bfloat16().to(gpu)
+    w = (torch.randn(G, n, k, generator=g) * 0.05).bfloat16().to(gpu)
+    gl = torch.tensor(LENS, dtype=torch.int64, device=gpu)
+    xq = K.quantize_mx_impl(x, afmt, rowwise=True, colwise=False, group_lens=gl, pad_to=128, kchunk=lay)
+    wq = K.quantize_mx_weight_2d_impl(w, wfmt, rowwise=True, colwise=False, pad_to=128, kchunk=lay)
+    want = K.grouped_gemm_mx_nt_impl(xq[0], xq[1], wq[0], wq[1], gl, kchunk=lay, tile="128")
+    buf = torch.full((GUARD + m * n + GUARD,), 7.0, dtype=torch.bfloat16, device=gpu)
+    out = buf[GUARD:GUARD + m * n]
+    p = ctypes.c_void_p
+    rc = _lib.load().mxl_grouped_gemm_nt_ex(p(xq[0].data_ptr()), p(xq[1].data_ptr()), afmt, p(wq[0].data_ptr()), p(wq[1].data_ptr()), wfmt,
+                                            p(out.data_ptr()), p(gl.data_ptr()), G, m, n, k, _lib.GF_KSTEP | _lib.GF_TILES["256"],
+                                            p(torch.cuda.current_stream().cuda_stream))
+    assert rc == 0
+    assert torch.equal(out.view(m, n).view(torch.int16), want.view(torch.int16))
+    assert bool((buf[:GUARD] == 7.0).all()) and bool((buf[GUARD + m * n:] == 7.0).all())
+
+
+@pytest.mark.parametrize("recipe", ["mxfp8", "mxfp4"])
+@pytest.mark.parametrize("n,k", [(32, 64), (96, 320), (288, 160), (416, 480)])
+def test_weight_gradient_edges(gpu, recipe, n, k):
+    from primus_amd.pytorch import kernels as K
+
+    fmt, lay = {"mxfp8": (0, 2), "mxfp4": (1, 3)}[recipe]
+    lens = [130, 0, 513, 64, 128, 1]
+    g = torch.Generator().manual_seed(n * k)
+    m, G = sum(lens), len(lens)
+    x = torch.randn(m, k, generator=g).bfloat16().to(gpu)
+    dy = torch.randn(m, n, generator=g).bfloat16().to(gpu)
+    gl = torch.tensor(lens, dtype=torch.int64, device=gpu)
+    xq = K.quantize_mx_impl(x, fmt, rowwise=False, colwise=True, group_lens=gl, pad_to=128, kchunk=lay)
+    dq = K.quantize_mx_impl(dy, fmt, rowwise=False, colwise=True, group_lens=gl, pad_to=128, kchunk=lay)
+    want = K.grouped_gemm_mx_wgrad_impl(dq[2], dq[3], xq[2], xq[3], gl, m, kchunk=lay, tile="128")
+    got = K.grouped_gemm_mx_wgrad_impl(dq[2], dq[3], xq[2], xq[3], gl, m, kchunk=lay, tile="256")
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
