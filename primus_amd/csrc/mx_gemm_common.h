@@ -78,6 +78,16 @@ __device__ __forceinline__ void store16_streaming(uint8_t* dst, const uint4& v) 
     __builtin_nontemporal_store(t, (u32x4*)dst);
 }
 
+// The same through a buffer descriptor (base and size uniform): a lane whose offsets pass its end stores nothing.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_store_rsrc(void* base, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000);
+}
+__device__ __forceinline__ void buffer_store16_streaming(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t soff, const uint4& v) {
+    const u32x4 t = {v.x, v.y, v.z, v.w};
+    constexpr int kNonTemporal = 2;
+    __builtin_amdgcn_raw_buffer_store_b128(t, rsrc, (int)voff, (int)soff, kNonTemporal);
+}
+
 // compile-time loop: f(integral_constant<int, I>) for I .. N - 1
 template <int I, int N, class F>
 __device__ __forceinline__ void static_for(F&& f) {
