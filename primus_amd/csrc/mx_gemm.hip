@@ -570,6 +570,7 @@ constexpr int RING_MAX_GROUPS = 256;          // what the group tables may take 
 constexpr int RING_PANEL = 256 * 16;              // scale panel of one operand: 16 bytes per row = 8 K steps
 constexpr int RING_PANEL_BUFS = 3;
 constexpr int RING_TBL = RING_MAX_GROUPS + 2;
+constexpr int EPI_STORES = 32;                    // a wave's stores of a tile, dropped ones included
 constexpr int HALF_ROWS = 128;                    // rows of a tile that the first two of every wave's fragments hold
 
 // The tile's accumulators are in the accumulation registers here, and leave them behind this point only.
@@ -609,10 +610,15 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
     // PEEL: a tile's first MFMAs start from the constant 0 instead of cleared accumulators.  The compiler clears the 256
     // accumulators of an E2M1 tile twice over, 2048 clocks that nothing covers (one wave per SIMD).  Launches alone, 1024
     // rows in each of 8 groups: weight gradient [8, 28672, 4096] 814 -> 776 us, [8, 4096, 14336] 370 -> 348; dgrad on the
-    // row-wise codes of the same weights 523 -> 516 and 260 -> 262.
-    // The peeled step is another copy of the loop body, which the forward GEMM gains nothing from and the FP8
-    // instantiations do not survive (16 -> 160 spilled registers, 1081 -> 1236 us).
-    constexpr bool PEEL = F44 && (MODE == MODE_WGRAD || BT);
+    // row-wise codes of the same weights 523 -> 516 and 260 -> 262; forward of 8 groups of about 1024 rows, [28672, 4096],
+    // 510 -> 499; E2M1 weights against FP8 rows, 128 groups of about 512 rows, [5760, 2880], 1046 -> 1024 and back 1015 -> 1008.
+    // The peeled step is another copy of the loop body, which the FP8 instantiations do not survive (up to 240 spilled
+    // registers; weight gradient 460 -> 613 us).
+    constexpr bool PEEL = BFMT == kFmtE2M1;
+    // SLACK: the first two steps behind an epilogue do not wait for its 32 stores (they are younger than the requests those
+    // steps need).  FP8 weight gradients of 32 groups of 2 .. 777 rows, [4096, 7168], 460 -> 442 us, [7168, 2048] 231 -> 221;
+    // [4096, 4096] x [14336, 4096] 200 -> 197.  E2M1 x E2M1 ones lose 1 %, the forward gains nothing.
+    constexpr bool SLACK = MODE == MODE_WGRAD && !ACCUM && !F44;
     constexpr int KS = F44 ? 2 * BK : BK;             // elements of the contraction per step
     constexpr int PSTEPS = 512 / KS;                  // steps per scale panel
     constexpr int B_ROW = B4 ? BK / 2 : BK;           // bytes of a row of b in a K step
@@ -986,6 +992,7 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
     wait_vm<2 * ROUNDS + 6>();       // everything up to K step 0 has landed
     __syncthreads();
 
+    int slack = 0;       // steps that may leave the last epilogue's stores on their way
     while (true) {
         v16f acc[4][4];
         Frags f0, f1;
@@ -1037,7 +1044,13 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
                 MXL_MFMA(cur, 1, 0); MXL_PIN;
                 MXL_MFMA(cur, 2, 0); if (ROUNDS == 8) issue_e(E7{}, slot_prev); MXL_PIN;
                 MXL_MFMA(cur, 3, 0); MXL_PIN;
-                wait_vm<2 * ROUNDS>();       // the group of step gs + 1 has landed (two younger groups may be in flight)
+                // the group of step gs + 1 has landed (two younger groups may be in flight)
+                if (SLACK && slack > 0) {
+                    --slack;
+                    wait_vm<2 * ROUNDS + EPI_STORES>();
+                } else {
+                    wait_vm<2 * ROUNDS>();
+                }
                 __syncthreads();
                 MXL_PIN;
                 // bookkeeping between the barrier and the first read: panel of the next step, stream hand-over
@@ -1157,7 +1170,7 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
                 const int cc = wn * 128 + rch * 8;
                 const uint32_t off0 = cc < n_valid ? lane_off : addr::kDropped, off1 = cc + 64 < n_valid ? lane_off + 128 : addr::kDropped;
                 uint4 v[4];
-                static_for<0, 9>([&](auto it_tag) {
+                static_for<0, 9>([&](auto it_tag) {      // 8 patches x 4 = EPI_STORES stores
                     constexpr int it = decltype(it_tag)::value;
                     if constexpr (it < 8) {
                         constexpr int i = it >> 1, jh = it & 1;
@@ -1241,6 +1254,7 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
             }
         }
         if (tile_n >= total_tiles) break;
+        if (SLACK) slack = 2;
         __syncthreads();      // every wave has left the patch: its slot takes K step 3 of the next tile
         // (the stream entered the next tile four steps ago; the group of its step 3 begins here)
         group_begin();

@@ -1,7 +1,8 @@
 """The ring kernel's tiles at a group's ragged end: row counts on both sides of every number of live fragments (64, 128, 192,
 256 rows), alone and behind a whole tile, and column counts on both sides of the output patches (64 and 128 columns).  Compared
 bit for bit with the 128 x 128 tile, which runs the same MFMAs per output element; rows and columns next to the tile must stay
-untouched, so the output is one part of a larger buffer filled beforehand."""
+untouched, so the output is one part of a larger buffer filled beforehand.  The last sizes of each list give a workgroup
+several tiles, one behind the other's stores."""
 
 import ctypes
 
@@ -17,7 +18,7 @@ GUARD = 512
 
 
 @pytest.mark.parametrize("recipe", ["mxfp8", "mxfp4w8", "mxfp4"])
-@pytest.mark.parametrize("n,k", [(32, 128), (64, 256), (96, 384), (160, 128), (320, 640), (512, 128)])
+@pytest.mark.parametrize("n,k", [(32, 128), (64, 256), (96, 384), (160, 128), (320, 640), (512, 128), (4096, 128)])
 def test_ragged_tiles(gpu, recipe, n, k):
     from primus_amd.pytorch import kernels as K
 
@@ -42,7 +43,7 @@ def test_ragged_tiles(gpu, recipe, n, k):
 
 
 @pytest.mark.parametrize("recipe", ["mxfp8", "mxfp4"])
-@pytest.mark.parametrize("n,k", [(32, 64), (96, 320), (288, 160), (416, 480)])
+@pytest.mark.parametrize("n,k", [(32, 64), (96, 320), (288, 160), (416, 480), (2080, 2048)])
 def test_weight_gradient_edges(gpu, recipe, n, k):
     from primus_amd.pytorch import kernels as K
 
