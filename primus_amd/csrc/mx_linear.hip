@@ -5,6 +5,7 @@
 // caller allocates three buffers -- what the backward needs, and a scratch buffer per direction -- and makes one call per
 // direction; the layout of the buffers is arithmetic on the sizes and is worked out again in every call.
 #include "mx_gemm_tile.h"
+#include "mx_quantize.h"
 
 namespace {
 
@@ -152,12 +153,15 @@ extern "C" int mxl_linear_forward(const mxl_linear* p, const void* x, const void
     const int af = (int)p->act_fmt, wf = (int)p->w_fmt;
     const bool from_rows = p->need_dx && p->dx_from_rows;
     const Copy wr = from_rows ? sv.w_row : f.w_row;
+    const bool rht = p->rht_signs >= 0 && p->need_dw && !l.tensorwise();
+    const mxl::LinearOperands both = {x, w, p->rows, l.batch, p->n, p->k, l.k_ld, l.n_ld,
+                                      l.tensorwise() && !p->need_dw ? nullptr : lens, l.tensorwise() && !p->need_dw ? 0 : G,
+                                      af, wf, (int)p->scale_mode, l.qf() | (rht ? MXL_QF_RHT_COL : 0u), rht ? (uint32_t)p->rht_signs : 0u,
+                                      f.x_amax, f.w_amax, sv.x_si, sv.w_si,
+                                      f.x_row.q, f.x_row.s, sv.x_col.q, sv.x_col.s, wr.q, wr.s, sv.w_col.q, sv.w_col.s};
     if (l.tensorwise()) {
         MXL_TRY(mxl::amax_pair(x, p->rows * p->k, f.x_amax, w, l.batch * p->n * p->k, f.w_amax, stream));
-        MXL_TRY(mxl_quantize_tensorwise(x, p->rows, p->k, l.k_ld, af, f.x_amax, p->need_dw ? lens : nullptr, p->need_dw ? G : 0, f.x_row.q, f.x_row.s,
-                                        sv.x_col.q, sv.x_col.s, sv.x_si, l.qf(), stream));
-        MXL_TRY(mxl_quantize_weight_tensorwise(w, l.batch, p->n, p->k, l.k_ld, l.n_ld, wf, f.w_amax, wr.q, wr.s, sv.w_col.q, sv.w_col.s, sv.w_si,
-                                               l.qf(), stream));
+        MXL_TRY(mxl::quantize_pair(both, stream));
         return mxl_grouped_gemm_nt_scaled(f.x_row.q, f.x_row.s, af, wr.q, wr.s, wf, y, lens, batch, p->rows, p->n, l.k_ld, sv.x_si, sv.w_si,
                                           MXL_GF_KSTEP, stream);
     }
@@ -169,10 +173,12 @@ extern "C" int mxl_linear_forward(const mxl_linear* p, const void* x, const void
         MXL_TRY(mxl_glu_probs_quantize(x, aux0, (int)p->probs_dtype, (const uint8_t*)aux1, p->rows, p->k, l.k_ld,
                                        p->input == MXL_LINEAR_SILU ? MXL_ACT_SILU : MXL_ACT_GELU, af, (int)p->scale_mode, lens, G, f.x_row.q,
                                        f.x_row.s, sv.x_col.q, sv.x_col.s, l.qf(), stream));
+    } else if (!p->w_quantized) {
+        MXL_TRY(mxl::quantize_pair(both, stream));
+        return mxl_grouped_gemm_nt_ex(f.x_row.q, f.x_row.s, af, wr.q, wr.s, wf, y, lens, batch, p->rows, p->n, l.k_ld, MXL_GF_KSTEP, stream);
     } else {
-        const bool rht = p->rht_signs >= 0 && p->need_dw;
-        MXL_TRY(mxl_quantize_ex(x, p->rows, p->k, l.k_ld, af, (int)p->scale_mode, lens, G, f.x_row.q, f.x_row.s, sv.x_col.q, sv.x_col.s,
-                                l.qf() | (rht ? MXL_QF_RHT_COL : 0u), 0, rht ? (uint32_t)p->rht_signs : 0u, stream));
+        MXL_TRY(mxl_quantize_ex(x, p->rows, p->k, l.k_ld, af, (int)p->scale_mode, lens, G, f.x_row.q, f.x_row.s, sv.x_col.q, sv.x_col.s, both.flags, 0,
+                                both.rht_signs, stream));
     }
     if (p->w_quantized) {
         if (!w_scales) return MXL_EINVAL;

@@ -1,0 +1,24 @@
+// Both operands of a linear's forward, quantised (mx_quantize.hip) for the calls in mx_linear.hip.
+#pragma once
+#include <stdint.h>
+
+namespace mxl {
+
+struct LinearOperands {
+    // activations [rows, k] (ragged groups: group_lens, num_groups; 0 and null: one), weights [batch, n, k]
+    const void *x, *w;
+    int64_t rows, batch, n, k, k_ld, n_ld;
+    const int64_t* group_lens;
+    int num_groups;
+    int x_fmt, w_fmt, scale_mode;
+    uint32_t flags, rht_signs;          // MXL_QF_* of mxl_quantize_ex (no stochastic rounding)
+    // tensor-wise scaling: abs-max of each on the device, and where 1 / scale goes; null otherwise
+    const float *x_amax, *w_amax;
+    float *x_scale_inv, *w_scale_inv;
+    // the copies; transposed ones may be null as mxl_quantize_ex and mxl_quantize_weight_2d_ex allow
+    uint8_t *xq_row, *xs_row, *xq_col, *xs_col, *wq_row, *ws_row, *wq_col, *ws_col;
+};
+// in one launch where there is a kernel for the two, else one after the other; the same bytes
+int quantize_pair(const LinearOperands& o, void* stream);
+
+}  // namespace mxl

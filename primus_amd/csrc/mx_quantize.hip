@@ -15,6 +15,7 @@
 // the 4 lane groups.  The transposed codes go through an LDS tile so that the
 // global stores are 128 contiguous bytes per output row.
 #include "mx_device.h"
+#include "mx_quantize.h"
 
 namespace mxl {
 
@@ -56,24 +57,28 @@ struct QuantArgs {
     uint64_t sr_seed;       // SR kernels: seed of the stochastic rounding
     uint32_t rht_signs;     // RHT kernels: sign bit i flips row i of every 16-row group before the transform
     int tiles_r, tiles_c;   // tile grid: row tiles (upper bound when grouped) x column tiles
-    int super_c, n_super;   // 8x8-tile supertiles: count along the columns, total
+    int super_c, n_super;   // supertiles: count along the columns, total
+    int super_log;          // log2 of a supertile's edge in tiles
 };
 
 // Workgroup -> tile.  Workgroups are dealt to the 8 XCDs round robin, so workgroup L is the
-// (L / 8)-th one of XCD L % 8.  Each XCD walks whole 8x8-tile supertiles, column tile fastest:
-//  - the 4-byte scale pieces that 8 neighbouring tiles write (32 contiguous bytes, along the columns
-//    for the row-wise copy and along the rows for the transposed one) meet in one L2 and leave it as
-//    one write instead of eight partial ones;
+// (L / 8)-th one of XCD L % 8.  Each XCD walks whole supertiles, column tile fastest:
+//  - the pieces of the scale arrays that neighbouring tiles write meet in one L2 and leave it as one write instead
+//    of several partial ones: 4 bytes of each of 8 neighbours in the row-major layouts, 2 + 2 bytes of each of 4 in a
+//    16-byte panel row;
 //  - the workgroups resident at any moment cover long contiguous row spans instead of one 256-byte
 //    column slice at a power-of-two stride, which would camp on a few memory channels.
-constexpr int QSUPER = 8;
-__device__ __forceinline__ bool quant_tile_of_workgroup(const QuantArgs& a, int& pt, int& ct) {
-    const int L = blockIdx.x, xcd = L & 7, k = L >> 3;
-    const int s = (k / (QSUPER * QSUPER)) * 8 + xcd;
+// 4 x 4 tiles with scale panels, 8 x 8 without: the XCDs' shares of a small tensor are the more even the smaller the
+// supertile (both copies of [1999, 5760]: 14.7 us on 8 x 8, 12.2 on 4 x 4 and on 2 x 2; [1000, 1024] 8.9, 7.2, 7.3; weight
+// [5760, 2880] 15.0, 13.8, 13.9; [8192, 14336] 93.3, 90.3, 91.7).
+__device__ __forceinline__ bool quant_tile_of_workgroup(const QuantArgs& a, int L, int& pt, int& ct) {
+    const int xcd = L & 7, k = L >> 3;
+    const int lg = a.super_log;
+    const int s = (k >> (2 * lg)) * 8 + xcd;
     if (s >= a.n_super) return false;
-    const int within = k % (QSUPER * QSUPER);
-    pt = (s / a.super_c) * QSUPER + within / QSUPER;
-    ct = (s % a.super_c) * QSUPER + within % QSUPER;
+    const int within = k & ((1 << (2 * lg)) - 1);
+    pt = ((s / a.super_c) << lg) + (within >> lg);
+    ct = ((s % a.super_c) << lg) + (within & ((1 << lg) - 1));
     return pt < a.tiles_r && ct < a.tiles_c;
 }
 
@@ -110,7 +115,7 @@ __device__ __forceinline__ void store_panel_scales(uint8_t* row16, int quarter, 
 }
 
 template <int FMT, int SMODE, bool ROW, bool COL, bool TWOD, int ACT = -1, bool SR = false, bool RHT = false>
-__global__ __launch_bounds__(QTHREADS) void mx_quant_kernel(QuantArgs a) {
+__device__ __forceinline__ void quant_workgroup(const QuantArgs& a, int block) {
     constexpr bool FP4 = (FMT == kFmtE2M1);
     constexpr bool TENSOR = (SMODE == SCALE_TENSOR);
     static_assert(TENSOR || FMT != kFmtE5M2, "E5M2 exists for tensor-wise scaling only");
@@ -130,10 +135,10 @@ __global__ __launch_bounds__(QTHREADS) void mx_quant_kernel(QuantArgs a) {
         const float amax = *a.tensor_amax;
         tensor_bad = !(amax < __uint_as_float(0x7F800000u));
         tscale = (FMT == kFmtE5M2 ? 57344.f : 448.f) / fmaxf(amax, 1e-12f);
-        if (blockIdx.x == 0 && t == 0 && a.scale_inv_out) *a.scale_inv_out = 1.0f / tscale;
+        if (block == 0 && t == 0 && a.scale_inv_out) *a.scale_inv_out = 1.0f / tscale;
     }
     int pt, ct;
-    if (!quant_tile_of_workgroup(a, pt, ct)) return;   // uniform over the workgroup
+    if (!quant_tile_of_workgroup(a, block, pt, ct)) return;   // uniform over the workgroup
     const int64_t col0 = (int64_t)ct * QT;
 
     // ---- which source rows does this tile hold? ----
@@ -499,6 +504,23 @@ __global__ __launch_bounds__(QTHREADS) void mx_quant_kernel(QuantArgs a) {
     }
 }
 
+template <int FMT, int SMODE, bool ROW, bool COL, bool TWOD, int ACT = -1, bool SR = false, bool RHT = false>
+__global__ __launch_bounds__(QTHREADS) void mx_quant_kernel(QuantArgs a) {
+    quant_workgroup<FMT, SMODE, ROW, COL, TWOD, ACT, SR, RHT>(a, (int)blockIdx.x);
+}
+
+// Both operands of a linear's forward in one launch: the activations' two copies (the first x_wgs workgroups) and the
+// weight's (WCOL: its transposed codes too).  Neither fills the chip for long where the linear is small, and each launch
+// costs its fill and drain and the gap behind it.  Forward of a linear, quantisers and GEMM, two launches / one, us:
+// [256, 4096] x 4096 39.8 / 34.0; [1999, 2880] x 5760 67.9 / 62.8; [8192, 4096] x 14336 422 / 412; tensor-wise [4096, 14336] x
+// 4096 279 / 272; 8 experts of [2048, 2048], 2048 rows, 56 / 51.  Large experts read their weights at 108 registers a lane
+// instead of 58, which costs them nothing (32 x [4096, 7168], 8192 rows, 860 / 865; 8 x [28672, 4096], 512 rows, 694 / 668).
+template <int FMT, int SMODE, bool WCOL>
+__global__ __launch_bounds__(QTHREADS) void mx_quant_pair_kernel(QuantArgs x, QuantArgs w, unsigned x_wgs) {
+    if (blockIdx.x < x_wgs) quant_workgroup<FMT, SMODE, true, true, false>(x, (int)blockIdx.x);
+    else quant_workgroup<FMT, SMODE, true, WCOL, true>(w, (int)(blockIdx.x - x_wgs));
+}
+
 // ---------------------------------------------------------------------------
 // dequantise: codes + scales -> bf16 (row-wise layout)
 // ---------------------------------------------------------------------------
@@ -559,17 +581,34 @@ __global__ __launch_bounds__(256) void mx_dequant_kernel(const uint8_t* q, const
 // ---------------------------------------------------------------------------
 // host-side dispatch
 // ---------------------------------------------------------------------------
-template <int FMT, int SMODE, bool TWOD, int ACT = -1, bool SR = false, bool RHT = false>
-static int launch_quant(QuantArgs& a, int64_t tiles_r, int64_t tiles_c, hipStream_t st) {
-    const int64_t super_r = (tiles_r + QSUPER - 1) / QSUPER, super_c = (tiles_c + QSUPER - 1) / QSUPER;
+// the activations of a pair, prepared and not yet launched; lives on the stack of the call that launches both
+struct HeldQuant {
+    bool held = false;
+    int fmt, smode;          // smode: SCALE_TENSOR or an MXL_SCALE_*
+    QuantArgs a;
+    int64_t wgs;
+};
+
+// fills in the launch's tile grid; its workgroups
+static int quant_grid(QuantArgs& a, int64_t tiles_r, int64_t tiles_c, int64_t* wgs) {
+    const int lg = a.kchunk >= 2 ? 2 : 3;
+    const int64_t side = (int64_t)1 << lg, super_r = (tiles_r + side - 1) / side, super_c = (tiles_c + side - 1) / side;
     const int64_t n_super = super_r * super_c;
-    const int64_t wgs = (n_super + 7) / 8 * 8 * QSUPER * QSUPER;
-    if (tiles_r > 0x7FFFFFFF || tiles_c > 0x7FFFFFFF || wgs > 0x7FFFFFFF) return MXL_EINVAL;
+    *wgs = (n_super + 7) / 8 * 8 * side * side;
+    if (tiles_r > 0x7FFFFFFF || tiles_c > 0x7FFFFFFF || *wgs > 0x7FFFFFFF) return MXL_EINVAL;
     if (!device_is_gfx950()) return MXL_ENODEV;
     a.tiles_r = (int)tiles_r;
     a.tiles_c = (int)tiles_c;
     a.super_c = (int)super_c;
+    a.super_log = lg;
     a.n_super = (int)n_super;
+    return MXL_OK;
+}
+
+template <int FMT, int SMODE, bool TWOD, int ACT = -1, bool SR = false, bool RHT = false>
+static int launch_quant(QuantArgs& a, int64_t tiles_r, int64_t tiles_c, hipStream_t st) {
+    int64_t wgs;
+    if (const int rc = quant_grid(a, tiles_r, tiles_c, &wgs)) return rc;
     const dim3 grid((unsigned)wgs);
     const bool row = a.q_row != nullptr, col = a.q_colT != nullptr;
     if (row && col)
@@ -613,6 +652,29 @@ template <bool TWOD>
 static int dispatch_quant_tensor(int fmt, QuantArgs& a, int64_t tiles_r, int64_t tiles_c, hipStream_t st) {
     if (fmt == MXL_FMT_E4M3) return launch_quant<MXL_FMT_E4M3, SCALE_TENSOR, TWOD>(a, tiles_r, tiles_c, st);
     if (fmt == MXL_FMT_E5M2) return launch_quant<MXL_FMT_E5M2, SCALE_TENSOR, TWOD>(a, tiles_r, tiles_c, st);
+    return MXL_EINVAL;
+}
+
+// both launches of a pair in one; false: there is no kernel for it
+static bool pair_taken(const HeldQuant& x, int fmt, int smode, const QuantArgs& w) {
+    return x.fmt == fmt && x.smode == smode && (smode == MXL_SCALE_OCP_FLOOR || smode == SCALE_TENSOR) && x.a.q_row && x.a.q_colT && w.q_row &&
+           (fmt == MXL_FMT_E4M3 || (fmt == MXL_FMT_E2M1 && smode == MXL_SCALE_OCP_FLOOR));
+}
+static int launch_quant_pair(const HeldQuant& x, QuantArgs& w, int64_t tiles_r, int64_t tiles_c, hipStream_t st) {
+    int64_t wgs;
+    if (const int rc = quant_grid(w, tiles_r, tiles_c, &wgs)) return rc;
+    if (x.wgs + wgs > 0x7FFFFFFF) return MXL_EINVAL;
+    const dim3 grid((unsigned)(x.wgs + wgs));
+#define MXL_QP(F, S)                                                                                                                      \
+    if (x.fmt == F && x.smode == S) {                                                                                                     \
+        if (w.q_colT) hipLaunchKernelGGL((mx_quant_pair_kernel<F, S, true>), grid, dim3(QTHREADS), 0, st, x.a, w, (unsigned)x.wgs);       \
+        else hipLaunchKernelGGL((mx_quant_pair_kernel<F, S, false>), grid, dim3(QTHREADS), 0, st, x.a, w, (unsigned)x.wgs);              \
+        return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;                                                                    \
+    }
+    MXL_QP(MXL_FMT_E4M3, MXL_SCALE_OCP_FLOOR)
+    MXL_QP(MXL_FMT_E2M1, MXL_SCALE_OCP_FLOOR)
+    MXL_QP(MXL_FMT_E4M3, SCALE_TENSOR)
+#undef MXL_QP
     return MXL_EINVAL;
 }
 
@@ -718,7 +780,7 @@ static int quantize_1d(const void* x_bf16, int64_t rows, int64_t cols, int64_t r
                        int act, const void* probs, int probs_dtype, const uint8_t* row_mask, void* stream,
                        bool sr = false, uint64_t sr_seed = 0, bool rht = false, uint32_t rht_signs = 0,
                        int kchunk = 0, const void* norm_w = nullptr, const void* tensor_amax = nullptr,
-                       void* scale_inv_out = nullptr) {
+                       void* scale_inv_out = nullptr, HeldQuant* hold = nullptr) {
     if (row_ld == 0) row_ld = cols;
     if (kchunk < 0) return MXL_EINVAL;                  // contradictory layout flags
     if (kchunk == 2 && fmt == MXL_FMT_E2M1) kchunk = 3;  // E2M1 activations: the K step is 128 elements (64-byte rows)
@@ -757,6 +819,13 @@ static int quantize_1d(const void* x_bf16, int64_t rows, int64_t cols, int64_t r
     a.chunk_rows_col = cols;
     const int64_t gx = q_colT ? a.W / QT : (rows + QT - 1) / QT;
     const int64_t gy = ((q_row ? row_ld : cols) + QT - 1) / QT;
+    if (hold && gx > 0 && !sr && !rht && act < 0) {
+        hold->held = true;
+        hold->fmt = fmt;
+        hold->smode = tensor_amax ? SCALE_TENSOR : scale_mode;
+        hold->a = a;
+        return quant_grid(hold->a, gx, gy, &hold->wgs);
+    }
     if (tensor_amax) {
         if (sr || rht || act >= 0) return MXL_EINVAL;
         if (gx == 0) return MXL_OK;   // nothing to quantise (scale_inv_out is then left unwritten)
@@ -812,7 +881,8 @@ extern "C" int mxl_rmsnorm_quantize(const void* x_bf16, const void* w_bf16, cons
 
 static int quantize_weight_2d(const void* w_bf16, int64_t batch, int64_t n, int64_t k, int64_t k_ld, int64_t n_ld, int fmt,
                               int scale_mode, void* q_row, void* s_row, void* q_colT, void* s_colT, int kchunk,
-                              void* stream, const void* tensor_amax = nullptr, void* scale_inv_out = nullptr) {
+                              void* stream, const void* tensor_amax = nullptr, void* scale_inv_out = nullptr,
+                              const HeldQuant* pair = nullptr, bool* paired = nullptr) {
     if (k_ld == 0) k_ld = k;
     if (n_ld == 0) n_ld = n;
     if (kchunk < 0 || (kchunk == 3 && fmt != MXL_FMT_E2M1)) return MXL_EINVAL;
@@ -850,9 +920,37 @@ static int quantize_weight_2d(const void* w_bf16, int64_t batch, int64_t n, int6
     a.chunk_rows_col = batch * k;
     const int64_t gx = batch * ((n + QT - 1) / QT);
     const int64_t gy = ((q_row ? k_ld : k) + QT - 1) / QT;
+    if (pair) {
+        *paired = pair->held && pair_taken(*pair, fmt, tensor_amax ? SCALE_TENSOR : scale_mode, a);
+        return *paired ? launch_quant_pair(*pair, a, gx, gy, (hipStream_t)stream) : MXL_OK;
+    }
     if (tensor_amax) return dispatch_quant_tensor<true>(fmt, a, gx, gy, (hipStream_t)stream);
     return dispatch_quant<true>(fmt, scale_mode, a, gx, gy, (hipStream_t)stream);
 }
+
+namespace mxl {
+int quantize_pair(const LinearOperands& o, void* stream) {
+    const int lay = qf_layout(o.flags);
+    const bool rht = (o.flags & MXL_QF_RHT_COL) != 0;
+    auto x = [&](HeldQuant* hold) {
+        return quantize_1d(o.x, o.rows, o.k, o.k_ld, o.x_fmt, o.scale_mode, o.group_lens, o.num_groups, o.xq_row, o.xs_row, o.xq_col, o.xs_col, -1,
+                           nullptr, MXL_PROBS_F32, nullptr, stream, false, 0, rht, o.rht_signs, lay, nullptr, o.x_amax, o.x_scale_inv, hold);
+    };
+    auto w = [&](const HeldQuant* pair, bool* paired) {
+        return quantize_weight_2d(o.w, o.batch, o.n, o.k, o.k_ld, o.n_ld, o.w_fmt, o.scale_mode, o.wq_row, o.ws_row, o.wq_col, o.ws_col, lay,
+                                  stream, o.w_amax, o.w_scale_inv, pair, paired);
+    };
+    HeldQuant hold;
+    bool paired = false;
+    if (!rht && o.xq_col) {
+        if (const int rc = x(&hold)) return rc;
+        if (const int rc = w(&hold, &paired)) return rc;
+        if (paired) return MXL_OK;
+    }
+    if (const int rc = x(nullptr)) return rc;
+    return w(nullptr, nullptr);
+}
+}  // namespace mxl
 
 extern "C" int mxl_quantize_weight_2d(const void* w_bf16, int64_t batch, int64_t n, int64_t k, int64_t k_ld,
                                       int64_t n_ld, int fmt, int scale_mode, void* q_row, void* s_row, void* q_colT,
