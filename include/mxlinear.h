@@ -505,9 +505,12 @@ int mxl_shuffle_scales(const void* src, int64_t rows, int64_t cols, void* dst, i
  *   w         bf16 [groups, n, k], or with w_quantized the row-wise codes (w_scales: their scales); the backward is then
  *             given the transposed copy (wt, wt_scales).
  *   dx_from_rows  the backward reads the row-wise codes transposed (MXL_GF_B_TRANSPOSED); n and k multiples of 128.
- * recipe MXL_LINEAR_TENSORWISE takes plain inputs and bf16 weights.  rows > 0. */
+ * recipe MXL_LINEAR_TENSORWISE takes plain inputs and bf16 weights.  MXL_LINEAR_BLOCKWISE (the 128-blockwise recipe: row-major
+ * copies, n and k multiples of 128, no fused accumulation) does too; its backward starts from the bf16 tensors again and is
+ * given x and, as wt, w.  rows > 0. */
 #define MXL_LINEAR_MX 0
 #define MXL_LINEAR_TENSORWISE 1
+#define MXL_LINEAR_BLOCKWISE 2
 #define MXL_LINEAR_PLAIN 0
 #define MXL_LINEAR_SILU 1
 #define MXL_LINEAR_GELU 2

@@ -100,7 +100,7 @@ class Linear(ctypes.Structure):
         (name, ctypes.c_int64) for name in ("saved_bytes", "fwd_bytes", "bwd_bytes")]
 
 
-LINEAR_MX, LINEAR_TENSORWISE = 0, 1
+LINEAR_MX, LINEAR_TENSORWISE, LINEAR_BLOCKWISE = 0, 1, 2
 LINEAR_PLAIN, LINEAR_SILU, LINEAR_GELU, LINEAR_RMSNORM = 0, 1, 2, 3
 LINEAR_QUANTIZE, LINEAR_DX, LINEAR_DW = 1, 2, 4
 

@@ -15,6 +15,7 @@
 // kernels, both of 8 waves, two per SIMD: a 128 x 256 tile with all four partial tiles of a wave's 64 x 64 at once
 // (small problems), and a 256 x 256 tile whose waves own 64 x 128 and keep one column of partial tiles at a time.
 #include "mx_device.h"
+#include "mx_blockwise.h"
 
 namespace mxl {
 
@@ -53,7 +54,7 @@ struct BwQuantArgs {
     const int64_t* group_lens;
     int num_groups;
     int64_t W;
-    int tiles_r, tiles_c, super_c, n_super;   // the launch's tile grid and its 8 x 8 supertiles
+    int tiles_r, tiles_c, super_c, n_super;   // a matrix's tile grid and its 4 x 4 supertiles
 };
 
 constexpr int BW_MAX_GROUPS = 1024;
@@ -136,28 +137,39 @@ template <int FMT> __device__ __forceinline__ uint2 bw_cvt8(uint32_t p0, uint32_
     return o;
 }
 
+struct BwQuantLds {
+    __attribute__((aligned(16))) uint8_t t_tile[BW * BW_TPITCH];
+    __attribute__((aligned(16))) uint32_t amax_r[BW];         // per row
+    __attribute__((aligned(16))) uint32_t amax_c[4][BW / 2];  // per wave: column pairs, packed 16-bit maxima
+    __attribute__((aligned(16))) uint32_t scale_r[BW], scale_c[BW];
+    int64_t grp_red[4];
+    uint32_t amax_w[4];
+    int grp_pre[BW_MAX_GROUPS + 1];
+};
+
+// workgroup L of matrix zoff (TWOD) of tensor `a`
 template <int FMT, bool TWOD>
-__global__ __launch_bounds__(BW_THREADS) void bw_quant_kernel(BwQuantArgs a) {
-    __shared__ __attribute__((aligned(16))) uint8_t t_tile[BW * BW_TPITCH];
-    __shared__ __attribute__((aligned(16))) uint32_t amax_r[BW];         // per row
-    __shared__ __attribute__((aligned(16))) uint32_t amax_c[4][BW / 2];  // per wave: column pairs, packed 16-bit maxima
-    __shared__ __attribute__((aligned(16))) uint32_t scale_r[BW], scale_c[BW];
-    __shared__ uint32_t amax_w[4];
-    __shared__ int grp_pre[BW_MAX_GROUPS + 1];
-    __shared__ int64_t grp_red[4];
+__device__ __forceinline__ void bw_quant_workgroup(const BwQuantArgs& a, int L, int64_t zoff, BwQuantLds& lds) {
+    auto& t_tile = lds.t_tile;
+    auto& amax_r = lds.amax_r;
+    auto& amax_c = lds.amax_c;
+    auto& scale_r = lds.scale_r;
+    auto& scale_c = lds.scale_c;
+    auto& amax_w = lds.amax_w;
+    auto& grp_pre = lds.grp_pre;
+    auto& grp_red = lds.grp_red;
     const int t = threadIdx.x;
     const int w = t >> 6, l = t & 63, c16 = l & 15, rg = l >> 4, rbase = 32 * w + 8 * rg;
-    // Tile order: consecutive workgroup ids land on different XCDs, and every XCD walks whole 8 x 8 supertiles (column
-    // tile fastest): the 4-byte factors that 8 neighbouring tiles write into one row of sinv_row (32 contiguous bytes)
-    // then meet in one L2, and the resident workgroups of an XCD cover long contiguous row spans.
-    const int L = blockIdx.x, xcd = L & 7, kk = L >> 3;
-    const int sup = (kk >> 6) * 8 + xcd;
+    // Tile order: consecutive workgroup ids land on different XCDs, and every XCD walks whole 4 x 4 supertiles (column
+    // tile fastest): the 4-byte factors that neighbouring tiles write into one row of sinv_row then meet in one L2, the
+    // resident workgroups of an XCD cover long contiguous row spans, and the XCDs' shares of a small tensor are even.
+    const int xcd = L & 7, kk = L >> 3;
+    const int sup = (kk >> 4) * 8 + xcd;
     if (sup >= a.n_super) return;
-    const int bx = (sup % a.super_c) * 8 + (kk & 7), by = (sup / a.super_c) * 8 + ((kk >> 3) & 7);
+    const int bx = (sup % a.super_c) * 4 + (kk & 3), by = (sup / a.super_c) * 4 + ((kk >> 2) & 3);
     if (bx >= a.tiles_c || by >= a.tiles_r) return;
     const int64_t col0 = (int64_t)bx * BW;
     // the tile's rows: rows [row0, row0 + valid) of this matrix land in columns [prow0, prow0 + 128) of the transposed copy
-    const int64_t zoff = TWOD ? (int64_t)blockIdx.y : 0;          // matrix of a batch of weights
     int64_t row0 = (int64_t)by * BW, prow0 = row0, rows_pad = (a.rows + BW - 1) / BW * BW;
     int64_t valid64 = a.rows - row0 < BW ? a.rows - row0 : BW;
     if (!TWOD && a.group_lens != nullptr) {
@@ -316,6 +328,29 @@ __global__ __launch_bounds__(BW_THREADS) void bw_quant_kernel(BwQuantArgs a) {
             store16_streaming(dst + (int64_t)c * rows_pad + 16 * ch, *(const uint4*)(t_tile + c * BW_TPITCH + 16 * ch));
         }
     }
+}
+
+// Up to three tensors in one launch: a linear's forward quantises its input and its weight, its backward the gradient, the
+// input again and the weight again, none of which waits for another.  Workgroups [0, end[0]) are the first tensor's, and so
+// on; those of a batch of weights go through its matrices one after the other.  A launch of an ordinary linear's tensor
+// lasts 12 to 17 us, of which a third is filling and draining the chip and the gap to the next one.  Five launches to two
+// over a forward and backward: [3000, 7168] x 2048 250 -> 236 us, [4096, 4096] x 4096 299 -> 288, [8192, 4096] x 14336 1665 -> 1638;
+// what small linears gain on top of that is host time (mx_linear.hip).
+constexpr int BW_SEVERAL = 3;
+struct BwQuantSeveral {
+    BwQuantArgs a[BW_SEVERAL];
+    int end[BW_SEVERAL];        // first workgroup behind each
+    int per_mat[BW_SEVERAL];    // workgroups of a matrix; 0: 1-D blocks
+};
+template <int FMT>
+__global__ __launch_bounds__(BW_THREADS) void bw_quant_kernel(BwQuantSeveral s) {
+    __shared__ BwQuantLds lds;
+    const int block = (int)blockIdx.x;
+    int i = 0, first = 0;
+    while (i < BW_SEVERAL - 1 && block >= s.end[i]) first = s.end[i++];
+    const int per = s.per_mat[i];
+    if (per == 0) bw_quant_workgroup<FMT, false>(s.a[i], block - first, 0, lds);
+    else bw_quant_workgroup<FMT, true>(s.a[i], (block - first) % per, (block - first) / per, lds);
 }
 
 // ------------------------------------------------------------------------------------------------------------
@@ -874,36 +909,46 @@ __global__ __launch_bounds__(BWG_THREADS) void bw_gemm256_kernel(BwGemmArgs p) {
         }
 }
 
-template <bool TWOD>
-static int launch_bw_quant(const BwQuantArgs& a, int fmt, int64_t row_tiles, int batch, hipStream_t st) {
-    const int64_t wgs = (int64_t)(a.n_super + 7) / 8 * 8 * 64;
-    if (wgs > 0x7FFFFFFF) return MXL_EINVAL;
-    const dim3 grid((unsigned)wgs, (unsigned)batch);
-    if (fmt == MXL_FMT_E4M3) hipLaunchKernelGGL((bw_quant_kernel<MXL_FMT_E4M3, TWOD>), grid, dim3(BW_THREADS), 0, st, a);
-    else hipLaunchKernelGGL((bw_quant_kernel<MXL_FMT_E5M2, TWOD>), grid, dim3(BW_THREADS), 0, st, a);
-    return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;
-}
-
-static int bw_quant(const void* x, int64_t rows, int64_t cols, int fmt, const int64_t* group_lens, int num_groups, int batch,
-                    void* q_row, void* sinv_row, void* q_colT, void* sinv_colT, bool twod, void* stream) {
-    if (rows < 0 || cols <= 0 || cols % BW != 0 || (fmt != MXL_FMT_E4M3 && fmt != MXL_FMT_E5M2)) return MXL_EINVAL;
-    if ((q_row == nullptr) != (sinv_row == nullptr) || (q_colT == nullptr) != (sinv_colT == nullptr)) return MXL_EINVAL;
-    if (!q_row && !q_colT) return MXL_EINVAL;
-    if (batch < 1 || batch > 65535 || (twod && rows % BW != 0) || (!twod && batch != 1)) return MXL_EINVAL;
-    if (num_groups < 0 || num_groups > BW_MAX_GROUPS || (num_groups > 0) != (group_lens != nullptr) || (twod && num_groups)) return MXL_EINVAL;
-    const int64_t W = num_groups ? mxl_padded_width(rows, num_groups) : (rows + BW - 1) / BW * BW;
+// checks one tensor and adds it to the launch (nothing to add: MXL_OK)
+static int bw_quant_add(BwQuantSeveral& s, int& count, const BwTensor& o, int fmt) {
+    const bool twod = o.batch > 0;
+    const int batch = twod ? (int)o.batch : 1, num_groups = o.num_groups;
+    if (o.rows < 0 || o.cols <= 0 || o.cols % BW != 0 || (fmt != MXL_FMT_E4M3 && fmt != MXL_FMT_E5M2)) return MXL_EINVAL;
+    if ((o.q_row == nullptr) != (o.sinv_row == nullptr) || (o.q_colT == nullptr) != (o.sinv_colT == nullptr)) return MXL_EINVAL;
+    if (!o.q_row && !o.q_colT) return MXL_EINVAL;
+    if (o.batch < 0 || o.batch > 65535 || (twod && o.rows % BW != 0)) return MXL_EINVAL;
+    if (o.num_groups < 0 || o.num_groups > BW_MAX_GROUPS || (num_groups > 0) != (o.group_lens != nullptr) || (twod && num_groups)) return MXL_EINVAL;
+    const int64_t W = num_groups ? mxl_padded_width(o.rows, num_groups) : (o.rows + BW - 1) / BW * BW;
     const int64_t row_tiles = W / BW;       // with groups: the 128-column pieces of the padded transposed copy
     if (row_tiles == 0) return MXL_OK;
-    if (!x && rows > 0) return MXL_EINVAL;
-    if (((uintptr_t)x & 15) != 0 || row_tiles > 65535) return MXL_EINVAL;
-    if ((((uintptr_t)q_row | (uintptr_t)q_colT) & 15) != 0) return MXL_EINVAL;
-    if (!device_is_gfx950()) return MXL_ENODEV;
-    const int tiles_c = (int)(cols / BW), super_c = (tiles_c + 7) / 8, super_r = (int)((row_tiles + 7) / 8);
+    if (!o.x && o.rows > 0) return MXL_EINVAL;
+    if (((uintptr_t)o.x & 15) != 0 || row_tiles > 65535) return MXL_EINVAL;
+    if ((((uintptr_t)o.q_row | (uintptr_t)o.q_colT) & 15) != 0) return MXL_EINVAL;
+    const int tiles_c = (int)(o.cols / BW), super_c = (tiles_c + 3) / 4, super_r = (int)((row_tiles + 3) / 4);
     if ((int64_t)super_c * super_r > 0x7FFFFFF) return MXL_EINVAL;
-    BwQuantArgs a{(const uint16_t*)x, rows, cols, (uint8_t*)q_row, (float*)sinv_row, (uint8_t*)q_colT, (float*)sinv_colT,
-                  group_lens, num_groups, W, (int)row_tiles, tiles_c, super_c, super_c * super_r};
-    return twod ? launch_bw_quant<true>(a, fmt, row_tiles, batch, (hipStream_t)stream)
-                : launch_bw_quant<false>(a, fmt, row_tiles, 1, (hipStream_t)stream);
+    const int64_t per_mat = ((int64_t)super_c * super_r + 7) / 8 * 8 * 16, first = count ? s.end[count - 1] : 0;
+    if (first + per_mat * batch > 0x7FFFFFFF) return MXL_EINVAL;
+    s.a[count] = BwQuantArgs{(const uint16_t*)o.x, o.rows, o.cols, (uint8_t*)o.q_row, (float*)o.sinv_row, (uint8_t*)o.q_colT, (float*)o.sinv_colT,
+                             o.group_lens, num_groups, W, (int)row_tiles, tiles_c, super_c, super_c * super_r};
+    s.per_mat[count] = twod ? (int)per_mat : 0;
+    s.end[count] = (int)(first + per_mat * batch);
+    ++count;
+    return MXL_OK;
+}
+
+int bw_quantize(const BwTensor* tensors, int n, int fmt, void* stream) {
+    if (n < 1 || n > BW_SEVERAL || !tensors) return MXL_EINVAL;
+    BwQuantSeveral s{};
+    int count = 0;
+    for (int i = 0; i < n; ++i)
+        if (const int rc = bw_quant_add(s, count, tensors[i], fmt)) return rc;
+    if (count == 0) return MXL_OK;
+    if (!device_is_gfx950()) return MXL_ENODEV;
+    const int wgs = s.end[count - 1];
+    for (int i = count; i < BW_SEVERAL; ++i) s.end[i] = wgs;
+    if (fmt == MXL_FMT_E4M3) hipLaunchKernelGGL((bw_quant_kernel<MXL_FMT_E4M3>), dim3((unsigned)wgs), dim3(BW_THREADS), 0, (hipStream_t)stream, s);
+    else hipLaunchKernelGGL((bw_quant_kernel<MXL_FMT_E5M2>), dim3((unsigned)wgs), dim3(BW_THREADS), 0, (hipStream_t)stream, s);
+    return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;
 }
 
 // The dynamic LDS size is above the default limit.  The attribute belongs to the (kernel, device) pair and is set at
@@ -1031,13 +1076,15 @@ using namespace mxl;
 
 extern "C" int mxl_quantize_blockwise(const void* x_bf16, int64_t rows, int64_t cols, int fmt, const int64_t* group_lens,
                                       int num_groups, void* q_row, void* sinv_row, void* q_colT, void* sinv_colT, void* stream) {
-    return bw_quant(x_bf16, rows, cols, fmt, group_lens, num_groups, 1, q_row, sinv_row, q_colT, sinv_colT, false, stream);
+    const BwTensor o = {x_bf16, rows, cols, 0, group_lens, num_groups, q_row, sinv_row, q_colT, sinv_colT};
+    return bw_quantize(&o, 1, fmt, stream);
 }
 
 extern "C" int mxl_quantize_blockwise_weight(const void* w_bf16, int64_t batch, int64_t n, int64_t k, int fmt, void* q, void* sinv,
                                              void* q_T, void* sinv_T, void* stream) {
     if (batch < 1 || batch > 65535) return MXL_EINVAL;
-    return bw_quant(w_bf16, n, k, fmt, nullptr, 0, (int)batch, q, sinv, q_T, sinv_T, true, stream);
+    const BwTensor o = {w_bf16, n, k, batch, nullptr, 0, q, sinv, q_T, sinv_T};
+    return bw_quantize(&o, 1, fmt, stream);
 }
 
 extern "C" int mxl_blockwise_gemm_tile(int rows) {

@@ -6,6 +6,7 @@
 // direction; the layout of the buffers is arithmetic on the sizes and is worked out again in every call.
 #include "mx_gemm_tile.h"
 #include "mx_quantize.h"
+#include "mx_blockwise.h"
 
 namespace {
 
@@ -40,6 +41,7 @@ struct Linear {
     }
     bool mx() const { return p.recipe == MXL_LINEAR_MX; }
     bool tensorwise() const { return p.recipe == MXL_LINEAR_TENSORWISE; }
+    bool blockwise() const { return p.recipe == MXL_LINEAR_BLOCKWISE; }
     uint32_t qf() const { return MXL_QF_KSTEP | (f44 ? MXL_QF_KSTEP128 : 0u); }
 
     // K-step-major copies of [rows, ld] (ld padded): codes, scale panels
@@ -112,8 +114,41 @@ struct BackwardScratch {
     }
 };
 
+// The 128-blockwise recipe (forward and backward of [1024, 2048] x 2048 190 -> 108 us in two calls, [256, 4096] x 4096 191 ->
+// 119; launch by launch it is bound by the host there).  Forward: row-wise copies of x and w.  Backward, from the bf16 tensors: both copies of dy, the
+// transposed ones of x and w.
+struct BwForward {
+    Copy x, w;
+    BwForward(const Linear& l, Arena& a) {
+        const mxl_linear& p = l.p;
+        x.q = a.take(p.rows * p.k);
+        x.s = a.take(p.rows * (p.k / 128) * 4);
+        w.q = a.take(l.batch * p.n * p.k);
+        w.s = a.take(l.batch * (p.n / 128) * (p.k / 128) * 4);
+    }
+};
+struct BwBackward {
+    Copy d_row, d_col, x_col, w_col;
+    BwBackward(const Linear& l, Arena& a) {
+        const mxl_linear& p = l.p;
+        if (p.need_dx) {
+            d_row.q = a.take(p.rows * p.n);
+            d_row.s = a.take(p.rows * (p.n / 128) * 4);
+            w_col.q = a.take(l.batch * p.k * p.n);
+            w_col.s = a.take(l.batch * (p.k / 128) * (p.n / 128) * 4);
+        }
+        if (p.need_dw) {
+            d_col.q = a.take(p.n * l.width);
+            d_col.s = a.take(p.n * (l.width / 128) * 4);
+            x_col.q = a.take(p.k * l.width);
+            x_col.s = a.take(p.k * (l.width / 128) * 4);
+        }
+    }
+};
+
 bool valid(const mxl_linear* p) {
     if (!p || p->rows <= 0 || p->n <= 0 || p->k <= 0 || p->n % MXL_BLOCK || p->k % MXL_BLOCK || p->groups < 0 || p->groups > MXL_MAX_GROUPS) return false;
+    if (p->recipe == MXL_LINEAR_BLOCKWISE) return p->input == MXL_LINEAR_PLAIN && !p->w_quantized && p->n % 128 == 0 && p->k % 128 == 0;
     if (p->recipe != MXL_LINEAR_MX && p->recipe != MXL_LINEAR_TENSORWISE) return false;
     if (p->recipe == MXL_LINEAR_TENSORWISE && (p->input != MXL_LINEAR_PLAIN || p->w_quantized)) return false;
     if (p->input < MXL_LINEAR_PLAIN || p->input > MXL_LINEAR_RMSNORM) return false;
@@ -128,10 +163,60 @@ bool valid(const mxl_linear* p) {
         if (rc_ != MXL_OK) return rc_;   \
     } while (0)
 
+namespace {
+
+int bw_forward(const Linear& l, const void* x, const void* w, const int64_t* lens, void* scratch, void* y, void* stream) {
+    const mxl_linear& p = l.p;
+    Arena a(scratch);
+    const BwForward f(l, a);
+    const int fmt = (int)p.act_fmt;
+    const mxl::BwTensor in[2] = {{x, p.rows, p.k, 0, nullptr, 0, f.x.q, f.x.s, nullptr, nullptr},
+                                 {w, p.n, p.k, l.batch, nullptr, 0, f.w.q, f.w.s, nullptr, nullptr}};
+    MXL_TRY(mxl::bw_quantize(in, 2, fmt, stream));
+    if (p.groups) return mxl_grouped_gemm_nt_blockwise(f.x.q, f.x.s, fmt, f.w.q, f.w.s, fmt, y, lens, (int)p.groups, p.rows, p.n, p.k, stream);
+    return mxl_gemm_nt_blockwise(f.x.q, f.x.s, fmt, f.w.q, f.w.s, fmt, 128, y, p.rows, p.n, p.k, stream);
+}
+
+int bw_backward(const Linear& l, int parts, const void* dy, const void* x, const void* w, const int64_t* lens, void* scratch, void* dx, void* dw,
+                void* stream) {
+    const mxl_linear& p = l.p;
+    Arena a(scratch);
+    const BwBackward b(l, a);
+    const int fmt = (int)p.grad_fmt, G = (int)p.groups;
+    if ((parts & MXL_LINEAR_QUANTIZE) && (p.need_dx || p.need_dw)) {
+        if (!dy || (p.need_dw && !x) || (p.need_dx && !w)) return MXL_EINVAL;
+        mxl::BwTensor in[3];
+        int count = 0;
+        in[count++] = {dy, p.rows, p.n, 0, p.need_dw ? lens : nullptr, p.need_dw ? G : 0, b.d_row.q, b.d_row.s, b.d_col.q, b.d_col.s};
+        if (p.need_dw) in[count++] = {x, p.rows, p.k, 0, lens, G, nullptr, nullptr, b.x_col.q, b.x_col.s};
+        if (p.need_dx) in[count++] = {w, p.n, p.k, l.batch, nullptr, 0, nullptr, nullptr, b.w_col.q, b.w_col.s};
+        MXL_TRY(mxl::bw_quantize(in, count, fmt, stream));
+    }
+    if ((parts & MXL_LINEAR_DX) && p.need_dx) {
+        if (G) MXL_TRY(mxl_grouped_gemm_nt_blockwise(b.d_row.q, b.d_row.s, fmt, b.w_col.q, b.w_col.s, fmt, dx, lens, G, p.rows, p.k, p.n, stream));
+        else MXL_TRY(mxl_gemm_nt_blockwise(b.d_row.q, b.d_row.s, fmt, b.w_col.q, b.w_col.s, fmt, 128, dx, p.rows, p.k, p.n, stream));
+    }
+    if ((parts & MXL_LINEAR_DW) && p.need_dw) {
+        if (G) return mxl_grouped_gemm_wgrad_blockwise(b.d_col.q, b.d_col.s, fmt, b.x_col.q, b.x_col.s, fmt, dw, lens, G, p.rows, p.n, p.k, stream);
+        return mxl_gemm_nt_blockwise(b.d_col.q, b.d_col.s, fmt, b.x_col.q, b.x_col.s, fmt, 1, dw, p.n, p.k, l.width, stream);
+    }
+    return MXL_OK;
+}
+
+}  // namespace
+
 extern "C" int mxl_linear_sizes(mxl_linear* p) {
     if (!valid(p)) return MXL_EINVAL;
     const Linear l(p);
     Arena s(nullptr), f(nullptr), b(nullptr);
+    if (l.blockwise()) {
+        BwForward fwd(l, f);
+        BwBackward bwd(l, b);
+        p->saved_bytes = 0;
+        p->fwd_bytes = f.used;
+        p->bwd_bytes = b.used;
+        return MXL_OK;
+    }
     Saved saved(l, s);
     ForwardScratch fwd(l, f);
     BackwardScratch bwd(l, b);
@@ -146,6 +231,7 @@ extern "C" int mxl_linear_forward(const mxl_linear* p, const void* x, const void
                                   void* stream) {
     if (!valid(p) || !x || !w || !scratch || !y || (p->saved_bytes > 0 && !saved_buf)) return MXL_EINVAL;
     const Linear l(p);
+    if (l.blockwise()) return bw_forward(l, x, w, lens, scratch, y, stream);
     const int G = (int)p->groups, batch = (int)l.batch;
     Arena sa(saved_buf), fa(scratch);
     const Saved sv(l, sa);
@@ -194,6 +280,7 @@ extern "C" int mxl_linear_backward(const mxl_linear* p, int parts, const void* d
                                    void* daux, void* dw, uint32_t dw_flags, uint64_t sr_seed, void* stream) {
     if (!valid(p) || !scratch || (dw_flags & ~(uint32_t)MXL_GF_ACCUM_F32)) return MXL_EINVAL;
     const Linear l(p);
+    if (l.blockwise()) return dw_flags ? MXL_EINVAL : bw_backward(l, parts, dy, x, wt, lens, scratch, dx, dw, stream);
     const int G = (int)p->groups, batch = (int)l.batch;
     Arena sa(saved_buf), ba(scratch);
     const Saved sv(l, sa);

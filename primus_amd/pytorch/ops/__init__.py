@@ -608,6 +608,16 @@ class _BWLinearFunction(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, a, b, group_lens, fwd_fmt, bwd_fmt, accum=None):
+        ctx.plan = None
+        if a.shape[0] > 0 and _two_calls(a, b, b.shape[-2], b.shape[-1], group_lens) and a.device == b.device:
+            n, k = b.shape[-2:]
+            plan = K.linear_plan(a.shape[0], n, k, 0 if group_lens is None else b.shape[0], _lib.LINEAR_BLOCKWISE, fwd_fmt, fwd_fmt, bwd_fmt, 0,
+                                 a.requires_grad, b.requires_grad)
+            y, _ = K.linear_forward_impl(plan, a, b, None, group_lens)
+            if a.requires_grad or b.requires_grad:
+                ctx.plan, ctx.accum = plan, accum
+                ctx.save_for_backward(a, b, group_lens)
+            return y
         a_row, a_s, _, _ = K.quantize_blockwise_impl(a, fwd_fmt, rowwise=True, colwise=False)
         w_row, w_s, _, _ = K.quantize_blockwise_weight_impl(b.detach(), fwd_fmt, rowwise=True, colwise=False)
         y = K.gemm_blockwise_nt_impl(a_row, a_s, w_row, w_s, group_lens, b_rows_per_scale=None if group_lens is not None else 128)
@@ -619,10 +629,20 @@ class _BWLinearFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dy):
         a, b, group_lens = ctx.saved_tensors
-        bwd_fmt, need_dgrad, need_wgrad = ctx.cfg
         dy = dy.contiguous()
         if dy.dtype != torch.bfloat16:
             dy = dy.to(torch.bfloat16)
+        if ctx.plan is not None:
+            plan = ctx.plan
+            scratch = torch.empty(plan.bwd_bytes, dtype=torch.uint8, device=dy.device)
+            grad_a = torch.empty_like(a) if plan.struct.need_dx else None
+            grad_b = torch.empty_like(b) if plan.struct.need_dw else None
+            K.linear_backward_impl(plan, _lib.LINEAR_QUANTIZE | _lib.LINEAR_DX | _lib.LINEAR_DW, dy, None, scratch, grad_a, grad_b, x=a, wt=b,
+                                   group_lens=group_lens)
+            if grad_b is not None:
+                grad_b = _finish_wgrad(grad_b, ctx.accum, False, tuple(b.shape))
+            return grad_a, grad_b, None, None, None, None
+        bwd_fmt, need_dgrad, need_wgrad = ctx.cfg
         d_row, d_s, d_col, d_cs = K.quantize_blockwise_impl(dy, bwd_fmt, rowwise=need_dgrad, colwise=need_wgrad,
                                                             group_lens=group_lens)
         grad_a = grad_b = None
