@@ -593,13 +593,17 @@ constexpr int ring_lds_bytes() {
 // With both operands E2M1 (128-element steps, 64-byte rows) a plane of the row-wise codes holds 128 output columns, a K
 // step is 128 contraction rows of the tile's two planes (four rounds of 64 rows x 64 bytes), and the fragments come
 // through ds_read_b64_tr_b4, a 16 x 16 nibble transpose inside each block of 16 lanes.
-template <int AFMT, int BFMT, int MODE, bool ALPHA, bool ACCUM = false, bool BT = false>
+// HALVES: tiles of at most HALF_ROWS rows run on half of every wave's fragments (LIVE), and a nearly empty last round is
+// split into such tiles.  Forward / dgrad, and the dense weight gradient; grouped ones, where a copy of the tile loop for it
+// would cost more than it gives (32 groups of 2 .. 777 rows, [4096, 7168], 445 -> 477 us), go without.
+template <int AFMT, int BFMT, int MODE, bool ALPHA, bool ACCUM = false, bool BT = false, bool HALVES = MODE == MODE_FWD>
 __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
     static_assert(!BT || (MODE == MODE_FWD && ((AFMT != kFmtE2M1 && BFMT != kFmtE2M1) || (AFMT == kFmtE2M1 && BFMT == kFmtE2M1))),
                   "transposed weight codes: forward / dgrad, both operands FP8 formats or both E2M1");
     // ACCUM (wgrad): p.c is a float32 buffer the result is ADDED to (one workgroup per output tile: no race, and the
     // sum does not depend on any order)
     static_assert(!ACCUM || MODE == MODE_WGRAD, "the accumulating epilogue belongs to the weight-gradient GEMM");
+    static_assert(!HALVES || !ACCUM, "halves: not built for the accumulating epilogue");
     // F44: both operands FP4, stored like FP8 operands byte for byte -- 64-byte rows per K step, which then hold 128
     // elements: a step is two MFMA K steps (the low and the high half of every fragment register group), scale panels
     // cover 4 steps instead of 8, and a contraction range may be an odd number of steps.
@@ -689,15 +693,24 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
     }
 
     const int tiles_n = (int)((p.n + BN - 1) / BN);
+    const int nwg = gridDim.x;
     int tiles_m, total_tiles;
     if (MODE == MODE_FWD) {
-        tiles_m = pre_tiles[G];
+        tiles_m = __builtin_amdgcn_readfirstlane(pre_tiles[G]);
         total_tiles = tiles_m * tiles_n;
     } else {
         tiles_m = (int)((p.m + BM - 1) / BM);
         total_tiles = G * tiles_m * tiles_n;
     }
-    const int nwg = gridDim.x;
+    // A last round that would occupy at most half of the workgroups is run on halves of its tiles, 128 rows each: tile
+    // numbers from split_from on stand for an upper and a lower half in turn (neighbours, on the same XCD).  3.5 rounds, us:
+    // tensor-wise sized FP8 dgrad [4096, 4096] x 14336 217 -> 199, forward 198 -> 188, weight gradients of 4096 and 8192 tokens,
+    // 14336 x 4096, 214 -> 200 and 373 -> 355; E2M1 x E2M1 forward 127 -> 117; grouped, 8 groups of about 1024 rows,
+    // [28672, 4096], dgrad 563 -> 514 (E2M1) and 904 -> 851 (FP8).  A half costs about 0.56 of a tile, and a partly filled round
+    // runs at a higher clock: more than half of the workgroups are better off with whole tiles.
+    const int rest = total_tiles % nwg;
+    const int split_from = HALVES && 2 * rest <= nwg ? total_tiles - rest : total_tiles;
+    total_tiles += total_tiles - split_from;
     const int per_xcd = nwg >> 3;
     const int vwg = (nwg & 7) ? (int)blockIdx.x : ((int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3));
 
@@ -740,7 +753,12 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
     auto decode = [&](int tile) __attribute__((always_inline)) {
         Tile d;
         int grp = 0, pid_m, pid_n;
-        int tl = tile;
+        int tl = tile, lower = 0;
+        const bool split = HALVES && tile >= split_from;
+        if (split) {
+            lower = (tile - split_from) & 1;
+            tl = split_from + ((tile - split_from) >> 1);
+        }
         if (MODE == MODE_WGRAD) {
             const int pos = tl / (tiles_m * tiles_n);
             tl -= pos * tiles_m * tiles_n;
@@ -755,6 +773,7 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
             pid_n = (tl % width) / gsz;
         }
         int64_t a_row0, b_row0, c_row0, k0, k1;
+        const int most = split ? HALF_ROWS : BM;      // (a lower half may hold no rows: nothing of it is stored)
         if (MODE == MODE_FWD) {
             int lo = 0, hi = G;
             while (hi - lo > 1) {
@@ -763,16 +782,16 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
             }
             grp = lo;
             const int64_t g_row0 = pre_rows[grp], g_rows = pre_rows[grp + 1] - g_row0;
-            const int64_t r = (int64_t)(pid_m - pre_tiles[grp]) * BM;
+            const int64_t r = (int64_t)(pid_m - pre_tiles[grp]) * BM + lower * HALF_ROWS;
             a_row0 = g_row0 + r;
-            d.m_valid = __builtin_amdgcn_readfirstlane((g_rows - r) < BM ? (int)(g_rows - r) : BM);
+            d.m_valid = __builtin_amdgcn_readfirstlane((g_rows - r) < most ? (int)(g_rows - r) : most);
             b_row0 = (int64_t)grp * p.n + (int64_t)pid_n * BN;
             c_row0 = a_row0;
             k0 = 0;
             k1 = p.k;
         } else {
-            a_row0 = (int64_t)pid_m * BM;
-            d.m_valid = __builtin_amdgcn_readfirstlane((p.m - a_row0) < BM ? (int)(p.m - a_row0) : BM);
+            a_row0 = (int64_t)pid_m * BM + lower * HALF_ROWS;
+            d.m_valid = __builtin_amdgcn_readfirstlane((p.m - a_row0) < most ? (int)(p.m - a_row0) : most);
             b_row0 = (int64_t)pid_n * BN;
             c_row0 = (int64_t)grp * p.m + a_row0;
             k0 = pre_rows[grp];
@@ -822,7 +841,7 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
     uint32_t lca, lcb, lla, llb, ga = 0, gb = 0, cgb = 0, gup = 0, lup = 0;
     auto stream_enter = [&](const Tile& d) __attribute__((always_inline)) {
         lra = d.ra; lrb = d.rb; lca = d.ca0; lcb = d.cb0; lla = d.cal; llb = d.cbl;
-        if (MODE == MODE_FWD) lup = d.m_valid > HALF_ROWS ? 0u : addr::kDropped;
+        if (HALVES) lup = d.m_valid > HALF_ROWS ? 0u : addr::kDropped;
     };
     // start the group of the stream's next K step: fixes ga / gb and moves the stream on.  A step past the tile's
     // contraction range (a range of two steps is padded to four) requests the range's last step again: every
@@ -843,7 +862,7 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
     auto issue_e = [&](auto e_tag, uint32_t slot_base) __attribute__((always_inline)) {
         constexpr int e = decltype(e_tag)::value;
         if constexpr (e < 2) dma16_at<e * 4096>(lra, slot_base, va[e], ga);
-        else if constexpr (e < 4) dma16_at<e * 4096>(lra, slot_base, va[e], MODE == MODE_FWD ? gup : ga);
+        else if constexpr (e < 4) dma16_at<e * 4096>(lra, slot_base, va[e], HALVES ? gup : ga);
         else if constexpr (e >= 6) dma16_at<A_BYTES + (e - 4) * 4096>(crb, slot_base, vb[e - 4], cgb);
         else dma16_at<A_BYTES + (e - 4) * 4096>(lrb, slot_base, vb[e - 4], gb);
     };
@@ -946,7 +965,7 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
     int round = 0;
     auto next_tile = [&]() __attribute__((always_inline)) {
         int tl = tile_at(round);
-        if (MODE == MODE_WGRAD) {
+        if (MODE == MODE_WGRAD && !HALVES) {
             while (tl < total_tiles) {
                 const int pos = tl / (tiles_m * tiles_n);
                 const int grp = __builtin_amdgcn_readfirstlane(by_len[pos]);
@@ -1118,8 +1137,8 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
             }
         };
         {
-            if (MODE != MODE_FWD || d.m_valid > HALF_ROWS + 64) run_tile(std::integral_constant<int, 4>{});
-            else if (d.m_valid > HALF_ROWS) run_tile(std::integral_constant<int, 3>{});
+            if (!HALVES || d.m_valid > HALF_ROWS + (MODE == MODE_FWD ? 64 : 0)) run_tile(std::integral_constant<int, 4>{});
+            else if (MODE == MODE_FWD && d.m_valid > HALF_ROWS) run_tile(std::integral_constant<int, 3>{});
             else run_tile(std::integral_constant<int, 2>{});
         }
         // K step 0 of the next tile (and its scale panel) has landed; every wave is done reading the ring
@@ -1321,13 +1340,16 @@ static int launch_gemm(const GemmArgs& a, int64_t max_tiles, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;
 }
 
-template <int AFMT, int BFMT, int MODE, bool ALPHA, bool ACCUM = false, bool BT = false>
+template <int AFMT, int BFMT, int MODE, bool ALPHA, bool ACCUM = false, bool BT = false, bool HALVES = MODE == MODE_FWD>
 static int launch_gemm_ring(const GemmArgs& a, int64_t max_tiles, hipStream_t st) {
+    if constexpr (MODE == MODE_WGRAD && !ACCUM && !HALVES) {
+        if (a.group_lens == nullptr) return launch_gemm_ring<AFMT, BFMT, MODE, ALPHA, ACCUM, BT, true>(a, max_tiles, st);
+    }
     constexpr int lds = ring_lds_bytes();
     if (!device_is_gfx950()) return MXL_ENODEV;
     static std::atomic<bool> attr_set[64];
     const int slot = current_device_slot();
-    auto kern = mx_gemm_ring_kernel<AFMT, BFMT, MODE, ALPHA, ACCUM, BT>;
+    auto kern = mx_gemm_ring_kernel<AFMT, BFMT, MODE, ALPHA, ACCUM, BT, HALVES>;
     if (!attr_set[slot].load(std::memory_order_acquire)) {
         if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
             return MXL_ELAUNCH;

@@ -59,3 +59,48 @@ def test_weight_gradient_edges(gpu, recipe, n, k):
     want = K.grouped_gemm_mx_wgrad_impl(dq[2], dq[3], xq[2], xq[3], gl, m, kchunk=lay, tile="128")
     got = K.grouped_gemm_mx_wgrad_impl(dq[2], dq[3], xq[2], xq[3], gl, m, kchunk=lay, tile="256")
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+# 11 x 24 tiles on 256 workgroups (a last round of 8, run as 16 halves): a last row tile with rows in both halves, in one
+# (exactly full, and not), and a ragged last column tile; and fewer tiles than half of the workgroups a grouped launch has
+@pytest.mark.parametrize("recipe", ["mxfp8", "mxfp4w8", "mxfp4"])
+@pytest.mark.parametrize("lens,n", [((2700,), 6112), ((2688,), 6144), ((2590,), 6112), ((2800, 16), 5984), ((0, 3, 0, 0, 300, 0, 1, 0), 480)])
+def test_last_round_in_halves(gpu, recipe, lens, n):
+    from primus_amd.pytorch import kernels as K
+
+    afmt, wfmt, lay = {"mxfp8": (0, 0, 2), "mxfp4w8": (0, 1, 2), "mxfp4": (1, 1, 3)}[recipe]
+    m, k, G = sum(lens), 128, len(lens)
+    g = torch.Generator().manual_seed(n + m)
+    x = torch.randn(m, k, generator=g).bfloat16().to(gpu)
+    w = (torch.randn(G, n, k, generator=g) * 0.05).bfloat16().to(gpu)
+    gl = torch.tensor(lens, dtype=torch.int64, device=gpu)
+    xq = K.quantize_mx_impl(x, afmt, rowwise=True, colwise=False, group_lens=gl, pad_to=128, kchunk=lay)
+    wq = K.quantize_mx_weight_2d_impl(w, wfmt, rowwise=True, colwise=False, pad_to=128, kchunk=lay)
+    got, want = (K.grouped_gemm_mx_nt_impl(xq[0], xq[1], wq[0], wq[1], gl, kchunk=lay, tile=t) for t in ("256", "128"))
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("recipe", ["mxfp8", "mxfp4", "tensorwise"])
+@pytest.mark.parametrize("m,n,k,grouped", [(70, 2720, 6112, False), (300, 2592, 6144, False), (640, 2688, 6112, False), (300, 2720, 6112, True)])
+def test_weight_gradient_in_halves(gpu, recipe, m, n, k, grouped):
+    from primus_amd.pytorch import kernels as K
+
+    g = torch.Generator().manual_seed(n + m)
+    x = torch.randn(m, k, generator=g).bfloat16().to(gpu)
+    dy = torch.randn(m, n, generator=g).bfloat16().to(gpu)
+    gl = torch.tensor([m], dtype=torch.int64, device=gpu) if grouped else None      # (a single group: the tile order of groups)
+    if recipe == "tensorwise":
+        xq = K.quantize_tensorwise_impl(x, 0, rowwise=False, colwise=True, group_lens=gl, pad_to=128, kchunk=2)
+        dq = K.quantize_tensorwise_impl(dy, 2, rowwise=False, colwise=True, group_lens=gl, pad_to=128, kchunk=2)
+        run = lambda t, into=None: K.gemm_tw_wgrad_impl(dq[2], dq[3], dq[4], xq[2], xq[3], xq[4], gl, m, kchunk=2, tile=t, accum_into=into)
+    else:
+        fmt, lay = {"mxfp8": (0, 2), "mxfp4": (1, 3)}[recipe]
+        xq = K.quantize_mx_impl(x, fmt, rowwise=False, colwise=True, group_lens=gl, pad_to=128, kchunk=lay)
+        dq = K.quantize_mx_impl(dy, fmt, rowwise=False, colwise=True, group_lens=gl, pad_to=128, kchunk=lay)
+        run = lambda t, into=None: K.grouped_gemm_mx_wgrad_impl(dq[2], dq[3], xq[2], xq[3], gl, m, kchunk=lay, tile=t, accum_into=into)
+    got, want = run("256"), run("128")
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    # added to a float32 buffer of zeros: the same sums before their rounding to bf16
+    into = torch.zeros(want.shape, dtype=torch.float32, device=gpu)
+    run(None, into)
+    assert torch.equal(into.bfloat16().view(torch.int16), want.view(torch.int16))
