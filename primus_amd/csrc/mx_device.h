@@ -28,9 +28,6 @@ inline bool device_is_gfx950() {
     return v == 1;
 }
 
-// abs-max of one or two bf16 tensors in two launches (mx_quantize.hip); b null: one tensor
-int amax_pair(const void* a, int64_t na, void* out_a, const void* b, int64_t nb, void* out_b, void* stream);
-
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));

@@ -87,8 +87,8 @@ struct ForwardScratch {
         x_row = l.x_row(a);
         if (!l.p.w_quantized && !(l.p.need_dx && l.p.dx_from_rows)) w_row = l.w_row(a);
         if (l.tensorwise()) {
-            x_amax = (float*)a.take(4);
-            w_amax = (float*)a.take(4);
+            x_amax = (float*)a.take(4 * mxl::AMAX_PARTS);
+            w_amax = (float*)a.take(4 * mxl::AMAX_PARTS);
         }
     }
 };
@@ -102,7 +102,7 @@ struct BackwardScratch {
         if (p.need_dx) d_row = Linear::rows_copy(a, p.rows, l.n_ld, p.grad_fmt);
         if (p.need_dw) d_col = l.cols_copy(a, p.n, p.grad_fmt);
         if (l.tensorwise()) {
-            amax = (float*)a.take(4);
+            amax = (float*)a.take(4 * mxl::AMAX_PARTS);
             d_si = (float*)a.take(4);
         }
         if (p.input != MXL_LINEAR_PLAIN && p.need_dx) dxi = a.take(p.rows * p.k * 2);
@@ -246,7 +246,7 @@ extern "C" int mxl_linear_forward(const mxl_linear* p, const void* x, const void
                                       f.x_amax, f.w_amax, sv.x_si, sv.w_si,
                                       f.x_row.q, f.x_row.s, sv.x_col.q, sv.x_col.s, wr.q, wr.s, sv.w_col.q, sv.w_col.s};
     if (l.tensorwise()) {
-        MXL_TRY(mxl::amax_pair(x, p->rows * p->k, f.x_amax, w, l.batch * p->n * p->k, f.w_amax, stream));
+        MXL_TRY(mxl::amax_pair(x, p->rows * p->k, f.x_amax, w, l.batch * p->n * p->k, f.w_amax, true, stream));
         MXL_TRY(mxl::quantize_pair(both, stream));
         return mxl_grouped_gemm_nt_scaled(f.x_row.q, f.x_row.s, af, wr.q, wr.s, wf, y, lens, batch, p->rows, p->n, l.k_ld, sv.x_si, sv.w_si,
                                           MXL_GF_KSTEP, stream);
@@ -290,8 +290,8 @@ extern "C" int mxl_linear_backward(const mxl_linear* p, int parts, const void* d
     if (parts & MXL_LINEAR_QUANTIZE) {
         if (!dy) return MXL_EINVAL;
         if (l.tensorwise()) {
-            MXL_TRY(mxl_amax(dy, p->rows * p->n, b.amax, stream));
-            MXL_TRY(mxl_quantize_tensorwise(dy, p->rows, p->n, p->need_dx ? l.n_ld : 0, gf, b.amax, p->need_dw ? lens : nullptr, p->need_dw ? G : 0,
+            MXL_TRY(mxl::amax_pair(dy, p->rows * p->n, b.amax, nullptr, 0, nullptr, true, stream));
+            MXL_TRY(mxl::quantize_tensorwise_parts(dy, p->rows, p->n, p->need_dx ? l.n_ld : 0, gf, b.amax, p->need_dw ? lens : nullptr, p->need_dw ? G : 0,
                                             b.d_row.q, b.d_row.s, b.d_col.q, b.d_col.s, b.d_si, l.qf(), stream));
         } else {
             const bool rht = p->rht_signs >= 0 && p->need_dw;

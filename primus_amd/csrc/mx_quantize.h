@@ -4,6 +4,15 @@
 
 namespace mxl {
 
+// An abs-max launch leaves one value per workgroup (amax_parts(n) of them for n elements), at most this many.
+constexpr int AMAX_PARTS = 512;
+int amax_parts(int64_t n);
+int amax_pair(const void* a, int64_t na, void* out_a, const void* b, int64_t nb, void* out_b, bool parts, void* stream);
+// mxl_quantize_tensorwise on such parts of x
+int quantize_tensorwise_parts(const void* x, int64_t rows, int64_t cols, int64_t row_ld, int fmt, const float* amax, const int64_t* group_lens,
+                              int num_groups, void* q_row, void* s_row, void* q_colT, void* s_colT, float* scale_inv, uint32_t flags,
+                              void* stream);
+
 struct LinearOperands {
     // activations [rows, k] (ragged groups: group_lens, num_groups; 0 and null: one), weights [batch, n, k]
     const void *x, *w;
@@ -12,7 +21,7 @@ struct LinearOperands {
     int num_groups;
     int x_fmt, w_fmt, scale_mode;
     uint32_t flags, rht_signs;          // MXL_QF_* of mxl_quantize_ex (no stochastic rounding)
-    // tensor-wise scaling: abs-max of each on the device, and where 1 / scale goes; null otherwise
+    // tensor-wise scaling: abs-max of each on the device (the parts of amax_pair), and where 1 / scale goes; null otherwise
     const float *x_amax, *w_amax;
     float *x_scale_inv, *w_scale_inv;
     // the copies; transposed ones may be null as mxl_quantize_ex and mxl_quantize_weight_2d_ex allow

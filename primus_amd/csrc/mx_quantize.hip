@@ -21,6 +21,7 @@ namespace mxl {
 
 constexpr int QT = 128;       // tile edge
 constexpr int QTHREADS = 256;
+constexpr int AMAX_MAX_WG = AMAX_PARTS;     // workgroups of an abs-max launch per tensor
 
 struct QuantArgs {
     const uint16_t* x;
@@ -46,6 +47,7 @@ struct QuantArgs {
     // from the tensor's abs-max on the device; its reciprocal is written to scale_inv_out (may be null).  The
     // block-scale arrays are filled with 127 (2^0), so the scaled GEMM reads the codes unchanged.
     const float* tensor_amax;
+    int amax_parts;         // number of values at tensor_amax, whose maximum it is
     float* scale_inv_out;
     // Code layout of both copies.  0: row-major [rows, ld].  1: K-chunk-major [ld / 128][rows][128 elements]:
     // the 128 elements of a row that one GEMM K slot consumes stay together and consecutive rows follow
@@ -129,13 +131,12 @@ __device__ __forceinline__ void quant_workgroup(const QuantArgs& a, int block) {
 
     const int t = threadIdx.x;
     const int w = t >> 6, l = t & 63, c16 = l & 15, rg = l >> 4;
-    float tscale = 1.f;
-    bool tensor_bad = false;   // abs-max is NaN or Inf: every code becomes NaN
+    // tensor-wise: the abs-max is the maximum of amax_parts values, eight to a lane, which every wave takes for itself; they
+    // are requested here and looked at behind the tile's own loads
+    uint32_t part[TENSOR ? AMAX_MAX_WG / 64 : 1];
     if (TENSOR) {
-        const float amax = *a.tensor_amax;
-        tensor_bad = !(amax < __uint_as_float(0x7F800000u));
-        tscale = (FMT == kFmtE5M2 ? 57344.f : 448.f) / fmaxf(amax, 1e-12f);
-        if (block == 0 && t == 0 && a.scale_inv_out) *a.scale_inv_out = 1.0f / tscale;
+#pragma unroll
+        for (int u = 0; u < AMAX_MAX_WG / 64; ++u) part[u] = u * 64 + l < a.amax_parts ? ((const uint32_t*)a.tensor_amax)[u * 64 + l] : 0u;
     }
     int pt, ct;
     if (!quant_tile_of_workgroup(a, block, pt, ct)) return;   // uniform over the workgroup
@@ -229,6 +230,21 @@ __device__ __forceinline__ void quant_workgroup(const QuantArgs& a, int block) {
                 }
             }
         }
+    }
+
+    float tscale = 1.f;
+    bool tensor_bad = false;   // abs-max is NaN or Inf: every code becomes NaN
+    if (TENSOR) {
+        // bit patterns of non-negative floats order like integers, a NaN above every number
+        uint32_t bits = part[0];
+#pragma unroll
+        for (int u = 1; u < AMAX_MAX_WG / 64; ++u) bits = max(bits, part[u]);
+#pragma unroll
+        for (int s = 32; s > 0; s >>= 1) bits = max(bits, (uint32_t)__shfl_xor((int)bits, s));
+        const float amax = __uint_as_float(bits);
+        tensor_bad = !(amax < __uint_as_float(0x7F800000u));
+        tscale = (FMT == kFmtE5M2 ? 57344.f : 448.f) / fmaxf(amax, 1e-12f);
+        if (block == 0 && t == 0 && a.scale_inv_out) *a.scale_inv_out = 1.0f / tscale;     // (workgroup 0 always has a tile)
     }
 
     if (ACT == PRO_RMSNORM) {
@@ -687,12 +703,13 @@ static int launch_quant_pair(const HeldQuant& x, QuantArgs& w, int64_t tiles_r, 
 // [4096, 4096]: 17.4 -> 11.8 us (16.6 with 1024 workgroups).
 // The loads are ordinary ones: the quantiser reads the same tensor next, and up to 256 MiB of it then come from the
 // memory-side cache.
-constexpr int AMAX_LOADS = 8, AMAX_PIECE = 256 * AMAX_LOADS, AMAX_MAX_WG = 512;
+constexpr int AMAX_LOADS = 8, AMAX_PIECE = 256 * AMAX_LOADS;
 struct AmaxArgs {
     const uint16_t* x[2];
     int64_t n[2];
     uint32_t* out[2];
     uint32_t wg[2];          // workgroups of each tensor
+    int parts;               // every workgroup stores its own maximum, out[tensor][workgroup]; nothing is initialised
 };
 __global__ __launch_bounds__(256) void amax_kernel(AmaxArgs p) {
     __shared__ uint32_t part[4];
@@ -722,7 +739,9 @@ __global__ __launch_bounds__(256) void amax_kernel(AmaxArgs p) {
     __syncthreads();
     if (threadIdx.x == 0) {
         m = max(max(part[0], part[1]), max(part[2], part[3]));
-        atomicMax(p.out[second], m << 16);   // bf16 pattern -> fp32 pattern
+        // bf16 pattern -> fp32 pattern
+        if (p.parts) p.out[second][blk] = m << 16;
+        else atomicMax(p.out[second], m << 16);
     }
 }
 
@@ -738,17 +757,23 @@ static uint32_t amax_workgroups(int64_t n) {
     return (uint32_t)((pieces + rounds - 1) / rounds);      // every workgroup the same number of pieces
 }
 
-// out_a = max |a| over na values, out_b = max |b| (b may be null: one tensor), in two launches
-int amax_pair(const void* a, int64_t na, void* out_a, const void* b, int64_t nb, void* out_b, void* stream) {
+int amax_parts(int64_t n) { return (int)amax_workgroups(n); }
+
+// out_a = max |a| over na values, out_b = max |b| (b may be null: one tensor), in two launches; with `parts` the
+// amax_parts(na) and amax_parts(nb) maxima of the workgroups, na and nb > 0, in one (the initialising launch costs a linear
+// 5 us in each direction, more than the quantiser's look at 512 values)
+int amax_pair(const void* a, int64_t na, void* out_a, const void* b, int64_t nb, void* out_b, bool parts, void* stream) {
     if (na < 0 || nb < 0 || !out_a || (na > 0 && !a) || ((uintptr_t)a & 15) != 0) return MXL_EINVAL;
     if (nb > 0 && (!b || !out_b || ((uintptr_t)b & 15) != 0)) return MXL_EINVAL;
     if (!device_is_gfx950()) return MXL_ENODEV;
     hipStream_t st = (hipStream_t)stream;
     AmaxArgs p{{(const uint16_t*)a, (const uint16_t*)b}, {na, nb}, {(uint32_t*)out_a, (uint32_t*)(out_b ? out_b : out_a)},
-               {amax_workgroups(na), amax_workgroups(nb)}};
-    // a fill kernel, not a memset: callers may be capturing the stream into a graph
-    hipLaunchKernelGGL(amax_init_kernel, dim3(1), dim3(1), 0, st, p.out[0], p.out[1]);
-    if (hipGetLastError() != hipSuccess) return MXL_ELAUNCH;
+               {amax_workgroups(na), amax_workgroups(nb)}, parts};
+    if (!parts) {
+        // a fill kernel, not a memset: callers may be capturing the stream into a graph
+        hipLaunchKernelGGL(amax_init_kernel, dim3(1), dim3(1), 0, st, p.out[0], p.out[1]);
+        if (hipGetLastError() != hipSuccess) return MXL_ELAUNCH;
+    }
     if (p.wg[0] + p.wg[1] == 0) return MXL_OK;
     hipLaunchKernelGGL(amax_kernel, dim3(p.wg[0] + p.wg[1]), dim3(256), 0, st, p);
     return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;
@@ -759,7 +784,7 @@ int amax_pair(const void* a, int64_t na, void* out_a, const void* b, int64_t nb,
 using namespace mxl;
 
 extern "C" int mxl_amax(const void* x_bf16, int64_t n, void* amax_f32, void* stream) {
-    return amax_pair(x_bf16, n, amax_f32, nullptr, 0, nullptr, stream);
+    return amax_pair(x_bf16, n, amax_f32, nullptr, 0, nullptr, false, stream);
 }
 
 extern "C" int64_t mxl_padded_width(int64_t total_rows, int num_groups) {
@@ -780,7 +805,7 @@ static int quantize_1d(const void* x_bf16, int64_t rows, int64_t cols, int64_t r
                        int act, const void* probs, int probs_dtype, const uint8_t* row_mask, void* stream,
                        bool sr = false, uint64_t sr_seed = 0, bool rht = false, uint32_t rht_signs = 0,
                        int kchunk = 0, const void* norm_w = nullptr, const void* tensor_amax = nullptr,
-                       void* scale_inv_out = nullptr, HeldQuant* hold = nullptr) {
+                       void* scale_inv_out = nullptr, HeldQuant* hold = nullptr, int parts = 1) {
     if (row_ld == 0) row_ld = cols;
     if (kchunk < 0) return MXL_EINVAL;                  // contradictory layout flags
     if (kchunk == 2 && fmt == MXL_FMT_E2M1) kchunk = 3;  // E2M1 activations: the K step is 128 elements (64-byte rows)
@@ -811,6 +836,7 @@ static int quantize_1d(const void* x_bf16, int64_t rows, int64_t cols, int64_t r
     a.row_mask = row_mask;
     a.norm_w = (const uint16_t*)norm_w;
     a.tensor_amax = (const float*)tensor_amax;
+    a.amax_parts = parts;
     a.scale_inv_out = (float*)scale_inv_out;
     a.sr_seed = sr_seed;
     a.rht_signs = rht_signs & 0xFFFFu;
@@ -882,7 +908,7 @@ extern "C" int mxl_rmsnorm_quantize(const void* x_bf16, const void* w_bf16, cons
 static int quantize_weight_2d(const void* w_bf16, int64_t batch, int64_t n, int64_t k, int64_t k_ld, int64_t n_ld, int fmt,
                               int scale_mode, void* q_row, void* s_row, void* q_colT, void* s_colT, int kchunk,
                               void* stream, const void* tensor_amax = nullptr, void* scale_inv_out = nullptr,
-                              const HeldQuant* pair = nullptr, bool* paired = nullptr) {
+                              const HeldQuant* pair = nullptr, bool* paired = nullptr, int parts = 1) {
     if (k_ld == 0) k_ld = k;
     if (n_ld == 0) n_ld = n;
     if (kchunk < 0 || (kchunk == 3 && fmt != MXL_FMT_E2M1)) return MXL_EINVAL;
@@ -912,6 +938,7 @@ static int quantize_weight_2d(const void* w_bf16, int64_t batch, int64_t n, int6
     a.row_mask = nullptr;
     a.norm_w = nullptr;
     a.tensor_amax = (const float*)tensor_amax;
+    a.amax_parts = parts;
     a.scale_inv_out = (float*)scale_inv_out;
     a.sr_seed = 0;
     a.rht_signs = 0;
@@ -934,11 +961,11 @@ int quantize_pair(const LinearOperands& o, void* stream) {
     const bool rht = (o.flags & MXL_QF_RHT_COL) != 0;
     auto x = [&](HeldQuant* hold) {
         return quantize_1d(o.x, o.rows, o.k, o.k_ld, o.x_fmt, o.scale_mode, o.group_lens, o.num_groups, o.xq_row, o.xs_row, o.xq_col, o.xs_col, -1,
-                           nullptr, MXL_PROBS_F32, nullptr, stream, false, 0, rht, o.rht_signs, lay, nullptr, o.x_amax, o.x_scale_inv, hold);
+                           nullptr, MXL_PROBS_F32, nullptr, stream, false, 0, rht, o.rht_signs, lay, nullptr, o.x_amax, o.x_scale_inv, hold, o.x_amax ? amax_parts(o.rows * o.k) : 1);
     };
     auto w = [&](const HeldQuant* pair, bool* paired) {
         return quantize_weight_2d(o.w, o.batch, o.n, o.k, o.k_ld, o.n_ld, o.w_fmt, o.scale_mode, o.wq_row, o.ws_row, o.wq_col, o.ws_col, lay,
-                                  stream, o.w_amax, o.w_scale_inv, pair, paired);
+                                  stream, o.w_amax, o.w_scale_inv, pair, paired, o.w_amax ? amax_parts(o.batch * o.n * o.k) : 1);
     };
     HeldQuant hold;
     bool paired = false;
@@ -965,6 +992,16 @@ extern "C" int mxl_quantize_weight_2d_ex(const void* w_bf16, int64_t batch, int6
     return quantize_weight_2d(w_bf16, batch, n, k, k_ld, n_ld, fmt, scale_mode, q_row, s_row, q_colT, s_colT,
                               qf_layout(flags), stream);
 }
+
+namespace mxl {
+int quantize_tensorwise_parts(const void* x, int64_t rows, int64_t cols, int64_t row_ld, int fmt, const float* amax, const int64_t* group_lens,
+                              int num_groups, void* q_row, void* s_row, void* q_colT, void* s_colT, float* scale_inv, uint32_t flags,
+                              void* stream) {
+    return quantize_1d(x, rows, cols, row_ld, fmt, MXL_SCALE_OCP_FLOOR, group_lens, num_groups, q_row, s_row, q_colT, s_colT, -1, nullptr,
+                       MXL_PROBS_F32, nullptr, stream, false, 0, false, 0, qf_layout(flags), nullptr, amax, scale_inv, nullptr,
+                       amax_parts(rows * cols));
+}
+}  // namespace mxl
 
 extern "C" int mxl_quantize_tensorwise(const void* x_bf16, int64_t rows, int64_t cols, int64_t row_ld, int fmt,
                                        const void* amax_f32, const int64_t* group_lens, int num_groups, void* q_row,
