@@ -244,6 +244,7 @@ extern "C" int mxl_linear_forward(const mxl_linear* p, const void* x, const void
                                       l.tensorwise() && !p->need_dw ? nullptr : lens, l.tensorwise() && !p->need_dw ? 0 : G,
                                       af, wf, (int)p->scale_mode, l.qf() | (rht ? MXL_QF_RHT_COL : 0u), rht ? (uint32_t)p->rht_signs : 0u,
                                       f.x_amax, f.w_amax, sv.x_si, sv.w_si,
+                                      p->input == MXL_LINEAR_RMSNORM ? aux0 : nullptr, sv.rstd,
                                       f.x_row.q, f.x_row.s, sv.x_col.q, sv.x_col.s, wr.q, wr.s, sv.w_col.q, sv.w_col.s};
     if (l.tensorwise()) {
         MXL_TRY(mxl::amax_pair(x, p->rows * p->k, f.x_amax, w, l.batch * p->n * p->k, f.w_amax, true, stream));
@@ -253,6 +254,10 @@ extern "C" int mxl_linear_forward(const mxl_linear* p, const void* x, const void
     }
     if (p->input == MXL_LINEAR_RMSNORM) {
         MXL_TRY(mxl_rmsnorm_fwd(x, aux0, (float)p->eps, p->rows, p->k, nullptr, sv.rstd, stream));
+        if (!p->w_quantized && G == 0 && aux0) {
+            MXL_TRY(mxl::quantize_pair(both, stream));
+            return mxl_grouped_gemm_nt_ex(f.x_row.q, f.x_row.s, af, wr.q, wr.s, wf, y, lens, batch, p->rows, p->n, l.k_ld, MXL_GF_KSTEP, stream);
+        }
         MXL_TRY(mxl_rmsnorm_quantize(x, aux0, sv.rstd, p->rows, p->k, l.k_ld, af, (int)p->scale_mode, nullptr, 0, f.x_row.q, f.x_row.s,
                                      sv.x_col.q, sv.x_col.s, l.qf(), stream));
     } else if (p->input != MXL_LINEAR_PLAIN) {

@@ -24,6 +24,8 @@ struct LinearOperands {
     // tensor-wise scaling: abs-max of each on the device (the parts of amax_pair), and where 1 / scale goes; null otherwise
     const float *x_amax, *w_amax;
     float *x_scale_inv, *w_scale_inv;
+    // the input an RMSNorm forms from x, its weight and the rows' statistics (mxl_rmsnorm_fwd); null: x itself
+    const void *norm_w, *rstd;
     // the copies; transposed ones may be null as mxl_quantize_ex and mxl_quantize_weight_2d_ex allow
     uint8_t *xq_row, *xs_row, *xq_col, *xs_col, *wq_row, *ws_row, *wq_col, *ws_col;
 };

@@ -530,10 +530,11 @@ __global__ __launch_bounds__(QTHREADS) void mx_quant_kernel(QuantArgs a) {
 // costs its fill and drain and the gap behind it.  Forward of a linear, quantisers and GEMM, two launches / one, us:
 // [256, 4096] x 4096 39.8 / 34.0; [1999, 2880] x 5760 67.9 / 62.8; [8192, 4096] x 14336 422 / 412; tensor-wise [4096, 14336] x
 // 4096 279 / 272; 8 experts of [2048, 2048], 2048 rows, 56 / 51.  Large experts read their weights at 108 registers a lane
-// instead of 58, which costs them nothing (32 x [4096, 7168], 8192 rows, 860 / 865; 8 x [28672, 4096], 512 rows, 694 / 668).
-template <int FMT, int SMODE, bool WCOL>
+// instead of 58, which costs them nothing (the input may be transformed by Hadamard, or formed by an RMSNorm from statistics
+// that are there already; 32 x [4096, 7168], 8192 rows, 860 / 865; 8 x [28672, 4096], 512 rows, 694 / 668).
+template <int FMT, int SMODE, bool WCOL, int ACT = -1, bool RHT = false>
 __global__ __launch_bounds__(QTHREADS) void mx_quant_pair_kernel(QuantArgs x, QuantArgs w, unsigned x_wgs) {
-    if (blockIdx.x < x_wgs) quant_workgroup<FMT, SMODE, true, true, false>(x, (int)blockIdx.x);
+    if (blockIdx.x < x_wgs) quant_workgroup<FMT, SMODE, true, true, false, ACT, false, RHT>(x, (int)blockIdx.x);
     else quant_workgroup<FMT, SMODE, true, WCOL, true>(w, (int)(blockIdx.x - x_wgs));
 }
 
@@ -601,6 +602,8 @@ __global__ __launch_bounds__(256) void mx_dequant_kernel(const uint8_t* q, const
 struct HeldQuant {
     bool held = false;
     int fmt, smode;          // smode: SCALE_TENSOR or an MXL_SCALE_*
+    int act;                 // -1 or PRO_RMSNORM
+    bool rht;
     QuantArgs a;
     int64_t wgs;
 };
@@ -674,22 +677,24 @@ static int dispatch_quant_tensor(int fmt, QuantArgs& a, int64_t tiles_r, int64_t
 // both launches of a pair in one; false: there is no kernel for it
 static bool pair_taken(const HeldQuant& x, int fmt, int smode, const QuantArgs& w) {
     return x.fmt == fmt && x.smode == smode && (smode == MXL_SCALE_OCP_FLOOR || smode == SCALE_TENSOR) && x.a.q_row && x.a.q_colT && w.q_row &&
-           (fmt == MXL_FMT_E4M3 || (fmt == MXL_FMT_E2M1 && smode == MXL_SCALE_OCP_FLOOR));
+           (fmt == MXL_FMT_E4M3 || (fmt == MXL_FMT_E2M1 && smode == MXL_SCALE_OCP_FLOOR && x.act < 0));
 }
 static int launch_quant_pair(const HeldQuant& x, QuantArgs& w, int64_t tiles_r, int64_t tiles_c, hipStream_t st) {
     int64_t wgs;
     if (const int rc = quant_grid(w, tiles_r, tiles_c, &wgs)) return rc;
     if (x.wgs + wgs > 0x7FFFFFFF) return MXL_EINVAL;
     const dim3 grid((unsigned)(x.wgs + wgs));
-#define MXL_QP(F, S)                                                                                                                      \
-    if (x.fmt == F && x.smode == S) {                                                                                                     \
-        if (w.q_colT) hipLaunchKernelGGL((mx_quant_pair_kernel<F, S, true>), grid, dim3(QTHREADS), 0, st, x.a, w, (unsigned)x.wgs);       \
-        else hipLaunchKernelGGL((mx_quant_pair_kernel<F, S, false>), grid, dim3(QTHREADS), 0, st, x.a, w, (unsigned)x.wgs);              \
-        return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;                                                                    \
+#define MXL_QP(F, S, ACT, RHT)                                                                                                              \
+    if (x.fmt == F && x.smode == S && x.act == ACT && x.rht == RHT) {                                                                       \
+        if (w.q_colT) hipLaunchKernelGGL((mx_quant_pair_kernel<F, S, true, ACT, RHT>), grid, dim3(QTHREADS), 0, st, x.a, w, (unsigned)x.wgs); \
+        else hipLaunchKernelGGL((mx_quant_pair_kernel<F, S, false, ACT, RHT>), grid, dim3(QTHREADS), 0, st, x.a, w, (unsigned)x.wgs);        \
+        return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;                                                                      \
     }
-    MXL_QP(MXL_FMT_E4M3, MXL_SCALE_OCP_FLOOR)
-    MXL_QP(MXL_FMT_E2M1, MXL_SCALE_OCP_FLOOR)
-    MXL_QP(MXL_FMT_E4M3, SCALE_TENSOR)
+    MXL_QP(MXL_FMT_E4M3, MXL_SCALE_OCP_FLOOR, -1, false)
+    MXL_QP(MXL_FMT_E4M3, MXL_SCALE_OCP_FLOOR, PRO_RMSNORM, false)
+    MXL_QP(MXL_FMT_E2M1, MXL_SCALE_OCP_FLOOR, -1, false)
+    MXL_QP(MXL_FMT_E2M1, MXL_SCALE_OCP_FLOOR, -1, true)
+    MXL_QP(MXL_FMT_E4M3, SCALE_TENSOR, -1, false)
 #undef MXL_QP
     return MXL_EINVAL;
 }
@@ -845,8 +850,10 @@ static int quantize_1d(const void* x_bf16, int64_t rows, int64_t cols, int64_t r
     a.chunk_rows_col = cols;
     const int64_t gx = q_colT ? a.W / QT : (rows + QT - 1) / QT;
     const int64_t gy = ((q_row ? row_ld : cols) + QT - 1) / QT;
-    if (hold && gx > 0 && !sr && !rht && act < 0) {
+    if (hold && gx > 0 && !sr && (act < 0 || act == PRO_RMSNORM)) {
         hold->held = true;
+        hold->act = act;
+        hold->rht = rht;
         hold->fmt = fmt;
         hold->smode = tensor_amax ? SCALE_TENSOR : scale_mode;
         hold->a = a;
@@ -960,8 +967,8 @@ int quantize_pair(const LinearOperands& o, void* stream) {
     const int lay = qf_layout(o.flags);
     const bool rht = (o.flags & MXL_QF_RHT_COL) != 0;
     auto x = [&](HeldQuant* hold) {
-        return quantize_1d(o.x, o.rows, o.k, o.k_ld, o.x_fmt, o.scale_mode, o.group_lens, o.num_groups, o.xq_row, o.xs_row, o.xq_col, o.xs_col, -1,
-                           nullptr, MXL_PROBS_F32, nullptr, stream, false, 0, rht, o.rht_signs, lay, nullptr, o.x_amax, o.x_scale_inv, hold, o.x_amax ? amax_parts(o.rows * o.k) : 1);
+        return quantize_1d(o.x, o.rows, o.k, o.k_ld, o.x_fmt, o.scale_mode, o.group_lens, o.num_groups, o.xq_row, o.xs_row, o.xq_col, o.xs_col,
+                           o.norm_w ? PRO_RMSNORM : -1, o.rstd, MXL_PROBS_F32, nullptr, stream, false, 0, rht, o.rht_signs, lay, o.norm_w, o.x_amax, o.x_scale_inv, hold, o.x_amax ? amax_parts(o.rows * o.k) : 1);
     };
     auto w = [&](const HeldQuant* pair, bool* paired) {
         return quantize_weight_2d(o.w, o.batch, o.n, o.k, o.k_ld, o.n_ld, o.w_fmt, o.scale_mode, o.wq_row, o.ws_row, o.wq_col, o.ws_col, lay,
@@ -969,7 +976,8 @@ int quantize_pair(const LinearOperands& o, void* stream) {
     };
     HeldQuant hold;
     bool paired = false;
-    if (!rht && o.xq_col) {
+    if (o.norm_w && !o.rstd) return MXL_EINVAL;
+    if (o.xq_col) {
         if (const int rc = x(&hold)) return rc;
         if (const int rc = w(&hold, &paired)) return rc;
         if (paired) return MXL_OK;
