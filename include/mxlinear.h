@@ -288,6 +288,8 @@ int mxl_grouped_gemm_bf16_wgrad(const void* p_bf16, const void* q_bf16, void* c,
  * computed in fp32, rounded once to bf16.  row_mask (one byte per row, may be NULL = all rows live):
  * a row with mask 0 yields zeros (tokens_per_expert_to_mask marks the rows past the routed tokens
  * of a worst-case sized buffer).  probs is fp32 or bf16 per probs_dtype.  Requires f % 8 == 0. */
+/* mask[i] = i < lens[0] + ... + lens[count - 1] (0 or 1 per byte, 16-byte aligned), on the device. */
+int mxl_row_mask(const int64_t* lens, int64_t count, int64_t rows, uint8_t* mask, void* stream);
 int mxl_glu_probs_fwd(const void* x_bf16, const void* probs, int probs_dtype, const uint8_t* row_mask,
                       int64_t rows, int64_t f, int act, void* y_bf16, void* stream);
 

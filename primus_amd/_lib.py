@@ -52,6 +52,7 @@ EXPORTS = (
     "mxl_grouped_gemm_wgrad_ex",
     "mxl_grouped_gemm_bf16",
     "mxl_grouped_gemm_bf16_wgrad",
+    "mxl_row_mask",
     "mxl_glu_probs_fwd",
     "mxl_glu_probs_bwd",
     "mxl_glu_probs_quantize",
@@ -160,6 +161,8 @@ def load() -> ctypes.CDLL:
         lib.mxl_grouped_gemm_bf16.argtypes = [vp, vp, vp, vp, i32, i64, i64, i64, u32, vp]
         lib.mxl_grouped_gemm_bf16_wgrad.restype = i32
         lib.mxl_grouped_gemm_bf16_wgrad.argtypes = [vp, vp, vp, vp, i32, i64, i64, i64, u32, vp]
+        lib.mxl_row_mask.restype = i32
+        lib.mxl_row_mask.argtypes = [vp, i64, i64, vp, vp]
         lib.mxl_glu_probs_fwd.restype = i32
         lib.mxl_glu_probs_fwd.argtypes = [vp, vp, i32, vp, i64, i64, i32, vp, vp]
         lib.mxl_glu_probs_bwd.restype = i32

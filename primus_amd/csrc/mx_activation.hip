@@ -111,6 +111,42 @@ static bool act_args_ok(const void* a, const void* b, const void* probs, int pro
     return rows == 0 || (a && b && probs);
 }
 
+// mask[i] = i < sum of the lens: which rows of a buffer sized for the worst case hold tokens.  A few kilobytes, so the launch is
+// all it costs: one instead of the three of a sum, a range and a comparison (32 groups, 8192 rows: 15.4 -> 6.7 us).
+constexpr int MASK_ROWS = 16;      // rows per thread, one 16-byte store
+__global__ __launch_bounds__(ATHREADS) void row_mask_kernel(const int64_t* lens, int64_t count, int64_t rows, uint8_t* mask) {
+    __shared__ int64_t part[ATHREADS / 64];
+    const int t = threadIdx.x;
+    int64_t sum = 0;
+    for (int64_t i = t; i < count; i += ATHREADS) sum += lens[i];
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) sum += __shfl_xor(sum, s);
+    if ((t & 63) == 0) part[t >> 6] = sum;
+    __syncthreads();
+    sum = 0;
+#pragma unroll
+    for (int w = 0; w < ATHREADS / 64; ++w) sum += part[w];
+    const int64_t row0 = ((int64_t)blockIdx.x * ATHREADS + t) * MASK_ROWS;
+    if (row0 + MASK_ROWS <= rows) {
+        uint32_t v[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int j = 0; j < MASK_ROWS; ++j) v[j >> 2] |= (row0 + j < sum ? 1u : 0u) << (8 * (j & 3));
+        *(uint4*)(mask + row0) = make_uint4(v[0], v[1], v[2], v[3]);
+    } else {
+        for (int64_t i = row0; i < rows; ++i) mask[i] = i < sum ? 1 : 0;
+    }
+}
+
+extern "C" int mxl_row_mask(const int64_t* lens, int64_t count, int64_t rows, uint8_t* mask, void* stream) {
+    if (count < 1 || rows < 0 || !lens || (rows > 0 && !mask) || ((uintptr_t)mask & 15) != 0) return MXL_EINVAL;
+    if (rows == 0) return MXL_OK;
+    const int64_t grid = (rows + ATHREADS * MASK_ROWS - 1) / (ATHREADS * MASK_ROWS);
+    if (grid > 0x7FFFFFFF) return MXL_EINVAL;
+    if (!device_is_gfx950()) return MXL_ENODEV;
+    hipLaunchKernelGGL(row_mask_kernel, dim3((unsigned)grid), dim3(ATHREADS), 0, (hipStream_t)stream, lens, count, rows, mask);
+    return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;
+}
+
 extern "C" int mxl_glu_probs_fwd(const void* x_bf16, const void* probs, int probs_dtype, const uint8_t* row_mask,
                                  int64_t rows, int64_t f, int act, void* y_bf16, void* stream) {
     if (!act_args_ok(x_bf16, y_bf16, probs, probs_dtype, rows, f, act)) return MXL_EINVAL;

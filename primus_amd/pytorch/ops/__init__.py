@@ -1015,9 +1015,23 @@ def grouped_gemm(a, b, group_lens: torch.Tensor, trans_b: bool = True,
 # Gated activation fused with the router probability and the row mask: the three operators the
 # reference's fused_bias_act_with_probs calls (primus_turbo.py:1954-1980).
 # ---------------------------------------------------------------------------
+def _plain_cuda_lens(t) -> bool:
+    """Whether native code may be handed the address of the counts ``t`` behind torch's back: an ordinary int64 vector on
+    the current GPU, and nothing traces, transforms or watches torch's calls."""
+    return (type(t) is torch.Tensor and t.is_cuda and t.dtype == torch.int64 and t.dim() == 1 and t.numel() > 0 and t.is_contiguous()
+            and t.get_device() == torch._C._cuda_getDevice() and not torch.compiler.is_compiling()
+            and torch._C._get_tracing_state() is None and not torch._C._are_functorch_transforms_active()
+            and torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0)
+
+
 def tokens_per_expert_to_mask(tokens_per_expert: torch.Tensor, num_tokens: int) -> torch.Tensor:
     """``mask[i] = i < sum(tokens_per_expert)``: the live rows of a buffer sized for the worst case.
     Stays on the device (no host read of the counts)."""
+    if _plain_cuda_lens(tokens_per_expert) and type(num_tokens) is int and num_tokens > 0:
+        mask = torch.empty((num_tokens,), dtype=torch.bool, device=tokens_per_expert.device)
+        _lib.check(_lib.load().mxl_row_mask(tokens_per_expert.data_ptr(), tokens_per_expert.numel(), num_tokens, mask.data_ptr(), K._stream()),
+                   "mxl_row_mask")
+        return mask
     total = tokens_per_expert.sum()
     return torch.arange(num_tokens, device=tokens_per_expert.device) < total
 
