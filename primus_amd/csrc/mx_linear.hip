@@ -1,6 +1,6 @@
 // One linear as two calls: everything its forward launches, and everything its backward launches (host code only).
 //
-// A linear is 3 to 5 launches forward and 4 to 7 backward, and a dozen buffers.  Issued one by one from Python, with an
+// A linear is 2 to 4 launches forward and 3 to 6 backward, and a dozen buffers.  Issued one by one from Python, with an
 // allocation per buffer and a stream look-up per launch, they take 230 us for a pass whose kernels need 60.  Here the
 // caller allocates three buffers -- what the backward needs, and a scratch buffer per direction -- and makes one call per
 // direction; the layout of the buffers is arithmetic on the sizes and is worked out again in every call.
