@@ -637,7 +637,7 @@ class LinearPlan:
     """Sizes and options of one linear and of the buffers its two calls work in; depends on nothing else, so linears of
     the same sizes share it."""
 
-    __slots__ = ("struct", "ptr", "saved_bytes", "fwd_bytes", "bwd_bytes", "rows", "n", "k", "groups")
+    __slots__ = ("struct", "ptr", "saved_bytes", "fwd_bytes", "bwd_bytes", "rows", "n", "k", "groups", "kept")
 
     def __init__(self, **fields):
         self.struct = _lib.Linear(**fields)
@@ -645,6 +645,14 @@ class LinearPlan:
         _lib.check(_lib.load().mxl_linear_sizes(self.ptr), "mxl_linear_sizes")
         self.saved_bytes, self.fwd_bytes, self.bwd_bytes = self.struct.saved_bytes, self.struct.fwd_bytes, self.struct.bwd_bytes
         self.rows, self.n, self.k, self.groups = self.struct.rows, self.struct.n, self.struct.k, self.struct.groups
+        # dtype (None: any) and bytes of what autograd keeps for the backward: saved, x, wt, wt_scales, group_lens, aux0, aux1
+        p, batch, ld, bf16 = self.struct, self.groups or 1, _round_up(self.n, GEMM_K_ALIGN), torch.bfloat16
+        glu = p.input in (_lib.LINEAR_SILU, _lib.LINEAR_GELU)
+        wt = (bf16, batch * self.n * self.k * 2) if p.recipe == _lib.LINEAR_BLOCKWISE else (_code_dtype(p.w_fmt), batch * self.k * ld // _per_byte(p.w_fmt))
+        probs = (bf16, 2) if p.probs_dtype == _lib.PROBS_BF16 else (torch.float32, 4)
+        self.kept = ((torch.uint8, self.saved_bytes), (bf16, self.rows * self.k * (4 if glu else 2)), wt,
+                     (None, (ld + PANEL - 1) // PANEL * batch * self.k * 16), (torch.int64, 8 * self.groups),
+                     (probs[0], probs[1] * self.rows) if glu else (bf16, 2 * self.k), (torch.uint8, self.rows))
 
 
 @functools.lru_cache(maxsize=512)
@@ -675,10 +683,18 @@ def linear_forward_impl(plan: LinearPlan, x, w, w_scales=None, group_lens=None, 
 def linear_backward_impl(plan: LinearPlan, parts: int, dy, saved, scratch, dx=None, dw=None, daux=None, x=None, wt=None, wt_scales=None,
                          group_lens=None, aux0=None, aux1=None, accumulate: bool = False, sr_seed: int = 0) -> None:
     """``parts`` of the linear's backward (``_lib.LINEAR_*``, or'ed) on the current stream; ``scratch``
-    (``plan.bwd_bytes``) carries the quantised gradient from one part to the others."""
+    (``plan.bwd_bytes``) carries the quantised gradient from one part to the others.
+
+    What autograd kept comes back through the saved-tensor hooks of whoever set some, and a hook may return the values
+    with other strides, or not what it was given: everything is looked at before its address is handed over."""
     def ptr(t):
         return None if t is None else t.data_ptr()
 
+    device = scratch.get_device()
+    for t, (dtype, nbytes) in zip((saved, x, wt, wt_scales, group_lens, aux0, aux1), plan.kept):
+        if t is not None and (t.get_device() != device or not t.is_contiguous() or t.nbytes != nbytes or (dtype is not None and t.dtype != dtype)):
+            raise ValueError(f"the linear's backward needs the tensors its forward kept as they were: contiguous, {nbytes} bytes"
+                             f"{'' if dtype is None else f' of {dtype}'} on GPU {device} (got {t.nbytes} of {t.dtype} on {t.device}, strides {t.stride()})")
     rc = _lib.load().mxl_linear_backward(
         plan.ptr, parts, ptr(dy), ptr(x), ptr(aux0), ptr(aux1), ptr(wt), ptr(wt_scales), ptr(group_lens), ptr(saved), ptr(scratch),
         ptr(dx), ptr(daux), ptr(dw), _lib.GF_ACCUM_F32 if accumulate else 0, sr_seed, _stream())
