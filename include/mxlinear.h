@@ -529,7 +529,7 @@ typedef struct mxl_linear {
     int64_t input, probs_dtype;
     int64_t need_dx, need_dw, w_quantized, dx_from_rows;
     int64_t grad_sr;                     /* E2M1 gradients rounded stochastically (sr_seed of the backward) */
-    int64_t rht_signs;                   /* Hadamard signs of both wgrad operands, or -1 */
+    int64_t rht_signs;                   /* plain inputs: Hadamard signs of both wgrad operands, or -1 */
     double eps;                          /* of the RMSNorm */
     int64_t saved_bytes, fwd_bytes, bwd_bytes;   /* written by mxl_linear_sizes */
 } mxl_linear;
