@@ -529,9 +529,10 @@ __global__ __launch_bounds__(QTHREADS) void mx_quant_kernel(QuantArgs a) {
 // weight's (WCOL: its transposed codes too).  Neither fills the chip for long where the linear is small, and each launch
 // costs its fill and drain and the gap behind it.  Forward of a linear, quantisers and GEMM, two launches / one, us:
 // [256, 4096] x 4096 39.8 / 34.0; [1999, 2880] x 5760 67.9 / 62.8; [8192, 4096] x 14336 422 / 412; tensor-wise [4096, 14336] x
-// 4096 279 / 272; 8 experts of [2048, 2048], 2048 rows, 56 / 51.  Large experts read their weights at 108 registers a lane
-// instead of 58, which costs them nothing (the input may be transformed by Hadamard, or formed by an RMSNorm from statistics
-// that are there already; 32 x [4096, 7168], 8192 rows, 860 / 865; 8 x [28672, 4096], 512 rows, 694 / 668).
+// 4096 279 / 272; 8 experts of [2048, 2048], 2048 rows, 56 / 51.  The weight's workgroups hold the activations' 108 registers
+// a lane instead of 58, 4 waves per SIMD instead of 8, and large experts are mostly weight: 32 x [4096, 7168], 8192 rows, 860 /
+// 865; 8 x [28672, 4096], 512 rows, 694 / 668.  The input may be transformed by Hadamard, or formed by an RMSNorm from
+// statistics that are there already.
 template <int FMT, int SMODE, bool WCOL, int ACT = -1, bool RHT = false>
 __global__ __launch_bounds__(QTHREADS) void mx_quant_pair_kernel(QuantArgs x, QuantArgs w, unsigned x_wgs) {
     if (blockIdx.x < x_wgs) quant_workgroup<FMT, SMODE, true, true, false, ACT, false, RHT>(x, (int)blockIdx.x);
@@ -674,29 +675,27 @@ static int dispatch_quant_tensor(int fmt, QuantArgs& a, int64_t tiles_r, int64_t
     return MXL_EINVAL;
 }
 
-// both launches of a pair in one; false: there is no kernel for it
-static bool pair_taken(const HeldQuant& x, int fmt, int smode, const QuantArgs& w) {
-    return x.fmt == fmt && x.smode == smode && (smode == MXL_SCALE_OCP_FLOOR || smode == SCALE_TENSOR) && x.a.q_row && x.a.q_colT && w.q_row &&
-           (fmt == MXL_FMT_E4M3 || (fmt == MXL_FMT_E2M1 && smode == MXL_SCALE_OCP_FLOOR && x.act < 0));
-}
-static int launch_quant_pair(const HeldQuant& x, QuantArgs& w, int64_t tiles_r, int64_t tiles_c, hipStream_t st) {
-    int64_t wgs;
-    if (const int rc = quant_grid(w, tiles_r, tiles_c, &wgs)) return rc;
-    if (x.wgs + wgs > 0x7FFFFFFF) return MXL_EINVAL;
-    const dim3 grid((unsigned)(x.wgs + wgs));
-#define MXL_QP(F, S, ACT, RHT)                                                                                                              \
-    if (x.fmt == F && x.smode == S && x.act == ACT && x.rht == RHT) {                                                                       \
-        if (w.q_colT) hipLaunchKernelGGL((mx_quant_pair_kernel<F, S, true, ACT, RHT>), grid, dim3(QTHREADS), 0, st, x.a, w, (unsigned)x.wgs); \
-        else hipLaunchKernelGGL((mx_quant_pair_kernel<F, S, false, ACT, RHT>), grid, dim3(QTHREADS), 0, st, x.a, w, (unsigned)x.wgs);        \
-        return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;                                                                      \
-    }
+// the kernel for both quantisations of a pair; null: there is none, and each is launched by itself
+typedef void (*QuantPairKernel)(QuantArgs, QuantArgs, unsigned);
+static QuantPairKernel pair_kernel(const HeldQuant& x, int fmt, int smode, const QuantArgs& w) {
+    if (x.fmt != fmt || x.smode != smode || !x.a.q_row || !x.a.q_colT || !w.q_row) return nullptr;
+#define MXL_QP(F, S, ACT, RHT)                                              \
+    if (fmt == F && smode == S && x.act == ACT && x.rht == RHT)             \
+        return w.q_colT ? (QuantPairKernel)mx_quant_pair_kernel<F, S, true, ACT, RHT> : (QuantPairKernel)mx_quant_pair_kernel<F, S, false, ACT, RHT>;
     MXL_QP(MXL_FMT_E4M3, MXL_SCALE_OCP_FLOOR, -1, false)
     MXL_QP(MXL_FMT_E4M3, MXL_SCALE_OCP_FLOOR, PRO_RMSNORM, false)
     MXL_QP(MXL_FMT_E2M1, MXL_SCALE_OCP_FLOOR, -1, false)
     MXL_QP(MXL_FMT_E2M1, MXL_SCALE_OCP_FLOOR, -1, true)
     MXL_QP(MXL_FMT_E4M3, SCALE_TENSOR, -1, false)
 #undef MXL_QP
-    return MXL_EINVAL;
+    return nullptr;
+}
+static int launch_quant_pair(QuantPairKernel kern, const HeldQuant& x, QuantArgs& w, int64_t tiles_r, int64_t tiles_c, hipStream_t st) {
+    int64_t wgs;
+    if (const int rc = quant_grid(w, tiles_r, tiles_c, &wgs)) return rc;
+    if (x.wgs + wgs > 0x7FFFFFFF) return MXL_EINVAL;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(x.wgs + wgs)), dim3(QTHREADS), 0, st, x.a, w, (unsigned)x.wgs);
+    return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;
 }
 
 // abs-max of one or two bf16 tensors: non-negative floats order like their bit patterns, so an integer atomic max on
@@ -955,8 +954,9 @@ static int quantize_weight_2d(const void* w_bf16, int64_t batch, int64_t n, int6
     const int64_t gx = batch * ((n + QT - 1) / QT);
     const int64_t gy = ((q_row ? k_ld : k) + QT - 1) / QT;
     if (pair) {
-        *paired = pair->held && pair_taken(*pair, fmt, tensor_amax ? SCALE_TENSOR : scale_mode, a);
-        return *paired ? launch_quant_pair(*pair, a, gx, gy, (hipStream_t)stream) : MXL_OK;
+        const QuantPairKernel kern = pair->held ? pair_kernel(*pair, fmt, tensor_amax ? SCALE_TENSOR : scale_mode, a) : nullptr;
+        *paired = kern != nullptr;
+        return kern ? launch_quant_pair(kern, *pair, a, gx, gy, (hipStream_t)stream) : MXL_OK;
     }
     if (tensor_amax) return dispatch_quant_tensor<true>(fmt, a, gx, gy, (hipStream_t)stream);
     return dispatch_quant<true>(fmt, scale_mode, a, gx, gy, (hipStream_t)stream);
