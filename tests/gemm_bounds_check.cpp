@@ -36,6 +36,16 @@ static void request(const Desc& d, uint32_t voff, uint32_t soff, int64_t bytes, 
     }
 }
 
+// A request that is to read nothing (past a contraction range, rounds of a half tile) carries a scalar offset with kDropped
+// in it and has to be dropped whole.
+static void dropped(const Desc& d, uint32_t voff, const char* what, uint32_t soff = kDropped) {
+    for (int c = 0; c < 4; ++c) {
+        ++n_checked;
+        if (accepted(d, voff, soff, c)) fail(what, d.base, d.records, voff, c);
+        else ++n_dropped;
+    }
+}
+
 static void check_slot2(int layout, int kb_row /* bytes of a row per K slot: 128 FP8, 64 FP4 */, int64_t rows_total, int64_t k_slots,
                         int64_t row0) {
     const int cpr = kb_row / 16, rows_per_ld = 256 / cpr, rounds = cpr;   // cpr rounds cover 256 rows
@@ -84,6 +94,8 @@ static void check_ring(int row_bytes, int64_t rows_total, int64_t steps, int64_t
                 const uint32_t voff = ring_code_lane(t, e, half);
                 const int row = half ? (t >> 1) + 128 * e : (t >> 2) + 64 * e;
                 request(d, voff, (uint32_t)(st * rows_total * row_bytes), bytes, row0 + row < rows_total && st < steps, "ring codes");
+                // a tile of at most 128 rows sends its other rounds to a scalar offset that has kDropped in it
+                if (!half && e >= 2) dropped(d, voff, "ring codes, rounds of a half tile", (uint32_t)(st * rows_total * row_bytes) | kDropped);
             }
     const int64_t panels = (steps * 64 + 511) / 512, pbytes = panels * rows_total * 16;
     const Desc dp = ring_panel_desc(rows_total, panels, row0);
@@ -131,16 +143,7 @@ static void check_ring_bt4(int64_t groups, int64_t kc, int64_t planes, int64_t g
                 request(d, ring_bt4_lane(t, e, rows_total), (uint32_t)(st * 128 * 64), bytes, plane0 + (e >> 1) < planes, "ring E2M1 codes transposed");
 }
 
-// ---- small-tile kernel (mx_gemm_tile_body.h): TM or TN rows per tile, ST K steps requested ahead.  A request past the
-// contraction range carries the scalar offset kDropped and has to be dropped whole. ----
-static void dropped(const Desc& d, uint32_t voff, const char* what) {
-    for (int c = 0; c < 4; ++c) {
-        ++n_checked;
-        if (accepted(d, voff, kDropped, c)) fail(what, d.base, d.records, voff, c);
-        else ++n_dropped;
-    }
-}
-
+// ---- small-tile kernel (mx_gemm_tile_body.h): TM or TN rows per tile, ST K steps requested ahead ----
 // codes of one operand: `rows` tile rows from row0 on, K steps st0 .. st0 + nst - 1 of `steps`
 static void check_tile_codes(int rows, int row_bytes, int64_t rows_total, int64_t steps, int64_t row0, int64_t st0, int64_t nst) {
     const bool half = row_bytes == 32;
@@ -201,7 +204,10 @@ static void check_tiles() {
                     }
     // the largest operand the entry points admit: num_records 32 bytes short of 2^32
     for (int t = 0; t < 256; ++t)
-        for (int e = 0; e < 2; ++e) dropped(Desc{0, (1ll << 32) - 32}, ring_code_lane(t, e, false), "largest operand");
+        for (int e = 0; e < 4; ++e) {
+            dropped(Desc{0, (1ll << 32) - 32}, ring_code_lane(t, e, false), "largest operand");
+            if (e >= 2) dropped(Desc{0, (1ll << 32) - 32}, ring_code_lane(t, e, false), "largest operand, rounds of a half tile", (1u << 20) | kDropped);
+        }
 }
 
 // ---- the 256-row bf16 tile (bf16_gemm_tall_kernel): slots of 64 contraction elements, eight requests a slot and wave and
@@ -282,9 +288,13 @@ int main() {
             for (int64_t k_slots : {1, 2, 5})
                 for (int layout = 0; layout < 2; ++layout)
                     for (int kb_row : {128, 64}) check_slot2(layout, kb_row, rows_total, k_slots, row0);
-            for (int64_t steps : {2, 4, 9})
+            for (int64_t steps : {1, 2, 4, 9})
                 for (int row_bytes : {64, 32}) check_ring(row_bytes, rows_total, steps, row0);
         }
+    // the lower half of a last round's tile may begin up to 127 rows behind the operand's last row
+    for (int64_t rows_total : {1, 31, 128, 255, 256, 257, 300})
+        for (int64_t past : {0, 1, 63, 127})
+            for (int64_t steps : {1, 2, 4, 9}) check_ring(64, rows_total, steps, rows_total + past);
     // the last rows of a large operand (descriptor fields near their limits; nothing is dereferenced)
     check_ring(64, (1ll << 31) / 64 / 16 + 3, 16, (1ll << 31) / 64 / 16 - 200);
     check_slot2(1, 128, (1ll << 24) - 5, 1, (1ll << 24) - 250);

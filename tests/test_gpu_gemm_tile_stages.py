@@ -1,5 +1,6 @@
 """The small tiles with eight stages (one workgroup to a CU, contractions from 48 K steps on) against the ring kernel, bit for
-bit: contractions on both sides of that line and of a scale panel, ragged rows and groups, transposed weight codes."""
+bit: contractions on both sides of that line (contractions are multiples of 128, so 47 steps of 64 are 48, and 46 the last
+number below it) and of a scale panel, more than 256 tiles, ragged rows and groups, transposed weight codes."""
 
 import pytest
 import torch
@@ -9,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("recipe", ["mxfp8", "mxfp4w8", "mxfp4"])
 @pytest.mark.parametrize("tile", ["64", "64x128"])
-@pytest.mark.parametrize("lens,n,steps", [(None, 96, 47), (None, 256, 48), (None, 128, 53), (None, 160, 64), ([33, 0, 130, 1], 128, 50), ([0, 70], 96, 72)])
+@pytest.mark.parametrize("lens,n,steps", [(None, 128, 46), (None, 96, 47), (None, 256, 48), (None, 11296, 48), (None, 128, 53), (None, 160, 64), ([33, 0, 130, 1], 128, 50), ([0, 70], 96, 72)])
 def test_eight_stages_give_the_same_bits(gpu, recipe, tile, lens, n, steps):
     from primus_amd.pytorch import kernels as K
 

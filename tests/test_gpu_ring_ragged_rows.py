@@ -104,3 +104,47 @@ def test_weight_gradient_in_halves(gpu, recipe, m, n, k, grouped):
     into = torch.zeros(want.shape, dtype=torch.float32, device=gpu)
     run(None, into)
     assert torch.equal(into.bfloat16().view(torch.int16), want.view(torch.int16))
+
+
+# the same splits on transposed weight codes (every input gradient) and under per-tensor factors
+@pytest.mark.parametrize("kind", ["mxfp8 transposed", "mxfp4 transposed", "e4m3 scaled", "e5m2 scaled", "e4m3 scaled transposed", "e5m2 scaled transposed"])
+@pytest.mark.parametrize("lens,n", [((2700,), 6112), ((2688,), 6144), ((2590,), 6112), ((2800, 16), 5984), ((0, 3, 0, 0, 300, 0, 1, 0), 480)])
+def test_last_round_in_halves_other_kernels(gpu, kind, lens, n):
+    from primus_amd.pytorch import kernels as K
+
+    m, k, G, bt = sum(lens), 128, len(lens), "transposed" in kind
+    g = torch.Generator().manual_seed(n + m)
+    x = torch.randn(m, k, generator=g).bfloat16().to(gpu)
+    w = (torch.randn(G, *((k, n) if bt else (n, k)), generator=g) * 0.05).bfloat16().to(gpu)
+    gl = torch.tensor(lens, dtype=torch.int64, device=gpu)
+    if "scaled" in kind:
+        xq = K.quantize_tensorwise_impl(x, _lib.FMT_E5M2 if "e5m2" in kind else _lib.FMT_E4M3, rowwise=True, colwise=False, pad_to=128, kchunk=2)
+        wq = K.quantize_weight_tensorwise_impl(w, _lib.FMT_E4M3, rowwise=True, colwise=False, pad_to=128, kchunk=2)
+        run = lambda t: K.gemm_tw_nt_impl(xq[0], xq[1], xq[4], wq[0], wq[1], wq[4], gl, kchunk=2, b_transposed_n=n if bt else None, tile=t)
+    else:
+        fmt, lay = {"mxfp8": (0, 2), "mxfp4": (1, 3)}[kind.split()[0]]
+        xq = K.quantize_mx_impl(x, fmt, rowwise=True, colwise=False, group_lens=gl, pad_to=128, kchunk=lay)
+        wq = K.quantize_mx_weight_2d_impl(w, fmt, rowwise=True, colwise=True, pad_to=128, kchunk=lay, col_scales_only=True)
+        run = lambda t: K.grouped_gemm_mx_nt_impl(xq[0], xq[1], wq[0], wq[3], gl, kchunk=lay, b_transposed=True, tile=t)
+    got, want = run("256"), run("128")
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+# an output aligned to less than the stores' 16 bytes, inside a larger buffer
+@pytest.mark.parametrize("offset", [0, 1, 2, 4])
+@pytest.mark.parametrize("m,n", [(300, 96), (33, 320)])
+def test_output_alignment(gpu, offset, m, n):
+    from primus_amd.pytorch import kernels as K
+
+    k = 256
+    g = torch.Generator().manual_seed(n)
+    xq = K.quantize_mx_impl(torch.randn(m, k, generator=g).bfloat16().to(gpu), 0, rowwise=True, colwise=False, pad_to=128, kchunk=2)
+    wq = K.quantize_mx_weight_2d_impl(torch.randn(n, k, generator=g).bfloat16().to(gpu), 0, rowwise=True, colwise=False, pad_to=128, kchunk=2)
+    want = K.gemm_mx_nt_impl(xq[0], xq[1], wq[0], wq[1], kchunk=2)
+    buf = torch.full((GUARD + m * n + GUARD,), 7.0, dtype=torch.bfloat16, device=gpu)
+    at = GUARD // 2 + offset
+    rc = _lib.load().mxl_grouped_gemm_nt_ex(xq[0].data_ptr(), xq[1].data_ptr(), 0, wq[0].data_ptr(), wq[1].data_ptr(), 0, buf[at:].data_ptr(),
+                                            None, 1, m, n, k, _lib.GF_KSTEP | _lib.GF_TILES["256"], torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    assert torch.equal(buf[at:at + m * n].view(m, n).view(torch.int16), want.view(torch.int16))
+    assert bool((buf[:at] == 7.0).all()) and bool((buf[at + m * n:] == 7.0).all())
