@@ -281,6 +281,10 @@ int mxl_grouped_gemm_bf16(const void* a_bf16, const void* b_bf16, void* c_bf16, 
 int mxl_grouped_gemm_bf16_wgrad(const void* p_bf16, const void* q_bf16, void* c, const int64_t* group_lens, int num_groups,
                                 int64_t total_m, int64_t m_out, int64_t n_out, uint32_t flags, void* stream);
 
+/* mask[i] = i < lens[0] + ... + lens[count - 1], 0 or 1 per byte (tokens_per_expert_to_mask), from counts on the device.
+ * count >= 1, rows >= 0, mask 16-byte aligned. */
+int mxl_row_mask(const int64_t* lens, int64_t count, int64_t rows, uint8_t* mask, void* stream);
+
 /* Gated activation of the expert MLP fused with the router probability and the row mask
  * (swiglu_with_probs / geglu_with_probs behind fused_bias_act_with_probs, primus_turbo.py:1954-1980;
  * the unfused arithmetic is experts.py:100-118):
@@ -288,8 +292,6 @@ int mxl_grouped_gemm_bf16_wgrad(const void* p_bf16, const void* q_bf16, void* c,
  * computed in fp32, rounded once to bf16.  row_mask (one byte per row, may be NULL = all rows live):
  * a row with mask 0 yields zeros (tokens_per_expert_to_mask marks the rows past the routed tokens
  * of a worst-case sized buffer).  probs is fp32 or bf16 per probs_dtype.  Requires f % 8 == 0. */
-/* mask[i] = i < lens[0] + ... + lens[count - 1] (0 or 1 per byte, 16-byte aligned), on the device. */
-int mxl_row_mask(const int64_t* lens, int64_t count, int64_t rows, uint8_t* mask, void* stream);
 int mxl_glu_probs_fwd(const void* x_bf16, const void* probs, int probs_dtype, const uint8_t* row_mask,
                       int64_t rows, int64_t f, int act, void* y_bf16, void* stream);
 

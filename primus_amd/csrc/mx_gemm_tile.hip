@@ -17,9 +17,9 @@ static int launch_tile(const GemmArgs& a, hipStream_t st) {
 }
 
 // Forward and input gradients: eight stages where every CU has at most one workgroup and its contraction is at least 48 K
-// steps long, else four.  Alone on
-// its CU a workgroup waits for memory at the distance it asks ahead: a K step's MFMAs are over in a quarter of a microsecond,
-// and with four stages 224 CUs keep 5 MB on their way, which over the latency is half of what the memory delivers.
+// steps long, else four.  Alone on its CU a workgroup waits for memory at the distance it asks ahead: a K step's MFMAs are
+// over in a quarter of a microsecond, and with four stages 224 CUs keep 5 MB on their way, which over the latency is half of
+// what the memory delivers.
 // us, four / eight stages, weights from memory: 64 x 64 tiles, [64, 4096] x 14336 16.8 / 13.7, [64, 14336] x 4096 44.2 / 31.4,
 // [32, 8192] x 8192 28.8 / 19.4, [256, 4096] x 4096 10.6 / 8.5; with more than 256 tiles [512, 4096] x 4096 13.8 / 14.3.
 // 64 x 128 tiles, [512, 4096] x 4096 13.3 / 12.3; E2M1 weights against FP8 rows, [64, 4096] x 14336 14.5 / 11.5.

@@ -1,6 +1,6 @@
 // One linear as two calls: everything its forward launches, and everything its backward launches (host code only).
 //
-// A linear is 2 to 4 launches forward and 3 to 6 backward, and a dozen buffers.  Issued one by one from Python, with an
+// A linear is 2 to 4 launches forward and 2 to 5 backward, and a dozen buffers.  Issued one by one from Python, with an
 // allocation per buffer and a stream look-up per launch, they take 230 us for a pass whose kernels need 60.  Here the
 // caller allocates three buffers -- what the backward needs, and a scratch buffer per direction -- and makes one call per
 // direction; the layout of the buffers is arithmetic on the sizes and is worked out again in every call.
@@ -115,8 +115,8 @@ struct BackwardScratch {
 };
 
 // The 128-blockwise recipe (forward and backward of [1024, 2048] x 2048 190 -> 108 us in two calls, [256, 4096] x 4096 191 ->
-// 119; launch by launch it is bound by the host there).  Forward: row-wise copies of x and w.  Backward, from the bf16 tensors: both copies of dy, the
-// transposed ones of x and w.
+// 119; launch by launch it is bound by the host there).  Forward: row-wise copies of x and w.  Backward, from the bf16
+// tensors: both copies of dy, the transposed ones of x and w.
 struct BwForward {
     Copy x, w;
     BwForward(const Linear& l, Arena& a) {
