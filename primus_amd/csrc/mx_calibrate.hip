@@ -105,7 +105,7 @@ __global__ __launch_bounds__(256) void mfma_only_bf16_kernel(int iters) {
 // The traffic of the dual quantiser without its arithmetic: every workgroup reads a 128 x 128 bf16 tile (16 bytes per
 // lane, rows adjacent) and writes one byte per element at the tile's place in a row-major array and one byte per
 // element at its place in the transposed array (16-byte stores; the bytes are XORs of the input, nothing is
-// transposed or converted), streaming loads and stores, tiles walked in the quantiser's order (8 x 8 supertiles, one
+// transposed or converted), streaming loads and stores, tiles walked in the quantiser's order (4 x 4 supertiles, one
 // XCD each).  What this moves per second is what the quantiser's access pattern allows on the board.
 typedef uint32_t cu32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t cu32x2 __attribute__((ext_vector_type(2)));
@@ -114,10 +114,10 @@ __global__ __launch_bounds__(256) void tile_copy_kernel(const uint16_t* in, uint
                                                         int64_t w_ld, int tiles_r, int tiles_c, int super_c, int n_super) {
     constexpr int TR = 128, TC = 128;
     const int L = blockIdx.x, xcd = L & 7, k = L >> 3;
-    const int sup = (k / 64) * 8 + xcd;
+    const int sup = (k / 16) * 8 + xcd;
     if (sup >= n_super) return;
-    const int within = k % 64;
-    const int pt = (sup / super_c) * 8 + within / 8, ct = (sup % super_c) * 8 + within % 8;
+    const int within = k % 16;
+    const int pt = (sup / super_c) * 4 + within / 4, ct = (sup % super_c) * 4 + within % 4;
     if (pt >= tiles_r || ct >= tiles_c) return;
     const int t = threadIdx.x;
     constexpr int LPR = TC * 2 / 16, RPI = 256 / LPR, NIT = TR / RPI;   // 16 lanes a row, 16 rows a pass, 8 passes
@@ -190,17 +190,17 @@ extern "C" int mxl_calibrate_tile_copy(const void* in_bf16, int64_t rows, int64_
     if ((((uintptr_t)in_bf16 | (uintptr_t)out_row | (uintptr_t)out_colT) & 15) != 0) return MXL_EINVAL;
     if (!device_is_gfx950()) return MXL_ENODEV;
     const int tiles_r = (int)(rows / 128), tiles_c = (int)(cols / 128);
-    const int super_r = (tiles_r + 7) / 8, super_c = (tiles_c + 7) / 8, n_super = super_r * super_c;
-    const int64_t wgs = (int64_t)(n_super + 7) / 8 * 8 * 64;
+    const int64_t super_r = (tiles_r + 3) / 4, super_c = (tiles_c + 3) / 4, n_super = super_r * super_c;
+    const int64_t wgs = (n_super + 7) / 8 * 8 * 16;
     if (wgs > 0x7FFFFFFF) return MXL_EINVAL;
     hipStream_t st = (hipStream_t)stream;
     const dim3 grid((unsigned)wgs), block(256);
     const uint16_t* in = (const uint16_t*)in_bf16;
     uint8_t *o1 = (uint8_t*)out_row, *o2 = (uint8_t*)out_colT;
-    if (o1 && o2) hipLaunchKernelGGL((tile_copy_kernel<true, true>), grid, block, 0, st, in, o1, o2, cols, rows, tiles_r, tiles_c, super_c, n_super);
-    else if (o1) hipLaunchKernelGGL((tile_copy_kernel<true, false>), grid, block, 0, st, in, o1, o2, cols, rows, tiles_r, tiles_c, super_c, n_super);
-    else if (o2) hipLaunchKernelGGL((tile_copy_kernel<false, true>), grid, block, 0, st, in, o1, o2, cols, rows, tiles_r, tiles_c, super_c, n_super);
-    else hipLaunchKernelGGL((tile_copy_kernel<false, false>), grid, block, 0, st, in, o1, o2, cols, rows, tiles_r, tiles_c, super_c, n_super);
+    if (o1 && o2) hipLaunchKernelGGL((tile_copy_kernel<true, true>), grid, block, 0, st, in, o1, o2, cols, rows, tiles_r, tiles_c, (int)super_c, (int)n_super);
+    else if (o1) hipLaunchKernelGGL((tile_copy_kernel<true, false>), grid, block, 0, st, in, o1, o2, cols, rows, tiles_r, tiles_c, (int)super_c, (int)n_super);
+    else if (o2) hipLaunchKernelGGL((tile_copy_kernel<false, true>), grid, block, 0, st, in, o1, o2, cols, rows, tiles_r, tiles_c, (int)super_c, (int)n_super);
+    else hipLaunchKernelGGL((tile_copy_kernel<false, false>), grid, block, 0, st, in, o1, o2, cols, rows, tiles_r, tiles_c, (int)super_c, (int)n_super);
     return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;
 }
 
