@@ -330,12 +330,19 @@ __device__ __forceinline__ void bw_quant_workgroup(const BwQuantArgs& a, int L, 
     }
 }
 
+template <int FMT, bool TWOD>
+__global__ __launch_bounds__(BW_THREADS) void bw_quant_kernel(BwQuantArgs a) {
+    __shared__ BwQuantLds lds;
+    bw_quant_workgroup<FMT, TWOD>(a, (int)blockIdx.x, TWOD ? (int64_t)blockIdx.y : 0, lds);
+}
+
 // Up to three tensors in one launch: a linear's forward quantises its input and its weight, its backward the gradient, the
 // input again and the weight again, none of which waits for another.  Workgroups [0, end[0]) are the first tensor's, and so
 // on; those of a batch of weights go through its matrices one after the other.  A launch of an ordinary linear's tensor
 // lasts 12 to 17 us, of which a third is filling and draining the chip and the gap to the next one.  Five launches to two
 // over a forward and backward: [3000, 7168] x 2048 250 -> 236 us, [4096, 4096] x 4096 299 -> 288, [8192, 4096] x 14336 1665 -> 1638;
-// what small linears gain on top of that is host time (mx_linear.hip).
+// what small linears gain on top of that is host time (mx_linear.hip).  A tensor alone has the kernel above: picking its
+// arguments out of three costs a small one up to half a microsecond (row-wise copy of [2048, 4096] 5.9 / 6.3 us).
 constexpr int BW_SEVERAL = 3;
 struct BwQuantSeveral {
     BwQuantArgs a[BW_SEVERAL];
@@ -343,7 +350,7 @@ struct BwQuantSeveral {
     int per_mat[BW_SEVERAL];    // workgroups of a matrix; 0: 1-D blocks
 };
 template <int FMT>
-__global__ __launch_bounds__(BW_THREADS) void bw_quant_kernel(BwQuantSeveral s) {
+__global__ __launch_bounds__(BW_THREADS) void bw_quant_several_kernel(BwQuantSeveral s) {
     __shared__ BwQuantLds lds;
     const int block = (int)blockIdx.x;
     int i = 0, first = 0;
@@ -945,9 +952,22 @@ int bw_quantize(const BwTensor* tensors, int n, int fmt, void* stream) {
     if (count == 0) return MXL_OK;
     if (!device_is_gfx950()) return MXL_ENODEV;
     const int wgs = s.end[count - 1];
+    hipStream_t st = (hipStream_t)stream;
+    if (count == 1) {
+        const int per = s.per_mat[0];
+        const dim3 grid((unsigned)(per ? per : wgs), (unsigned)(per ? wgs / per : 1));
+        if (fmt == MXL_FMT_E4M3) {
+            if (per) hipLaunchKernelGGL((bw_quant_kernel<MXL_FMT_E4M3, true>), grid, dim3(BW_THREADS), 0, st, s.a[0]);
+            else hipLaunchKernelGGL((bw_quant_kernel<MXL_FMT_E4M3, false>), grid, dim3(BW_THREADS), 0, st, s.a[0]);
+        } else {
+            if (per) hipLaunchKernelGGL((bw_quant_kernel<MXL_FMT_E5M2, true>), grid, dim3(BW_THREADS), 0, st, s.a[0]);
+            else hipLaunchKernelGGL((bw_quant_kernel<MXL_FMT_E5M2, false>), grid, dim3(BW_THREADS), 0, st, s.a[0]);
+        }
+        return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;
+    }
     for (int i = count; i < BW_SEVERAL; ++i) s.end[i] = wgs;
-    if (fmt == MXL_FMT_E4M3) hipLaunchKernelGGL((bw_quant_kernel<MXL_FMT_E4M3>), dim3((unsigned)wgs), dim3(BW_THREADS), 0, (hipStream_t)stream, s);
-    else hipLaunchKernelGGL((bw_quant_kernel<MXL_FMT_E5M2>), dim3((unsigned)wgs), dim3(BW_THREADS), 0, (hipStream_t)stream, s);
+    if (fmt == MXL_FMT_E4M3) hipLaunchKernelGGL((bw_quant_several_kernel<MXL_FMT_E4M3>), dim3((unsigned)wgs), dim3(BW_THREADS), 0, st, s);
+    else hipLaunchKernelGGL((bw_quant_several_kernel<MXL_FMT_E5M2>), dim3((unsigned)wgs), dim3(BW_THREADS), 0, st, s);
     return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;
 }
 
