@@ -240,8 +240,9 @@ extern "C" int mxl_linear_forward(const mxl_linear* p, const void* x, const void
     const bool from_rows = p->need_dx && p->dx_from_rows;
     const Copy wr = from_rows ? sv.w_row : f.w_row;
     const bool rht = p->rht_signs >= 0 && p->need_dw && p->input == MXL_LINEAR_PLAIN && !l.tensorwise();
-    const mxl::LinearOperands both = {x, w, p->rows, l.batch, p->n, p->k, l.k_ld, l.n_ld,
-                                      l.tensorwise() && !p->need_dw ? nullptr : lens, l.tensorwise() && !p->need_dw ? 0 : G,
+    // (a tensor-wise scaled row-wise copy by itself knows no groups, nor do the copies of an input that an RMSNorm forms)
+    const bool ungrouped = (l.tensorwise() && !p->need_dw) || p->input == MXL_LINEAR_RMSNORM;
+    const mxl::LinearOperands both = {x, w, p->rows, l.batch, p->n, p->k, l.k_ld, l.n_ld, ungrouped ? nullptr : lens, ungrouped ? 0 : G,
                                       af, wf, (int)p->scale_mode, l.qf() | (rht ? MXL_QF_RHT_COL : 0u), rht ? (uint32_t)p->rht_signs : 0u,
                                       f.x_amax, f.w_amax, sv.x_si, sv.w_si,
                                       p->input == MXL_LINEAR_RMSNORM ? aux0 : nullptr, sv.rstd,
