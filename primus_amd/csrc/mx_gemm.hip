@@ -1372,22 +1372,26 @@ static bool tile_flag_ok(uint32_t flags) {
 // 256 x 256 53 -- per flop the ring kernel is the cheapest (1 : 0.93 : 0.69 : 0.51), but it needs 256 tiles to occupy the
 // chip, and its launches cost whole rounds of 256.  A dense launch takes the tile with the least ceil(tiles / 256) * cost.
 // Only the first two rounds are priced as whole ones: from the third on a partly filled round runs at a higher clock, and at
-// the board's power limit the small tiles' LDS reads cost what the empty CUs would ([4096, 14336] x [4096, 14336]
-// tensor-wise, 3.5 rounds each in the backward, whole linear 699 us on ring tiles, 746 on 128 x 128 ones; 1.08 rounds, the
-// weight gradient of 1999 tokens, 5760 x 2880: 57 and 41 us; 1.5 rounds, 3333 tokens, 3072 x 8192: 96 and 76).
-//   [256, 4096] x [4096, 4096]: ring 41.2 us, 128 13.2, 64 x 128 10.4, 64 x 64 8.9.   [1024, ...]: 42.4, 18.4, 22.2, 27.6
-//   [1999, 2880] x [5760, 2880]: 39.2, 34.0, 45.7, 54.4.   [4096, 4096] x [4096, 4096]: 56.3, 60.1, 80.6, 106
+// the board's power limit the small tiles' LDS reads cost what the empty CUs would (3.5 rounds, [4096, 4096] x 14336: 186 us
+// on ring tiles, 207 on 128 x 128 ones; the weight gradient of 4096 tokens, 4096 x 14336: 186 and 207).  Since the ring
+// kernel runs a last round of at most half the workgroups on halves of its tiles, its second round costs about half of what
+// the rule takes it for, and 128 x 128 tiles chosen there are ahead by less, or by nothing:
+//   ring / 128, us: 1.08 rounds, weight gradient of 1999 tokens, 5760 x 2880, 45 / 40; 1.13 and 1.25, [4096, 4096] x 4608 and 5120,
+//   78 / 72 and 80 / 75; 1.5, x 6144, 85 / 89, and weight gradients of 3333 tokens, 3072 x 8192 and 8192 x 3072, 77 / 76 and 75 / 78
+// All four, operands in the cache where they fit:
+//   [256, 4096] x [4096, 4096]: ring 28 us, 128 13, 64 x 128 11.2, 64 x 64 8.4.   [1024, ...]: 41, 19-21, 23, 28
+//   [1999, 2880] x [5760, 2880]: 37, 35, 45, 55.   [4096, 4096] x [4096, 4096]: 57, 61, 80, 102
 // A grouped launch does not know its tile counts (they are on the device): a group's last row tile is taken as half full.
 // Up to about one round of the ring kernel the same rule holds.  Beyond that a launch is bound by reading the weights,
 // which the ring kernel does best from about 32 rows per group on; with fewer its two and a half rounds of mostly empty
 // tiles cost more than the smaller tiles' shorter reads.  E2M1 weights against FP8 rows are half the bytes, which shifts
 // the line up.
-//   128 groups, [5760, 2880]: 4 rows per group ring 378 us, 64 x 128 317 (E2M1 weights 272, 183); 64 rows 474, 530 (413, 333)
-//   32 groups, [4096, 7168]: 32 rows per group ring 185, 128 180 (transposed codes 238, 196); 64 rows 187, 208 (243, 217)
+//   128 groups, [5760, 2880]: 4 rows per group ring 418 us, 64 x 128 377 (E2M1 weights 308, 217); 64 rows 433, 467 (317, 267)
+//   32 groups, [4096, 7168]: 32 rows per group ring 169, 128 175 (transposed codes 206, 183); 64 rows 169, 174 (212, 180)
 // The weight gradient's tiles are all output and little contraction: dense ones take 128 x 128 while the contraction is
-// short (256 tokens, 14336 x 4096: 43 -> 29 us).  Grouped ones run the ring kernel, which writes more per second on
-// expert-sized gradients, if far from what a fill does (256 rows in each of 32 groups, [4096, 7168]: 458 us, a fill of its
-// 1.9 GB 273; skewed rows, ring 474, 128 x 128 tiles 541), except where the gradient is a few tiles.
+// short (256 tokens, 14336 x 4096: ring 38 us, 128 x 128 31).  Grouped ones run the ring kernel, which writes more per second on
+// expert-sized gradients, if far from what a fill does (256 rows in each of 32 groups, [4096, 7168]: ring 404 us, 128 x 128
+// tiles 494, a fill of its 1.9 GB 277; skewed rows 444 and 573), except where the gradient is a few tiles.
 template <int MODE> static int tile_choice(const GemmArgs& a, bool e2m1_weights, bool bt, uint32_t flags) {
     switch (flags & MXL_GF_TILE_MASK) {
         case MXL_GF_TILE_64: return TILE_64;

@@ -155,10 +155,11 @@ def _overlaps(plan) -> bool:
     """Whether the weight gradient runs on the side stream next to dgrad.  Both are persistent kernels on every CU, so what
     the overlap gives is their last, partial rounds of tiles and their epilogues under the other's MFMAs; what it costs is
     the events between the streams, operand panels of two GEMMs in the same L2s, and buffers the allocator must keep for
-    two streams.  Measured, together / one after the other: dense [8192, 4096] x 14336 1.29 / 1.28 ms, [2048, 4096] x 4096
-    217 / 144 us; Mixtral experts MXFP8, 16384 tokens, 16.5 / 16.3 ms.  Grouped E2M1 operands gain (Mixtral MXFP4, 4096
-    tokens 3.81 / 3.88 ms, 16384 10.6 / 10.7; at 2048 tokens and 4096 x 4096 experts 936 / 936 us), FP8 ones with groups of up
-    to about 1000 rows a little (DeepSeek shard, 4096 tokens, 5.59 / 5.63; 8192 tokens 9.39 / 9.37)."""
+    two streams.  Measured, together / one after the other: dense [8192, 4096] x 14336 1.22 / 1.20 ms, [2048, 4096] x 4096
+    210 / 140 us, E2M1 [4096, 4096] x 14336 451 / 437.  Grouped E2M1 operands gain (Mixtral MXFP4, 4096 tokens 3.71 / 3.75 ms,
+    16384 10.4 / 10.5; not yet at 2048 tokens and 4096 x 4096 experts, 869 / 863 us), FP8 ones with groups of up to about 1000
+    rows a little (DeepSeek shard, 4096 tokens, 5.51 / 5.57; 8192 tokens, 2048 rows a group, 9.33 / 9.37).  Mixtral experts MXFP8,
+    16384 tokens, 4096 rows a group, gain too (16.15 / 16.5 ms), which this line, drawn when they lost (16.5 / 16.3), leaves out."""
     flops = 2.0 * plan.rows * plan.n * plan.k
     if plan.groups == 0:
         return False
