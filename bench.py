@@ -70,7 +70,7 @@ WORKLOADS = {
 # elementwise kernel: 2.000 and 1.000).  The counter summary is committed as
 # profiles/bench_mixtral_mxfp8_hbm_traffic.txt.
 TRAFFIC_BYTES_PER_LAUNCH = {
-    "mixtral_8x7b_moe_mxfp8": (3099696.1 * 2.000 + 821230.5 * 1.000) * 1024,
+    "mixtral_8x7b_moe_mxfp8": (3553658.9 * 2.000 + 819303.1 * 1.000) * 1024,
 }
 
 
