@@ -508,7 +508,7 @@ int mxl_shuffle_scales(const void* src, int64_t rows, int64_t cols, void* dst, i
  *             into it (aux0 = norm weight; daux = its bf16 gradient).
  *   w         bf16 [groups, n, k], or with w_quantized the row-wise codes (w_scales: their scales); the backward is then
  *             given the transposed copy (wt, wt_scales).
- *   dx_from_rows  the backward reads the row-wise codes transposed (MXL_GF_B_TRANSPOSED); n and k multiples of 128.
+ *   dx_from_rows  the backward reads the row-wise codes transposed (MXL_GF_B_TRANSPOSED).
  * recipe MXL_LINEAR_TENSORWISE takes plain inputs and bf16 weights.  MXL_LINEAR_BLOCKWISE (the 128-blockwise recipe: row-major
  * copies, n and k multiples of 128, no fused accumulation) does too; its backward starts from the bf16 tensors again and is
  * given x and, as wt, w.  rows > 0. */

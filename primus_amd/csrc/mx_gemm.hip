@@ -715,7 +715,7 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
     const int vwg = (nwg & 7) ? (int)blockIdx.x : ((int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3));
 
     const int64_t a_rows_total = (MODE == MODE_FWD) ? p.total_m : p.m;
-    const int64_t b_rows_total = (MODE == MODE_FWD) ? (int64_t)G * p.n : p.n;
+    const int64_t b_rows_total = (MODE == MODE_FWD) ? (int64_t)G * p.b_rows : p.n;
     // K-step-major codes: [k / 64][rows][64]; scales: [ceil(k / 512)][rows][16] (16 bytes = 8 K steps of a row)
     const uint32_t a_cstride = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a_rows_total * BK));
     // BT: the rows of b's code array are the contraction index (G * k of them); a K step moves on by 64 rows inside
@@ -785,7 +785,7 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
             const int64_t r = (int64_t)(pid_m - pre_tiles[grp]) * BM + lower * HALF_ROWS;
             a_row0 = g_row0 + r;
             d.m_valid = __builtin_amdgcn_readfirstlane((g_rows - r) < most ? (int)(g_rows - r) : most);
-            b_row0 = (int64_t)grp * p.n + (int64_t)pid_n * BN;
+            b_row0 = (int64_t)grp * p.b_rows + (int64_t)pid_n * BN;
             c_row0 = a_row0;
             k0 = 0;
             k1 = p.k;
@@ -1590,7 +1590,10 @@ __global__ __launch_bounds__(256) void zero_fill_kernel(uint32_t* dst, int64_t w
 
 static int grouped_gemm_nt(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes, const void* b_scales,
                            int b_fmt, void* c_bf16, const int64_t* group_lens, int num_groups, int64_t total_m, int64_t n,
-                           int64_t k, const float* alpha_a, const float* alpha_b, uint32_t flags, void* stream, HeldGemm* hold = nullptr) {
+                           int64_t k, const float* alpha_a, const float* alpha_b, uint32_t flags, void* stream, HeldGemm* hold = nullptr,
+                           int64_t b_rows = 0) {
+    if (b_rows == 0) b_rows = n;
+    if (b_rows < n || (b_rows > n && (!(flags & MXL_GF_KSTEP) || (flags & MXL_GF_B_TRANSPOSED)))) return MXL_EINVAL;
     if (flags & ~(uint32_t)(MXL_GF_KCHUNK | MXL_GF_KSTEP | MXL_GF_B_TRANSPOSED | MXL_GF_B_SHUFFLED | MXL_GF_TILE_MASK)) return MXL_EINVAL;
     if (!tile_flag_ok(flags)) return MXL_EINVAL;
     if ((flags & MXL_GF_KCHUNK) && (flags & MXL_GF_KSTEP)) return MXL_EINVAL;
@@ -1617,6 +1620,7 @@ static int grouped_gemm_nt(const void* a_codes, const void* a_scales, int a_fmt,
     a.total_m = total_m;
     a.m = 0;
     a.n = n;
+    a.b_rows = b_rows;
     a.k = k;
     a.alpha_a = alpha_a;
     a.alpha_b = alpha_b;
@@ -1630,7 +1634,7 @@ static int grouped_gemm_nt(const void* a_codes, const void* a_scales, int a_fmt,
         return dispatch_gemm_ring_bt(a_fmt, b_fmt, a, max_tiles, (hipStream_t)stream, flags, hold);
     }
     return dispatch_gemm<MODE_FWD>(a_fmt, b_fmt, a, max_tiles, (flags & MXL_GF_KSTEP) ? 2 : (flags & MXL_GF_KCHUNK) ? 1 : 0, total_m,
-                                   (int64_t)num_groups * n, (hipStream_t)stream, false, flags, hold);
+                                   (int64_t)num_groups * b_rows, (hipStream_t)stream, false, flags, hold);
 }
 
 extern "C" int mxl_grouped_gemm_nt_ex(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes,
@@ -1707,6 +1711,7 @@ static int grouped_gemm_wgrad(const void* a_codes, const void* a_scales, int a_f
     a.total_m = total_m;
     a.m = n;  // rows of the output per group
     a.n = k;  // columns of the output
+    a.b_rows = k;
     a.k = mxl_padded_width(total_m, G);
     a.alpha_a = alpha_a;
     a.alpha_b = alpha_b;
@@ -1718,9 +1723,9 @@ static int grouped_gemm_wgrad(const void* a_codes, const void* a_scales, int a_f
 namespace mxl {
 int gemm_nt_held(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes, const void* b_scales, int b_fmt, void* c,
                  const int64_t* group_lens, int num_groups, int64_t total_m, int64_t n, int64_t k, const float* alpha_a,
-                 const float* alpha_b, uint32_t flags, HeldGemm* hold, void* stream) {
+                 const float* alpha_b, uint32_t flags, HeldGemm* hold, void* stream, int64_t b_rows) {
     return grouped_gemm_nt(a_codes, a_scales, a_fmt, b_codes, b_scales, b_fmt, c, group_lens, num_groups, total_m, n, k, alpha_a, alpha_b, flags,
-                           stream, hold);
+                           stream, hold, b_rows);
 }
 int gemm_wgrad_held(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes, const void* b_scales, int b_fmt, void* c,
                     const int64_t* group_lens, int num_groups, int64_t total_m, int64_t n, int64_t k, const float* alpha_a,

@@ -24,7 +24,8 @@ struct GemmArgs {
     int num_groups;     // >= 1
     int64_t total_m;    // FWD: rows of a; WGRAD: tokens (sum of lens)
     int64_t m;          // WGRAD: rows of a (fixed)   | FWD: unused
-    int64_t n;          // columns of c / rows of b (per group in FWD)
+    int64_t n;          // columns of c / rows of b
+    int64_t b_rows;     // FWD: rows from one group's matrix in b to the next (n, or more where the matrices are padded)
     int64_t k;          // FWD: contraction length; WGRAD: padded width W
     const float* alpha_a;   // ALPHA kernels: the output is multiplied by *alpha_a * *alpha_b (per-tensor
     const float* alpha_b;   // scales of tensor-wise quantised operands) before it is rounded

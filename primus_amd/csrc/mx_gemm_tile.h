@@ -34,10 +34,11 @@ bool gemm_pair_takes(const HeldGemm& h);
 int gemm_pair(const HeldGemm& h, const GemmArgs& wgrad, hipStream_t st);
 
 // mxl_grouped_gemm_nt_ex / _scaled and mxl_grouped_gemm_wgrad_ex / _scaled (alpha null or given), with the former put off
-// into `hold` if it runs on small tiles, and the latter launched with what is held
+// into `hold` if it runs on small tiles, and the latter launched with what is held.  b_rows: rows from one group's matrix in b
+// to the next (0: n)
 int gemm_nt_held(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes, const void* b_scales, int b_fmt, void* c,
                  const int64_t* group_lens, int num_groups, int64_t total_m, int64_t n, int64_t k, const float* alpha_a,
-                 const float* alpha_b, uint32_t flags, HeldGemm* hold, void* stream);
+                 const float* alpha_b, uint32_t flags, HeldGemm* hold, void* stream, int64_t b_rows = 0);
 int gemm_wgrad_held(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes, const void* b_scales, int b_fmt, void* c,
                     const int64_t* group_lens, int num_groups, int64_t total_m, int64_t n, int64_t k, const float* alpha_a,
                     const float* alpha_b, uint32_t flags, HeldGemm* hold, void* stream);

@@ -175,9 +175,9 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, uint32_t block
     if (nst > 0) {
         // ---- descriptors and per-lane offsets (addr:: as the ring kernel) ----
         const int64_t a_rows_total = MODE == MODE_FWD ? p.total_m : p.m;
-        const int64_t b_rows_total = MODE == MODE_FWD ? (int64_t)G * p.n : p.n;
+        const int64_t b_rows_total = MODE == MODE_FWD ? (int64_t)G * p.b_rows : p.n;
         const int64_t bt_rows = (int64_t)G * p.k;
-        const int64_t b_row0 = (MODE == MODE_FWD ? (int64_t)grp * p.n : 0) + n0;
+        const int64_t b_row0 = (MODE == MODE_FWD ? (int64_t)grp * p.b_rows : 0) + n0;
         const addr::Desc da = addr::ring_code_desc(a_rows_total, p.k / KS, a_row0, BK);
         const addr::Desc db = BT ? addr::ring_bt_desc(bt_rows, (p.n + 127) / 128 * (F44 ? 1 : 2), (int64_t)grp * p.k, (int64_t)pid_n * (F44 ? TN / 128 : TN / 64))
                                  : addr::ring_code_desc(b_rows_total, p.k / KS, b_row0, B_ROW);

@@ -53,7 +53,14 @@ struct Linear {
     }
     Copy x_row(Arena& a) const { return rows_copy(a, p.rows, k_ld, p.act_fmt); }
     Copy cols_copy(Arena& a, int64_t cols, int64_t fmt) const { return rows_copy(a, cols, width, fmt, p.groups > 0 ? p.groups + 1 : 0); }
-    Copy w_row(Arena& a) const { return rows_copy(a, batch * p.n, k_ld, p.w_fmt); }
+    // Rows per matrix of the weight's row-wise copy: where the backward reads it transposed, its rows are a contraction and each
+    // matrix is filled up with zeros to whole K steps, which the forward steps over (a neighbouring expert's rows in their
+    // place would meet zero codes of dy, but NaN among them would stay NaN).  With a transposed copy of the codes instead, for
+    // widths that are no multiples of 128, the quantiser writes a byte more per element; a pass before and now, us: 32 experts of
+    // [4544, 1152] and [1152, 2272], 284 rows, 480 -> 422; of [2176, 6816] and [6816, 1088], 8460 rows, 1871 -> 1733; E2M1, of
+    // [4736, 2624] and [2624, 2368], 200 rows, 829 -> 770; dense, [1999, 2880] x 5760, 151 -> 143, E2M1 [2736, 8064] x 13408, 592 -> 578.
+    int64_t w_rows() const { return p.need_dx && p.dx_from_rows ? n_ld : p.n; }
+    Copy w_row(Arena& a) const { return rows_copy(a, batch * w_rows(), k_ld, p.w_fmt); }
     Copy w_col(Arena& a) const {
         Copy c;
         if (!p.dx_from_rows) c.q = a.take(batch * p.k * n_ld / (p.w_fmt == MXL_FMT_E2M1 ? 2 : 1));
@@ -152,7 +159,7 @@ bool valid(const mxl_linear* p) {
     if (p->recipe != MXL_LINEAR_MX && p->recipe != MXL_LINEAR_TENSORWISE) return false;
     if (p->recipe == MXL_LINEAR_TENSORWISE && (p->input != MXL_LINEAR_PLAIN || p->w_quantized)) return false;
     if (p->input < MXL_LINEAR_PLAIN || p->input > MXL_LINEAR_RMSNORM) return false;
-    return !(p->dx_from_rows && (p->n % 128 || p->k % 128 || p->w_quantized));
+    return !(p->dx_from_rows && p->w_quantized);
 }
 
 }  // namespace
@@ -242,22 +249,25 @@ extern "C" int mxl_linear_forward(const mxl_linear* p, const void* x, const void
     const bool rht = p->rht_signs >= 0 && p->need_dw && p->input == MXL_LINEAR_PLAIN && !l.tensorwise();
     // (a tensor-wise scaled row-wise copy by itself knows no groups, nor do the copies of an input that an RMSNorm forms)
     const bool ungrouped = (l.tensorwise() && !p->need_dw) || p->input == MXL_LINEAR_RMSNORM;
-    const mxl::LinearOperands both = {x, w, p->rows, l.batch, p->n, p->k, l.k_ld, l.n_ld, ungrouped ? nullptr : lens, ungrouped ? 0 : G,
+    const mxl::LinearOperands both = {x, w, p->rows, l.batch, p->n, p->k, l.k_ld, l.n_ld, l.w_rows(), ungrouped ? nullptr : lens, ungrouped ? 0 : G,
                                       af, wf, (int)p->scale_mode, l.qf() | (rht ? MXL_QF_RHT_COL : 0u), rht ? (uint32_t)p->rht_signs : 0u,
                                       f.x_amax, f.w_amax, sv.x_si, sv.w_si,
                                       p->input == MXL_LINEAR_RMSNORM ? aux0 : nullptr, sv.rstd,
                                       f.x_row.q, f.x_row.s, sv.x_col.q, sv.x_col.s, wr.q, wr.s, sv.w_col.q, sv.w_col.s};
+    auto product = [&](const Copy& wc, const float* alpha_a, const float* alpha_b) {
+        return mxl::gemm_nt_held(f.x_row.q, f.x_row.s, af, wc.q, wc.s, wf, y, lens, batch, p->rows, p->n, l.k_ld, alpha_a, alpha_b, MXL_GF_KSTEP, nullptr,
+                                 stream, l.w_rows());
+    };
     if (l.tensorwise()) {
         MXL_TRY(mxl::amax_pair(x, p->rows * p->k, f.x_amax, w, l.batch * p->n * p->k, f.w_amax, true, stream));
         MXL_TRY(mxl::quantize_pair(both, stream));
-        return mxl_grouped_gemm_nt_scaled(f.x_row.q, f.x_row.s, af, wr.q, wr.s, wf, y, lens, batch, p->rows, p->n, l.k_ld, sv.x_si, sv.w_si,
-                                          MXL_GF_KSTEP, stream);
+        return product(wr, sv.x_si, sv.w_si);
     }
     if (p->input == MXL_LINEAR_RMSNORM) {
         MXL_TRY(mxl_rmsnorm_fwd(x, aux0, (float)p->eps, p->rows, p->k, nullptr, sv.rstd, stream));
         if (!p->w_quantized && G == 0 && aux0) {
             MXL_TRY(mxl::quantize_pair(both, stream));
-            return mxl_grouped_gemm_nt_ex(f.x_row.q, f.x_row.s, af, wr.q, wr.s, wf, y, lens, batch, p->rows, p->n, l.k_ld, MXL_GF_KSTEP, stream);
+            return product(wr, nullptr, nullptr);
         }
         MXL_TRY(mxl_rmsnorm_quantize(x, aux0, sv.rstd, p->rows, p->k, l.k_ld, af, (int)p->scale_mode, nullptr, 0, f.x_row.q, f.x_row.s,
                                      sv.x_col.q, sv.x_col.s, l.qf(), stream));
@@ -267,7 +277,7 @@ extern "C" int mxl_linear_forward(const mxl_linear* p, const void* x, const void
                                        f.x_row.s, sv.x_col.q, sv.x_col.s, l.qf(), stream));
     } else if (!p->w_quantized) {
         MXL_TRY(mxl::quantize_pair(both, stream));
-        return mxl_grouped_gemm_nt_ex(f.x_row.q, f.x_row.s, af, wr.q, wr.s, wf, y, lens, batch, p->rows, p->n, l.k_ld, MXL_GF_KSTEP, stream);
+        return product(wr, nullptr, nullptr);
     } else {
         MXL_TRY(mxl_quantize_ex(x, p->rows, p->k, l.k_ld, af, (int)p->scale_mode, lens, G, f.x_row.q, f.x_row.s, sv.x_col.q, sv.x_col.s, both.flags, 0,
                                 both.rht_signs, stream));
@@ -276,9 +286,9 @@ extern "C" int mxl_linear_forward(const mxl_linear* p, const void* x, const void
         if (!w_scales) return MXL_EINVAL;
         return mxl_grouped_gemm_nt_ex(f.x_row.q, f.x_row.s, af, w, w_scales, wf, y, lens, batch, p->rows, p->n, l.k_ld, MXL_GF_KSTEP, stream);
     }
-    MXL_TRY(mxl_quantize_weight_2d_ex(w, l.batch, p->n, p->k, l.k_ld, l.n_ld, wf, (int)p->scale_mode, wr.q, wr.s, sv.w_col.q, sv.w_col.s, l.qf(),
-                                      stream));
-    return mxl_grouped_gemm_nt_ex(f.x_row.q, f.x_row.s, af, wr.q, wr.s, wf, y, lens, batch, p->rows, p->n, l.k_ld, MXL_GF_KSTEP, stream);
+    MXL_TRY(mxl::quantize_weight_rows(w, l.batch, p->n, p->k, l.k_ld, l.n_ld, l.w_rows(), wf, (int)p->scale_mode, wr.q, wr.s, sv.w_col.q, sv.w_col.s,
+                                      l.qf(), stream));
+    return product(wr, nullptr, nullptr);
 }
 
 extern "C" int mxl_linear_backward(const mxl_linear* p, int parts, const void* dy, const void* x, const void* aux0, const void* aux1,

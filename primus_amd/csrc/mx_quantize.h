@@ -17,6 +17,7 @@ struct LinearOperands {
     // activations [rows, k] (ragged groups: group_lens, num_groups; 0 and null: one), weights [batch, n, k]
     const void *x, *w;
     int64_t rows, batch, n, k, k_ld, n_ld;
+    int64_t w_rows;                     // rows per matrix of the weight's row-wise copy: n, or n_ld with zeros behind the n
     const int64_t* group_lens;
     int num_groups;
     int x_fmt, w_fmt, scale_mode;
@@ -31,5 +32,8 @@ struct LinearOperands {
 };
 // in one launch where there is a kernel for the two, else one after the other; the same bytes
 int quantize_pair(const LinearOperands& o, void* stream);
+// mxl_quantize_weight_2d_ex with `rows` rows per matrix in the row-wise copy
+int quantize_weight_rows(const void* w, int64_t batch, int64_t n, int64_t k, int64_t k_ld, int64_t n_ld, int64_t rows, int fmt, int scale_mode,
+                         void* q_row, void* s_row, void* q_colT, void* s_colT, uint32_t flags, void* stream);
 
 }  // namespace mxl

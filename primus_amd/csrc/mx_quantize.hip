@@ -35,6 +35,7 @@ struct QuantArgs {
     int64_t row_ld;     // columns of the row-wise copy (>= cols; the excess is zero-filled padding)
     int64_t W;          // padded width of the transposed copy (elements)
     int64_t mat_rows;   // TWOD: rows per matrix (n); otherwise unused
+    int64_t out_rows;   // TWOD: rows per matrix in the row-wise copy, n or n rounded up to whole tiles (the excess is written as zeros)
     // fused gated activation in front (ACT >= 0): x is fc1's output [rows, 2 * cols], the tensor that is
     // quantised is act(x[:, :cols]) * x[:, cols:] * probs[row], masked rows are zero
     const void* probs;
@@ -152,6 +153,8 @@ __device__ __forceinline__ void quant_workgroup(const QuantArgs& a, int block) {
     int64_t src_row0 = 0;
     int rows_valid = 0;
     int64_t batch_off_rows = 0;  // TWOD: first row of this matrix in the flattened input
+    int64_t out_row0;            // the tile's first row in the row-wise copy, and how many of its rows that has
+    int rows_out;
     // K-step-major scales of a grouped transposed copy: the 16-byte scale panels restart at every group
     int64_t seg_pan0 = 0;        // panels of the groups in front of this tile's group
     int seg_tile = -1;           // this tile's number inside its group's padded segment (-1: not grouped)
@@ -163,6 +166,9 @@ __device__ __forceinline__ void quant_workgroup(const QuantArgs& a, int block) {
         src_row0 = batch_off_rows + (int64_t)rt * QT;
         int64_t rem = a.mat_rows - (int64_t)rt * QT;
         rows_valid = rem < QT ? (int)rem : QT;
+        rem = a.out_rows - (int64_t)rt * QT;
+        rows_out = rem < QT ? (int)rem : QT;
+        out_row0 = (int64_t)mat * a.out_rows + (int64_t)rt * QT;
     } else if (!COL || a.group_lens == nullptr) {
         src_row0 = (int64_t)pt * QT;
         int64_t rem = a.rows - src_row0;
@@ -192,6 +198,8 @@ __device__ __forceinline__ void quant_workgroup(const QuantArgs& a, int block) {
             seg_tile = pt - pto;
         }
     }
+
+    if (!TWOD) out_row0 = src_row0, rows_out = rows_valid;
 
     // fused activation: the tile's 128 probabilities (and row-mask bits) are fetched once by 128 lanes and
     // handed round through LDS; fetched per lane and row they would double the number of load instructions
@@ -342,10 +350,10 @@ __device__ __forceinline__ void quant_workgroup(const QuantArgs& a, int block) {
                     const uint4 out = odd ? make_uint4(recv.x, recv.y, o.x, o.y) : make_uint4(o_even.x, o_even.y, recv.x, recv.y);
                     const int rr = odd ? r : r - 1;
                     const int cc = c16 & ~1;          // the pair's first 8-column piece
-                    if (out_ok && rr < rows_valid) {
-                        const int64_t at = a.kchunk == 2 ? ((int64_t)(2 * ct + (cc >> 3)) * a.chunk_rows_row + src_row0 + rr) * (QT / 2) + 8 * (cc & 7)
-                                         : a.kchunk  ? ((int64_t)ct * a.chunk_rows_row + src_row0 + rr) * QT + 8 * cc
-                                                     : (src_row0 + rr) * a.row_ld + col0 + 8 * cc;
+                    if (out_ok && rr < rows_out) {
+                        const int64_t at = a.kchunk == 2 ? ((int64_t)(2 * ct + (cc >> 3)) * a.chunk_rows_row + out_row0 + rr) * (QT / 2) + 8 * (cc & 7)
+                                         : a.kchunk  ? ((int64_t)ct * a.chunk_rows_row + out_row0 + rr) * QT + 8 * cc
+                                                     : (out_row0 + rr) * a.row_ld + col0 + 8 * cc;
                         store16_streaming(a.q_row + at, out);
                     }
                 }
@@ -363,11 +371,11 @@ __device__ __forceinline__ void quant_workgroup(const QuantArgs& a, int block) {
                     o = nonfinite2_e2m1(d[it].x) | (nonfinite2_e2m1(d[it].y) << 8) | (nonfinite2_e2m1(d[it].z) << 16) |
                         (nonfinite2_e2m1(d[it].w) << 24);
                 }
-                if (out_ok && r < rows_valid) {
+                if (out_ok && r < rows_out) {
                     // element offsets; K-step-major: 64 elements (32 bytes) of a row per K step
-                    const int64_t at = a.kchunk == 2 ? ((int64_t)(2 * ct + (c16 >> 3)) * a.chunk_rows_row + src_row0 + r) * (QT / 2) + 8 * (c16 & 7)
-                                     : a.kchunk ? ((int64_t)ct * a.chunk_rows_row + src_row0 + r) * QT + 8 * c16
-                                                : (src_row0 + r) * a.row_ld + col;
+                    const int64_t at = a.kchunk == 2 ? ((int64_t)(2 * ct + (c16 >> 3)) * a.chunk_rows_row + out_row0 + r) * (QT / 2) + 8 * (c16 & 7)
+                                     : a.kchunk ? ((int64_t)ct * a.chunk_rows_row + out_row0 + r) * QT + 8 * c16
+                                                : (out_row0 + r) * a.row_ld + col;
                     store4_streaming(a.q_row + at / 2, o);
                 }
             }
@@ -476,13 +484,13 @@ __device__ __forceinline__ void quant_workgroup(const QuantArgs& a, int block) {
     __syncthreads();
 
     // ---- scales: one dword (4 blocks) per row / per column of the tile ----
-    if (ROW && t < QT && t < rows_valid) {
+    if (ROW && t < QT && t < rows_out) {
         const int64_t sld = a.row_ld / 32;
         const int64_t nb = (a.row_ld - col0) / 32;  // valid blocks in this tile row
-        uint8_t* dst = a.s_row + (src_row0 + t) * sld + col0 / 32;
+        uint8_t* dst = a.s_row + (out_row0 + t) * sld + col0 / 32;
         const uint32_t v = srow_tile[t];
         if (a.kchunk >= 2) {
-            store_panel_scales(a.s_row + ((int64_t)(ct >> 2) * a.chunk_rows_row + src_row0 + t) * 16, ct & 3, v);
+            store_panel_scales(a.s_row + ((int64_t)(ct >> 2) * a.chunk_rows_row + out_row0 + t) * 16, ct & 3, v);
         } else if (nb >= 4 && (sld & 3) == 0) {
             *(uint32_t*)dst = v;
         } else {
@@ -844,6 +852,7 @@ static int quantize_1d(const void* x_bf16, int64_t rows, int64_t cols, int64_t r
     a.row_ld = row_ld;
     a.W = mxl_padded_width(rows, num_groups);
     a.mat_rows = 0;
+    a.out_rows = 0;
     a.probs = probs;
     a.probs_bf16 = probs_dtype == MXL_PROBS_BF16;
     a.row_mask = row_mask;
@@ -923,9 +932,11 @@ extern "C" int mxl_rmsnorm_quantize(const void* x_bf16, const void* w_bf16, cons
 static int quantize_weight_2d(const void* w_bf16, int64_t batch, int64_t n, int64_t k, int64_t k_ld, int64_t n_ld, int fmt,
                               int scale_mode, void* q_row, void* s_row, void* q_colT, void* s_colT, int kchunk,
                               void* stream, const void* tensor_amax = nullptr, void* scale_inv_out = nullptr,
-                              const HeldQuant* pair = nullptr, bool* paired = nullptr, int parts = 1) {
+                              const HeldQuant* pair = nullptr, bool* paired = nullptr, int parts = 1, int64_t out_rows = 0) {
     if (k_ld == 0) k_ld = k;
     if (n_ld == 0) n_ld = n;
+    if (out_rows == 0) out_rows = n;
+    if (out_rows < n || out_rows > (n + QT - 1) / QT * QT) return MXL_EINVAL;   // the excess stays inside the last tile
     if (kchunk < 0 || (kchunk == 3 && fmt != MXL_FMT_E2M1)) return MXL_EINVAL;
     if (kchunk && ((q_row && k_ld % QT != 0) || (q_colT && n_ld % QT != 0))) return MXL_EINVAL;   // whole chunks
     if (k_ld < k || n_ld < n || k_ld % MXL_BLOCK != 0 || n_ld % MXL_BLOCK != 0) return MXL_EINVAL;
@@ -948,6 +959,7 @@ static int quantize_weight_2d(const void* w_bf16, int64_t batch, int64_t n, int6
     a.row_ld = k_ld;
     a.W = n_ld;  // transposed copy of each matrix is [k, n_ld]
     a.mat_rows = n;
+    a.out_rows = out_rows;
     a.probs = nullptr;
     a.probs_bf16 = 0;
     a.row_mask = nullptr;
@@ -958,7 +970,7 @@ static int quantize_weight_2d(const void* w_bf16, int64_t batch, int64_t n, int6
     a.sr_seed = 0;
     a.rht_signs = 0;
     a.kchunk = kchunk;
-    a.chunk_rows_row = batch * n;   // the batch is one operand of batch * n rows (resp. batch * k for the transposed copy)
+    a.chunk_rows_row = batch * out_rows;   // the batch is one operand of that many rows (batch * k for the transposed copy)
     a.chunk_rows_col = batch * k;
     const int64_t gx = batch * ((n + QT - 1) / QT);
     const int64_t gy = ((q_row ? k_ld : k) + QT - 1) / QT;
@@ -981,7 +993,7 @@ int quantize_pair(const LinearOperands& o, void* stream) {
     };
     auto w = [&](const HeldQuant* pair, bool* paired) {
         return quantize_weight_2d(o.w, o.batch, o.n, o.k, o.k_ld, o.n_ld, o.w_fmt, o.scale_mode, o.wq_row, o.ws_row, o.wq_col, o.ws_col, lay,
-                                  stream, o.w_amax, o.w_scale_inv, pair, paired, o.w_amax ? amax_parts(o.batch * o.n * o.k) : 1);
+                                  stream, o.w_amax, o.w_scale_inv, pair, paired, o.w_amax ? amax_parts(o.batch * o.n * o.k) : 1, o.w_rows);
     };
     HeldQuant hold;
     bool paired = false;
@@ -993,6 +1005,11 @@ int quantize_pair(const LinearOperands& o, void* stream) {
     }
     if (const int rc = x(nullptr)) return rc;
     return w(nullptr, nullptr);
+}
+int quantize_weight_rows(const void* w, int64_t batch, int64_t n, int64_t k, int64_t k_ld, int64_t n_ld, int64_t rows, int fmt, int scale_mode,
+                         void* q_row, void* s_row, void* q_colT, void* s_colT, uint32_t flags, void* stream) {
+    return quantize_weight_2d(w, batch, n, k, k_ld, n_ld, fmt, scale_mode, q_row, s_row, q_colT, s_colT, qf_layout(flags), stream, nullptr, nullptr,
+                              nullptr, nullptr, 1, rows);
 }
 }  // namespace mxl
 

@@ -224,7 +224,7 @@ def _mx_forward(ctx, a, b, w_shape, b_t, group_lens, act_fmt, w_fmt, scale_mode,
             wt, wt_scales = _cached_codes(b_t, kc), _cached_scales(b_t, kc)
     n, k = w_shape[-2], w_shape[-1]
     # dgrad on the row-wise weight codes: see the launch-by-launch route below
-    bt = (need_dgrad and not cached and _dgrad_reads_rowwise and act_fmt == w_fmt and n % K.GEMM_K_ALIGN == 0 and k % K.GEMM_K_ALIGN == 0)
+    bt = need_dgrad and not cached and _dgrad_reads_rowwise and act_fmt == w_fmt
     inp, pd, aux0, aux1 = _lib.LINEAR_PLAIN, 0, None, None
     if activation is not None:
         act, pd, row_mask = K._glu_args(a, probs, row_mask, activation)
@@ -517,7 +517,7 @@ class _TWLinearFunction(torch.autograd.Function):
             kc = K.pick_layout(groups, b.shape[-2], b.shape[-1], a.shape[0], fp8=True)
         if kc == K.LAYOUT_KSTEP and a.shape[0] > 0 and not isinstance(b, QuantizedTensor) and _two_calls(a, b, b.shape[-2], b.shape[-1], group_lens):
             n, k = b.shape[-2], b.shape[-1]
-            bt = need_dgrad and _dgrad_reads_rowwise and fwd_fmt == _lib.FMT_E4M3 and n % K.GEMM_K_ALIGN == 0 and k % K.GEMM_K_ALIGN == 0
+            bt = need_dgrad and _dgrad_reads_rowwise and fwd_fmt == _lib.FMT_E4M3
             plan = K.linear_plan(a.shape[0], n, k, groups if grouped else 0, _lib.LINEAR_TENSORWISE, fwd_fmt, fwd_fmt, bwd_fmt, 0,
                                  need_dgrad, need_wgrad, bt)
             y, saved = K.linear_forward_impl(plan, a, b, None, group_lens)
