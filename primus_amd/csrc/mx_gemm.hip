@@ -115,31 +115,16 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_kernel(GemmArgs p) {
     const uint32_t smem_base = (uint32_t)(uintptr_t)smem;  // LDS byte address of the ring
 
     // ---- per-workgroup group tables (device-side, no host sync) ----
-    // The lens are fetched by all threads at once and summed by one.  They are clamped to what the
-    // operands hold (no negative length; the running sum never passes total_m, resp. the padded width),
-    // so that lens which do not match the buffers cannot send a tile outside them.
-    for (int i = t; i < G; i += GTHREADS) pre_rows[i + 1] = p.group_lens ? p.group_lens[i] : p.total_m;
-    __syncthreads();
-    if (t == 0) {
-        int tiles = 0;
-        int64_t rows = 0;
-        const int64_t cap = (MODE == MODE_FWD) ? p.total_m : p.k;
-        pre_tiles[0] = 0;
-        pre_rows[0] = 0;
-        for (int i = 0; i < G; ++i) {
-            int64_t len = pre_rows[i + 1];
-            len = len < 0 ? 0 : len;
-            if (MODE == MODE_FWD) {
-                len = len > cap - rows ? cap - rows : len;
-                tiles += (int)((len + BM - 1) / BM);
-                rows += len;
-            } else {
-                int64_t seg = (len + MXL_SEG_ALIGN - 1) / MXL_SEG_ALIGN * MXL_SEG_ALIGN;
-                seg = seg > cap - rows ? cap - rows : seg;
-                rows += seg;
-            }
-            pre_tiles[i + 1] = tiles;
-            pre_rows[i + 1] = rows;
+    if (w == 0) {
+        GroupScan<MODE == MODE_FWD ? 1 : MXL_SEG_ALIGN> scan(MODE == MODE_FWD ? p.total_m : p.k, G, l);
+        uint32_t tiles = 0;
+        if (l == 0) pre_tiles[0] = 0, pre_rows[0] = 0;
+        for (int c = 0; c < G; c += 64) {
+            uint32_t first, end;
+            scan.step(p.group_lens, c, first, end);
+            const uint32_t te = wave_prefix((end - first + BM - 1) / BM) + tiles;
+            if (c + l < G) pre_tiles[c + l + 1] = MODE == MODE_FWD ? (int)te : 0, pre_rows[c + l + 1] = end;
+            tiles = (uint32_t)__builtin_amdgcn_readlane((int)te, 63);
         }
     }
     __syncthreads();
@@ -646,31 +631,16 @@ __global__ __launch_bounds__(GTHREADS) void mx_gemm_ring_kernel(GemmArgs p) {
     const uint32_t smem_base = (uint32_t)(uintptr_t)smem;
 
     // ---- per-workgroup group tables (as in mx_gemm_kernel, plus the scale-panel prefix) ----
-    for (int i = t; i < G; i += GTHREADS) pre_rows[i + 1] = p.group_lens ? p.group_lens[i] : p.total_m;
-    __syncthreads();
-    if (t == 0) {
-        int tiles = 0, pans = 0;
-        int64_t rows = 0;
-        const int64_t cap = (MODE == MODE_FWD) ? p.total_m : p.k;
-        pre_tiles[0] = 0;
-        pre_rows[0] = 0;
-        pre_pan[0] = 0;
-        for (int i = 0; i < G; ++i) {
-            int64_t len = pre_rows[i + 1];
-            len = len < 0 ? 0 : len;
-            if (MODE == MODE_FWD) {
-                len = len > cap - rows ? cap - rows : len;
-                tiles += (int)((len + BM - 1) / BM);
-                rows += len;
-            } else {
-                int64_t seg = (len + MXL_SEG_ALIGN - 1) / MXL_SEG_ALIGN * MXL_SEG_ALIGN;
-                seg = seg > cap - rows ? cap - rows : seg;
-                rows += seg;
-                pans += (int)((seg + 511) / 512);
-            }
-            pre_tiles[i + 1] = tiles;
-            pre_rows[i + 1] = rows;
-            pre_pan[i + 1] = pans;
+    if (w == 0) {
+        GroupScan<MODE == MODE_FWD ? 1 : MXL_SEG_ALIGN> scan(MODE == MODE_FWD ? p.total_m : p.k, G, l);
+        uint32_t tiles = 0;                  // row tiles (forward) or scale panels (weight gradient) so far
+        if (l == 0) pre_tiles[0] = 0, pre_rows[0] = 0, pre_pan[0] = 0;
+        for (int c = 0; c < G; c += 64) {
+            uint32_t first, end;
+            scan.step(p.group_lens, c, first, end);
+            const uint32_t te = wave_prefix(MODE == MODE_FWD ? (end - first + BM - 1) / BM : (end - first + 511) / 512) + tiles;
+            if (c + l < G) (MODE == MODE_FWD ? pre_tiles : pre_pan)[c + l + 1] = (int)te, pre_rows[c + l + 1] = end;
+            tiles = (uint32_t)__builtin_amdgcn_readlane((int)te, 63);
         }
     }
     __syncthreads();

@@ -97,23 +97,17 @@ __device__ __forceinline__ void bf_wait_vm() {
 
 // prefix sums over the groups of their rows and of their row tiles; lens clamped to what the buffers hold
 template <int BM>
-__device__ __forceinline__ void bf16_group_table(const Bf16Args& p, int64_t* pre_rows, int* pre_tiles, int t, int threads) {
-    const int G = p.num_groups;
-    for (int i = t; i < G; i += threads) pre_rows[i + 1] = p.group_lens ? p.group_lens[i] : p.total_m;
-    __syncthreads();
-    if (t == 0) {
-        int tiles = 0;
-        int64_t rows = 0;
-        pre_tiles[0] = 0;
-        pre_rows[0] = 0;
-        for (int i = 0; i < G; ++i) {
-            int64_t len = pre_rows[i + 1];
-            len = len < 0 ? 0 : len;
-            len = len > p.total_m - rows ? p.total_m - rows : len;
-            tiles += (int)((len + BM - 1) / BM);
-            rows += len;
-            pre_tiles[i + 1] = tiles;
-            pre_rows[i + 1] = rows;
+__device__ __forceinline__ void bf16_group_table(const Bf16Args& p, int64_t* pre_rows, int* pre_tiles, int t) {
+    if (t < 64) {
+        GroupScan<> scan(p.total_m, p.num_groups, t);
+        uint32_t tiles = 0;
+        if (t == 0) pre_tiles[0] = 0, pre_rows[0] = 0;
+        for (int c = 0; c < p.num_groups; c += 64) {
+            uint32_t first, end;
+            scan.step(p.group_lens, c, first, end);
+            const uint32_t te = wave_prefix((end - first + BM - 1) / BM) + tiles;
+            if (c + t < p.num_groups) pre_tiles[c + t + 1] = (int)te, pre_rows[c + t + 1] = end;
+            tiles = (uint32_t)__builtin_amdgcn_readlane((int)te, 63);
         }
     }
     __syncthreads();
@@ -153,7 +147,7 @@ __global__ __launch_bounds__(BF_THREADS, 2) void bf16_gemm_kernel(Bf16Args p) {
     const int G = p.num_groups;
     const uint32_t smem_base = (uint32_t)(uintptr_t)smem;
 
-    bf16_group_table<BF_BM>(p, pre_rows, pre_tiles, t, BF_THREADS);
+    bf16_group_table<BF_BM>(p, pre_rows, pre_tiles, t);
 
     const int tiles_n = (int)((p.n + BF_BN - 1) / BF_BN);
     const int tiles_m = WGRAD ? (int)((p.m + BF_BM - 1) / BF_BM) : pre_tiles[G];
@@ -433,7 +427,7 @@ __global__ __launch_bounds__(TL_THREADS, 2) void bf16_gemm_tall_kernel(Bf16Args 
     const int wm = w >> 2, wn = w & 3;      // the two waves of a SIMD hold different rows: a tile of <= 128 rows keeps one busy on each
     const int G = p.num_groups;
     const uint32_t smem_base = (uint32_t)(uintptr_t)smem;
-    bf16_group_table<256>(p, pre_rows, pre_tiles, t, TL_THREADS);
+    bf16_group_table<256>(p, pre_rows, pre_tiles, t);
 
     const int tiles_n = (int)((p.n + BF_BN - 1) / BF_BN);
     const int tiles_m = WGRAD ? (int)((p.m + 255) / 256) : pre_tiles[G];

@@ -23,16 +23,6 @@ namespace mxl {
 
 constexpr int TILE_MAX_GROUPS = 256;      // four per lane in the scan
 
-// inclusive sum over the lanes of a wave, saturating at cap (all values in [0, cap], cap < 2^31)
-__device__ __forceinline__ uint32_t wave_scan_sat(uint32_t v, uint32_t cap, int lane) {
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t o = (uint32_t)__shfl_up((int)v, d);
-        if (lane >= d) v = v + o < cap ? v + o : cap;
-    }
-    return v;
-}
-
 // f(0), f(1), ... f(n - 1) for a run-time n < N, each call inside the previous one's branch (no joins in between)
 template <int I, int N, class F> __device__ __forceinline__ void nested_steps(int n, F&& f) {
     if constexpr (I < N - 1) {
@@ -79,27 +69,18 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p, uint32_t block
     const uint32_t cap = (uint32_t)(MODE == MODE_FWD ? p.total_m : p.k);
     int tiles_m;
     if (p.group_lens) {
-        uint32_t base = 0, tbase = 0;
+        GroupScan<MODE == MODE_FWD ? 1 : MXL_SEG_ALIGN> scan(cap, G, l);
+        uint32_t tbase = 0;
 #pragma unroll
         for (int c = 0; c < TILE_MAX_GROUPS / 64; ++c) {
             cum[c] = tcum[c] = own[c] = town[c] = 0;
             if (c * 64 < G) {
-                const int i = c * 64 + l;
-                int64_t len = i < G ? p.group_lens[i] : 0;
-                len = len < 0 ? 0 : len;
-                uint32_t v = len > (int64_t)cap ? cap : (uint32_t)len;
-                if (MODE == MODE_WGRAD) v = (v + MXL_SEG_ALIGN - 1) / MXL_SEG_ALIGN * MXL_SEG_ALIGN, v = v > cap ? cap : v;
-                uint32_t s = wave_scan_sat(v, cap, l);
-                uint32_t before = s;                    // rows up to this group, clamped to what the operand has
-                s = base + s < cap ? base + s : cap;
-                before = (uint32_t)__shfl_up((int)s, 1);
-                before = l ? before : base;
-                own[c] = s - before;
-                cum[c] = before;
-                base = (uint32_t)__builtin_amdgcn_readlane((int)s, 63);
+                uint32_t end;
+                scan.step(p.group_lens, c * 64, cum[c], end);
+                own[c] = end - cum[c];
                 // row tiles (forward) or scale panels (weight gradient) of the groups in front of this one
                 town[c] = MODE == MODE_FWD ? (own[c] + TM - 1) / TM : (own[c] + 511) / 512;
-                const uint32_t ts = wave_scan_sat(town[c], 0x7FFFFFFFu, l) + tbase;
+                const uint32_t ts = wave_prefix(town[c]) + tbase;
                 tcum[c] = ts - town[c];
                 tbase = (uint32_t)__builtin_amdgcn_readlane((int)ts, 63);
             }

@@ -174,31 +174,32 @@ __device__ __forceinline__ void quant_workgroup(const QuantArgs& a, int block) {
         int64_t rem = a.rows - src_row0;
         rows_valid = rem <= 0 ? 0 : (rem < QT ? (int)rem : QT);
     } else {
-        int64_t off = 0, ppo = 0;
-        int pto = 0;
-        for (int g = 0; g < a.num_groups; ++g) {
-            // clamped to the rows that exist, so that lens which do not match the buffer cannot read outside it
-            int64_t len = a.group_lens[g];
-            len = len < 0 ? 0 : (len > a.rows - off ? a.rows - off : len);
-            const int nt = (int)((len + QT - 1) / QT);
-            if (pt < pto + nt) {
-                const int64_t r = (int64_t)(pt - pto) * QT;
-                src_row0 = off + r;
-                rows_valid = (len - r) < QT ? (int)(len - r) : QT;
-                seg_pan0 = ppo;
-                seg_tile = pt - pto;
+        // every wave looks the tile's group up for itself
+        GroupScan<> scan(a.rows, a.num_groups, l);
+        uint32_t tiles = 0, pans = 0;
+        for (int c = 0; c < a.num_groups; c += 64) {
+            uint32_t first, end;
+            scan.step(a.group_lens, c, first, end);
+            const uint32_t nt = (end - first + QT - 1) / QT, np = (nt + 3) / 4;
+            const uint32_t te = wave_prefix(nt) + tiles, pe = wave_prefix(np) + pans;
+            const uint64_t hit = __ballot((uint32_t)pt >= te - nt && (uint32_t)pt < te);
+            if (hit) {
+                const int src = __builtin_ctzll(hit);
+                seg_tile = pt - __builtin_amdgcn_readlane((int)(te - nt), src);
+                seg_pan0 = (uint32_t)__builtin_amdgcn_readlane((int)(pe - np), src);
+                const uint32_t len = (uint32_t)__builtin_amdgcn_readlane((int)(end - first), src), r = (uint32_t)seg_tile * QT;
+                src_row0 = (int64_t)(uint32_t)__builtin_amdgcn_readlane((int)first, src) + r;
+                rows_valid = len - r < QT ? (int)(len - r) : QT;
                 break;
             }
-            off += len;
-            pto += nt;
-            ppo += (nt + 3) / 4;
+            tiles = (uint32_t)__builtin_amdgcn_readlane((int)te, 63);
+            pans = (uint32_t)__builtin_amdgcn_readlane((int)pe, 63);
         }
         if (seg_tile < 0) {   // a padding tile behind the last group: its scales go behind the last group's panels
-            seg_pan0 = ppo;
-            seg_tile = pt - pto;
+            seg_pan0 = pans;
+            seg_tile = pt - (int)tiles;
         }
     }
-
     if (!TWOD) out_row0 = src_row0, rows_out = rows_valid;
 
     // fused activation: the tile's 128 probabilities (and row-mask bits) are fetched once by 128 lanes and
