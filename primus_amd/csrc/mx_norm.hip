@@ -73,6 +73,12 @@ __global__ __launch_bounds__(NTHREADS) void rmsnorm_fwd_kernel(const uint16_t* x
 
 // CH: 8-column chunks per lane (k <= CH * 2048).  The weight chunks are loaded once per workgroup and a
 // row's x and dy stay in registers between the reduction and the output pass.
+//
+// Bound by memory, 6 bytes an element.  x and dy are read for the last time here: loaded past the caches, and, where a row is
+// more than one chunk a lane (a workgroup to a CU or two, whose next row would otherwise wait for the present one's output), a
+// row ahead.  us from memory, caches full of other data, ordinary loads / streaming / streaming a row ahead: [8192, 4096] 65 / 38 /
+// 38, [32768, 4096] 202 / 144 / 142 (5.7 TB/s), [4096, 8192] 65 / 37 / 38, [12995, 11328] 215 / 197 / 152, [8192, 16384] 197 / 162 /
+// 138; one chunk a lane, [16384, 1024], 31 / 21 / 24.
 template <int CH>
 __global__ __launch_bounds__(NTHREADS) void rmsnorm_bwd_kernel(const uint16_t* dy, const uint16_t* x, const uint16_t* w,
                                                                const float* rstd, int64_t rows, int64_t k, uint16_t* dx,
@@ -87,20 +93,31 @@ __global__ __launch_bounds__(NTHREADS) void rmsnorm_bwd_kernel(const uint16_t* d
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[j][e] = 0.f;
     }
-    for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
+    uint4 xn[CH], dn[CH];
+    float rn = 0.f;
+    auto request = [&](int64_t row) {
         const uint16_t *xr = x + row * k, *dr = dy + row * k;
-        uint16_t* dxr = dx + row * k;
-        uint4 xv[CH], dv[CH];
 #pragma unroll
         for (int j = 0; j < CH; ++j) {
             const int64_t c = ((int64_t)j * NTHREADS + threadIdx.x) * 8;
-            xv[j] = dv[j] = make_uint4(0, 0, 0, 0);
+            xn[j] = dn[j] = make_uint4(0, 0, 0, 0);
             if (c < k) {
-                xv[j] = norm_load16(xr + c);
-                dv[j] = norm_load16(dr + c);
+                xn[j] = load16_streaming(xr + c);
+                dn[j] = load16_streaming(dr + c);
             }
         }
-        const float r = rstd[row];
+        rn = rstd[row];
+    };
+    constexpr bool AHEAD = CH > 1;
+    if (AHEAD && blockIdx.x < rows) request(blockIdx.x);
+    for (int64_t row = blockIdx.x; row < rows; row += gridDim.x) {
+        uint16_t* dxr = dx + row * k;
+        if (!AHEAD) request(row);
+        uint4 xv[CH], dv[CH];
+#pragma unroll
+        for (int j = 0; j < CH; ++j) xv[j] = xn[j], dv[j] = dn[j];
+        const float r = rn;
+        if (AHEAD && row + gridDim.x < rows) request(row + gridDim.x);
         // sum_j g * xh, and the column sums (chunks past k hold zeros)
         float dot = 0.f;
 #pragma unroll
@@ -147,19 +164,29 @@ __global__ __launch_bounds__(NTHREADS) void rmsnorm_bwd_kernel(const uint16_t* d
 }
 
 // dw[j] = sum over the blocks' partial rows.  A workgroup owns 32 columns: thread (bg, cg) adds rows
-// bg, bg + 32, ... of column group cg (4 columns) in order, then the 32 partial sums are added in order.
+// bg, bg + 32, ... of column group cg (4 columns) in order, then the 32 partial sums are added in order.  A chain of up to
+// 64 loads that wait for one another took 22 us; sixteen at a time: 2048 rows of 1696 columns 21.9 -> 6.9 us, 1024 of 4096 10.8 -> 5.5.
+constexpr int DW_LOADS = 16;     // rows a thread asks for before it adds the first
 __global__ __launch_bounds__(NTHREADS) void rmsnorm_dw_kernel(const float* partial, int blocks, int64_t k, uint16_t* dw) {
     __shared__ float4 part[32][8];
     const int cg = threadIdx.x & 7, bg = threadIdx.x >> 3;
     const int64_t c = (int64_t)blockIdx.x * 32 + 4 * cg;
     float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
     if (c < k) {
-        for (int b = bg; b < blocks; b += 32) {
-            const float4 v = *(const float4*)(partial + (int64_t)b * k + c);
-            s.x += v.x;
-            s.y += v.y;
-            s.z += v.z;
-            s.w += v.w;
+        for (int b0 = bg; b0 < blocks; b0 += 32 * DW_LOADS) {
+            float4 v[DW_LOADS];
+#pragma unroll
+            for (int u = 0; u < DW_LOADS; ++u) {
+                v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (b0 + 32 * u < blocks) v[u] = *(const float4*)(partial + (int64_t)(b0 + 32 * u) * k + c);
+            }
+#pragma unroll
+            for (int u = 0; u < DW_LOADS; ++u) {
+                s.x += v[u].x;
+                s.y += v[u].y;
+                s.z += v[u].z;
+                s.w += v[u].w;
+            }
         }
     }
     part[bg][cg] = s;
