@@ -7,11 +7,19 @@
 //
 // for bf16 x[rows, 2F], computed in fp32 and rounded once to bf16.  Backward returns dx[rows, 2F]
 // and dp[rows] (fp32).  Both kernels stream: one workgroup per row, 16 bytes per lane and access.
+//
+// Bound by memory (6 and 10 bytes per output element), at 6.0-6.4 TB/s where a workgroup gets through its row in one to two
+// passes: with 256 threads a long row is many short visits to each of its pieces of memory while thousands of others are open.
+// Hence 256, 512 or 1024 threads by the row's length.  us, 256 / 512 / 1024 threads: backward [32768, 14336] 882 / 846 / 813,
+// [8192, 14336] 219 / 208 / 194, [8192, 7168] 105 / 98 / 95, [8192, 5760] 83 / 77 / 83, [16384, 3584] 97 / 91 / 117, [65536, 2880]
+// 311 / 306 / 408, [32768, 2048] 106 / 114 / 172; forward 506 / 481 / 461, 127 / 116 / 111, 60 / 56 / 57, 47 / 45 / 47, 55 / 57 / 59,
+// 176 / 175 / 188, 64 / 64 / 64.
+#include "mx_activation.h"
 #include "mx_device.h"
 
 namespace mxl {
 
-constexpr int ATHREADS = 256;
+constexpr int ATHREADS = 256;     // (row_mask_kernel)
 
 typedef uint32_t au32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ uint4 act_load16(const void* s) {
@@ -35,15 +43,15 @@ template <int ACT> __device__ __forceinline__ void act_both(float g, float& a, f
     }
 }
 
-template <int ACT>
-__global__ __launch_bounds__(ATHREADS) void glu_probs_fwd_kernel(const uint16_t* x, const void* probs, int probs_bf16,
+template <int ACT, int THREADS>
+__global__ __launch_bounds__(THREADS) void glu_probs_fwd_kernel(const uint16_t* x, const void* probs, int probs_bf16,
                                                                  const uint8_t* row_mask, int64_t f, uint16_t* y) {
     const int64_t row = blockIdx.x;
     const bool live = row_mask == nullptr || row_mask[row] != 0;
     const float p = live ? load_prob(probs, probs_bf16, row) : 0.f;
     const uint16_t* xg = x + row * 2 * f;
     uint16_t* yr = y + row * f;
-    for (int64_t c = (int64_t)threadIdx.x * 8; c < f; c += ATHREADS * 8) {
+    for (int64_t c = (int64_t)threadIdx.x * 8; c < f; c += THREADS * 8) {
         uint4 o = make_uint4(0, 0, 0, 0);
         if (live) {
             o = glu8<ACT>(act_load16(xg + c), act_load16(xg + f + c), p);
@@ -52,11 +60,11 @@ __global__ __launch_bounds__(ATHREADS) void glu_probs_fwd_kernel(const uint16_t*
     }
 }
 
-template <int ACT>
-__global__ __launch_bounds__(ATHREADS) void glu_probs_bwd_kernel(const uint16_t* dy, const uint16_t* x, const void* probs,
+template <int ACT, int THREADS>
+__global__ __launch_bounds__(THREADS) void glu_probs_bwd_kernel(const uint16_t* dy, const uint16_t* x, const void* probs,
                                                                  int probs_bf16, const uint8_t* row_mask, int64_t f,
                                                                  uint16_t* dx, float* dprobs) {
-    __shared__ float part[ATHREADS / 64];
+    __shared__ float part[THREADS / 64];
     const int64_t row = blockIdx.x;
     const bool live = row_mask == nullptr || row_mask[row] != 0;
     const float p = live ? load_prob(probs, probs_bf16, row) : 0.f;
@@ -64,7 +72,7 @@ __global__ __launch_bounds__(ATHREADS) void glu_probs_bwd_kernel(const uint16_t*
     const uint16_t* dyr = dy + row * f;
     uint16_t* dxr = dx + row * 2 * f;
     float acc = 0.f;
-    for (int64_t c = (int64_t)threadIdx.x * 8; c < f; c += ATHREADS * 8) {
+    for (int64_t c = (int64_t)threadIdx.x * 8; c < f; c += THREADS * 8) {
         uint4 o1 = make_uint4(0, 0, 0, 0), o2 = o1;
         if (live) {
             const uint4 g = act_load16(xg + c), u = act_load16(xg + f + c), d = act_load16(dyr + c);
@@ -95,7 +103,7 @@ __global__ __launch_bounds__(ATHREADS) void glu_probs_bwd_kernel(const uint16_t*
     if (threadIdx.x == 0) {
         float t = 0.f;
 #pragma unroll
-        for (int i = 0; i < ATHREADS / 64; ++i) t += part[i];
+        for (int i = 0; i < THREADS / 64; ++i) t += part[i];
         dprobs[row] = live ? t : 0.f;
     }
 }
@@ -147,38 +155,55 @@ extern "C" int mxl_row_mask(const int64_t* lens, int64_t count, int64_t rows, ui
     return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;
 }
 
+template <int ACT, int THREADS>
+static void launch_glu_fwd(const void* x, const void* probs, int probs_dtype, const uint8_t* row_mask, int64_t rows, int64_t f, void* y, hipStream_t st) {
+    hipLaunchKernelGGL((glu_probs_fwd_kernel<ACT, THREADS>), dim3((unsigned)rows), dim3(THREADS), 0, st, (const uint16_t*)x, probs, probs_dtype, row_mask,
+                       f, (uint16_t*)y);
+}
+template <int ACT, int THREADS>
+static void launch_glu_bwd(const void* dy, const void* x, const void* probs, int probs_dtype, const uint8_t* row_mask, int64_t rows, int64_t f,
+                           void* dx, void* dprobs, hipStream_t st) {
+    hipLaunchKernelGGL((glu_probs_bwd_kernel<ACT, THREADS>), dim3((unsigned)rows), dim3(THREADS), 0, st, (const uint16_t*)dy, (const uint16_t*)x, probs,
+                       probs_dtype, row_mask, f, (uint16_t*)dx, (float*)dprobs);
+}
+constexpr int64_t GLU_LONG_ROW = 6656;                                   // 1024 threads from here on
+constexpr int64_t GLU_FWD_MIDDLE_ROW = 4096, GLU_BWD_MIDDLE_ROW = 2560;  // 512 threads
+
 extern "C" int mxl_glu_probs_fwd(const void* x_bf16, const void* probs, int probs_dtype, const uint8_t* row_mask,
                                  int64_t rows, int64_t f, int act, void* y_bf16, void* stream) {
     if (!act_args_ok(x_bf16, y_bf16, probs, probs_dtype, rows, f, act)) return MXL_EINVAL;
     if (rows == 0) return MXL_OK;
     if (!device_is_gfx950()) return MXL_ENODEV;
-    const dim3 grid((unsigned)rows), block(ATHREADS);
-    hipStream_t st = (hipStream_t)stream;
-    if (act == MXL_ACT_SILU)
-        hipLaunchKernelGGL((glu_probs_fwd_kernel<MXL_ACT_SILU>), grid, block, 0, st, (const uint16_t*)x_bf16, probs,
-                           probs_dtype, row_mask, f, (uint16_t*)y_bf16);
-    else
-        hipLaunchKernelGGL((glu_probs_fwd_kernel<MXL_ACT_GELU>), grid, block, 0, st, (const uint16_t*)x_bf16, probs,
-                           probs_dtype, row_mask, f, (uint16_t*)y_bf16);
+    const bool silu = act == MXL_ACT_SILU;
+    const auto launch = f >= GLU_LONG_ROW         ? (silu ? launch_glu_fwd<MXL_ACT_SILU, 1024> : launch_glu_fwd<MXL_ACT_GELU, 1024>)
+                        : f >= GLU_FWD_MIDDLE_ROW ? (silu ? launch_glu_fwd<MXL_ACT_SILU, 512> : launch_glu_fwd<MXL_ACT_GELU, 512>)
+                                                  : (silu ? launch_glu_fwd<MXL_ACT_SILU, 256> : launch_glu_fwd<MXL_ACT_GELU, 256>);
+    launch(x_bf16, probs, probs_dtype, row_mask, rows, f, y_bf16, (hipStream_t)stream);
     return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;
 }
 
-extern "C" int mxl_glu_probs_bwd(const void* dy_bf16, const void* x_bf16, const void* probs, int probs_dtype,
-                                 const uint8_t* row_mask, int64_t rows, int64_t f, int act, void* dx_bf16,
-                                 void* dprobs_f32, void* stream) {
+namespace mxl {
+// `shared`: another launch that fills the chip runs on another stream.  Its workgroups leave room here and there, which small
+// workgroups use better: a pass of 8 experts [28672, 4096], E2M1, 8192 rows, whose weight gradients run beside it, 3735 us with
+// 256 threads, 3767 with 1024.
+int glu_probs_bwd(const void* dy_bf16, const void* x_bf16, const void* probs, int probs_dtype, const uint8_t* row_mask, int64_t rows, int64_t f, int act,
+                  void* dx_bf16, void* dprobs_f32, bool shared, void* stream) {
     if (!act_args_ok(x_bf16, dx_bf16, probs, probs_dtype, rows, f, act)) return MXL_EINVAL;
     if (rows == 0) return MXL_OK;
     if (!dy_bf16 || !dprobs_f32) return MXL_EINVAL;
     if (!device_is_gfx950()) return MXL_ENODEV;
-    const dim3 grid((unsigned)rows), block(ATHREADS);
-    hipStream_t st = (hipStream_t)stream;
-    if (act == MXL_ACT_SILU)
-        hipLaunchKernelGGL((glu_probs_bwd_kernel<MXL_ACT_SILU>), grid, block, 0, st, (const uint16_t*)dy_bf16,
-                           (const uint16_t*)x_bf16, probs, probs_dtype, row_mask, f, (uint16_t*)dx_bf16,
-                           (float*)dprobs_f32);
-    else
-        hipLaunchKernelGGL((glu_probs_bwd_kernel<MXL_ACT_GELU>), grid, block, 0, st, (const uint16_t*)dy_bf16,
-                           (const uint16_t*)x_bf16, probs, probs_dtype, row_mask, f, (uint16_t*)dx_bf16,
-                           (float*)dprobs_f32);
+    const bool silu = act == MXL_ACT_SILU;
+    const auto launch = shared                    ? (silu ? launch_glu_bwd<MXL_ACT_SILU, 256> : launch_glu_bwd<MXL_ACT_GELU, 256>)
+                        : f >= GLU_LONG_ROW       ? (silu ? launch_glu_bwd<MXL_ACT_SILU, 1024> : launch_glu_bwd<MXL_ACT_GELU, 1024>)
+                        : f >= GLU_BWD_MIDDLE_ROW ? (silu ? launch_glu_bwd<MXL_ACT_SILU, 512> : launch_glu_bwd<MXL_ACT_GELU, 512>)
+                                                  : (silu ? launch_glu_bwd<MXL_ACT_SILU, 256> : launch_glu_bwd<MXL_ACT_GELU, 256>);
+    launch(dy_bf16, x_bf16, probs, probs_dtype, row_mask, rows, f, dx_bf16, dprobs_f32, (hipStream_t)stream);
     return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;
+}
+}  // namespace mxl
+
+extern "C" int mxl_glu_probs_bwd(const void* dy_bf16, const void* x_bf16, const void* probs, int probs_dtype,
+                                 const uint8_t* row_mask, int64_t rows, int64_t f, int act, void* dx_bf16,
+                                 void* dprobs_f32, void* stream) {
+    return mxl::glu_probs_bwd(dy_bf16, x_bf16, probs, probs_dtype, row_mask, rows, f, act, dx_bf16, dprobs_f32, false, stream);
 }

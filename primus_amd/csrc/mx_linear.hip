@@ -4,6 +4,7 @@
 // allocation per buffer and a stream look-up per launch, they take 230 us for a pass whose kernels need 60.  Here the
 // caller allocates three buffers -- what the backward needs, and a scratch buffer per direction -- and makes one call per
 // direction; the layout of the buffers is arithmetic on the sizes and is worked out again in every call.
+#include "mx_activation.h"
 #include "mx_gemm_tile.h"
 #include "mx_quantize.h"
 #include "mx_blockwise.h"
@@ -344,8 +345,8 @@ extern "C" int mxl_linear_backward(const mxl_linear* p, int parts, const void* d
         if (p->input == MXL_LINEAR_RMSNORM)
             MXL_TRY(mxl_rmsnorm_bwd(b.dxi, x, aux0, sv.rstd, p->rows, p->k, dx, daux, b.norm_ws, b.norm_bytes, stream));
         else if (p->input != MXL_LINEAR_PLAIN)
-            MXL_TRY(mxl_glu_probs_bwd(b.dxi, x, aux0, (int)p->probs_dtype, (const uint8_t*)aux1, p->rows, p->k,
-                                      p->input == MXL_LINEAR_SILU ? MXL_ACT_SILU : MXL_ACT_GELU, dx, daux, stream));
+            MXL_TRY(mxl::glu_probs_bwd(b.dxi, x, aux0, (int)p->probs_dtype, (const uint8_t*)aux1, p->rows, p->k,
+                                       p->input == MXL_LINEAR_SILU ? MXL_ACT_SILU : MXL_ACT_GELU, dx, daux, p->need_dw && !dw_part, stream));
     }
     return MXL_OK;
 }
