@@ -43,6 +43,19 @@ struct Linear {
     bool mx() const { return p.recipe == MXL_LINEAR_MX; }
     bool tensorwise() const { return p.recipe == MXL_LINEAR_TENSORWISE; }
     bool blockwise() const { return p.recipe == MXL_LINEAR_BLOCKWISE; }
+    // Whether codes go through the caches (as far as they fit, mx_quantize.hip) or are streamed past them.  The GEMM behind reads
+    // them next; what it does not find in the cache any more was written to memory while it multiplied instead of before.  So:
+    // everything where a linear's operands fit the 256 MiB memory-side cache together, and beyond that where the GEMMs multiply
+    // rather than read weights.  Not with tensor-wise scaling, whose quantiser finds its input in that cache, left there by the
+    // abs-max pass.  us a pass, streamed / row-wise copies kept / both copies kept: [1999, 2880] x 5760 143 / 134 / 132, [8192, 4096] x
+    // 4096 386 / 380 / 377, [4096, 4096] x 14336 639 / 631 / 623, [16384, 4096] x 14336 2296 / 2274 / 2283; E2M1 [8192, 8192] x 8192 828 /
+    // 817 / 815; 16 experts of 1408, 2048 wide, 256 and 1024 rows each, 372 / 354 / 347 and 785 / 762 / 763; E2M1 weights, 128 experts
+    // [5760, 2880], 512 rows each, 3996 / 3969 / 3970.  Bound by their weights: 32 experts [4096, 7168] and [7168, 2048], 256 rows each,
+    // 2690 / 2740 / 2745 (forward GEMM 319 -> 352).  Tensor-wise, [4096, 4096] x 8192, 383 / 385 / 383.
+    bool keeps() const {
+        const int64_t copies = p.rows * (k_ld + n_ld) * 2 / (p.act_fmt == MXL_FMT_E2M1 ? 2 : 1) + batch * n_ld * k_ld / (p.w_fmt == MXL_FMT_E2M1 ? 2 : 1);
+        return mx() && (p.rows >= 512 * batch || copies <= (int64_t)256 << 20);
+    }
     uint32_t qf() const { return MXL_QF_KSTEP | (f44 ? MXL_QF_KSTEP128 : 0u); }
 
     // K-step-major copies of [rows, ld] (ld padded): codes, scale panels
@@ -251,7 +264,7 @@ extern "C" int mxl_linear_forward(const mxl_linear* p, const void* x, const void
     // (a tensor-wise scaled row-wise copy by itself knows no groups, nor do the copies of an input that an RMSNorm forms)
     const bool ungrouped = (l.tensorwise() && !p->need_dw) || p->input == MXL_LINEAR_RMSNORM;
     const mxl::LinearOperands both = {x, w, p->rows, l.batch, p->n, p->k, l.k_ld, l.n_ld, l.w_rows(), ungrouped ? nullptr : lens, ungrouped ? 0 : G,
-                                      af, wf, (int)p->scale_mode, l.qf() | (rht ? MXL_QF_RHT_COL : 0u), rht ? (uint32_t)p->rht_signs : 0u,
+                                      af, wf, (int)p->scale_mode, l.qf() | (rht ? MXL_QF_RHT_COL : 0u), rht ? (uint32_t)p->rht_signs : 0u, l.keeps(),
                                       f.x_amax, f.w_amax, sv.x_si, sv.w_si,
                                       p->input == MXL_LINEAR_RMSNORM ? aux0 : nullptr, sv.rstd,
                                       f.x_row.q, f.x_row.s, sv.x_col.q, sv.x_col.s, wr.q, wr.s, sv.w_col.q, sv.w_col.s};
@@ -270,25 +283,34 @@ extern "C" int mxl_linear_forward(const mxl_linear* p, const void* x, const void
             MXL_TRY(mxl::quantize_pair(both, stream));
             return product(wr, nullptr, nullptr);
         }
-        MXL_TRY(mxl_rmsnorm_quantize(x, aux0, sv.rstd, p->rows, p->k, l.k_ld, af, (int)p->scale_mode, nullptr, 0, f.x_row.q, f.x_row.s,
-                                     sv.x_col.q, sv.x_col.s, l.qf(), stream));
+        if (!aux0 || !sv.rstd) return MXL_EINVAL;
+        mxl::LinearInput in{x};
+        in.norm_w = aux0;
+        in.rstd = sv.rstd;
+        MXL_TRY(mxl::quantize_input(in, p->rows, p->k, l.k_ld, af, (int)p->scale_mode, nullptr, 0, f.x_row.q, f.x_row.s, sv.x_col.q, sv.x_col.s, l.qf(), 0,
+                                    0, l.keeps(), stream));
     } else if (p->input != MXL_LINEAR_PLAIN) {
-        MXL_TRY(mxl_glu_probs_quantize(x, aux0, (int)p->probs_dtype, (const uint8_t*)aux1, p->rows, p->k, l.k_ld,
-                                       p->input == MXL_LINEAR_SILU ? MXL_ACT_SILU : MXL_ACT_GELU, af, (int)p->scale_mode, lens, G, f.x_row.q,
-                                       f.x_row.s, sv.x_col.q, sv.x_col.s, l.qf(), stream));
+        if (!aux0 || (p->probs_dtype != MXL_PROBS_F32 && p->probs_dtype != MXL_PROBS_BF16)) return MXL_EINVAL;
+        mxl::LinearInput in{x};
+        in.act = p->input == MXL_LINEAR_SILU ? MXL_ACT_SILU : MXL_ACT_GELU;
+        in.probs = aux0;
+        in.probs_dtype = (int)p->probs_dtype;
+        in.row_mask = (const uint8_t*)aux1;
+        MXL_TRY(mxl::quantize_input(in, p->rows, p->k, l.k_ld, af, (int)p->scale_mode, lens, G, f.x_row.q, f.x_row.s, sv.x_col.q, sv.x_col.s, l.qf(), 0, 0,
+                                    l.keeps(), stream));
     } else if (!p->w_quantized) {
         MXL_TRY(mxl::quantize_pair(both, stream));
         return product(wr, nullptr, nullptr);
     } else {
-        MXL_TRY(mxl_quantize_ex(x, p->rows, p->k, l.k_ld, af, (int)p->scale_mode, lens, G, f.x_row.q, f.x_row.s, sv.x_col.q, sv.x_col.s, both.flags, 0,
-                                both.rht_signs, stream));
+        MXL_TRY(mxl::quantize_input({x}, p->rows, p->k, l.k_ld, af, (int)p->scale_mode, lens, G, f.x_row.q, f.x_row.s, sv.x_col.q, sv.x_col.s, both.flags, 0,
+                                    both.rht_signs, l.keeps(), stream));
     }
     if (p->w_quantized) {
         if (!w_scales) return MXL_EINVAL;
         return mxl_grouped_gemm_nt_ex(f.x_row.q, f.x_row.s, af, w, w_scales, wf, y, lens, batch, p->rows, p->n, l.k_ld, MXL_GF_KSTEP, stream);
     }
     MXL_TRY(mxl::quantize_weight_rows(w, l.batch, p->n, p->k, l.k_ld, l.n_ld, l.w_rows(), wf, (int)p->scale_mode, wr.q, wr.s, sv.w_col.q, sv.w_col.s,
-                                      l.qf(), stream));
+                                      l.qf(), l.keeps(), stream));
     return product(wr, nullptr, nullptr);
 }
 
@@ -312,9 +334,9 @@ extern "C" int mxl_linear_backward(const mxl_linear* p, int parts, const void* d
                                             b.d_row.q, b.d_row.s, b.d_col.q, b.d_col.s, b.d_si, l.qf(), stream));
         } else {
             const bool rht = p->rht_signs >= 0 && p->need_dw;
-            MXL_TRY(mxl_quantize_ex(dy, p->rows, p->n, l.n_ld, gf, (int)p->scale_mode, lens, G, b.d_row.q, b.d_row.s, b.d_col.q, b.d_col.s,
-                                    l.qf() | (rht ? MXL_QF_RHT_COL : 0u) | (sr ? MXL_QF_SR : 0u), sr ? sr_seed : 0,
-                                    rht ? (uint32_t)p->rht_signs : 0u, stream));
+            MXL_TRY(mxl::quantize_input({dy}, p->rows, p->n, l.n_ld, gf, (int)p->scale_mode, lens, G, b.d_row.q, b.d_row.s, b.d_col.q, b.d_col.s,
+                                        l.qf() | (rht ? MXL_QF_RHT_COL : 0u) | (sr ? MXL_QF_SR : 0u), sr ? sr_seed : 0,
+                                        rht ? (uint32_t)p->rht_signs : 0u, l.keeps(), stream));
         }
     }
     // the two GEMMs: where both run on small tiles, in one launch

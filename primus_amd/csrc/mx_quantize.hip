@@ -59,6 +59,7 @@ struct QuantArgs {
     int64_t chunk_rows_row, chunk_rows_col;
     uint64_t sr_seed;       // SR kernels: seed of the stochastic rounding
     uint32_t rht_signs;     // RHT kernels: sign bit i flips row i of every 16-row group before the transform
+    bool keep_row, keep_col;    // codes are stored through the caches (keep_in_cache)
     int tiles_r, tiles_c;   // tile grid: row tiles (upper bound when grouped) x column tiles
     int super_c, n_super;   // supertiles: count along the columns, total
     int super_log;          // log2 of a supertile's edge in tiles
@@ -115,6 +116,26 @@ template <int FMT, int SMODE> __device__ __forceinline__ uint32_t block_byte(uin
 __device__ __forceinline__ void store_panel_scales(uint8_t* row16, int quarter, uint32_t v) {
     *(uint16_t*)(row16 + 2 * quarter) = (uint16_t)((v & 0xFFu) | ((v >> 8) & 0xFF00u));
     *(uint16_t*)(row16 + 8 + 2 * quarter) = (uint16_t)(((v >> 8) & 0xFFu) | ((v >> 16) & 0xFF00u));
+}
+
+// (the empty statements keep the compiler from making one store of the two, which would not be a streaming one)
+__device__ __forceinline__ void store16(uint8_t* d, const uint4& v, bool keep) {
+    if (keep) {
+        asm volatile("");
+        *(uint4*)d = v;
+        asm volatile("");
+    } else {
+        store16_streaming(d, v);
+    }
+}
+__device__ __forceinline__ void store4(uint8_t* d, uint32_t v, bool keep) {
+    if (keep) {
+        asm volatile("");
+        *(uint32_t*)d = v;
+        asm volatile("");
+    } else {
+        store4_streaming(d, v);
+    }
 }
 
 template <int FMT, int SMODE, bool ROW, bool COL, bool TWOD, int ACT = -1, bool SR = false, bool RHT = false>
@@ -355,7 +376,7 @@ __device__ __forceinline__ void quant_workgroup(const QuantArgs& a, int block) {
                         const int64_t at = a.kchunk == 2 ? ((int64_t)(2 * ct + (cc >> 3)) * a.chunk_rows_row + out_row0 + rr) * (QT / 2) + 8 * (cc & 7)
                                          : a.kchunk  ? ((int64_t)ct * a.chunk_rows_row + out_row0 + rr) * QT + 8 * cc
                                                      : (out_row0 + rr) * a.row_ld + col0 + 8 * cc;
-                        store16_streaming(a.q_row + at, out);
+                        store16(a.q_row + at, out, a.keep_row);
                     }
                 }
             } else {
@@ -377,7 +398,7 @@ __device__ __forceinline__ void quant_workgroup(const QuantArgs& a, int block) {
                     const int64_t at = a.kchunk == 2 ? ((int64_t)(2 * ct + (c16 >> 3)) * a.chunk_rows_row + out_row0 + r) * (QT / 2) + 8 * (c16 & 7)
                                      : a.kchunk ? ((int64_t)ct * a.chunk_rows_row + out_row0 + r) * QT + 8 * c16
                                                 : (out_row0 + r) * a.row_ld + col;
-                    store4_streaming(a.q_row + at / 2, o);
+                    store4(a.q_row + at / 2, o, a.keep_row);
                 }
             }
         }
@@ -532,7 +553,7 @@ __device__ __forceinline__ void quant_workgroup(const QuantArgs& a, int block) {
                                        ? ((2 * (m0 / QT) + (ch >> 2)) * a.chunk_rows_col + out_rows_base + col0 + c) * (QT / 2) + 16 * (ch & 3)
                                    : a.kchunk ? ((m0 / QT) * a.chunk_rows_col + out_rows_base + col0 + c) * ROWB + 16 * ch
                                               : (out_rows_base + col0 + c) * wbytes + m0b + 16 * ch;
-                store16_streaming(a.q_colT + at, v);
+                store16(a.q_colT + at, v, a.keep_col);
             }
         }
     }
@@ -626,6 +647,16 @@ struct HeldQuant {
     QuantArgs a;
     int64_t wgs;
 };
+
+// `keep`: the caller's word that codes stored through the caches are found there by the GEMM behind (mx_linear.hip: keeps), for
+// copies that fit the 256 MiB memory-side cache; the transposed ones are read later, the activations' not before the backward,
+// and may take a quarter of it.
+constexpr int64_t KEEP_ROW_BYTES = (int64_t)256 << 20, KEEP_COL_BYTES = KEEP_ROW_BYTES / 4;
+static void keep_in_cache(QuantArgs& a, bool keep, int fmt, int64_t row_codes, int64_t col_codes) {
+    const int per = fmt == MXL_FMT_E2M1 ? 2 : 1;
+    a.keep_row = keep && row_codes / per <= KEEP_ROW_BYTES;
+    a.keep_col = keep && col_codes / per <= KEEP_COL_BYTES;
+}
 
 // fills in the launch's tile grid; its workgroups
 static int quant_grid(QuantArgs& a, int64_t tiles_r, int64_t tiles_c, int64_t* wgs) {
@@ -827,7 +858,7 @@ static int quantize_1d(const void* x_bf16, int64_t rows, int64_t cols, int64_t r
                        int act, const void* probs, int probs_dtype, const uint8_t* row_mask, void* stream,
                        bool sr = false, uint64_t sr_seed = 0, bool rht = false, uint32_t rht_signs = 0,
                        int kchunk = 0, const void* norm_w = nullptr, const void* tensor_amax = nullptr,
-                       void* scale_inv_out = nullptr, HeldQuant* hold = nullptr, int parts = 1) {
+                       void* scale_inv_out = nullptr, HeldQuant* hold = nullptr, int parts = 1, bool keep = false) {
     if (row_ld == 0) row_ld = cols;
     if (kchunk < 0) return MXL_EINVAL;                  // contradictory layout flags
     if (kchunk == 2 && fmt == MXL_FMT_E2M1) kchunk = 3;  // E2M1 activations: the K step is 128 elements (64-byte rows)
@@ -866,6 +897,7 @@ static int quantize_1d(const void* x_bf16, int64_t rows, int64_t cols, int64_t r
     a.kchunk = kchunk;
     a.chunk_rows_row = rows;
     a.chunk_rows_col = cols;
+    keep_in_cache(a, keep, fmt, rows * row_ld, cols * a.W);
     const int64_t gx = q_colT ? a.W / QT : (rows + QT - 1) / QT;
     const int64_t gy = ((q_row ? row_ld : cols) + QT - 1) / QT;
     if (hold && gx > 0 && !sr && (act < 0 || act == PRO_RMSNORM)) {
@@ -933,7 +965,7 @@ extern "C" int mxl_rmsnorm_quantize(const void* x_bf16, const void* w_bf16, cons
 static int quantize_weight_2d(const void* w_bf16, int64_t batch, int64_t n, int64_t k, int64_t k_ld, int64_t n_ld, int fmt,
                               int scale_mode, void* q_row, void* s_row, void* q_colT, void* s_colT, int kchunk,
                               void* stream, const void* tensor_amax = nullptr, void* scale_inv_out = nullptr,
-                              const HeldQuant* pair = nullptr, bool* paired = nullptr, int parts = 1, int64_t out_rows = 0) {
+                              const HeldQuant* pair = nullptr, bool* paired = nullptr, int parts = 1, int64_t out_rows = 0, bool keep = false) {
     if (k_ld == 0) k_ld = k;
     if (n_ld == 0) n_ld = n;
     if (out_rows == 0) out_rows = n;
@@ -973,6 +1005,7 @@ static int quantize_weight_2d(const void* w_bf16, int64_t batch, int64_t n, int6
     a.kchunk = kchunk;
     a.chunk_rows_row = batch * out_rows;   // the batch is one operand of that many rows (batch * k for the transposed copy)
     a.chunk_rows_col = batch * k;
+    keep_in_cache(a, keep, fmt, a.chunk_rows_row * k_ld, a.chunk_rows_col * n_ld);
     const int64_t gx = batch * ((n + QT - 1) / QT);
     const int64_t gy = ((q_row ? k_ld : k) + QT - 1) / QT;
     if (pair) {
@@ -990,11 +1023,11 @@ int quantize_pair(const LinearOperands& o, void* stream) {
     const bool rht = (o.flags & MXL_QF_RHT_COL) != 0;
     auto x = [&](HeldQuant* hold) {
         return quantize_1d(o.x, o.rows, o.k, o.k_ld, o.x_fmt, o.scale_mode, o.group_lens, o.num_groups, o.xq_row, o.xs_row, o.xq_col, o.xs_col,
-                           o.norm_w ? PRO_RMSNORM : -1, o.rstd, MXL_PROBS_F32, nullptr, stream, false, 0, rht, o.rht_signs, lay, o.norm_w, o.x_amax, o.x_scale_inv, hold, o.x_amax ? amax_parts(o.rows * o.k) : 1);
+                           o.norm_w ? PRO_RMSNORM : -1, o.rstd, MXL_PROBS_F32, nullptr, stream, false, 0, rht, o.rht_signs, lay, o.norm_w, o.x_amax, o.x_scale_inv, hold, o.x_amax ? amax_parts(o.rows * o.k) : 1, o.keep);
     };
     auto w = [&](const HeldQuant* pair, bool* paired) {
         return quantize_weight_2d(o.w, o.batch, o.n, o.k, o.k_ld, o.n_ld, o.w_fmt, o.scale_mode, o.wq_row, o.ws_row, o.wq_col, o.ws_col, lay,
-                                  stream, o.w_amax, o.w_scale_inv, pair, paired, o.w_amax ? amax_parts(o.batch * o.n * o.k) : 1, o.w_rows);
+                                  stream, o.w_amax, o.w_scale_inv, pair, paired, o.w_amax ? amax_parts(o.batch * o.n * o.k) : 1, o.w_rows, o.keep);
     };
     HeldQuant hold;
     bool paired = false;
@@ -1008,9 +1041,15 @@ int quantize_pair(const LinearOperands& o, void* stream) {
     return w(nullptr, nullptr);
 }
 int quantize_weight_rows(const void* w, int64_t batch, int64_t n, int64_t k, int64_t k_ld, int64_t n_ld, int64_t rows, int fmt, int scale_mode,
-                         void* q_row, void* s_row, void* q_colT, void* s_colT, uint32_t flags, void* stream) {
+                         void* q_row, void* s_row, void* q_colT, void* s_colT, uint32_t flags, bool keep, void* stream) {
     return quantize_weight_2d(w, batch, n, k, k_ld, n_ld, fmt, scale_mode, q_row, s_row, q_colT, s_colT, qf_layout(flags), stream, nullptr, nullptr,
-                              nullptr, nullptr, 1, rows);
+                              nullptr, nullptr, 1, rows, keep);
+}
+int quantize_input(const LinearInput& o, int64_t rows, int64_t cols, int64_t row_ld, int fmt, int scale_mode, const int64_t* group_lens, int num_groups,
+                   void* q_row, void* s_row, void* q_colT, void* s_colT, uint32_t flags, uint64_t sr_seed, uint32_t rht_signs, bool keep, void* stream) {
+    return quantize_1d(o.x, rows, cols, row_ld, fmt, scale_mode, group_lens, num_groups, q_row, s_row, q_colT, s_colT,
+                       o.norm_w ? PRO_RMSNORM : o.act, o.norm_w ? o.rstd : o.probs, o.probs_dtype, o.row_mask, stream, (flags & MXL_QF_SR) != 0, sr_seed,
+                       (flags & MXL_QF_RHT_COL) != 0, rht_signs, qf_layout(flags), o.norm_w, nullptr, nullptr, nullptr, 1, keep);
 }
 }  // namespace mxl
 
