@@ -54,6 +54,7 @@ struct BwQuantArgs {
     const int64_t* group_lens;
     int num_groups;
     int64_t W;
+    bool keep;                  // codes are stored through the caches
     int tiles_r, tiles_c, super_c, n_super;   // a matrix's tile grid and its 4 x 4 supertiles
 };
 
@@ -295,7 +296,7 @@ __device__ __forceinline__ void bw_quant_workgroup(const BwQuantArgs& a, int L, 
                 const uint2 recv = make_uint2(dpp_xor1(send.x), dpp_xor1(send.y));
                 const uint4 out = odd ? make_uint4(recv.x, recv.y, o.x, o.y) : make_uint4(o_even.x, o_even.y, recv.x, recv.y);
                 const int rr = odd ? it : it - 1;
-                if (rbase + rr < valid) store16_streaming(dst + (int64_t)rr * a.cols, out);
+                if (rbase + rr < valid) store16(dst + (int64_t)rr * a.cols, out, a.keep);
             }
         }
     }
@@ -325,7 +326,7 @@ __device__ __forceinline__ void bw_quant_workgroup(const BwQuantArgs& a, int L, 
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int c = (t >> 3) + 32 * i, ch = t & 7;
-            store16_streaming(dst + (int64_t)c * rows_pad + 16 * ch, *(const uint4*)(t_tile + c * BW_TPITCH + 16 * ch));
+            store16(dst + (int64_t)c * rows_pad + 16 * ch, *(const uint4*)(t_tile + c * BW_TPITCH + 16 * ch), a.keep);
         }
     }
 }
@@ -936,7 +937,7 @@ static int bw_quant_add(BwQuantSeveral& s, int& count, const BwTensor& o, int fm
     const int64_t per_mat = ((int64_t)super_c * super_r + 7) / 8 * 8 * 16, first = count ? s.end[count - 1] : 0;
     if (first + per_mat * batch > 0x7FFFFFFF) return MXL_EINVAL;
     s.a[count] = BwQuantArgs{(const uint16_t*)o.x, o.rows, o.cols, (uint8_t*)o.q_row, (float*)o.sinv_row, (uint8_t*)o.q_colT, (float*)o.sinv_colT,
-                             o.group_lens, num_groups, W, (int)row_tiles, tiles_c, super_c, super_c * super_r};
+                             o.group_lens, num_groups, W, o.keep, (int)row_tiles, tiles_c, super_c, super_c * super_r};
     s.per_mat[count] = twod ? (int)per_mat : 0;
     s.end[count] = (int)(first + per_mat * batch);
     ++count;
@@ -1096,14 +1097,14 @@ using namespace mxl;
 
 extern "C" int mxl_quantize_blockwise(const void* x_bf16, int64_t rows, int64_t cols, int fmt, const int64_t* group_lens,
                                       int num_groups, void* q_row, void* sinv_row, void* q_colT, void* sinv_colT, void* stream) {
-    const BwTensor o = {x_bf16, rows, cols, 0, group_lens, num_groups, q_row, sinv_row, q_colT, sinv_colT};
+    const BwTensor o = {x_bf16, rows, cols, 0, group_lens, num_groups, q_row, sinv_row, q_colT, sinv_colT, false};
     return bw_quantize(&o, 1, fmt, stream);
 }
 
 extern "C" int mxl_quantize_blockwise_weight(const void* w_bf16, int64_t batch, int64_t n, int64_t k, int fmt, void* q, void* sinv,
                                              void* q_T, void* sinv_T, void* stream) {
     if (batch < 1 || batch > 65535) return MXL_EINVAL;
-    const BwTensor o = {w_bf16, n, k, batch, nullptr, 0, q, sinv, q_T, sinv_T};
+    const BwTensor o = {w_bf16, n, k, batch, nullptr, 0, q, sinv, q_T, sinv_T, false};
     return bw_quantize(&o, 1, fmt, stream);
 }
 

@@ -277,6 +277,26 @@ __device__ __forceinline__ void store8_streaming(void* d, const uint2& v) {
     __builtin_nontemporal_store(t, (qu32x2*)d);
 }
 __device__ __forceinline__ void store4_streaming(void* d, uint32_t v) { __builtin_nontemporal_store(v, (uint32_t*)d); }
+// Through the caches (`keep`) or past them.  The empty statements keep the compiler from making one store of the two, which would
+// not be a streaming one.
+__device__ __forceinline__ void store16(void* d, const uint4& v, bool keep) {
+    if (keep) {
+        asm volatile("");
+        *(uint4*)d = v;
+        asm volatile("");
+    } else {
+        store16_streaming(d, v);
+    }
+}
+__device__ __forceinline__ void store4(void* d, uint32_t v, bool keep) {
+    if (keep) {
+        asm volatile("");
+        *(uint32_t*)d = v;
+        asm volatile("");
+    } else {
+        store4_streaming(d, v);
+    }
+}
 __device__ __forceinline__ uint4 load16_streaming(const void* s) {
     const qu32x4 t = __builtin_nontemporal_load((const qu32x4*)s);
     return make_uint4(t.x, t.y, t.z, t.w);

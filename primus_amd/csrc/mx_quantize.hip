@@ -118,26 +118,6 @@ __device__ __forceinline__ void store_panel_scales(uint8_t* row16, int quarter, 
     *(uint16_t*)(row16 + 8 + 2 * quarter) = (uint16_t)(((v >> 8) & 0xFFu) | ((v >> 16) & 0xFF00u));
 }
 
-// (the empty statements keep the compiler from making one store of the two, which would not be a streaming one)
-__device__ __forceinline__ void store16(uint8_t* d, const uint4& v, bool keep) {
-    if (keep) {
-        asm volatile("");
-        *(uint4*)d = v;
-        asm volatile("");
-    } else {
-        store16_streaming(d, v);
-    }
-}
-__device__ __forceinline__ void store4(uint8_t* d, uint32_t v, bool keep) {
-    if (keep) {
-        asm volatile("");
-        *(uint32_t*)d = v;
-        asm volatile("");
-    } else {
-        store4_streaming(d, v);
-    }
-}
-
 template <int FMT, int SMODE, bool ROW, bool COL, bool TWOD, int ACT = -1, bool SR = false, bool RHT = false>
 __device__ __forceinline__ void quant_workgroup(const QuantArgs& a, int block) {
     constexpr bool FP4 = (FMT == kFmtE2M1);
