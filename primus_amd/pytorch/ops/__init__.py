@@ -157,15 +157,17 @@ def _overlaps(plan) -> bool:
     the events between the streams, operand panels of two GEMMs in the same L2s, and buffers the allocator must keep for
     two streams.  Measured, together / one after the other: dense [8192, 4096] x 14336 1.22 / 1.20 ms, [2048, 4096] x 4096
     210 / 140 us, E2M1 [4096, 4096] x 14336 451 / 437.  Grouped E2M1 operands gain (Mixtral MXFP4, 4096 tokens 3.71 / 3.75 ms,
-    16384 10.4 / 10.5; not yet at 2048 tokens and 4096 x 4096 experts, 869 / 863 us), FP8 ones with groups of up to about 1000
-    rows a little (DeepSeek shard, 4096 tokens, 5.51 / 5.57; 8192 tokens, 2048 rows a group, 9.33 / 9.37).  Mixtral experts MXFP8,
-    16384 tokens, 4096 rows a group, gain too (16.15 / 16.5 ms), which this line, drawn when they lost (16.5 / 16.3), leaves out."""
+    16384 10.4 / 10.5; not yet at 2048 tokens and 4096 x 4096 experts, 869 / 863 us), and so do FP8 ones: Mixtral, 4096, 8192 and
+    16384 tokens, 5.28 / 5.31, 8.84 / 8.99 and 16.13 / 16.34 ms; 8 experts [11264, 2048] and [2048, 5632], 4096 rows each, 3.81 / 3.87; 16
+    experts of 8192, 2048 wide, 2048 rows each, 5.91 / 5.95; DeepSeek shard, 4096 tokens, 5.51 / 5.57, 8192 tokens 9.33 / 9.37; tensor-wise
+    Mixtral, 8192 tokens, 9.29 / 9.33.  Below the line they gain nothing that can be told from noise (DeepSeek shard, 1024 tokens,
+    2.674 / 2.683)."""
     flops = 2.0 * plan.rows * plan.n * plan.k
     if plan.groups == 0:
         return False
     if plan.struct.act_fmt == _lib.FMT_E2M1:
         return flops >= 5e11
-    return flops >= 1.5e12 and plan.rows <= 1024 * plan.groups
+    return flops >= 1.5e12
 
 
 _CODE_DTYPES = {fmt: K._code_dtype(fmt) for fmt in (_lib.FMT_E4M3, _lib.FMT_E2M1, _lib.FMT_E5M2)}
