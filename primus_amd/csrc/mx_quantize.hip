@@ -544,6 +544,82 @@ __global__ __launch_bounds__(QTHREADS) void mx_quant_kernel(QuantArgs a) {
     quant_workgroup<FMT, SMODE, ROW, COL, TWOD, ACT, SR, RHT>(a, (int)blockIdx.x);
 }
 
+// The row-wise copy alone of few rows, K-step-major: a wave takes two rows of a 512-element scale panel, a lane 8 columns of both.
+// A 128 x 128 tile's workgroup has four times the rows to a lane, one after the other, two barriers and a search for its tile, and
+// few rows are few workgroups: what such a launch lasts is that chain.  Linear on cached weights, us on tiles / so: 64 rows of 4096 to 14336
+// columns (as a graph, the host takes 18) 17.0 / 15.2, 256 rows 22.0 / 20.2, 512 33.1 / 31.9, [1024, 4096] x 4096 23.5 / 22.8, [2048, 4096] x
+// 4096 39.8 / 38.8; E2M1, [512, 4096] x 14336 23.1 / 20.9, [1024, 4096] x 4096 18.9 / 17.5.  From 4096 rows of 2880 on, where the chip is
+// full, tiles are ahead: to 256 columns 23.9 / 24.8, E2M1 17.7 / 18.3.
+constexpr int64_t FEW_ROWS_ELEMENTS = (int64_t)8 << 20;
+template <int FMT, int SMODE, int ACT>
+__global__ __launch_bounds__(64) void mx_quant_few_rows_kernel(QuantArgs a) {
+    constexpr bool FP4 = (FMT == kFmtE2M1);
+    const int l = threadIdx.x;
+    const int64_t row0 = 2 * (int64_t)blockIdx.y, col = 512 * (int64_t)blockIdx.x + 8 * l;
+    const bool two = row0 + 1 < a.rows;
+    if (col >= a.row_ld) return;          // (row_ld is a multiple of 128: the 16 lanes of a K step stay or go together)
+    uint4 d[2] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
+    if (col < a.cols) {
+        if (ACT < 0 || ACT == PRO_RMSNORM) {
+            const uint16_t* x = a.x + row0 * a.cols + col;
+            d[0] = load16_streaming(x);
+            if (two) d[1] = load16_streaming(x + a.cols);
+        }
+        if (ACT == PRO_RMSNORM) {
+            const uint4 wv = *(const uint4*)(a.norm_w + col);
+            const float* rstd = (const float*)a.probs + row0;
+            d[0] = norm8(d[0], wv, rstd[0]);
+            if (two) d[1] = norm8(d[1], wv, rstd[1]);
+        } else if (ACT >= 0) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                if ((i == 0 || two) && (a.row_mask == nullptr || a.row_mask[row0 + i] != 0)) {
+                    const uint16_t* x = a.x + (row0 + i) * 2 * a.cols + col;
+                    d[i] = glu8<(ACT == MXL_ACT_GELU ? MXL_ACT_GELU : MXL_ACT_SILU)>(load16_streaming(x), load16_streaming(x + a.cols),
+                                                                                      load_prob(a.probs, a.probs_bf16, row0 + i));
+                }
+            }
+        }
+    }
+    uint32_t byte[2];
+    uint2 o[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        uint32_t m = hmax16(pk_max16(pk_max16(d[i].x & 0x7FFF7FFFu, d[i].y & 0x7FFF7FFFu), pk_max16(d[i].z & 0x7FFF7FFFu, d[i].w & 0x7FFF7FFFu)));
+        m = max(m, dpp_xor1(m));
+        m = max(m, dpp_xor2(m));
+        byte[i] = scale_byte<FMT, SMODE>(m);
+        if (FP4) {
+            const float sc = fwd_scale(byte[i]);
+            o[i].x = byte[i] != 255u ? cvt2_e2m1(d[i].x, sc) | (cvt2_e2m1(d[i].y, sc) << 8) | (cvt2_e2m1(d[i].z, sc) << 16) | (cvt2_e2m1(d[i].w, sc) << 24)
+                                     : nonfinite2_e2m1(d[i].x) | (nonfinite2_e2m1(d[i].y) << 8) | (nonfinite2_e2m1(d[i].z) << 16) |
+                                           (nonfinite2_e2m1(d[i].w) << 24);
+        } else if (byte[i] != 255u) {
+            const float inv = inv_scale(byte[i]);
+            o[i] = make_uint2(cvt4_e4m3(d[i].x, d[i].y, inv), cvt4_e4m3(d[i].z, d[i].w, inv));
+        } else {
+            o[i] = make_uint2(nonfinite4_e4m3(d[i].x, d[i].y), nonfinite4_e4m3(d[i].z, d[i].w));
+        }
+    }
+    const int64_t step = FP4 ? col >> 7 : col >> 6;                  // 64 bytes of a row either way
+    uint8_t* q = a.q_row + (step * a.chunk_rows_row + row0) * 64;
+    if (FP4) {
+        store4(q + 4 * (l & 15), o[0].x, a.keep_row);
+        if (two) store4(q + 64 + 4 * (l & 15), o[1].x, a.keep_row);
+    } else {
+        // a lane pair swaps 8-byte pieces: the even lane 16 codes of the first row, the odd lane 16 of the second
+        const bool odd = (l & 1) != 0;
+        const uint2 send = odd ? o[0] : o[1];
+        const uint2 recv = make_uint2(dpp_xor1(send.x), dpp_xor1(send.y));
+        if (!odd || two)
+            store16(q + (odd ? 64 : 0) + 8 * (l & 6), odd ? make_uint4(recv.x, recv.y, o[1].x, o[1].y) : make_uint4(o[0].x, o[0].y, recv.x, recv.y), a.keep_row);
+    }
+    // block b = l / 4 of the panel at [block parity][K step]; the second lane of a block writes the second row's byte
+    const int sub = l & 3, b = l >> 2;
+    if (sub == 0 || (sub == 1 && two))
+        a.s_row[((int64_t)blockIdx.x * a.chunk_rows_row + row0 + sub) * 16 + 8 * (b & 1) + (b >> 1)] = (uint8_t)(sub ? byte[1] : byte[0]);
+}
+
 // Both operands of a linear's forward in one launch: the activations' two copies (the first x_wgs workgroups) and the
 // weight's (WCOL: its transposed codes too).  Neither fills the chip for long where the linear is small, and each launch
 // costs its fill and drain and the gap behind it.  Forward of a linear, quantisers and GEMM, two launches / one, us:
@@ -660,6 +736,13 @@ static int launch_quant(QuantArgs& a, int64_t tiles_r, int64_t tiles_c, hipStrea
     if (const int rc = quant_grid(a, tiles_r, tiles_c, &wgs)) return rc;
     const dim3 grid((unsigned)wgs);
     const bool row = a.q_row != nullptr, col = a.q_colT != nullptr;
+    if constexpr (FMT != MXL_FMT_E5M2 && SMODE != SCALE_TENSOR && !TWOD && !SR && !RHT) {
+        if (row && !col && a.kchunk >= 2 && a.rows * a.row_ld <= FEW_ROWS_ELEMENTS) {      // (at most 65536 rows: 32768 pairs of them)
+            const dim3 pairs((unsigned)((a.row_ld + 511) / 512), (unsigned)((a.rows + 1) / 2));
+            hipLaunchKernelGGL((mx_quant_few_rows_kernel<FMT, SMODE, ACT>), pairs, dim3(64), 0, st, a);
+            return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;
+        }
+    }
     if (row && col)
         hipLaunchKernelGGL((mx_quant_kernel<FMT, SMODE, true, true, TWOD, ACT, SR, RHT>), grid, dim3(QTHREADS), 0, st, a);
     else if (row && !RHT)
