@@ -176,16 +176,20 @@ __device__ __forceinline__ uint32_t sr_high(uint64_t key, uint64_t seed, uint32_
     return (uint32_t)(key >> 32) * 0x9E3779B9u + (uint32_t)(seed >> 32) + stream * 0x85EBCA6Bu;
 }
 __device__ __forceinline__ uint32_t sr_word(uint32_t low, uint32_t i, uint32_t high) { return sr_mix(sr_mix(low ^ i) + high); }
-// (The products of the counter and the shared part are worked out once: the random words are four 32-bit multiplications a pair, each the
-// time of four other instructions, and bound the kernel.  Quantising [4096, 14336] both ways with stochastic rounding and
-// the Hadamard transform: 90 -> 79 us, 46 without stochastic rounding.)
-// The magnitude without a branch: in units of 2^-23, w itself below 1 and its fp32 pattern (less that of 0.5) from 1 on.
-// The pattern is the smaller of the two from 1 on and the larger never below, so the one wanted is the median with 1.
-__device__ __forceinline__ uint32_t sr_mag_e2m1(float x, float inv, uint32_t rnd16) {
+// (The products of the counter and the shared part are worked out once.  The kernel is bound by instructions, 148 for eight codes:
+// quantising [4096, 14336] both ways with stochastic rounding and the Hadamard transform takes 87 us, 46 without stochastic rounding; 91
+// with a conversion to integers and a median per magnitude and the nibbles put together one by one, 163 instructions.  The four
+// words' first products out of one multiplication are 8 additions for 3 multiplications: 89.5; products out of 16-bit dot products: 101.)
+// The magnitude without a branch, in bits 26:24 of the result (the caller takes the upper byte).  In units of 2^-23 it is w below 1
+// and w's fp32 pattern, less that of 0.5, from 1 on.  The first comes out of the pattern of (w + 1) 2^23 - 0.5, less that of 2^23 and
+// not below it.  The sum may round to the integer below, but never across a multiple of 64 (w has 8 bits: 63.25 to 63.75 and 127.5
+// stay below, 64 and 128 do not), and what is added is a multiple of 64.  The larger of the two is the one wanted: below 1 the pattern of w is
+// the smaller, from 1 on that of w + 1 is.  Both carry the pattern of 2^23 here, which the random bits' upper byte takes off again.
+constexpr uint32_t SR_RND_TOP = 0xD4000000u;      // -(0x4B000000 << 2)
+__device__ __forceinline__ uint32_t sr_mag_e2m1(float x, float inv, uint32_t rnd8) {
     const float w = fabsf(x) * inv;
-    const int fixed = (int)(w * 8388608.f), line = (int)__float_as_uint(w) - 0x3F000000;
-    const int base = max(min(line, fixed), min(max(line, fixed), 1 << 23));
-    return (uint32_t)min(base + (int)(rnd16 << 6), 0x1FFFFFF) >> 22;
+    const uint32_t fixed = __float_as_uint(fmaf(w, 8388608.f, 8388607.5f)), line = __float_as_uint(w) + (0x4B000000u - 0x3F000000u);
+    return min((max(max(fixed, line), 0x4B000000u) << 2) + rnd8, 0x7FFFFFFu);
 }
 // four packed bf16 pairs -> eight nibbles, element 0 (random bits 15:0 of the first word) in bits 3:0; the signs are
 // gathered for all eight at once.  key: the first pair's counter, a multiple of 4
@@ -193,13 +197,16 @@ __device__ __forceinline__ uint32_t sr8_e2m1(uint32_t p0, uint32_t p1, uint32_t 
                                              uint64_t seed, uint32_t stream) {
     const uint32_t p[4] = {p0, p1, p2, p3};
     const uint32_t low = (uint32_t)key ^ (uint32_t)seed, high = sr_high(key, seed, stream);
-    uint32_t o = 0;
+    uint32_t e[4], d[4];
 #pragma unroll
-    for (int i = 3; i >= 0; --i) {
+    for (int i = 0; i < 4; ++i) {
         const uint32_t rnd = sr_word(low, (uint32_t)i, high);
-        o = (o << 4) | sr_mag_e2m1(bf16_hi(p[i]), inv, rnd >> 16);
-        o = (o << 4) | sr_mag_e2m1(bf16_lo(p[i]), inv, rnd & 0xFFFFu);
+        e[i] = sr_mag_e2m1(bf16_lo(p[i]), inv, __builtin_amdgcn_perm(SR_RND_TOP, rnd, 0x0701000Cu));      // bits 15:0, from bit 8 on
+        d[i] = sr_mag_e2m1(bf16_hi(p[i]), inv, __builtin_amdgcn_perm(SR_RND_TOP, rnd, 0x0703020Cu));      // bits 31:16
     }
+    const uint32_t e_all = __builtin_amdgcn_perm(__builtin_amdgcn_perm(e[3], e[2], 0x07030C0Cu), __builtin_amdgcn_perm(e[1], e[0], 0x0C0C0703u), 0x07060100u);
+    const uint32_t d_all = __builtin_amdgcn_perm(__builtin_amdgcn_perm(d[3], d[2], 0x07030C0Cu), __builtin_amdgcn_perm(d[1], d[0], 0x0C0C0703u), 0x07060100u);
+    const uint32_t o = e_all | (d_all << 4);
     const uint32_t x = __builtin_amdgcn_perm(p1, p0, 0x07030501u), y = __builtin_amdgcn_perm(p3, p2, 0x07030501u);
     const uint32_t even = __builtin_amdgcn_perm(y, x, 0x05040100u), odd = __builtin_amdgcn_perm(y, x, 0x07060302u);
     return o | ((even >> 4) & 0x08080808u) | (odd & 0x80808080u);
