@@ -1352,17 +1352,24 @@ static bool tile_flag_ok(uint32_t flags) {
 //   [256, 4096] x [4096, 4096]: ring 28 us, 128 13, 64 x 128 11.2, 64 x 64 8.4.   [1024, ...]: 41, 19-21, 23, 28
 //   [1999, 2880] x [5760, 2880]: 37, 35, 45, 55.   [4096, 4096] x [4096, 4096]: 57, 61, 80, 102
 // A grouped launch does not know its tile counts (they are on the device): a group's last row tile is taken as half full.
-// Up to about one round of the ring kernel the same rule holds.  Beyond that a launch is bound by reading the weights,
-// which the ring kernel does best from about 32 rows per group on; with fewer its two and a half rounds of mostly empty
-// tiles cost more than the smaller tiles' shorter reads.  E2M1 weights against FP8 rows are half the bytes, which shifts
-// the line up.
-//   128 groups, [5760, 2880]: 4 rows per group ring 418 us, 64 x 128 377 (E2M1 weights 308, 217); 64 rows 433, 467 (317, 267)
-//   32 groups, [4096, 7168]: 32 rows per group ring 169, 128 175 (transposed codes 206, 183); 64 rows 169, 174 (212, 180)
+// Up to about one round of the ring kernel the same rule holds.  Beyond that a launch is bound by reading the weights.  Up to 192 MiB
+// of codes come out of the memory-side cache, where the quantiser has just put them, and what counts is how soon a workgroup is
+// through: 64 x 64 tiles up to 32 rows per group (transposed codes: 128 x 128), 128 x 128 up to 192.  Larger ones come from memory,
+// which the ring kernel reads best from about 32 rows per group on; with fewer, and short contractions, its rounds of mostly empty
+// tiles cost more than 64 x 128 ones.  E2M1 weights against FP8 rows are half the bytes, which shifts the line up.  us, ring / 128 x 128 / 64 x
+// 128 / 64 x 64, groups of uneven size:
+//   64 groups, [2048, 1024], 32 rows per group 31.7 / 23.9 / 24.2 / 23.1, 64 rows 32.0 / 25.8 / 28.4 / 28.1, 192 rows 47.8 / 39.8 / 48.6 / 53.6, 256 rows
+//   51.5 / 49.1 / 63.2 / 67.0; E2M1, 16 groups, [14336, 2048], 8 rows 51.9 / 38.5 / 40.4 / 37.0, 160 rows 75.5 / 66.6 / 79.6 / 88.9, 256 rows 92.7 / 89.5 / ..
+//   64 groups, [6144, 3584], 8 rows 252 / 263 / 250 / 272, 32 rows 253 / 288 / 271 / 308 (transposed 262 / 285 / 266), 64 rows 255 / 304 / 332 / 374;
+//   E2M1, 128 groups, [2304, 2304], 32 rows 82.8 / 80.6 / 73.9 / 83.0, 64 rows 84.9 / 84.4 / 91.1 / 98.8
+//   E2M1 weights, FP8 rows: 64 groups, [3072, 1280], 160 rows 63.0 / 54.2 / 49.7 / ..; [6144, 3584], 160 rows 266 / 308 / 325 / ..
+// A pass of 64 experts of 1408, 2048 wide, 96 and 192 rows each, with these lines and the earlier ones (128 x 128 up to 32 rows, 64 with
+// transposed codes, ring behind): E2M1 823 -> 786 and 941 -> 891, FP8 1031 -> 1007 and 1201 -> 1190, tensor-wise 1189 -> 1158.
 // The weight gradient's tiles are all output and little contraction: dense ones take 128 x 128 while the contraction is
 // short (256 tokens, 14336 x 4096: ring 38 us, 128 x 128 31).  Grouped ones run the ring kernel, which writes more per second on
 // expert-sized gradients, if far from what a fill does (256 rows in each of 32 groups, [4096, 7168]: ring 404 us, 128 x 128
 // tiles 494, a fill of its 1.9 GB 277; skewed rows 444 and 573), except where the gradient is a few tiles.
-template <int MODE> static int tile_choice(const GemmArgs& a, bool e2m1_weights, bool bt, uint32_t flags) {
+template <int MODE> static int tile_choice(const GemmArgs& a, bool act_e2m1, bool e2m1_weights, bool bt, uint32_t flags) {
     switch (flags & MXL_GF_TILE_MASK) {
         case MXL_GF_TILE_64: return TILE_64;
         case MXL_GF_TILE_64X128: return TILE_64x128;
@@ -1379,11 +1386,18 @@ template <int MODE> static int tile_choice(const GemmArgs& a, bool e2m1_weights,
         return (a.total_m / tm + (live + 1) / 2) * cols;
     };
     const int64_t ring_tiles = tiles(256, 256);
+    const int64_t rows = a.total_m / a.num_groups;
     if (MODE == MODE_WGRAD && grouped) return ring_tiles < 256 ? TILE_128 : TILE_RING;
     if (grouped && ring_tiles > 300) {
-        const int64_t rows = a.total_m / a.num_groups;
-        if (e2m1_weights) return rows <= 96 ? TILE_64x128 : rows <= 192 ? TILE_128 : TILE_RING;
-        return rows <= 16 ? TILE_64x128 : rows <= (bt ? 64 : 32) ? TILE_128 : TILE_RING;
+        const int64_t steps = a.k / (act_e2m1 ? 2 * BK : BK);
+        if (e2m1_weights) return rows <= 96 || (rows <= 192 && steps < 40) ? TILE_64x128 : TILE_RING;
+        if ((int64_t)a.num_groups * a.n * a.k / (act_e2m1 ? 2 : 1) <= (int64_t)192 << 20) {
+            if (rows <= 32) return bt ? TILE_128 : TILE_64;
+            return rows <= 192 ? TILE_128 : TILE_RING;
+        }
+        if (rows <= 16) return TILE_64x128;
+        if (rows <= 32) return bt || act_e2m1 || steps < 40 ? TILE_64x128 : TILE_RING;
+        return bt && rows <= 64 ? TILE_128 : TILE_RING;
     }
     auto cost = [&](int64_t tm, int64_t tn, double c) { return (double)cdiv(tiles(tm, tn), 256) * c; };
     int best = TILE_RING;
@@ -1494,7 +1508,7 @@ static int hold_or_launch(bool bt, int afmt, int bfmt, const GemmArgs& a, int ti
 // rows, or E2M1 weights with E2M1 rows (128-element steps)
 static int dispatch_gemm_ring_bt(int afmt, int bfmt, const GemmArgs& a, int64_t max_tiles, hipStream_t st, uint32_t flags, HeldGemm* hold) {
     if (a.num_groups > RING_MAX_GROUPS) return MXL_EINVAL;
-    const int tile = tile_choice<MODE_FWD>(a, false, true, flags);
+    const int tile = tile_choice<MODE_FWD>(a, afmt == MXL_FMT_E2M1, false, true, flags);
     if (bfmt == MXL_FMT_E2M1) {
         if (afmt != MXL_FMT_E2M1 || a.alpha_a != nullptr) return MXL_EINVAL;
         if (tile != TILE_RING) return hold_or_launch(true, afmt, bfmt, a, tile, hold, st);
@@ -1522,7 +1536,7 @@ static int dispatch_gemm(int afmt, int bfmt, const GemmArgs& a, int64_t max_tile
         // the kernel keeps a tile's first output row in 32 bits
         if ((MODE == MODE_WGRAD ? (int64_t)a.num_groups * a.m : a.total_m) >= ((int64_t)1 << 31)) return MXL_EINVAL;
         if (accum) return dispatch_wgrad_accum_ring(afmt, bfmt, a, max_tiles, st);
-        const int tile = tile_choice<MODE>(a, bfmt == MXL_FMT_E2M1 && afmt != MXL_FMT_E2M1, false, flags);
+        const int tile = tile_choice<MODE>(a, afmt == MXL_FMT_E2M1, bfmt == MXL_FMT_E2M1 && afmt != MXL_FMT_E2M1, false, flags);
         if (tile != TILE_RING && MODE == MODE_FWD) return hold_or_launch(false, afmt, bfmt, a, tile, hold, st);
         // the weight gradient of what is held: the same rows' format, and the columns' is the weight's
         if (tile != TILE_RING && hold && hold->held && hold->afmt == afmt && hold->bfmt == bfmt) {
