@@ -169,6 +169,7 @@ def kchunk_default() -> bool:
     return _kchunk_default
 
 
+@functools.lru_cache(maxsize=512)
 def kchunk_fits(groups: int, n: int, k: int, rows: int = 0) -> bool:
     """The GEMMs address a K-chunk-major operand with 32-bit offsets from its base, so every operand of a
     linear with weights ``[groups, n, k]`` and ``rows`` tokens has to stay under 4 GiB."""

@@ -702,8 +702,10 @@ def _apply(fn, *args):
     transform or a forward-mode level ``apply`` is called all the same: it refuses what the operator has no rule for,
     where the forward alone would drop the tangent.  So it is under ``torch.jit.trace``, which records the function as one
     call; of the forward alone it would record the allocations and none of the launches."""
-    if torch.is_grad_enabled() and any(isinstance(t, torch.Tensor) and t.requires_grad for t in args):
-        return fn.apply(*args)
+    if torch.is_grad_enabled():
+        for t in args:      # (a generator costs a microsecond)
+            if t is not None and isinstance(t, torch.Tensor) and t.requires_grad:
+                return fn.apply(*args)
     if (torch._C._are_functorch_transforms_active() or torch.autograd.forward_ad._current_level >= 0
             or torch._C._get_tracing_state() is not None):
         return fn.apply(*args)
