@@ -60,24 +60,33 @@ __global__ __launch_bounds__(THREADS) void glu_probs_fwd_kernel(const uint16_t* 
     }
 }
 
-template <int ACT, int THREADS>
+// SUMS: partial sums a thread keeps.  The gradient of a row's probability is a sum over the row whose order is that of THREADS * SUMS
+// threads with one sum each: chunk i of a thread goes to sum i mod SUMS, which is what thread threadIdx.x + THREADS * (i mod SUMS) of
+// those has, and the waves' sums are added in their order.  So a smaller workgroup gives the bits of the one it stands in for.
+template <int ACT, int THREADS, int SUMS>
 __global__ __launch_bounds__(THREADS) void glu_probs_bwd_kernel(const uint16_t* dy, const uint16_t* x, const void* probs,
                                                                  int probs_bf16, const uint8_t* row_mask, int64_t f,
                                                                  uint16_t* dx, float* dprobs) {
-    __shared__ float part[THREADS / 64];
+    __shared__ float part[SUMS * THREADS / 64];
     const int64_t row = blockIdx.x;
     const bool live = row_mask == nullptr || row_mask[row] != 0;
     const float p = live ? load_prob(probs, probs_bf16, row) : 0.f;
     const uint16_t* xg = x + row * 2 * f;
     const uint16_t* dyr = dy + row * f;
     uint16_t* dxr = dx + row * 2 * f;
-    float acc = 0.f;
+    float sums[SUMS];
+#pragma unroll
+    for (int s = 0; s < SUMS; ++s) sums[s] = 0.f;
+    int turn = 0;
     for (int64_t c = (int64_t)threadIdx.x * 8; c < f; c += THREADS * 8) {
         uint4 o1 = make_uint4(0, 0, 0, 0), o2 = o1;
         if (live) {
             const uint4 g = act_load16(xg + c), u = act_load16(xg + f + c), d = act_load16(dyr + c);
             const uint32_t gw[4] = {g.x, g.y, g.z, g.w}, uw[4] = {u.x, u.y, u.z, u.w}, dw[4] = {d.x, d.y, d.z, d.w};
             uint32_t w1[4], w2[4];
+            float acc = sums[0];
+#pragma unroll
+            for (int s = 1; s < SUMS; ++s) acc = turn == s ? sums[s] : acc;
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 float a0, da0, a1, da1;
@@ -89,6 +98,9 @@ __global__ __launch_bounds__(THREADS) void glu_probs_bwd_kernel(const uint16_t* 
                 w1[k] = pack_bf16(d0 * p * u0 * da0, d1 * p * u1 * da1);
                 w2[k] = pack_bf16(d0 * p * a0, d1 * p * a1);
             }
+#pragma unroll
+            for (int s = 0; s < SUMS; ++s) sums[s] = SUMS == 1 || turn == s ? acc : sums[s];
+            turn = (turn + 1) & (SUMS - 1);
             o1 = make_uint4(w1[0], w1[1], w1[2], w1[3]);
             o2 = make_uint4(w2[0], w2[1], w2[2], w2[3]);
         }
@@ -97,13 +109,17 @@ __global__ __launch_bounds__(THREADS) void glu_probs_bwd_kernel(const uint16_t* 
     }
     // row sum of dy * act(g) * u over the workgroup
 #pragma unroll
-    for (int s = 32; s > 0; s >>= 1) acc += __shfl_xor(acc, s);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = acc;
+    for (int i = 0; i < SUMS; ++i) {
+        float acc = sums[i];
+#pragma unroll
+        for (int s = 32; s > 0; s >>= 1) acc += __shfl_xor(acc, s);
+        if ((threadIdx.x & 63) == 0) part[i * (THREADS / 64) + (threadIdx.x >> 6)] = acc;
+    }
     __syncthreads();
     if (threadIdx.x == 0) {
         float t = 0.f;
 #pragma unroll
-        for (int i = 0; i < THREADS / 64; ++i) t += part[i];
+        for (int i = 0; i < SUMS * THREADS / 64; ++i) t += part[i];
         dprobs[row] = live ? t : 0.f;
     }
 }
@@ -160,10 +176,10 @@ static void launch_glu_fwd(const void* x, const void* probs, int probs_dtype, co
     hipLaunchKernelGGL((glu_probs_fwd_kernel<ACT, THREADS>), dim3((unsigned)rows), dim3(THREADS), 0, st, (const uint16_t*)x, probs, probs_dtype, row_mask,
                        f, (uint16_t*)y);
 }
-template <int ACT, int THREADS>
+template <int ACT, int THREADS, int SUMS>
 static void launch_glu_bwd(const void* dy, const void* x, const void* probs, int probs_dtype, const uint8_t* row_mask, int64_t rows, int64_t f,
                            void* dx, void* dprobs, hipStream_t st) {
-    hipLaunchKernelGGL((glu_probs_bwd_kernel<ACT, THREADS>), dim3((unsigned)rows), dim3(THREADS), 0, st, (const uint16_t*)dy, (const uint16_t*)x, probs,
+    hipLaunchKernelGGL((glu_probs_bwd_kernel<ACT, THREADS, SUMS>), dim3((unsigned)rows), dim3(THREADS), 0, st, (const uint16_t*)dy, (const uint16_t*)x, probs,
                        probs_dtype, row_mask, f, (uint16_t*)dx, (float*)dprobs);
 }
 constexpr int64_t GLU_LONG_ROW = 6656;                                   // 1024 threads from here on
@@ -184,8 +200,8 @@ extern "C" int mxl_glu_probs_fwd(const void* x_bf16, const void* probs, int prob
 
 namespace mxl {
 // `shared`: another launch that fills the chip runs on another stream.  Its workgroups leave room here and there, which small
-// workgroups use better: a pass of 8 experts [28672, 4096], E2M1, 8192 rows, whose weight gradients run beside it, 3735 us with
-// 256 threads, 3767 with 1024.
+// workgroups use better: a pass of 8 experts [28672, 4096] and [4096, 14336] whose weight gradients run beside it, with 256 threads
+// (and four sums each) and with 1024: FP8, 32768 rows, 16.00 and 16.23 ms; E2M1, 8192 rows, 3.69 and 3.73.
 int glu_probs_bwd(const void* dy_bf16, const void* x_bf16, const void* probs, int probs_dtype, const uint8_t* row_mask, int64_t rows, int64_t f, int act,
                   void* dx_bf16, void* dprobs_f32, bool shared, void* stream) {
     if (!act_args_ok(x_bf16, dx_bf16, probs, probs_dtype, rows, f, act)) return MXL_EINVAL;
@@ -193,10 +209,12 @@ int glu_probs_bwd(const void* dy_bf16, const void* x_bf16, const void* probs, in
     if (!dy_bf16 || !dprobs_f32) return MXL_EINVAL;
     if (!device_is_gfx950()) return MXL_ENODEV;
     const bool silu = act == MXL_ACT_SILU;
-    const auto launch = shared                    ? (silu ? launch_glu_bwd<MXL_ACT_SILU, 256> : launch_glu_bwd<MXL_ACT_GELU, 256>)
-                        : f >= GLU_LONG_ROW       ? (silu ? launch_glu_bwd<MXL_ACT_SILU, 1024> : launch_glu_bwd<MXL_ACT_GELU, 1024>)
-                        : f >= GLU_BWD_MIDDLE_ROW ? (silu ? launch_glu_bwd<MXL_ACT_SILU, 512> : launch_glu_bwd<MXL_ACT_GELU, 512>)
-                                                  : (silu ? launch_glu_bwd<MXL_ACT_SILU, 256> : launch_glu_bwd<MXL_ACT_GELU, 256>);
+    const auto launch =
+        f >= GLU_LONG_ROW       ? (shared ? (silu ? launch_glu_bwd<MXL_ACT_SILU, 256, 4> : launch_glu_bwd<MXL_ACT_GELU, 256, 4>)
+                                          : (silu ? launch_glu_bwd<MXL_ACT_SILU, 1024, 1> : launch_glu_bwd<MXL_ACT_GELU, 1024, 1>))
+        : f >= GLU_BWD_MIDDLE_ROW ? (shared ? (silu ? launch_glu_bwd<MXL_ACT_SILU, 256, 2> : launch_glu_bwd<MXL_ACT_GELU, 256, 2>)
+                                          : (silu ? launch_glu_bwd<MXL_ACT_SILU, 512, 1> : launch_glu_bwd<MXL_ACT_GELU, 512, 1>))
+                                : (silu ? launch_glu_bwd<MXL_ACT_SILU, 256, 1> : launch_glu_bwd<MXL_ACT_GELU, 256, 1>);
     launch(dy_bf16, x_bf16, probs, probs_dtype, row_mask, rows, f, dx_bf16, dprobs_f32, (hipStream_t)stream);
     return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;
 }
