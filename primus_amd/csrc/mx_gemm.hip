@@ -1490,18 +1490,29 @@ static int dispatch_wgrad_accum_ring(int afmt, int bfmt, const GemmArgs& a, int6
     return MXL_EINVAL;
 }
 
-// an input gradient on small tiles: put off into `hold` where a launch with the weight gradient exists
-static int hold_or_launch(bool bt, int afmt, int bfmt, const GemmArgs& a, int tile, HeldGemm* hold, hipStream_t st) {
+// an input gradient: put off into `hold` where a launch with the weight gradient exists, or where it goes behind that
+static int hold_or_launch(bool bt, int afmt, int bfmt, const GemmArgs& a, int tile, int64_t max_tiles, HeldGemm* hold, hipStream_t st) {
     HeldGemm h;
     h.held = true;
     h.bt = bt;
     h.afmt = afmt;
     h.bfmt = bfmt;
     h.tile = tile;
+    h.max_tiles = max_tiles;
     h.args = a;
-    if (!hold || !gemm_pair_takes(h)) return h.flush(st);
+    if (!hold || !(hold->behind || gemm_pair_takes(h))) return h.flush(st);
     *hold = h;
     return MXL_OK;
+}
+
+int gemm_ring_fwd(bool bt, int afmt, int bfmt, const GemmArgs& a, int64_t max_tiles, hipStream_t st) {
+    if (!bt) return dispatch_gemm_ring<MODE_FWD>(afmt, bfmt, a, max_tiles, st);
+    if (bfmt == MXL_FMT_E2M1) return launch_gemm_ring<MXL_FMT_E2M1, MXL_FMT_E2M1, MODE_FWD, false, false, true>(a, max_tiles, st);
+    if (a.alpha_a != nullptr) {
+        if (afmt == MXL_FMT_E5M2) return launch_gemm_ring<MXL_FMT_E5M2, MXL_FMT_E4M3, MODE_FWD, true, false, true>(a, max_tiles, st);
+        return launch_gemm_ring<MXL_FMT_E4M3, MXL_FMT_E4M3, MODE_FWD, true, false, true>(a, max_tiles, st);
+    }
+    return launch_gemm_ring<MXL_FMT_E4M3, MXL_FMT_E4M3, MODE_FWD, false, false, true>(a, max_tiles, st);
 }
 
 // forward / dgrad on the row-wise codes of the transposed weight (MXL_GF_B_TRANSPOSED): E4M3 weights with E4M3 or E5M2
@@ -1509,18 +1520,10 @@ static int hold_or_launch(bool bt, int afmt, int bfmt, const GemmArgs& a, int ti
 static int dispatch_gemm_ring_bt(int afmt, int bfmt, const GemmArgs& a, int64_t max_tiles, hipStream_t st, uint32_t flags, HeldGemm* hold) {
     if (a.num_groups > RING_MAX_GROUPS) return MXL_EINVAL;
     const int tile = tile_choice<MODE_FWD>(a, afmt == MXL_FMT_E2M1, false, true, flags);
-    if (bfmt == MXL_FMT_E2M1) {
-        if (afmt != MXL_FMT_E2M1 || a.alpha_a != nullptr) return MXL_EINVAL;
-        if (tile != TILE_RING) return hold_or_launch(true, afmt, bfmt, a, tile, hold, st);
-        return launch_gemm_ring<MXL_FMT_E2M1, MXL_FMT_E2M1, MODE_FWD, false, false, true>(a, max_tiles, st);
-    }
-    if (bfmt != MXL_FMT_E4M3 || (afmt != MXL_FMT_E4M3 && (afmt != MXL_FMT_E5M2 || a.alpha_a == nullptr))) return MXL_EINVAL;
-    if (tile != TILE_RING) return hold_or_launch(true, afmt, bfmt, a, tile, hold, st);
-    if (a.alpha_a != nullptr) {
-        if (afmt == MXL_FMT_E5M2) return launch_gemm_ring<MXL_FMT_E5M2, MXL_FMT_E4M3, MODE_FWD, true, false, true>(a, max_tiles, st);
-        return launch_gemm_ring<MXL_FMT_E4M3, MXL_FMT_E4M3, MODE_FWD, true, false, true>(a, max_tiles, st);
-    }
-    return launch_gemm_ring<MXL_FMT_E4M3, MXL_FMT_E4M3, MODE_FWD, false, false, true>(a, max_tiles, st);
+    if (bfmt == MXL_FMT_E2M1 ? afmt != MXL_FMT_E2M1 || a.alpha_a != nullptr
+                             : bfmt != MXL_FMT_E4M3 || (afmt != MXL_FMT_E4M3 && (afmt != MXL_FMT_E5M2 || a.alpha_a == nullptr)))
+        return MXL_EINVAL;
+    return hold_or_launch(true, afmt, bfmt, a, tile, max_tiles, hold, st);
 }
 
 // a_rows / b_rows: rows of the whole operands (for the 4 GiB bound of the chunk-major layout)
@@ -1537,7 +1540,7 @@ static int dispatch_gemm(int afmt, int bfmt, const GemmArgs& a, int64_t max_tile
         if ((MODE == MODE_WGRAD ? (int64_t)a.num_groups * a.m : a.total_m) >= ((int64_t)1 << 31)) return MXL_EINVAL;
         if (accum) return dispatch_wgrad_accum_ring(afmt, bfmt, a, max_tiles, st);
         const int tile = tile_choice<MODE>(a, afmt == MXL_FMT_E2M1, bfmt == MXL_FMT_E2M1 && afmt != MXL_FMT_E2M1, false, flags);
-        if (tile != TILE_RING && MODE == MODE_FWD) return hold_or_launch(false, afmt, bfmt, a, tile, hold, st);
+        if (MODE == MODE_FWD) return hold_or_launch(false, afmt, bfmt, a, tile, max_tiles, hold, st);
         // the weight gradient of what is held: the same rows' format, and the columns' is the weight's
         if (tile != TILE_RING && hold && hold->held && hold->afmt == afmt && hold->bfmt == bfmt) {
             hold->held = false;

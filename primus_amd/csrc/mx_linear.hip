@@ -339,6 +339,7 @@ extern "C" int mxl_linear_backward(const mxl_linear* p, int parts, const void* d
     // So that one goes first and finds the gradient's transposed copy there.  us a pass: 32 experts of 2048, 7168 wide, 256 rows each, 2719 ->
     // 2692 (the order alone 2707, the copies kept alone 2740), E2M1 2036 -> 1994; 8 experts of 14336, 4096 wide, 256 rows each, E2M1 2007 ->
     // 1950, FP8 2681 -> 2672; no difference with 16 experts of 4096, 4096 wide.  (Dense gradients this small share a launch, below.)
+    // dgrad's operands are looked at before either is launched: a call that it refuses has added nothing to a weight gradient.
     const bool dw_first = dw_part && dx_part && p->groups > 0 && l.mx() && !l.keeps();
     if (parts & MXL_LINEAR_QUANTIZE) {
         if (!dy) return MXL_EINVAL;
@@ -355,14 +356,7 @@ extern "C" int mxl_linear_backward(const mxl_linear* p, int parts, const void* d
     }
     // the two GEMMs: where both run on small tiles, in one launch
     mxl::HeldGemm hold;
-    int rc = MXL_OK;
-    auto weight_gradient = [&]() {
-        const bool tw = l.tensorwise();
-        if (tw && (!b.d_si || !sv.x_si)) return (int)MXL_EINVAL;
-        return mxl::gemm_wgrad_held(b.d_col.q, b.d_col.s, gf, sv.x_col.q, sv.x_col.s, (int)p->act_fmt, dw, lens, G, p->rows, p->n, p->k,
-                                    tw ? b.d_si : nullptr, tw ? sv.x_si : nullptr, MXL_GF_KSTEP | dw_flags, &hold, stream);
-    };
-    if (dw_first) MXL_TRY(weight_gradient());
+    hold.behind = dw_first;
     if (dx_part) {
         void* out = b.dxi ? b.dxi : dx;
         if (!out) return MXL_EINVAL;
@@ -372,9 +366,16 @@ extern "C" int mxl_linear_backward(const mxl_linear* p, int parts, const void* d
         const bool tw = l.tensorwise();
         if (tw && (!b.d_si || !sv.w_si)) return MXL_EINVAL;
         MXL_TRY(mxl::gemm_nt_held(b.d_row.q, b.d_row.s, gf, bq, bs, wf, out, lens, batch, p->rows, p->k, l.n_ld, tw ? b.d_si : nullptr,
-                                  tw ? sv.w_si : nullptr, flags, dw_part && !dw_first ? &hold : nullptr, stream));
+                                  tw ? sv.w_si : nullptr, flags, dw_part ? &hold : nullptr, stream));
     }
-    if (dw_part && !dw_first) rc = weight_gradient();
+    int rc = MXL_OK;
+    if (dw_part) {
+        const bool tw = l.tensorwise();
+        if (tw && (!b.d_si || !sv.x_si)) rc = MXL_EINVAL;
+        else
+            rc = mxl::gemm_wgrad_held(b.d_col.q, b.d_col.s, gf, sv.x_col.q, sv.x_col.s, (int)p->act_fmt, dw, lens, G, p->rows, p->n, p->k,
+                                      tw ? b.d_si : nullptr, tw ? sv.x_si : nullptr, MXL_GF_KSTEP | dw_flags, dw_first ? nullptr : &hold, stream);
+    }
     MXL_TRY(hold.flush((hipStream_t)stream));
     MXL_TRY(rc);
     if (dx_part) {
