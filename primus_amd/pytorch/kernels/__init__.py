@@ -169,10 +169,16 @@ def kchunk_default() -> bool:
     return _kchunk_default
 
 
-@functools.lru_cache(maxsize=512)
 def kchunk_fits(groups: int, n: int, k: int, rows: int = 0) -> bool:
     """The GEMMs address a K-chunk-major operand with 32-bit offsets from its base, so every operand of a
     linear with weights ``[groups, n, k]`` and ``rows`` tokens has to stay under 4 GiB."""
+    # (worked out once per sizes: 1.3 us a call.  A tracer's sizes are symbols, which have no hash, or tensors: those are not kept.)
+    plain = type(groups) is type(n) is type(k) is type(rows) is int
+    return (_kchunk_fits if plain else _kchunk_fits.__wrapped__)(groups, n, k, rows)
+
+
+@functools.lru_cache(maxsize=512)
+def _kchunk_fits(groups, n, k, rows):
     np_, kp = _round_up(n, KCHUNK), _round_up(k, KCHUNK)
     limit = 1 << 32
     if groups * np_ * kp >= limit:
