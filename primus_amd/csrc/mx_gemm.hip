@@ -1352,23 +1352,12 @@ static bool tile_flag_ok(uint32_t flags) {
 //   [256, 4096] x [4096, 4096]: ring 28 us, 128 13, 64 x 128 11.2, 64 x 64 8.4.   [1024, ...]: 41, 19-21, 23, 28
 //   [1999, 2880] x [5760, 2880]: 37, 35, 45, 55.   [4096, 4096] x [4096, 4096]: 57, 61, 80, 102
 // A grouped launch does not know its tile counts (they are on the device): a group's last row tile is taken as half full.
-// Up to about one round of the ring kernel the same rule holds.  Beyond that a launch is bound by reading the weights.  Up to 192 MiB
-// of codes come out of the memory-side cache, where the quantiser has just put them, and what counts is how soon a workgroup is
-// through: 64 x 64 tiles up to 32 rows per group (transposed codes: 128 x 128), 128 x 128 up to 192.  Larger ones come from memory,
-// which the ring kernel reads best from about 32 rows per group on; with fewer, and short contractions, its rounds of mostly empty
-// tiles cost more than 64 x 128 ones.  E2M1 weights against FP8 rows are half the bytes, which shifts the line up.  us, ring / 128 x 128 / 64 x
-// 128 / 64 x 64, groups of uneven size:
-//   64 groups, [2048, 1024], 32 rows per group 31.7 / 23.9 / 24.2 / 23.1, 64 rows 32.0 / 25.8 / 28.4 / 28.1, 192 rows 47.8 / 39.8 / 48.6 / 53.6, 256 rows
-//   51.5 / 49.1 / 63.2 / 67.0; E2M1, 16 groups, [14336, 2048], 8 rows 51.9 / 38.5 / 40.4 / 37.0, 160 rows 75.5 / 66.6 / 79.6 / 88.9, 256 rows 92.7 / 89.5 / ..
-//   64 groups, [6144, 3584], 8 rows 252 / 263 / 250 / 272, 32 rows 253 / 288 / 271 / 308 (transposed 262 / 285 / 266), 64 rows 255 / 304 / 332 / 374;
-//   E2M1, 128 groups, [2304, 2304], 32 rows 82.8 / 80.6 / 73.9 / 83.0, 64 rows 84.9 / 84.4 / 91.1 / 98.8
-//   E2M1 weights, FP8 rows: 64 groups, [3072, 1280], 160 rows 63.0 / 54.2 / 49.7 / ..; [6144, 3584], 160 rows 266 / 308 / 325 / ..
-// A pass of 64 experts of 1408, 2048 wide, 96 and 192 rows each, with these lines and the earlier ones (128 x 128 up to 32 rows, 64 with
-// transposed codes, ring behind): E2M1 823 -> 786 and 941 -> 891, FP8 1031 -> 1007 and 1201 -> 1190, tensor-wise 1189 -> 1158.
+// Up to about one round of the ring kernel the same rule holds; what lies beyond is grouped_tile's (mx_gemm_choice.h).
 // The weight gradient's tiles are all output and little contraction: dense ones take 128 x 128 while the contraction is
 // short (256 tokens, 14336 x 4096: ring 38 us, 128 x 128 31).  Grouped ones run the ring kernel, which writes more per second on
 // expert-sized gradients, if far from what a fill does (256 rows in each of 32 groups, [4096, 7168]: ring 404 us, 128 x 128
 // tiles 494, a fill of its 1.9 GB 277; skewed rows 444 and 573), except where the gradient is a few tiles.
+constexpr uint32_t GF_B_FRESH = 1u << 31;      // gemm_nt_held's b_fresh on its way to tile_choice; no flag of the C entries
 template <int MODE> static int tile_choice(const GemmArgs& a, bool act_e2m1, bool e2m1_weights, bool bt, uint32_t flags) {
     switch (flags & MXL_GF_TILE_MASK) {
         case MXL_GF_TILE_64: return TILE_64;
@@ -1386,19 +1375,10 @@ template <int MODE> static int tile_choice(const GemmArgs& a, bool act_e2m1, boo
         return (a.total_m / tm + (live + 1) / 2) * cols;
     };
     const int64_t ring_tiles = tiles(256, 256);
-    const int64_t rows = a.total_m / a.num_groups;
     if (MODE == MODE_WGRAD && grouped) return ring_tiles < 256 ? TILE_128 : TILE_RING;
-    if (grouped && ring_tiles > 300) {
-        const int64_t steps = a.k / (act_e2m1 ? 2 * BK : BK);
-        if (e2m1_weights) return rows <= 96 || (rows <= 192 && steps < 40) ? TILE_64x128 : TILE_RING;
-        if ((int64_t)a.num_groups * a.n * a.k / (act_e2m1 ? 2 : 1) <= (int64_t)192 << 20) {
-            if (rows <= 32) return bt ? TILE_128 : TILE_64;
-            return rows <= 192 ? TILE_128 : TILE_RING;
-        }
-        if (rows <= 16) return TILE_64x128;
-        if (rows <= 32) return bt || act_e2m1 || steps < 40 ? TILE_64x128 : TILE_RING;
-        return bt && rows <= 64 ? TILE_128 : TILE_RING;
-    }
+    if (grouped && ring_tiles > 300)
+        return grouped_tile((int64_t)a.num_groups * a.n * a.k / (act_e2m1 || e2m1_weights ? 2 : 1), a.total_m / a.num_groups, a.k / (act_e2m1 ? 2 * BK : BK),
+                            act_e2m1, e2m1_weights, bt, (flags & GF_B_FRESH) != 0);
     auto cost = [&](int64_t tm, int64_t tn, double c) { return (double)cdiv(tiles(tm, tn), 256) * c; };
     int best = TILE_RING;
     double least = ring_tiles <= 512 ? cost(256, 256, 53.0) : ring_tiles / 256.0 * 53.0;
@@ -1578,7 +1558,7 @@ __global__ __launch_bounds__(256) void zero_fill_kernel(uint32_t* dst, int64_t w
 static int grouped_gemm_nt(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes, const void* b_scales,
                            int b_fmt, void* c_bf16, const int64_t* group_lens, int num_groups, int64_t total_m, int64_t n,
                            int64_t k, const float* alpha_a, const float* alpha_b, uint32_t flags, void* stream, HeldGemm* hold = nullptr,
-                           int64_t b_rows = 0) {
+                           int64_t b_rows = 0, bool b_fresh = false) {
     if (b_rows == 0) b_rows = n;
     if (b_rows < n || (b_rows > n && (!(flags & MXL_GF_KSTEP) || (flags & MXL_GF_B_TRANSPOSED)))) return MXL_EINVAL;
     if (flags & ~(uint32_t)(MXL_GF_KCHUNK | MXL_GF_KSTEP | MXL_GF_B_TRANSPOSED | MXL_GF_B_SHUFFLED | MXL_GF_TILE_MASK)) return MXL_EINVAL;
@@ -1612,6 +1592,7 @@ static int grouped_gemm_nt(const void* a_codes, const void* a_scales, int a_fmt,
     a.alpha_a = alpha_a;
     a.alpha_b = alpha_b;
     const int64_t max_tiles = (total_m / BM + num_groups) * ((n + BN - 1) / BN);
+    if (b_fresh) flags |= GF_B_FRESH;
     if (flags & MXL_GF_B_SHUFFLED) return launch_gemm<MXL_FMT_E2M1, MXL_FMT_E2M1, MODE_FWD, 0, false, false, true>(a, max_tiles, (hipStream_t)stream);
     if (flags & MXL_GF_B_TRANSPOSED) {
         // offsets inside an operand are 32-bit; the kernel keeps a tile's first output row in 32 bits
@@ -1710,9 +1691,9 @@ static int grouped_gemm_wgrad(const void* a_codes, const void* a_scales, int a_f
 namespace mxl {
 int gemm_nt_held(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes, const void* b_scales, int b_fmt, void* c,
                  const int64_t* group_lens, int num_groups, int64_t total_m, int64_t n, int64_t k, const float* alpha_a,
-                 const float* alpha_b, uint32_t flags, HeldGemm* hold, void* stream, int64_t b_rows) {
+                 const float* alpha_b, uint32_t flags, HeldGemm* hold, void* stream, int64_t b_rows, bool b_fresh) {
     return grouped_gemm_nt(a_codes, a_scales, a_fmt, b_codes, b_scales, b_fmt, c, group_lens, num_groups, total_m, n, k, alpha_a, alpha_b, flags,
-                           stream, hold, b_rows);
+                           stream, hold, b_rows, b_fresh);
 }
 int gemm_wgrad_held(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes, const void* b_scales, int b_fmt, void* c,
                     const int64_t* group_lens, int num_groups, int64_t total_m, int64_t n, int64_t k, const float* alpha_a,

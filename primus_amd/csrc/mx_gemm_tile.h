@@ -1,10 +1,9 @@
 // Entry points of the small-tile GEMM kernel (mx_gemm_tile.hip, mx_gemm_pair.hip) for the dispatch in mx_gemm.hip.
 #pragma once
+#include "mx_gemm_choice.h"
 #include "mx_gemm_common.h"
 
 namespace mxl {
-
-enum { TILE_RING = 0, TILE_64 = 1, TILE_64x128 = 2, TILE_128 = 3 };
 
 // A dense weight gradient over few tokens runs the 128 x 128 tile with two stages instead of four: more workgroups on a
 // CU overlap their outputs (1024 tokens, 14336 x 4096: 69 -> 64 us, 256 tokens 35 -> 29; 2048 tokens, 4096 x 4096: 33 -> 40).
@@ -40,10 +39,10 @@ int gemm_pair(const HeldGemm& h, const GemmArgs& wgrad, hipStream_t st);
 
 // mxl_grouped_gemm_nt_ex / _scaled and mxl_grouped_gemm_wgrad_ex / _scaled (alpha null or given), with the former put off
 // into `hold` if it runs on small tiles (or hold->behind), and the latter launched with what is held.  b_rows: rows from one group's matrix in b
-// to the next (0: n)
+// to the next (0: n); b_fresh: the caller has just quantised b
 int gemm_nt_held(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes, const void* b_scales, int b_fmt, void* c,
                  const int64_t* group_lens, int num_groups, int64_t total_m, int64_t n, int64_t k, const float* alpha_a,
-                 const float* alpha_b, uint32_t flags, HeldGemm* hold, void* stream, int64_t b_rows = 0);
+                 const float* alpha_b, uint32_t flags, HeldGemm* hold, void* stream, int64_t b_rows = 0, bool b_fresh = false);
 int gemm_wgrad_held(const void* a_codes, const void* a_scales, int a_fmt, const void* b_codes, const void* b_scales, int b_fmt, void* c,
                     const int64_t* group_lens, int num_groups, int64_t total_m, int64_t n, int64_t k, const float* alpha_a,
                     const float* alpha_b, uint32_t flags, HeldGemm* hold, void* stream);

@@ -278,7 +278,7 @@ extern "C" int mxl_linear_forward(const mxl_linear* p, const void* x, const void
                                       f.x_row.q, f.x_row.s, sv.x_col.q, sv.x_col.s, wr.q, wr.s, sv.w_col.q, sv.w_col.s};
     auto product = [&](const Copy& wc, const float* alpha_a, const float* alpha_b) {
         return mxl::gemm_nt_held(f.x_row.q, f.x_row.s, af, wc.q, wc.s, wf, y, lens, batch, p->rows, p->n, l.k_ld, alpha_a, alpha_b, MXL_GF_KSTEP, nullptr,
-                                 stream, l.w_rows());
+                                 stream, l.w_rows(), true);
     };
     if (l.tensorwise()) {
         MXL_TRY(mxl::amax_pair(x, p->rows * p->k, f.x_amax, w, l.batch * p->n * p->k, f.w_amax, true, stream));
