@@ -548,9 +548,17 @@ __global__ __launch_bounds__(QTHREADS) void mx_quant_kernel(QuantArgs a) {
 // A 128 x 128 tile's workgroup has four times the rows to a lane, one after the other, two barriers and a search for its tile, and
 // few rows are few workgroups: what such a launch lasts is that chain.  Linear on cached weights, us on tiles / so: 64 rows of 4096 to 14336
 // columns (as a graph, the host takes 18) 17.0 / 15.2, 256 rows 22.0 / 20.2, 512 33.1 / 31.9, [1024, 4096] x 4096 23.5 / 22.8, [2048, 4096] x
-// 4096 39.8 / 38.8; E2M1, [512, 4096] x 14336 23.1 / 20.9, [1024, 4096] x 4096 18.9 / 17.5.  From 4096 rows of 2880 on, where the chip is
-// full, tiles are ahead: to 256 columns 23.9 / 24.8, E2M1 17.7 / 18.3.
+// 4096 39.8 / 38.8; E2M1, [512, 4096] x 14336 23.1 / 20.9, [1024, 4096] x 4096 18.9 / 17.5.  With more waves than the chip holds at once
+// (32 to a CU: 8192) tiles are ahead, for narrow rows, whose waves are part empty, as for wide ones: quantiser alone, time so / on tiles, at
+// 6144 waves 0.88 (3072 rows of 2048) to 0.97 (12288 of 128), at 8192 1.01 to 1.08, 65536 rows of 128 columns 1.49.  An RMSNorm in front
+// moves the line up (8192 waves 0.90 to 1.00, 16384 1.15), a gated activation, which is what a tile's lane spends its time on, past the
+// sizes here: 0.84 at 32768 rows of 256, 0.74 at 8192 of 1024.
 constexpr int64_t FEW_ROWS_ELEMENTS = (int64_t)8 << 20;
+static bool few_rows(const QuantArgs& a, int act) {
+    if (a.rows * a.row_ld > FEW_ROWS_ELEMENTS) return false;      // (at most 65536 rows: 32768 pairs of them)
+    const int64_t waves = (a.rows + 1) / 2 * ((a.row_ld + 511) / 512);
+    return act == PRO_RMSNORM ? waves <= 8192 : act >= 0 || waves <= 6144;
+}
 template <int FMT, int SMODE, int ACT>
 __global__ __launch_bounds__(64) void mx_quant_few_rows_kernel(QuantArgs a) {
     constexpr bool FP4 = (FMT == kFmtE2M1);
@@ -737,7 +745,7 @@ static int launch_quant(QuantArgs& a, int64_t tiles_r, int64_t tiles_c, hipStrea
     const dim3 grid((unsigned)wgs);
     const bool row = a.q_row != nullptr, col = a.q_colT != nullptr;
     if constexpr (FMT != MXL_FMT_E5M2 && SMODE != SCALE_TENSOR && !TWOD && !SR && !RHT) {
-        if (row && !col && a.kchunk >= 2 && a.rows * a.row_ld <= FEW_ROWS_ELEMENTS) {      // (at most 65536 rows: 32768 pairs of them)
+        if (row && !col && a.kchunk >= 2 && few_rows(a, ACT)) {
             const dim3 pairs((unsigned)((a.row_ld + 511) / 512), (unsigned)((a.rows + 1) / 2));
             hipLaunchKernelGGL((mx_quant_few_rows_kernel<FMT, SMODE, ACT>), pairs, dim3(64), 0, st, a);
             return hipGetLastError() == hipSuccess ? MXL_OK : MXL_ELAUNCH;

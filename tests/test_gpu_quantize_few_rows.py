@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("fmt", [0, 1])
 @pytest.mark.parametrize("kind", ["plain", "norm", "silu", "gelu"])
-@pytest.mark.parametrize("rows,cols", [(1, 32), (2, 96), (3, 512), (64, 544), (129, 1120), (255, 2880), (2047, 4096), (2049, 4096)])
+@pytest.mark.parametrize("rows,cols", [(1, 32), (2, 96), (3, 512), (64, 544), (129, 1120), (255, 2880), (2047, 4096), (2049, 4096), (1536, 4096), (1537, 4096), (12288, 96), (12289, 96), (16384, 96), (16385, 96)])
 def test_row_wise_copy_alone(gpu, fmt, kind, rows, cols):
     from primus_amd.pytorch import kernels as K
 
