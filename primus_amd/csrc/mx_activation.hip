@@ -183,7 +183,9 @@ static void launch_glu_bwd(const void* dy, const void* x, const void* probs, int
                        probs_dtype, row_mask, f, (uint16_t*)dx, (float*)dprobs);
 }
 constexpr int64_t GLU_LONG_ROW = 6656;                                   // 1024 threads from here on
-constexpr int64_t GLU_FWD_MIDDLE_ROW = 4096, GLU_BWD_MIDDLE_ROW = 2560;  // 512 threads
+// 512 threads.  The forward of 4096 columns is whole passes of 256 threads: cold, 256 / 512, [2197, 4096] 13.0 / 14.1, [1098, 4096] 9.0 / 9.6,
+// [14160, 4096] 58.6 / 57.8, and one chunk more [2192, 4104] 14.0 / 14.0, [14132, 4104] 62.4 / 58.4.
+constexpr int64_t GLU_FWD_MIDDLE_ROW = 4104, GLU_BWD_MIDDLE_ROW = 2560;
 
 extern "C" int mxl_glu_probs_fwd(const void* x_bf16, const void* probs, int probs_dtype, const uint8_t* row_mask,
                                  int64_t rows, int64_t f, int act, void* y_bf16, void* stream) {

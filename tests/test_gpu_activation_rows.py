@@ -1,4 +1,4 @@
-"""swiglu_with_probs / geglu_with_probs at the row lengths where the workgroup's size changes (2560, 4096 and 6656 columns), one
+"""swiglu_with_probs / geglu_with_probs at the row lengths where the workgroup's size changes (2560, 4104 and 6656 columns), one
 chunk to either side of them and of whole passes of 512 and 1024 threads, against the oracle with test_gpu_activation's bounds."""
 
 import pytest
