@@ -80,14 +80,14 @@ __device__ __forceinline__ void store16_streaming(uint8_t* dst, const uint4& v) 
 }
 
 // The same through a buffer descriptor (base and size uniform): a lane whose offsets pass its end stores nothing.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_store_rsrc(void* base, int bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000);
+}
 // A store of more than 8 bytes fetches its data registers after it has issued: an instruction right behind it that writes
 // one of them changes what is stored, in some lanes and now and then (seen as single wrong dwords in lanes 12-15, 28-31, ..
 // of a store directly followed by a multiplication into its first data register).  The compiler puts the wait states in for
 // a store without a scalar offset register only, so they are written here: the statement takes the data as an operand, so
 // the registers cannot be handed on before it.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_store_rsrc(void* base, int bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(base, 0, bytes, 0x00020000);
-}
 __device__ __forceinline__ void buffer_store16_streaming(__amdgpu_buffer_rsrc_t rsrc, uint32_t voff, uint32_t soff, const uint4& v) {
     const u32x4 t = {v.x, v.y, v.z, v.w};
     constexpr int kNonTemporal = 2;
