@@ -182,7 +182,10 @@ static void launch_glu_bwd(const void* dy, const void* x, const void* probs, int
     hipLaunchKernelGGL((glu_probs_bwd_kernel<ACT, THREADS, SUMS>), dim3((unsigned)rows), dim3(THREADS), 0, st, (const uint16_t*)dy, (const uint16_t*)x, probs,
                        probs_dtype, row_mask, f, (uint16_t*)dx, (float*)dprobs);
 }
-constexpr int64_t GLU_LONG_ROW = 6656;                                   // 1024 threads from here on
+// 1024 threads from here on.  GELU, which computes more, has more than two passes of 512 threads in front of it: cold, 256 / 512 / 1024, forward
+// [1890, 6656] 16.8 / 15.1 / 16.1, [7561, 6656] 53.8 / 49.5 / 51.4, [16384, 8192] 142 / 132 / 131; backward 31.9 / 30.4 / 30.8, 107 / 104 / 108,
+// 273 / 276 / 281, and beyond [9830, 10240] 210 / 208 / 211, [585, 14336] 27.2 / 23.7 / 22.7.
+constexpr int64_t GLU_LONG_ROW[2] = {6656, 8200};
 // 512 threads.  The forward of 4096 columns is whole passes of 256 threads: cold, 256 / 512, [2197, 4096] 13.0 / 14.1, [1098, 4096] 9.0 / 9.6,
 // [14160, 4096] 58.6 / 57.8, and one chunk more [2192, 4104] 14.0 / 14.0, [14132, 4104] 62.4 / 58.4.
 constexpr int64_t GLU_FWD_MIDDLE_ROW = 4104, GLU_BWD_MIDDLE_ROW = 2560;
@@ -193,7 +196,7 @@ extern "C" int mxl_glu_probs_fwd(const void* x_bf16, const void* probs, int prob
     if (rows == 0) return MXL_OK;
     if (!device_is_gfx950()) return MXL_ENODEV;
     const bool silu = act == MXL_ACT_SILU;
-    const auto launch = f >= GLU_LONG_ROW         ? (silu ? launch_glu_fwd<MXL_ACT_SILU, 1024> : launch_glu_fwd<MXL_ACT_GELU, 1024>)
+    const auto launch = f >= GLU_LONG_ROW[act]    ? (silu ? launch_glu_fwd<MXL_ACT_SILU, 1024> : launch_glu_fwd<MXL_ACT_GELU, 1024>)
                         : f >= GLU_FWD_MIDDLE_ROW ? (silu ? launch_glu_fwd<MXL_ACT_SILU, 512> : launch_glu_fwd<MXL_ACT_GELU, 512>)
                                                   : (silu ? launch_glu_fwd<MXL_ACT_SILU, 256> : launch_glu_fwd<MXL_ACT_GELU, 256>);
     launch(x_bf16, probs, probs_dtype, row_mask, rows, f, y_bf16, (hipStream_t)stream);
@@ -212,7 +215,7 @@ int glu_probs_bwd(const void* dy_bf16, const void* x_bf16, const void* probs, in
     if (!device_is_gfx950()) return MXL_ENODEV;
     const bool silu = act == MXL_ACT_SILU;
     const auto launch =
-        f >= GLU_LONG_ROW       ? (shared ? (silu ? launch_glu_bwd<MXL_ACT_SILU, 256, 4> : launch_glu_bwd<MXL_ACT_GELU, 256, 4>)
+        f >= GLU_LONG_ROW[act]  ? (shared ? (silu ? launch_glu_bwd<MXL_ACT_SILU, 256, 4> : launch_glu_bwd<MXL_ACT_GELU, 256, 4>)
                                           : (silu ? launch_glu_bwd<MXL_ACT_SILU, 1024, 1> : launch_glu_bwd<MXL_ACT_GELU, 1024, 1>))
         : f >= GLU_BWD_MIDDLE_ROW ? (shared ? (silu ? launch_glu_bwd<MXL_ACT_SILU, 256, 2> : launch_glu_bwd<MXL_ACT_GELU, 256, 2>)
                                           : (silu ? launch_glu_bwd<MXL_ACT_SILU, 512, 1> : launch_glu_bwd<MXL_ACT_GELU, 512, 1>))

@@ -1,4 +1,4 @@
-"""swiglu_with_probs / geglu_with_probs at the row lengths where the workgroup's size changes (2560, 4104 and 6656 columns), one
+"""swiglu_with_probs / geglu_with_probs at the row lengths where the workgroup's size changes (2560, 4104, 6656 and 8200 columns), one
 chunk to either side of them and of whole passes of 512 and 1024 threads, against the oracle with test_gpu_activation's bounds."""
 
 import pytest
@@ -10,6 +10,6 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("activation", ["silu", "gelu"])
-@pytest.mark.parametrize("f", [2552, 2560, 4088, 4096, 4104, 6648, 6656, 8184, 8200])
+@pytest.mark.parametrize("f", [2552, 2560, 4088, 4096, 4104, 6648, 6656, 8184, 8192, 8200])
 def test_every_workgroup_size(gpu, activation, f):
     check(gpu, activation, 9, f, torch.float32)
