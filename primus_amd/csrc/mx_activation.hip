@@ -189,6 +189,14 @@ constexpr int64_t GLU_LONG_ROW[2] = {6656, 8200};
 // 512 threads.  The forward of 4096 columns is whole passes of 256 threads: cold, 256 / 512, [2197, 4096] 13.0 / 14.1, [1098, 4096] 9.0 / 9.6,
 // [14160, 4096] 58.6 / 57.8, and one chunk more [2192, 4104] 14.0 / 14.0, [14132, 4104] 62.4 / 58.4.
 constexpr int64_t GLU_FWD_MIDDLE_ROW = 4104, GLU_BWD_MIDDLE_ROW = 2560;
+// A workgroup takes half the threads its row's length gives it where whole workgroups are more waves than the chip holds (32 to a CU: 8192) and
+// halves are not, on rows that fill the halves' passes.  SILU, us, half / whole: backward [1638, 2560] 10.2 / 10.6, [1170, 3584] 10.2 / 10.8, [1536, 4096] 13.4 /
+// 14.0, [2048, 4096] 16.6 / 16.9, [768, 8192] 13.5 / 14.4, [1024, 8192] 17.4 / 17.9, but [1092, 2880] 9.2 / 8.9, [2184, 2880] 14.5 / 14.0, [1456, 5760]
+// 18.0 / 17.4; forward [768, 8192] 8.5 / 8.9, [1024, 8192] 10.6 / 11.0.  GELU loses: backward [1638, 2560] 12.8 / 12.2, [768, 8192] 16.2 / 15.7.
+static bool glu_halves(int act, int64_t rows, int64_t f) {
+    if (act != MXL_ACT_SILU) return false;
+    return f >= GLU_LONG_ROW[act] ? f <= 8192 && rows > 512 && rows <= 1024 : f <= 4096 && rows > 1152 && rows <= 2048;
+}
 
 extern "C" int mxl_glu_probs_fwd(const void* x_bf16, const void* probs, int probs_dtype, const uint8_t* row_mask,
                                  int64_t rows, int64_t f, int act, void* y_bf16, void* stream) {
@@ -196,7 +204,7 @@ extern "C" int mxl_glu_probs_fwd(const void* x_bf16, const void* probs, int prob
     if (rows == 0) return MXL_OK;
     if (!device_is_gfx950()) return MXL_ENODEV;
     const bool silu = act == MXL_ACT_SILU;
-    const auto launch = f >= GLU_LONG_ROW[act]    ? (silu ? launch_glu_fwd<MXL_ACT_SILU, 1024> : launch_glu_fwd<MXL_ACT_GELU, 1024>)
+    const auto launch = f >= GLU_LONG_ROW[act] && !glu_halves(act, rows, f) ? (silu ? launch_glu_fwd<MXL_ACT_SILU, 1024> : launch_glu_fwd<MXL_ACT_GELU, 1024>)
                         : f >= GLU_FWD_MIDDLE_ROW ? (silu ? launch_glu_fwd<MXL_ACT_SILU, 512> : launch_glu_fwd<MXL_ACT_GELU, 512>)
                                                   : (silu ? launch_glu_fwd<MXL_ACT_SILU, 256> : launch_glu_fwd<MXL_ACT_GELU, 256>);
     launch(x_bf16, probs, probs_dtype, row_mask, rows, f, y_bf16, (hipStream_t)stream);
@@ -214,10 +222,12 @@ int glu_probs_bwd(const void* dy_bf16, const void* x_bf16, const void* probs, in
     if (!dy_bf16 || !dprobs_f32) return MXL_EINVAL;
     if (!device_is_gfx950()) return MXL_ENODEV;
     const bool silu = act == MXL_ACT_SILU;
+    const bool halves = glu_halves(act, rows, f);
     const auto launch =
         f >= GLU_LONG_ROW[act]  ? (shared ? (silu ? launch_glu_bwd<MXL_ACT_SILU, 256, 4> : launch_glu_bwd<MXL_ACT_GELU, 256, 4>)
+                                 : halves ? launch_glu_bwd<MXL_ACT_SILU, 512, 2>
                                           : (silu ? launch_glu_bwd<MXL_ACT_SILU, 1024, 1> : launch_glu_bwd<MXL_ACT_GELU, 1024, 1>))
-        : f >= GLU_BWD_MIDDLE_ROW ? (shared ? (silu ? launch_glu_bwd<MXL_ACT_SILU, 256, 2> : launch_glu_bwd<MXL_ACT_GELU, 256, 2>)
+        : f >= GLU_BWD_MIDDLE_ROW ? (shared || halves ? (silu ? launch_glu_bwd<MXL_ACT_SILU, 256, 2> : launch_glu_bwd<MXL_ACT_GELU, 256, 2>)
                                           : (silu ? launch_glu_bwd<MXL_ACT_SILU, 512, 1> : launch_glu_bwd<MXL_ACT_GELU, 512, 1>))
                                 : (silu ? launch_glu_bwd<MXL_ACT_SILU, 256, 1> : launch_glu_bwd<MXL_ACT_GELU, 256, 1>);
     launch(dy_bf16, x_bf16, probs, probs_dtype, row_mask, rows, f, dx_bf16, dprobs_f32, (hipStream_t)stream);

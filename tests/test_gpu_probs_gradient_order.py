@@ -37,3 +37,18 @@ def test_two_calls_and_launch_by_launch(gpu, f, kind):
     gl = torch.tensor(lens, dtype=torch.int64, device=gpu)
     cfg = test_gpu_linear_two_calls._config("mxfp8")
     test_gpu_linear_two_calls._check(lambda: ops.glu_grouped_gemm_fp8(x, probs, w, gl, activation=kind, row_mask=mask, config=cfg), [x, probs, w])
+
+
+@pytest.mark.parametrize("f,rows", [(2560, 1152), (2560, 1153), (4096, 2048), (4096, 2049), (4104, 2048), (6656, 512), (6656, 513), (8192, 1024), (8192, 1025)])
+def test_whatever_the_number_of_rows(gpu, f, rows):
+    from primus_amd.pytorch import ops
+
+    g = torch.Generator(device=gpu).manual_seed(f)
+    x, dy = (torch.randn(rows, c, generator=g, device=gpu).bfloat16() for c in (2 * f, f))
+    probs = torch.rand(rows, generator=g, device=gpu)
+    out = []
+    for some in (slice(None), slice(0, 500)):
+        h, p = x[some].clone().requires_grad_(), probs[some].clone().requires_grad_()
+        out.append([t[:500] for t in torch.autograd.grad(ops.swiglu_with_probs(h, p), (h, p), dy[some])])
+    for a, b in zip(*out):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
