@@ -595,11 +595,20 @@ def _accum_target(accum_into, shape, kchunk, device):
     return accum_into
 
 
+def _wgrad_out(out, shape, device):
+    if out is None:
+        return torch.empty(shape, dtype=torch.bfloat16, device=device)
+    if out.dtype != torch.bfloat16 or not out.is_contiguous() or out.device != device:
+        raise ValueError("out must be a contiguous bfloat16 tensor on the operands' device")
+    return out.view(shape)
+
+
 def grouped_gemm_mx_wgrad_impl(a_t, a_t_scale, b_t, b_t_scale, group_lens, total_m, out_dtype=torch.bfloat16,
-                               kchunk=False, accum_into: Optional[torch.Tensor] = None, tile: Optional[str] = None) -> torch.Tensor:
+                               kchunk=False, accum_into: Optional[torch.Tensor] = None, tile: Optional[str] = None,
+                               out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Variable-K (wgrad) grouped GEMM on segment-padded transposed operands:
     ``a_t`` = dY^T codes ``[n, W]``, ``b_t`` = X^T codes ``[k, W]``; returns
-    ``[G, n, k]`` (``[n, k]`` when ``group_lens`` is None).  An expert with no
+    ``[G, n, k]`` (``[n, k]`` when ``group_lens`` is None), in ``out`` if given.  An expert with no
     tokens gets a zero gradient."""
     _check_out_dtype(out_dtype)
     _require_cuda(a_t, a_t_scale, b_t, b_t_scale, group_lens)
@@ -627,7 +636,7 @@ def grouped_gemm_mx_wgrad_impl(a_t, a_t_scale, b_t, b_t_scale, group_lens, total
         c = _accum_target(accum_into, shape, kchunk, a_t.device)
         flags |= _lib.GF_ACCUM_F32
     else:
-        c = torch.empty(shape, dtype=torch.bfloat16, device=a_t.device)
+        c = _wgrad_out(out, shape, a_t.device)
     with _hooked("grouped_gemm_wgrad", m=total_m, n=n, k=k):
         rc = _lib.load().mxl_grouped_gemm_wgrad_ex(
             _ptr(a_t), _ptr(a_t_scale), a_fmt, _ptr(b_t), _ptr(b_t_scale), b_fmt, _ptr(c), _ptr(group_lens), G, total_m, n, k,
@@ -1031,9 +1040,10 @@ def gemm_tw_nt_impl(a, a_unit, a_scale_inv, b, b_unit, b_scale_inv, group_lens=N
 
 
 def gemm_tw_wgrad_impl(a_t, a_t_unit, a_scale_inv, b_t, b_t_unit, b_scale_inv, group_lens, total_m,
-                       kchunk: bool = False, accum_into: Optional[torch.Tensor] = None, tile: Optional[str] = None) -> torch.Tensor:
+                       kchunk: bool = False, accum_into: Optional[torch.Tensor] = None, tile: Optional[str] = None,
+                       out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """Variable-K (wgrad) GEMM on tensor-wise scaled transposed operands, times the two factors; shapes as
-    ``grouped_gemm_mx_wgrad_impl`` (also ``accum_into``)."""
+    ``grouped_gemm_mx_wgrad_impl`` (also ``accum_into`` and ``out``)."""
     _require_cuda(a_t, a_t_unit, b_t, b_t_unit, group_lens)
     _alpha_ok(a_scale_inv, b_scale_inv)
     G = _check_group_lens(group_lens, a_t.device)
@@ -1058,7 +1068,7 @@ def gemm_tw_wgrad_impl(a_t, a_t_unit, a_scale_inv, b_t, b_t_unit, b_scale_inv, g
         c = _accum_target(accum_into, shape, kchunk, a_t.device)
         flags |= _lib.GF_ACCUM_F32
     else:
-        c = torch.empty(shape, dtype=torch.bfloat16, device=a_t.device)
+        c = _wgrad_out(out, shape, a_t.device)
     with _hooked("grouped_gemm_wgrad", m=total_m, n=n, k=k):
         rc = _lib.load().mxl_grouped_gemm_wgrad_scaled(
             _ptr(a_t), _ptr(a_t_unit), a_fmt, _ptr(b_t), _ptr(b_t_unit), b_fmt, _ptr(c), _ptr(group_lens), G, total_m, n, k,

@@ -20,6 +20,7 @@ Activations and gradients use 1-D blocks of 32, weights 2-D 32x32 blocks.
 
 from __future__ import annotations
 
+import contextlib
 from typing import Optional, Union
 
 import torch
@@ -82,6 +83,20 @@ def _side_stream(device: torch.device) -> "torch.cuda.Stream":
         st = torch.cuda.Stream(device=device)   # default priority
         _side_streams[key] = st
     return st
+
+
+@contextlib.contextmanager
+def _beside(main, side):
+    """Launches inside go to ``side``, and ``main`` waits for them at the end, also when one raises.  Nothing launched there may read
+    or write memory that is given back earlier than that, nor write memory taken from ``main``'s pool after ``side`` waited for
+    ``main``.  So every buffer is reused in ``main``'s order like any other.  (Marked with ``record_stream`` instead, none came back before
+    the device had got there: a loop of passes that nothing waits in grew until the card was full, 15 to 287 GiB in 40 passes of
+    8 experts of 14336, 4096 wide, 32768 rows, 16.5 to 128 ms each.)"""
+    try:
+        with torch.cuda.stream(side):
+            yield
+    finally:
+        main.wait_stream(side)
 
 
 _dummy_wgrads = {}
@@ -293,15 +308,11 @@ def _backward_in_parts(plan, dy, saved, group_lens, accum, need_dgrad, need_wgra
         K.linear_backward_impl(plan, _lib.LINEAR_QUANTIZE, dy, saved, scratch, group_lens=group_lens, sr_seed=sr_seed)
         main = torch.cuda.current_stream(dev)
         side = _side_stream(dev)
+        dw = target if fused else torch.empty(w_shape, dtype=torch.bfloat16, device=dev)
         side.wait_stream(main)   # the quantised operands are ready
         K.linear_backward_impl(plan, _lib.LINEAR_DX, None, saved, scratch, dx, None, daux, x, wt, wt_scales, group_lens, aux0, aux1)
-        with torch.cuda.stream(side):
-            dw = target if fused else torch.empty(w_shape, dtype=torch.bfloat16, device=dev)
+        with _beside(main, side):
             K.linear_backward_impl(plan, _lib.LINEAR_DW, None, saved, scratch, None, dw, group_lens=group_lens, accumulate=fused)
-        for t in (saved, scratch) + (() if group_lens is None else (group_lens,)):
-            t.record_stream(side)
-        dw.record_stream(main)
-        main.wait_stream(side)
     if need_wgrad and accum is not None:
         return _finish_wgrad(dw, accum, fused, w_shape)
     return dw
@@ -426,10 +437,14 @@ class _MXLinearFunction(torch.autograd.Function):
         )
         kc = ctx.kchunk
         grad_a = grad_b = None
+        target = ctx.accum[0] if need_wgrad and ctx.accum is not None else None
+        fused = _fusable(target) and kc != K.LAYOUT_ROWMAJOR   # the GEMM's epilogue adds into the float32 buffer
         overlap = _wgrad_overlap and need_dgrad and need_wgrad
+        out = None
         if overlap:
             main = torch.cuda.current_stream(dy.device)
             side = _side_stream(dy.device)
+            out = None if fused else torch.empty(w_shape, dtype=torch.bfloat16, device=dy.device)
             side.wait_stream(main)   # the quantised operands are ready
         if need_dgrad:
             if grouped:
@@ -437,22 +452,9 @@ class _MXLinearFunction(torch.autograd.Function):
             else:
                 grad_a = K.gemm_mx_nt_impl(d_row, d_rs, w_col, w_cs, kchunk=kc, b_transposed=ctx.b_transposed)
         if need_wgrad:
-            target = ctx.accum[0] if ctx.accum is not None else None
-            fused = _fusable(target) and kc != K.LAYOUT_ROWMAJOR   # the GEMM's epilogue adds into the float32 buffer
-
-            def wgrad():
-                return K.grouped_gemm_mx_wgrad_impl(d_col, d_cs, a_col, a_cs, group_lens, total_m, kchunk=kc,
-                                                    accum_into=target if fused else None)
-
-            if overlap:
-                with torch.cuda.stream(side):
-                    grad_b = wgrad()
-                for t in (d_col, d_cs, a_col, a_cs, grad_b):
-                    t.record_stream(side)
-                grad_b.record_stream(main)
-                main.wait_stream(side)
-            else:
-                grad_b = wgrad()
+            with _beside(main, side) if overlap else contextlib.nullcontext():
+                grad_b = K.grouped_gemm_mx_wgrad_impl(d_col, d_cs, a_col, a_cs, group_lens, total_m, kchunk=kc,
+                                                      accum_into=target if fused else None, out=out)
             grad_b = _finish_wgrad(grad_b, ctx.accum, fused, w_shape)
         grad_p = None
         if ctx.activation is not None and need_dgrad:
@@ -573,31 +575,22 @@ class _TWLinearFunction(torch.autograd.Function):
         d_row, d_ru, d_col, d_cu, d_si = K.quantize_tensorwise_impl(
             dy, bwd_fmt, rowwise=need_dgrad, colwise=need_wgrad, group_lens=group_lens, pad_to=K.GEMM_K_ALIGN, kchunk=kc)
         grad_a = grad_b = None
+        target = ctx.accum[0] if need_wgrad and ctx.accum is not None else None
+        fused = _fusable(target) and kc != K.LAYOUT_ROWMAJOR
         overlap = _wgrad_overlap and need_dgrad and need_wgrad
+        out = None
         if overlap:
             main = torch.cuda.current_stream(dy.device)
             side = _side_stream(dy.device)
+            out = None if fused else torch.empty(w_shape, dtype=torch.bfloat16, device=dy.device)
             side.wait_stream(main)
         if need_dgrad:
             grad_a = K.gemm_tw_nt_impl(d_row, d_ru, d_si, w_col, w_cu, w_si, group_lens, kchunk=kc,
                                        b_transposed_n=w_shape[-1] if ctx.b_transposed else None)
         if need_wgrad:
-            target = ctx.accum[0] if ctx.accum is not None else None
-            fused = _fusable(target) and kc != K.LAYOUT_ROWMAJOR
-
-            def wgrad():
-                return K.gemm_tw_wgrad_impl(d_col, d_cu, d_si, a_col, a_cu, a_si, group_lens, total_m, kchunk=kc,
-                                            accum_into=target if fused else None)
-
-            if overlap:
-                with torch.cuda.stream(side):
-                    grad_b = wgrad()
-                for t in (d_col, d_cu, d_si, a_col, a_cu, a_si, grad_b):
-                    t.record_stream(side)
-                grad_b.record_stream(main)
-                main.wait_stream(side)
-            else:
-                grad_b = wgrad()
+            with _beside(main, side) if overlap else contextlib.nullcontext():
+                grad_b = K.gemm_tw_wgrad_impl(d_col, d_cu, d_si, a_col, a_cu, a_si, group_lens, total_m, kchunk=kc,
+                                              accum_into=target if fused else None, out=out)
             grad_b = _finish_wgrad(grad_b, ctx.accum, fused, w_shape)
         return grad_a, grad_b, None, None, None, None, None, None
 
